@@ -8,6 +8,9 @@
 // offset of the device/host boundary, hence no chunk ever straddles the tiers
 // and a straddling ROW is still resolved exactly, chunk by chunk.
 //
+// Rows whose length is no multiple of 16 bytes (odd feature widths) go through a kernel of their own
+// that cuts the OUTPUT into 16-byte chunks instead and loads their bytes from wherever they lie.
+//
 // Index values are checked before they address anything: a row outside the rows the
 // requested tier holds is not read, its output row is filled with zero bytes and the
 // caller's flag word (if any) is set.
@@ -154,6 +157,161 @@ __global__ __launch_bounds__(kGatherThreads) void gather_flat_kernel(
   if (bad && bad_index) *bad_index = 1;
 }
 
+// ---- rows that are no multiple of 16 bytes -----------------------------------------------------
+//
+// Cutting such rows into the largest power of two that divides them leaves 8, 4 or 2 bytes per lane
+// and instruction, and the load/store units, not memory, bound the launch.  Here the output, which
+// is contiguous, is cut into aligned 16-byte chunks; a chunk's bytes lie at an arbitrary address in
+// its row, which global loads may name as it is, and a chunk that holds the end of one row and the
+// beginning of the next (one in row_bytes / 16) takes a second load, placed so that both line up
+// with the chunk.  Bound: HBM, plus the lines that a row's ends share with its neighbours.  300 MB
+// of rows, element-wide chunks against this kernel, us: 602 B (bf16 x301) 274 -> 123 = 4.9 TB/s, 1204 B
+// 163 -> 107, 404 B (f32 x101) 166 -> 121, 188 B 172 -> 140, 129 B (bytes) 509 -> 164, 2408 B (f32 x602)
+// 108 -> 96 = 6.2 TB/s.  (Three chunks a thread as in the kernel above; 49 VGPRs, eight blocks a CU.)
+constexpr int kRaggedBytesPerBlock = kChunksPerBlock * 16;
+// Rows of at least kRaggedMinChunks of the chunks they could be cut into evenly: on shorter ones a
+// second load comes with every few chunks, and wide enough even chunks are as fast (300 MB of rows, us,
+// even chunks against this kernel: 72 B 180 / 191, 52 B 228 / 234, 36 B 271 / 294, 28 B 314 / 352, all
+// of 4- or 8-byte chunks; 26 B 385 / 391 and 34 B 353 / 319 of 2-byte chunks; 17 B 653 / 571 of bytes).
+// The upper bound keeps the multiply-high division exact: (row + kRaggedBytesPerBlock) * row < 2^32.
+constexpr int64_t kRaggedMinChunks = 16, kRaggedMaxRow = 32768;
+
+typedef u32x4 __attribute__((aligned(1))) u32x4_anywhere;
+
+// What a launch may read: bytes [lo, hi) of the store, of which those below `thr` lie in the device
+// slice.  With TIER_ANY a load must not straddle `thr`.
+template <int TIER>
+__device__ __forceinline__ bool loadable16(int64_t g, int64_t lo, int64_t hi, int64_t thr) {
+  const bool inside = g >= lo && g + 16 <= hi;
+  return TIER == DGS_TIER_ANY ? inside && (g >= thr || g + 16 <= thr) : inside;
+}
+
+// Bytes [first, last) of a chunk whose byte 0 lies at store byte g, one by one (the few chunks at the
+// ends of a slice whose 16-byte load would leave it); the other bytes of the result are 0.
+template <int TIER>
+__device__ u32x4 bytes_of(const char* dev, const char* host, int64_t thr, int64_t g, int first, int last) {
+  uint64_t half[2] = {0, 0};
+  for (int i = first; i < last; ++i)
+    half[i >> 3] |= uint64_t(uint8_t(*resolve<TIER>(dev, host, thr, g + i))) << (8 * (i & 7));
+  u32x4 v;
+  v.x = uint32_t(half[0]); v.y = uint32_t(half[0] >> 32); v.z = uint32_t(half[1]); v.w = uint32_t(half[1] >> 32);
+  return v;
+}
+
+// All bytes of dword j of a chunk that lie below byte m of the chunk.
+__device__ __forceinline__ uint32_t mask_below(int m, int j) {
+  const int n = m - 4 * j;
+  return n >= 4 ? ~0u : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+}
+
+// One tile (kRaggedBytesPerBlock output bytes from byte b0 on), in the passes of gather_tile: row ids,
+// loads, stores.  Sizes are bytes: `readable` is what the index array covers, `total` what counts.
+template <int TIER, typename IndexT>
+__device__ __forceinline__ bool ragged_tile(const char* __restrict__ dev, const char* __restrict__ host, int64_t thr,
+                                            int64_t lo, int64_t hi, uint32_t row_bytes, uint32_t magic,
+                                            const IndexT* __restrict__ index, int64_t readable, int64_t total,
+                                            const int64_t* __restrict__ n_rows_dev, int64_t row_lo, int64_t row_hi,
+                                            char* __restrict__ out, int64_t b0, int64_t* counted) {
+  bool bad = false;
+  const int64_t row0 = b0 / row_bytes;
+  const uint32_t rem0 = uint32_t(b0 - row0 * row_bytes);
+  const IndexT* __restrict__ index0 = index + row0;
+  int64_t src[kGatherUnroll], next[kGatherUnroll];
+  uint32_t off[kGatherUnroll];
+#pragma unroll
+  for (int u = 0; u < kGatherUnroll; ++u) {
+    const uint32_t t = (u * kGatherThreads + threadIdx.x) * 16u;
+    const uint32_t q = __umulhi(rem0 + t, magic);
+    off[u] = rem0 + t - q * row_bytes;
+    const int64_t left = readable - (b0 + t);  // bytes from this chunk on
+    src[u] = left > 0 ? int64_t(index0[q]) : row_lo;
+    // the row that begins inside the chunk, if one does
+    const uint32_t m = row_bytes - off[u];
+    next[u] = m < 16u && left > int64_t(m) ? int64_t(index0[q + 1]) : row_lo;
+  }
+  if (n_rows_dev) {  // row count decided on the device; one that exceeds the output's rows gathers nothing
+    const int64_t rows = *n_rows_dev;
+    total = rows >= 0 && rows * row_bytes <= readable ? rows * row_bytes : 0;
+  }
+  *counted = total;
+  if (b0 >= total) return false;  // whole blocks leave together
+  u32x4 val[kGatherUnroll];
+  int64_t at[kGatherUnroll];
+  bool whole[kGatherUnroll], in_range[kGatherUnroll];
+#pragma unroll
+  for (int u = 0; u < kGatherUnroll; ++u) {
+    const bool counts = b0 + (u * kGatherThreads + threadIdx.x) * 16 < total;
+    in_range[u] = src[u] >= row_lo && src[u] < row_hi;
+    bad |= counts && !in_range[u];
+    if (!in_range[u] || !counts) src[u] = row_lo;
+    at[u] = src[u] * row_bytes + off[u];
+    whole[u] = loadable16<TIER>(at[u], lo, hi, thr);
+    // (the first 16 bytes a launch may read lie in one slice: the launcher sees to it)
+    val[u] = *reinterpret_cast<const u32x4_anywhere*>(resolve<TIER>(dev, host, thr, whole[u] ? at[u] : lo));
+  }
+  // the second loads, all requested before any of the first is used
+  u32x4 second[kGatherUnroll];
+#pragma unroll
+  for (int u = 0; u < kGatherUnroll; ++u) {
+    const int m = int(row_bytes - off[u]);  // chunk bytes from m on belong to the next row
+    second[u] = u32x4(0);
+    if (m >= 16 || total - (b0 + (u * kGatherThreads + threadIdx.x) * 16) <= m) continue;  // no next row in the chunk
+    if (next[u] >= row_lo && next[u] < row_hi) {
+      const int64_t g = next[u] * row_bytes - m;
+      second[u] = loadable16<TIER>(g, lo, hi, thr)
+                      ? *reinterpret_cast<const u32x4_anywhere*>(resolve<TIER>(dev, host, thr, g))
+                      : bytes_of<TIER>(dev, host, thr, g, m, 16);
+    } else {
+      bad = true;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kGatherUnroll; ++u) {
+    const int m = int(row_bytes - off[u]);
+    if (!whole[u]) val[u] = bytes_of<TIER>(dev, host, thr, at[u], 0, m < 16 ? m : 16);
+    if (!in_range[u]) val[u] = u32x4(0);
+    if (m < 16) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t mask = mask_below(m, j);
+        val[u][j] = (val[u][j] & mask) | (second[u][j] & ~mask);
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kGatherUnroll; ++u) {
+    const int64_t b = b0 + (u * kGatherThreads + threadIdx.x) * 16;
+    if (b + 16 <= total) {
+      __builtin_nontemporal_store(val[u], reinterpret_cast<u32x4*>(out + b));
+    } else if (b < total) {  // the output's last bytes
+      for (int i = 0; i < int(total - b); ++i) out[b + i] = char(val[u][i >> 2] >> (8 * (i & 3)));
+    }
+  }
+  return bad;
+}
+
+template <int TIER, typename IndexT, bool STRIDE>
+__global__ __launch_bounds__(kGatherThreads) void gather_ragged_kernel(
+    const char* __restrict__ dev, const char* __restrict__ host, int64_t thr, int64_t lo, int64_t hi,
+    uint32_t row_bytes, uint32_t magic, const IndexT* __restrict__ index, int64_t total,
+    const int64_t* __restrict__ n_rows_dev, int64_t row_lo, int64_t row_hi, int64_t* __restrict__ bad_index,
+    char* __restrict__ out) {
+  const int64_t first = int64_t(blockIdx.x) * kRaggedBytesPerBlock;
+  if (first >= total) return;
+  int64_t counted;
+  bool bad = ragged_tile<TIER, IndexT>(dev, host, thr, lo, hi, row_bytes, magic, index, total, total, n_rows_dev, row_lo,
+                                       row_hi, out, first, &counted);
+  if (STRIDE) {
+    for (int64_t b0 = first + int64_t(gridDim.x) * kRaggedBytesPerBlock; b0 < counted;
+         b0 += int64_t(gridDim.x) * kRaggedBytesPerBlock) {
+      int64_t unused;
+      bad |= ragged_tile<TIER, IndexT>(dev, host, thr, lo, hi, row_bytes, magic, index, counted, counted, nullptr, row_lo,
+                                       row_hi, out, b0, &unused);
+    }
+  }
+  if (bad && bad_index) *bad_index = 1;
+}
+
 // Rows wider than kMaxFlatChunksPerRow chunks, and any launch whose tier holds no whole row
 // (every id is refused): a block owns one segment of kChunksPerBlock chunks of one row.
 template <int VEC, int TIER, typename IndexT>
@@ -183,6 +341,26 @@ __global__ __launch_bounds__(kGatherThreads) void gather_wide_kernel(
   }
 }
 
+// Blocks of a launch that covers `tiles` tiles in the worst case (`expected` of them in the caller's
+// estimate, 0: no estimate); a launch whose row count is read on the device is sized for what the
+// caller expects, and blocks stride should there be more.
+inline int64_t gather_blocks(int64_t tiles, int64_t expected, bool counted_on_device) {
+  int64_t blocks = tiles;
+  if (counted_on_device) {
+    if (expected > 0 && expected < blocks) blocks = expected;
+    if (blocks > kMaxDynGrid) blocks = kMaxDynGrid;
+  }
+  return blocks > 0x7fffffff ? 0x7fffffff : blocks;
+}
+
+// LDS that a gather does not use, reserved so that fewer of its blocks fit a CU: a caller's limit
+// (dgs_gather_rows_dyn_shared), or the measurement hook's byte count.
+inline uint32_t reserved_lds(int32_t blocks_per_cu) {
+  int64_t lds = debug_option(DGS_DEBUG_GATHER_LDS_BYTES);
+  if (lds <= 0 && blocks_per_cu > 0 && blocks_per_cu < kGatherBlocksPerCu) lds = lds_per_cu() / blocks_per_cu / 256 * 256;
+  return uint32_t(lds < 0 ? 0 : (lds > 65536 ? 65536 : lds));
+}
+
 template <int VEC, int TIER, typename IndexT>
 dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index, int64_t n,
                          const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad_index, void* out, hipStream_t st) {
@@ -198,29 +376,17 @@ dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index
   if (cpr <= kMaxFlatChunksPerRow && row_lo < row_hi) {
     const int64_t total_chunks = n * cpr;
     const int64_t tiles = (total_chunks + kChunksPerBlock - 1) / kChunksPerBlock;
-    int64_t blocks = tiles;
-    if (n_dev != nullptr) {
-      // a count read on the device: the launch is sized for the rows the caller expects (all of
-      // them when it says nothing), and blocks stride should there be more
-      if (n_expected > 0 && n_expected < n) blocks = (n_expected * cpr + kChunksPerBlock - 1) / kChunksPerBlock;
-      if (blocks > kMaxDynGrid) blocks = kMaxDynGrid;
-      if (blocks > tiles) blocks = tiles;
-    }
-    if (blocks > 0x7fffffff) blocks = 0x7fffffff;
+    const int64_t blocks = gather_blocks(tiles, (n_expected * cpr + kChunksPerBlock - 1) / kChunksPerBlock, n_dev != nullptr);
     const uint32_t magic = cpr > 1 ? uint32_t((uint64_t(1) << 32) / uint64_t(cpr)) + 1u : 0u;
-    // LDS that the kernel does not use, reserved so that fewer of its blocks fit a CU: a caller's
-    // limit (dgs_gather_rows_dyn_shared), or the measurement hook's byte count
-    int64_t lds = debug_option(DGS_DEBUG_GATHER_LDS_BYTES);
-    if (lds <= 0 && blocks_per_cu > 0 && blocks_per_cu < kGatherBlocksPerCu) lds = lds_per_cu() / blocks_per_cu / 256 * 256;
-    lds = lds < 0 ? 0 : (lds > 65536 ? 65536 : lds);
+    const uint32_t lds = reserved_lds(blocks_per_cu);
     if (blocks < tiles)
       hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, true>), dim3(uint32_t(blocks)),
-                         dim3(kGatherThreads), uint32_t(lds), st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
+                         dim3(kGatherThreads), lds, st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
                          magic, static_cast<const IndexT*>(index), total_chunks, n_dev, row_lo, row_hi,
                          bad_index, static_cast<char*>(out));
     else
       hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, false>), dim3(uint32_t(blocks)),
-                         dim3(kGatherThreads), uint32_t(lds), st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
+                         dim3(kGatherThreads), lds, st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
                          magic, static_cast<const IndexT*>(index), total_chunks, n_dev, row_lo, row_hi,
                          bad_index, static_cast<char*>(out));
   } else {
@@ -232,6 +398,43 @@ dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index
                        static_cast<const IndexT*>(index), n, n_dev, row_lo, row_hi, bad_index,
                        static_cast<char*>(out));
   }
+  DGS_LAUNCH_CHECK();
+  return DGS_OK;
+}
+
+// Whether the launch goes to gather_ragged_kernel: rows that 16-byte chunks do not divide (or that
+// begin at odd addresses), unless they are very short (see kRaggedMinChunks); a row of
+// kRaggedMinChunks chunks has at least 16 bytes, so a 16-byte chunk meets two rows at most.
+bool is_ragged(const dgs_view& v, int64_t row_bytes, const void* out, int tier, int vec) {
+  if (vec == 16 || row_bytes < kRaggedMinChunks * vec || row_bytes > kRaggedMaxRow) return false;
+  if (reinterpret_cast<uintptr_t>(out) & 15) return false;
+  const int64_t thr = v.threshold * v.elem_bytes, all = v.total * v.elem_bytes / row_bytes * row_bytes;
+  if (tier == DGS_TIER_DEVICE) return thr >= row_bytes;
+  if (tier == DGS_TIER_HOST) return (thr + row_bytes - 1) / row_bytes * row_bytes < all;
+  return thr >= 16 && all >= row_bytes;
+}
+
+template <int TIER, typename IndexT>
+dgs_status launch_ragged(const dgs_view& v, int64_t row_bytes, const void* index, int64_t n, const int64_t* n_dev,
+                         int64_t n_expected, int32_t blocks_per_cu, int64_t* bad_index, void* out, hipStream_t st) {
+  const int64_t thr = v.threshold * v.elem_bytes;
+  const int64_t row_lo = TIER == DGS_TIER_HOST ? (thr + row_bytes - 1) / row_bytes : 0;
+  const int64_t row_hi = TIER == DGS_TIER_DEVICE ? thr / row_bytes : v.total * v.elem_bytes / row_bytes;
+  const int64_t lo = TIER == DGS_TIER_HOST ? thr : 0;
+  const int64_t hi = TIER == DGS_TIER_DEVICE ? thr : v.total * v.elem_bytes;
+  const int64_t total = n * row_bytes;
+  const int64_t tiles = (total + kRaggedBytesPerBlock - 1) / kRaggedBytesPerBlock;
+  const int64_t blocks = gather_blocks(tiles, (n_expected * row_bytes + kRaggedBytesPerBlock - 1) / kRaggedBytesPerBlock,
+                                       n_dev != nullptr);
+  const uint32_t magic = uint32_t((uint64_t(1) << 32) / uint64_t(row_bytes)) + 1u;
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks)), dim3(kGatherThreads), reserved_lds(blocks_per_cu), st,
+                       static_cast<const char*>(v.dev), static_cast<const char*>(v.host), thr, lo, hi, uint32_t(row_bytes),
+                       magic, static_cast<const IndexT*>(index), total, n_dev, row_lo, row_hi, bad_index,
+                       static_cast<char*>(out));
+  };
+  if (blocks < tiles) go(gather_ragged_kernel<TIER, IndexT, true>);
+  else go(gather_ragged_kernel<TIER, IndexT, false>);
   DGS_LAUNCH_CHECK();
   return DGS_OK;
 }
@@ -248,6 +451,9 @@ template <int TIER>
 dgs_status dispatch_vec(int vec, const dgs_view& v, int64_t row_bytes, const void* index,
                         int32_t index_bytes, int64_t n, const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad,
                         void* out, hipStream_t st) {
+  if (is_ragged(v, row_bytes, out, TIER, vec))
+    return index_bytes == 8 ? launch_ragged<TIER, int64_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st)
+                            : launch_ragged<TIER, int32_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
   switch (vec) {
     case 16: return dispatch_index<16, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
     case 8: return dispatch_index<8, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);

@@ -90,6 +90,47 @@ def test_index_every_split(pkg, oracle, dtype, rows, dim):
                 assert np.array_equal(o, got.cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 301), (torch.float32, 47), (torch.float32, 602), (torch.uint8, 16),
+                                       (torch.uint8, 17), (torch.uint8, 129), (torch.bfloat16, 17), (torch.float32, 8190)])
+def test_gather_of_rows_that_16_byte_chunks_do_not_divide(pkg, dtype, dim):
+    # every row length modulo 16 that a width can give, output chunks that hold the ends of two rows,
+    # the store's first and last bytes (where a 16-byte load would leave the slice), boundaries on a row,
+    # inside a row and near both ends, an output that ends inside a chunk, ids outside the store next to
+    # good ones, and launches sized for fewer rows than there are: bytes are moved, so all exactly
+    capi = pkg.capi
+    rows, eb = 300, torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator().manual_seed(dim)
+    full = torch.randint(0, 256, (rows, dim * eb), generator=g, dtype=torch.uint8).view(dtype)
+    idx = torch.cat([torch.tensor([0, rows - 1, rows - 1, 0, 1, rows - 2]), torch.randint(0, rows, (501,), generator=g)])
+    bad = torch.zeros(1, dtype=torch.int64, device="cuda")
+    for cap in (0, 16, dim * eb + eb, 123 * dim * eb, 123 * dim * eb + 5 * eb, rows * dim * eb - eb, rows * dim * eb):
+        st = capi.Store(rows * dim, eb, cap)
+        st.load(full)
+        for w in (torch.int64, torch.int32):
+            ids = idx.to(w).cuda()
+            for n in (1, 6, ids.numel()):
+                got = capi.gather_rows(st.view, dim, ids[:n], dtype, bad_index=bad)
+                assert bad.item() == 0 and torch.equal(_bits(got.cpu()), _bits(full[idx[:n]])), (cap, n)
+            wrong = ids.clone()
+            wrong[3], wrong[40], wrong[-1] = -1, rows, rows + 7
+            got = capi.gather_rows(st.view, dim, wrong, dtype, bad_index=bad).cpu()
+            want = full[idx].clone()
+            want[[3, 40, idx.numel() - 1]] = 0
+            assert bad.item() == 1 and torch.equal(_bits(got), _bits(want)), cap
+            bad.zero_()
+            out = torch.zeros((ids.numel() + 1, dim), dtype=dtype, device="cuda")
+            for count, expected in ((ids.numel(), 1), (29, 7), (0, 1), (ids.numel() + 1, 3)):
+                out.zero_()
+                n_dev = torch.tensor([count], dtype=torch.int64, device="cuda")
+                capi.check(capi.lib.dgs_gather_rows_dyn(st.view, dim, ids.data_ptr(), ids.element_size(), ids.numel(),
+                                                        n_dev.data_ptr(), expected, out.data_ptr(), capi.TIER_ANY,
+                                                        bad.data_ptr(), capi.stream_ptr()))
+                written = count if count <= ids.numel() else 0
+                assert torch.equal(_bits(out[:written].cpu()), _bits(full[idx[:written]])), (cap, count)
+                assert (_bits(out[written:]) == 0).all().item() and bad.item() == 0, (cap, count)
+        st.close()
+
+
 def test_index_1d_and_empty(pkg):
     full = torch.arange(1000, dtype=torch.int32)
     ct = pkg.ChunkTensor([1000], torch.int32, 1234)

@@ -24,28 +24,28 @@
 //
 // A large last hop of uniform picks does without the table altogether (see Buckets below): its
 // fill records the picked ids, two launches group them by id and take the smallest position of
-// every id in LDS, and flag / compact / relabel read the same slot words as on the table path.
+// every id in LDS, and compact / relabel read the same slot words as on the table path.
 //
-// Critical path per hop (3 launches): fill -> flag -> compact.
+// Critical path per hop (2 launches): fill -> compact.
 //   fill     G lanes per seed row (G = 8..64): indptr pair, picks by the dgs-philox-1
 //            contract, one insert_min per pick.
-//   flag     finalises the first-occurrence bit (hop 0, whose seed list may repeat ids and
-//            whose lost marks nobody cleared, asks the table instead) and counts per
-//            1024-position tile.
-//   compact  every block sums the tile counts before its own (the list is short), ranks
-//            its first occurrences, appends them to the frontier and records the rank
-//            at the position.
-// Off the critical path, as surplus blocks of later launches: per-row pick counts are
-// scanned per 256-row tile, and the packed edge list (src_local, dst_local) is written
-// (rank of a pick = rank recorded at its id's smallest position).
+//   compact  a block per tile of positions finalises the first-occurrence bits (hop 0, whose
+//            seed list may repeat ids, asks the table; later hops look at the lost marks),
+//            learns how many first occurrences lie in the tiles before (lookback.h), ranks its
+//            own, appends them to the frontier and records the rank at the position.
+// Off the critical path, as surplus blocks of later launches: the rows' pick counts are
+// scanned (blocks of the compact launch), and the packed edge list (src_local, dst_local) is
+// written (rank of a pick = rank recorded at its id's smallest position).
 //
 // These kernels are chains of dependent memory accesses, so what a thread will need is requested
 // as early as its address is known: a hop's length lives in device memory, but every buffer has
 // its worst-case size, so a thread asks for its own elements (inside the buffer whatever the
 // length turns out to be) together with the length and only then decides whether they count.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
+#include "lookback.h"
 #include "picks.h"
 #include "race.h"
 #include "table.h"
@@ -54,9 +54,23 @@ namespace dgs {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kRowTile = 256;                  // seed rows per offsets tile
-constexpr int kPosItems = 4;
-constexpr int kPosTile = kBlock * kPosItems;   // padded positions per flag/compact block
+constexpr int kRowTile = 256;                  // seed rows per relabel tile
+constexpr int kRowItems = 4;                   // rows a thread of a compact block takes
+// What a compact block's tile is, by the hop's worst case: NT threads x ITEMS consecutive positions x
+// GROUPS.  A few hundred tiles at most for the look-back (see lookback.h), but no fewer blocks than a
+// short list can use: hop 0 reads the table at random, and two CUs alone take 6 us longer over 6 k
+// positions than twelve.  Blocks of four waves as far as it goes: beside other batches' gathers, which
+// free a CU's wave slots four at a time, blocks of eight wait (8 batches through the loader 1394 us
+// against 1433).  The longest lists need eight: with four a thread's positions spill its registers
+// (2.1 M positions 28 us, 3.6 M 32 us, against 13 and 17).
+enum PosTile { kShortTile, kMiddleTile, kLongTile };  // NT x ITEMS x GROUPS = 256 x 1 x 1, 256 x 4 x 4, 512 x 4 x 4
+inline PosTile pos_tile_kind(int64_t len_max) { return len_max <= 131072 ? kShortTile : len_max <= 1310720 ? kMiddleTile : kLongTile; }
+inline int64_t pos_tile_size(int64_t len_max) {
+  const PosTile t = pos_tile_kind(len_max);
+  return t == kShortTile ? 256 : t == kMiddleTile ? 4096 : 8192;
+}
+inline int64_t row_tile_size(int64_t len_max) { return (pos_tile_kind(len_max) == kLongTile ? 512 : 256) * kRowItems; }
+constexpr int kMaxPosTile = 8192;
 constexpr uint32_t kFirstBit = 0x80000000u;
 constexpr uint32_t kInvalidSlot = 0xffffffffu; // padded position that holds no pick
 // row_cnt markers of rows that make the call fail (bit (kBadRow - marker) of the hop's flag word)
@@ -64,9 +78,9 @@ constexpr uint32_t kBadRow = 0xffffffffu;      // degree >= 2^32, or offsets out
 constexpr uint32_t kBadSeed = 0xfffffffeu;     // the seed id is not a row of the graph
 constexpr uint32_t kBadPick = 0xfffffffdu;     // a picked neighbour id is outside what the table holds
 __device__ __forceinline__ bool is_bad_row(uint32_t row_cnt) { return row_cnt >= kBadPick; }
+constexpr int kErrBucketOverflow = 8;          // hop flag bit: the ids of a bucket of the hashed pass did not fit its LDS table
 constexpr int kMaxPicks = 64;
 constexpr int64_t kMaxPositions = int64_t(1) << 30;
-constexpr int64_t kInlineTiles = 2048;         // above this a separate scan launch is used
 // Launches are sized for the worst case, which can exceed the real work many times over (a hub
 // graph deduplicates heavily).  Grids are capped and blocks stride over the virtual block index,
 // so a mostly empty worst case costs a few loop trips instead of 10^5 empty blocks.
@@ -77,6 +91,9 @@ constexpr int64_t kGridCap = 16384;
 // 0.167-0.178 / 0.165-0.169 / 0.183-0.187 ms per step, R-MAT [50,50] 0.342-0.352 / 0.345-0.356 /
 // 0.343-0.353 / 0.357-0.361; a batch alone is level or 2 % faster).
 constexpr int64_t kLoopGrid = 4096;
+// A compact launch that loops keeps to blocks that fit the GPU all at once: a tile's block waits for the
+// tiles before it (a bounded wait, see lookback.h), so those should not queue behind it for a slot.
+constexpr int64_t kLookbackGrid = 512;
 inline int64_t grid_cap() {
   const int64_t forced = debug_option(DGS_DEBUG_SAMPLER_GRID_CAP);
   return forced > 0 ? forced : kGridCap;
@@ -108,19 +125,16 @@ struct Hop {
   int64_t* flags;           // device scalar: bit 0 degree, bit 1 seed id, bit 2 picked id of a bad row
   int64_t* host_sizes;      // optional pinned mirror of the whole sizes array (NULL: none)
   int32_t n_hops;           // layout of the mirror: [0..H] seeds, then H edge counts, then H flags
-  int32_t pad0_;
+  int32_t look_polls;       // lookback_polls()
   uint32_t* row_cnt;        // [s_max] picks of every row (kBadRow on error)
-  uint32_t* row_off;        // [s_max] exclusive offset of the row inside its 256-row tile
-  int* tile_sum;            // [row tiles]
-  int* tile_flag;           // [row tiles]
-  int64_t* tile_off;        // [row tiles] only when row tiles > kInlineTiles
+  uint32_t* row_off;        // [s_max] first packed edge of the row
+  tile_state* row_state;    // [row tiles] the tiles' edge counts, in the course of their scan
   uint32_t* slot;           // [all positions] table slot of a position, bit 31 = first occurrence
   uint32_t* rank_at;        // [all positions] rank of the id first seen at that position
   uint8_t* lost;            // [all positions] non-zero: a smaller position of the same id exists
   int64_t* long_rows;       // weighted only: [s_max] rows handed to the block-per-row launch
   int64_t* long_count;      // weighted only: entries of long_rows
-  int* pos_cnt;             // [position tiles of this hop] first occurrences per tile
-  int64_t* pos_off;         // [position tiles] only when position tiles > kInlineTiles
+  tile_state* pos_state;    // [position tiles of this hop] first occurrences, in the course of their scan
   void* frontier;           // growing array of distinct ids
   void* src_local;          // out [nnz]
   void* dst_local;          // out [nnz]
@@ -191,7 +205,6 @@ constexpr uint32_t kRankBit = 0x40000000u;
 constexpr int kHashBlock = 1024;
 constexpr int kHashSlots = 16384;
 constexpr uint32_t kHashEmpty = 0xffffffffu;         // no id: ids are below 2^31
-constexpr int kErrBucketOverflow = 8;                // hop flag bit: a bucket's ids did not fit its LDS table
 
 struct Buckets {
   uint2* items;      // [tiles_max][kBucketTile] (id, order value), every tile's units in bucket order
@@ -240,40 +253,66 @@ __device__ __forceinline__ T block_sum(T v, T* lds /* NT/64 */) {
   return s;
 }
 
-template <int NT>
-__device__ __forceinline__ int block_or(int v, int* lds /* NT/64 */) {
-#pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) v |= __shfl_xor(v, d, kWave);
-  if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
-  __syncthreads();
-  int s = 0;
-#pragma unroll
-  for (int w = 0; w < NT / kWave; ++w) s |= lds[w];
-  __syncthreads();
-  return s;
-}
-
 // ---- packed edge list of one hop (off the critical path) -----------------------------
 
-// One block per 256-row tile: scan of the rows' pick counts.
-__device__ __forceinline__ void offsets_tile(const Hop& h, int tile) {
-  __shared__ int lds[kBlock / kWave];
+// One block per NT * kRowItems rows: scan of the rows' pick counts.  The block of the last row publishes the
+// hop's edge count and error bits.
+template <int NT, bool EARLY>
+__device__ __forceinline__ void offsets_tile(const Hop& h, int64_t tile) {
+  constexpr int64_t kRows = NT * kRowItems;
+  __shared__ int lds[NT / kWave];
+  __shared__ LookbackLds<NT> look;
   __shared__ int bad;
+  const int64_t s = seeds_of(h);
+  if (!EARLY && tile * kRows >= s) return;
+  const int64_t i = tile * kRows + threadIdx.x * kRowItems;
+  uint32_t rc[kRowItems];
+#pragma unroll
+  for (int j = 0; j < kRowItems; ++j) rc[j] = i + j < h.s_max ? h.row_cnt[i + j] : 0u;  // requested together with s
+  if (tile * kRows >= s) return;  // whole blocks leave together
   if (threadIdx.x == 0) bad = 0;
   __syncthreads();
-  const int64_t s = seeds_of(h);
-  const int64_t i = int64_t(tile) * kRowTile + threadIdx.x;
-  const uint32_t rc = i < h.s_max ? h.row_cnt[i] : 0u;  // requested together with s
   int c = 0;
-  if (i < s) {
-    if (is_bad_row(rc)) atomicOr(&bad, 1 << (kBadRow - rc)); else c = int(rc);
+#pragma unroll
+  for (int j = 0; j < kRowItems; ++j) {
+    if (i + j >= s) rc[j] = 0;
+    if (is_bad_row(rc[j])) {
+      atomicOr(&bad, 1 << (kBadRow - rc[j]));
+      rc[j] = 0;
+    }
+    c += int(rc[j]);
   }
   int total;
-  const int ex = block_exclusive_scan<kBlock, int>(c, &total, lds);
-  if (i < s) h.row_off[i] = uint32_t(ex);
-  if (threadIdx.x == 0) {
-    h.tile_sum[tile] = total;
-    h.tile_flag[tile] = bad;
+  const int ex = block_exclusive_scan<NT, int>(c, &total, lds);
+  const tile_state own = tile_word(total, uint32_t(bad));
+  const tile_state before = tile_exclusive_prefix<NT, true>(h.row_state, tile, own, h.look_polls, look, [&](int64_t t) {
+    __syncthreads();
+    if (threadIdx.x == 0) bad = 0;
+    __syncthreads();
+    int n = 0;
+    for (int j = 0; j < kRowItems; ++j) {  // (a tile before this one is full)
+      const uint32_t r = h.row_cnt[t * kRows + j * NT + threadIdx.x];
+      if (is_bad_row(r)) atomicOr(&bad, 1 << (kBadRow - r)); else n += int(r);
+    }
+    const int sum = block_sum<NT, int>(n, lds);
+    return tile_word(sum, uint32_t(bad));
+  });
+  uint32_t off = uint32_t(tile_sum_of(before)) + uint32_t(ex);
+#pragma unroll
+  for (int j = 0; j < kRowItems; ++j) {
+    if (i + j < s) h.row_off[i + j] = off;
+    off += rc[j];
+  }
+  if ((tile + 1) * kRows >= s && threadIdx.x == 0) {
+    const tile_state all = tile_add(before, own);
+    int64_t flags = tile_flags_of(all);
+    if (h.bucketed != 0 && *h.bucket_overflow != 0) flags |= kErrBucketOverflow;
+    *h.nnz = tile_sum_of(all);
+    *h.flags = flags;
+    if (h.host_sizes) {
+      mirror_to_host(h.host_sizes + h.n_hops + 1 + h.index, tile_sum_of(all));
+      mirror_to_host(h.host_sizes + 2 * h.n_hops + 1 + h.index, flags);
+    }
   }
 }
 
@@ -289,7 +328,6 @@ __device__ __forceinline__ void offsets_tile(const Hop& h, int tile) {
 // leave without having read anything.
 template <typename IdT, typename TableT, bool EARLY>
 __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, int64_t b) {
-  __shared__ int64_t lds[kBlock / kWave];
   const int k = h.k;
   if (k == 0) return;
   const int groups = relabel_groups(k);
@@ -321,17 +359,10 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
       if (h.index == 0) seed_word[j] = h.slot[h.pos_base + i[j]];
     }
   }
-  int64_t part = 0;
-  if (h.tile_off) {
-    if (threadIdx.x == 0) part = h.tile_off[tile];
-  } else {
-    for (int64_t j = threadIdx.x; j < tile; j += kBlock) part += h.tile_sum[j];
-  }
   if (tile * kRowTile >= s) return;  // whole blocks leave together
   // Rank of a pick = rank recorded at the smallest position of its id: its own position when it
   // is a first occurrence, else the position the table holds.  Two rounds of loads, each issued
-  // for all of the thread's picks before any is used, and both before the block adds up its
-  // prefix (whose barrier nothing here has to wait behind).
+  // for all of the thread's picks before any is used.
   const bool bucketed = bucketed_now(h, s);
   bool live[kRelabelItems];
   bool known[kRelabelItems];  // bucketed hop: the word of a repeat may be the rank itself
@@ -353,11 +384,10 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
   uint32_t rank[kRelabelItems];
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) rank[j] = !live[j] ? 0u : known[j] ? at[j] : h.rank_at[at[j]];
-  const int64_t prefix = block_sum<kBlock, int64_t>(part, lds);
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) {
     if (!live[j]) continue;
-    const int64_t o = prefix + off[j] + l[j];
+    const int64_t o = int64_t(off[j]) + l[j];
     static_cast<IdT*>(h.src_local)[o] = IdT(rank[j]);
     static_cast<IdT*>(h.dst_local)[o] =
         h.index == 0 ? IdT(rank_of(h, table, h.pos_base + i[j], seed_word[j])) : IdT(i[j]);
@@ -392,7 +422,7 @@ __device__ __forceinline__ bool place_pick(const Hop& h, const TableT& table, Id
   uint32_t displaced;
   uint32_t w = table.insert_min(col, uint32_t(p), &first, &displaced, look_first);
   if (h.index != 0) {
-    if (first) w |= kFirstBit;  // provisional: cleared by flag() if the position gets lost
+    if (first) w |= kFirstBit;  // provisional: void once the position is marked lost
     mark_lost(h, displaced);
   }
   *word = w;
@@ -464,7 +494,7 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   const bool bad = deg64 < 0 || deg64 > 0xffffffffLL || b < 0 || b + deg64 > indices.n;
   const uint32_t deg = bad ? 0u : uint32_t(deg64);
   const int k = h.k;
-  if (l == 0 && h.index == 0) {  // the caller's seeds open the mapping list; flag() decides their first bits
+  if (l == 0 && h.index == 0) {  // the caller's seeds open the mapping list; compact_tile decides their first bits
     bool first;
     uint32_t displaced;
     h.slot[h.pos_base + i] =
@@ -1030,152 +1060,157 @@ __global__ __launch_bounds__(kHashBlock) void bucket_first_hashed_kernel(Hop h, 
   }
 }
 
-// One virtual block of the flag launch: 1024 padded positions.
-template <typename IdT, typename TableT, bool EARLY>
-__device__ __forceinline__ void flag_tile(const Hop& h, int64_t tile, const TableT& table) {
-  __shared__ int lds[kBlock / kWave];
+// Whether the position `rel` of the hop, of slot word `word`, is the first one of its id (`rel` is below
+// the hop's length); the answer is the same before and after compact_tile has brought the word's bit
+// up to date.
+template <typename TableT>
+__device__ __forceinline__ bool is_first(const Hop& h, const TableT& table, int64_t rel, uint32_t word, bool lost) {
+  if (word == kInvalidSlot) return false;
+  return h.index == 0 ? table.value(word & ~kFirstBit) == uint32_t(h.pos_base + rel) : (word & kFirstBit) != 0 && !lost;
+}
+
+// ITEMS consecutive words of an array as one load or store.
+template <int ITEMS> struct Items;
+template <> struct Items<1> {
+  typedef uint32_t words __attribute__((ext_vector_type(1)));
+  static __device__ __forceinline__ uint32_t load_marks(const uint8_t* p) { return *p; }
+};
+template <> struct Items<4> {
+  typedef uint32_t words __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ uint32_t load_marks(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
+};
+
+// The first occurrences of one tile: counted, ranked, appended to the frontier.  A thread takes ITEMS
+// consecutive positions of every group: their slot words, their lost marks and their ranks move as
+// one load or store each, whether the positions count or not (the arrays reach a tile beyond the last
+// position).  Bound: the chain of waits (length and words, the tiles before, the stores), 6 us at the
+// floor; 13 bytes per position and 12 per first occurrence otherwise (2.1 M positions, 980 k of them
+// first: 13 us).
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool EARLY>
+__device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const TableT& table) {
+  using words = typename Items<ITEMS>::words;
+  constexpr int kWaves = NT / kWave;
+  constexpr int kGroup = NT * ITEMS;
+  constexpr int64_t kTile = int64_t(kGroup) * GROUPS;
+  __shared__ LookbackLds<NT> look;
+  __shared__ int wave_count[GROUPS * kWaves];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  // the hop's length and this thread's slot words (EARLY: requested together)
   const int64_t s = seeds_of(h);
   const int64_t len = seed_part(h, s) + s * h.k;
-  if (!EARLY && tile * kPosTile >= len) {
-    if (threadIdx.x == 0) h.pos_cnt[tile] = 0;
+  if (!EARLY && tile != 0 && tile * kTile >= len) return;
+  const int64_t base = tile * kTile + threadIdx.x * ITEMS;
+  words word[GROUPS];
+  uint32_t lost[GROUPS];
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const int64_t p = h.pos_base + base + g * kGroup;  // a multiple of ITEMS
+    word[g] = *reinterpret_cast<const words*>(h.slot + p);
+    lost[g] = h.index != 0 ? Items<ITEMS>::load_marks(h.lost + p) : 0u;
+  }
+  if (tile != 0 && tile * kTile >= len) return;  // whole blocks leave together
+  uint32_t first[GROUPS];   // bit j: position j of the group's is its id's first
+  int lane_before[GROUPS];  // first positions in the lanes below
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    first[g] = 0;
+    const int64_t rel = base + g * kGroup;
+    if (h.index == 0) {  // is_first's question to the table for all positions at once (slot 0 stands in where there is none)
+      uint32_t least[ITEMS];
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j) {
+        if (rel + j >= len) word[g][j] = kInvalidSlot;
+        least[j] = table.value(word[g][j] != kInvalidSlot ? word[g][j] & ~kFirstBit : 0u);
+      }
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j)
+        if (word[g][j] != kInvalidSlot && least[j] == uint32_t(h.pos_base + rel + j)) first[g] |= 1u << j;
+    } else {
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j)
+        if (rel + j < len && is_first(h, table, rel + j, word[g][j], ((lost[g] >> (8 * j)) & 0xffu) != 0)) first[g] |= 1u << j;
+    }
+    const int c = __builtin_popcount(first[g]);  // its bits are summed over the lanes by ballots
+    lane_before[g] = 0;
+    int sum = 0;
+#pragma unroll
+    for (int bit = 0; (1 << bit) <= ITEMS; ++bit) {
+      const uint64_t at = __ballot((c >> bit) & 1);
+      lane_before[g] += __builtin_popcountll(at & ((uint64_t(1) << lane) - 1)) << bit;
+      sum += __builtin_popcountll(at) << bit;
+    }
+    if (lane == 0) wave_count[g * kWaves + wave] = sum;
+  }
+  __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int q = 0; q < GROUPS * kWaves; ++q) {
+    if (q % kWaves == wave) lane_before[q / kWaves] += total;
+    total += wave_count[q];
+  }
+  const tile_state before = tile_exclusive_prefix<NT, false>(h.pos_state, tile, tile_word(total), h.look_polls, look, [&](int64_t t) {
+    int n = 0;
+    for (int j = 0; j < GROUPS * ITEMS; ++j) {  // (a tile before this one is full)
+      const int64_t rel = t * kTile + int64_t(j) * NT + threadIdx.x;
+      n += is_first(h, table, rel, h.slot[h.pos_base + rel], h.index != 0 && h.lost[h.pos_base + rel] != 0);
+    }
+    __syncthreads();
+    return tile_word(block_sum<NT, int>(n, wave_count));
+  });
+  const int64_t rank0 = first_rank(h, s) + tile_sum_of(before);
+  if ((tile + 1) * kTile >= len && threadIdx.x == 0) {  // the last tile: the frontier's size is known
+    *h.n_unique = rank0 + total;
+    if (h.host_sizes) {
+      if (h.index == 0) mirror_to_host(h.host_sizes, s);
+      mirror_to_host(h.host_sizes + h.index + 1, rank0 + total);
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const int64_t p = h.pos_base + base + g * kGroup;
+    uint32_t rank = uint32_t(rank0) + uint32_t(lane_before[g]);
+    words ranks;
+    bool changed = false;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      ranks[j] = rank;
+      const uint32_t bare = word[g][j] & ~kFirstBit;
+      if ((first[g] >> j) & 1) {
+        static_cast<IdT*>(h.frontier)[rank] = table.key(bare);
+        ++rank;
+        changed |= h.index == 0;
+        if (h.index == 0) word[g][j] = bare | kFirstBit;  // the bit as relabel_tile reads it
+      } else if (((lost[g] >> (8 * j)) & 0xffu) != 0) {
+        changed = true;
+        word[g][j] = bare;
+      }
+    }
+    *reinterpret_cast<words*>(h.rank_at + p) = ranks;  // (only the ones at first positions are ever read)
+    if (changed) *reinterpret_cast<words*>(h.slot + p) = word[g];
+  }
+}
+
+// Virtual blocks: one per NT * kRowItems rows (scan of the rows' pick counts), then one per position tile.  A
+// launch that fits the grid cap has a block for each in the worst case; a launch that loops (STRIDE)
+// goes over the tiles the hop really has.
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE>
+__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table) {
+  constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
+  if (!STRIDE) {
+    const int64_t vb = blockIdx.x;
+    if (vb < row_tiles) offsets_tile<NT, true>(h, vb);
+    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, true>(h, vb - row_tiles, table);
     return;
   }
-  const int64_t base = tile * kPosTile + threadIdx.x * kPosItems;
-  // this thread's slot words and lost marks (EARLY: requested together with the hop's length)
-  const int64_t readable = EARLY ? h.len_max : len;
-  uint32_t w[kPosItems];
-  uint8_t gone[kPosItems];
-#pragma unroll
-  for (int j = 0; j < kPosItems; ++j) {
-    const bool inside = base + j < readable;
-    w[j] = inside ? h.slot[h.pos_base + base + j] : kInvalidSlot;
-    gone[j] = inside && h.index != 0 ? h.lost[h.pos_base + base + j] : uint8_t(0);
-  }
-  int c = 0;
-  if (tile * kPosTile < len) {
-#pragma unroll
-    for (int j = 0; j < kPosItems; ++j) {
-      const int64_t rel = base + j;
-      if (rel < len && w[j] != kInvalidSlot) {
-        const int64_t p = h.pos_base + rel;
-        if (h.index == 0) {
-          if (table.value(w[j]) == uint32_t(p)) {
-            h.slot[p] = w[j] | kFirstBit;
-            ++c;
-          }
-        } else if (w[j] & kFirstBit) {
-          if (gone[j]) h.slot[p] = w[j] & ~kFirstBit; else ++c;
-        }
-      }
-    }
-    c = block_sum<kBlock, int>(c, lds);
-  }
-  if (threadIdx.x == 0) h.pos_cnt[tile] = c;
-}
-
-// Virtual blocks [0, flag_blocks): position tiles; then row_tiles blocks scanning the rows' pick
-// counts per 256-row tile (for the packed edge list, off the critical path).
-template <typename IdT, typename TableT, bool STRIDE>
-__global__ __launch_bounds__(kBlock) void hop_flag_kernel(Hop h, int64_t flag_blocks, int64_t row_tiles,
-                                                          TableT table) {
-  DGS_FOR_VIRTUAL_BLOCKS(vb, flag_blocks + row_tiles) {
-    if (vb < flag_blocks) flag_tile<IdT, TableT, !STRIDE>(h, vb, table);
-    else offsets_tile(h, int(vb - flag_blocks));
-  }
-}
-
-// Separate scans for very long tile lists (one block), over the tiles the hop really has.
-__device__ __forceinline__ int64_t real_pos_tiles(const Hop& h, int64_t s) {
-  return (seed_part(h, s) + s * h.k + kPosTile - 1) / kPosTile;
-}
-__global__ __launch_bounds__(1024) void pos_scan_kernel(Hop h) {
-  int64_t sum;
-  single_block_scan<1024, int, int64_t>(h.pos_cnt, h.pos_off, real_pos_tiles(h, seeds_of(h)), &sum);
-}
-__global__ __launch_bounds__(1024) void tile_scan_kernel(Hop h) {
-  int64_t sum;
-  single_block_scan<1024, int, int64_t>(h.tile_sum, h.tile_off, (seeds_of(h) + kRowTile - 1) / kRowTile, &sum);
-}
-
-// One virtual block of the compact launch: the first occurrences of one 1024-position tile.
-// `pos_tiles` / `row_tiles` are the worst-case tile counts the flag launch covered: the counts of
-// tiles beyond the hop's real length are zero there, so sums may run over all of them.
-template <typename IdT, typename TableT, bool EARLY>
-__device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, int64_t pos_tiles, int64_t row_tiles,
-                                             const TableT& table) {
-  __shared__ int64_t lds64[kBlock / kWave];
-  __shared__ int lds[kBlock / kWave];
-  // the hop's length, this thread's slot words and its share of the tile counts (EARLY: requested together)
   const int64_t s = seeds_of(h);
+  const int64_t rows = (s + NT * kRowItems - 1) / (NT * kRowItems);
   const int64_t len = seed_part(h, s) + s * h.k;
-  if (!EARLY && tile != 0 && tile * kPosTile >= len) return;
-  const int64_t base = tile * kPosTile + threadIdx.x * kPosItems;
-  const int64_t readable = EARLY ? h.len_max : len;
-  uint32_t w[kPosItems];
-#pragma unroll
-  for (int j = 0; j < kPosItems; ++j) w[j] = base + j < readable ? h.slot[h.pos_base + base + j] : kInvalidSlot;
-  // first occurrences in the tiles before this one (block 0 needs the grand total instead)
-  int64_t part = 0;
-  if (h.pos_off) {  // scanned by pos_scan_kernel over the hop's real tiles
-    const int64_t last = real_pos_tiles(h, s) - 1;
-    if (threadIdx.x == 0) part = tile != 0 ? h.pos_off[tile] : last >= 0 ? h.pos_off[last] + h.pos_cnt[last] : 0;
-  } else {
-    const int64_t upto = tile == 0 ? pos_tiles : tile;
-    for (int64_t j = threadIdx.x; j < upto; j += kBlock) part += h.pos_cnt[j];
+  const int64_t total = rows + (len > 0 ? (len + kTile - 1) / kTile : 1);
+  for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
+    if (vb < rows) offsets_tile<NT, false>(h, vb);
+    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table);
+    __syncthreads();  // the tiles' LDS is rewritten by the block's next one
   }
-  int64_t edges = 0;
-  int bad = 0;
-  if (tile == 0) {
-    for (int64_t j = threadIdx.x; j < row_tiles; j += kBlock) {
-      edges += h.tile_sum[j];
-      bad |= h.tile_flag[j];
-    }
-  }
-  const int64_t rank0 = first_rank(h, s);
-  if (tile != 0 && tile * kPosTile >= len) return;  // whole blocks leave together
-  part = block_sum<kBlock, int64_t>(part, lds64);
-  if (tile == 0) {
-    // this hop's lengths, written even when there is nothing to do: frontier size, edge count
-    // (row tiles were scanned by the surplus blocks of the flag launch) and error bits
-    edges = block_sum<kBlock, int64_t>(edges, lds64);
-    bad = block_or<kBlock>(bad, lds);
-    if (h.bucketed != 0 && *h.bucket_overflow != 0) bad |= kErrBucketOverflow;
-    if (threadIdx.x == 0) {
-      *h.n_unique = rank0 + part;
-      *h.nnz = edges;
-      *h.flags = bad;
-      if (h.host_sizes) {
-        if (h.index == 0) mirror_to_host(h.host_sizes, s);
-        mirror_to_host(h.host_sizes + h.index + 1, rank0 + part);
-        mirror_to_host(h.host_sizes + h.n_hops + 1 + h.index, edges);
-        mirror_to_host(h.host_sizes + 2 * h.n_hops + 1 + h.index, bad);
-      }
-    }
-    if (len <= 0) return;
-  }
-  const int64_t before = tile == 0 ? 0 : part;
-  int c = 0;
-#pragma unroll
-  for (int j = 0; j < kPosItems; ++j) {
-    if (base + j >= len || w[j] == kInvalidSlot) w[j] = 0;  // bit 31 clear: not a first occurrence
-    c += (w[j] & kFirstBit) != 0;
-  }
-  int total;
-  int64_t rank = rank0 + before + block_exclusive_scan<kBlock, int>(c, &total, lds);
-#pragma unroll
-  for (int j = 0; j < kPosItems; ++j) {
-    if (w[j] & kFirstBit) {
-      static_cast<IdT*>(h.frontier)[rank] = table.key(w[j] & ~kFirstBit);
-      h.rank_at[h.pos_base + base + j] = uint32_t(rank);
-      ++rank;
-    }
-  }
-}
-
-template <typename IdT, typename TableT, bool STRIDE>
-__global__ __launch_bounds__(kBlock) void hop_compact_kernel(Hop h, int64_t blocks, int64_t pos_tiles,
-                                                             int64_t row_tiles, TableT table) {
-  DGS_FOR_VIRTUAL_BLOCKS(vb, blocks) compact_tile<IdT, TableT, !STRIDE>(h, vb, pos_tiles, row_tiles, table);
 }
 
 template <typename IdT, typename TableT, bool STRIDE>
@@ -1288,36 +1323,47 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
   return DGS_OK;
 }
 
+inline int64_t row_tiles_of(int64_t rows, int64_t len_max) { return (rows + row_tile_size(len_max) - 1) / row_tile_size(len_max); }
+inline int64_t pos_tiles_of(int64_t len_max) {
+  return len_max > 0 ? (len_max + pos_tile_size(len_max) - 1) / pos_tile_size(len_max) : 1;
+}
+
 // Lays the workspace out; with base == nullptr only the size is computed.
 size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void** table,
               Buckets* buckets = nullptr) {
   Carver c(base);
   char* t = c.take<char>(p.table_bytes);
   if (table) *table = t;
-  const size_t positions = size_t(p.s_max[p.n_hops]);  // sum over hops of (seed part + s_max * k)
+  // sum over hops of (seed part + s_max * k), every hop's base rounded up to a multiple of 16, and a
+  // tile beyond the last position (see compact_tile)
+  const size_t positions = size_t(p.s_max[p.n_hops]) + 16 * size_t(p.n_hops) + kMaxPosTile;
   uint32_t* slot = c.take<uint32_t>(positions);
   uint32_t* rank_at = c.take<uint32_t>(positions);
-  uint8_t* lost = c.take<uint8_t>(positions + 16);
+  uint8_t* lost = c.take<uint8_t>(positions);
+  // the tile states of all hops, right behind the lost marks: cleared together by hop 0's fill launch
+  size_t tiles = 0;
+  for (int h = 0; h < p.n_hops; ++h) {
+    const int64_t len = (h == 0 ? p.s_max[0] : 0) + p.nnz_max[h];
+    tiles += row_tiles_of(p.s_max[h], len) + pos_tiles_of(len);
+  }
+  tile_state* states = c.take<tile_state>(tiles + 2);
   int64_t* long_counts = p.weighted ? c.take<int64_t>(DGS_MAX_HOPS) : nullptr;
   int64_t pos_base = 0;
   for (int h = 0; h < p.n_hops; ++h) {
     const size_t s = size_t(p.s_max[h]);
     const size_t len = (h == 0 ? s : 0) + size_t(p.nnz_max[h]);
-    const size_t row_tiles = (s + kRowTile - 1) / kRowTile;
-    const size_t pos_tiles = (len + kPosTile - 1) / kPosTile;
     Hop v{};
     v.row_cnt = c.take<uint32_t>(s);
     v.row_off = c.take<uint32_t>(s);
-    v.tile_sum = c.take<int>(row_tiles);
-    v.tile_flag = c.take<int>(row_tiles);
-    v.tile_off = row_tiles > size_t(kInlineTiles) ? c.take<int64_t>(row_tiles) : nullptr;
+    v.row_state = states;
+    states += row_tiles_of(int64_t(s), int64_t(len));
+    v.pos_state = states;
+    states += pos_tiles_of(int64_t(len));
     v.slot = slot;
     v.rank_at = rank_at;
     v.lost = lost;
     v.long_rows = p.weighted ? c.take<int64_t>(s) : nullptr;
     v.long_count = p.weighted ? long_counts + h : nullptr;
-    v.pos_cnt = c.take<int>(pos_tiles + 1);
-    v.pos_off = pos_tiles > size_t(kInlineTiles) ? c.take<int64_t>(pos_tiles) : nullptr;
     v.s_max = p.s_max[h];
     v.pos_base = pos_base;
     v.len_max = int64_t(len);
@@ -1326,7 +1372,7 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     v.bucketed = p.bucketed && h == p.n_hops - 1;
     v.bucket_pos_cap = int64_t(p.bucket_pos_tiles) * kBucketTile;
     if (hops) hops[h] = v;
-    pos_base += int64_t(len);
+    pos_base += (int64_t(len) + 15) / 16 * 16;
   }
   if (p.bucket_space) {
     Buckets b{};
@@ -1357,6 +1403,18 @@ void launch_relabel(const Hop& hop, const TableT& table, hipStream_t st) {
   else
     hipLaunchKernelGGL((hop_relabel_kernel<IdT, TableT, false>), dim3(capped_grid(blocks)), dim3(kBlock), 0, st, hop,
                        blocks, table);
+}
+
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
+void launch_compact(const Hop& hop, const TableT& table, hipStream_t st) {
+  const int64_t row_tiles = row_tiles_of(hop.s_max, hop.len_max);
+  const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max);
+  if (blocks > std::min(grid_cap(), kLookbackGrid))
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true>), dim3(uint32_t(std::min(grid_cap(), kLookbackGrid))),
+                       dim3(NT), 0, st, hop, row_tiles, table);
+  else
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false>), dim3(uint32_t(blocks)), dim3(NT), 0, st,
+                       hop, row_tiles, table);
 }
 
 template <typename IdT, typename PtrT, typename TableT, int G>
@@ -1417,15 +1475,15 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
     const Hop& cur = hops[h];
     const Hop prev = h > 0 ? hops[h - 1] : Hop{};
     const int64_t surplus = h > 0 ? relabel_blocks(prev.s_max, prev.k) : 0;
-    // the launch of hop 0 also clears the lost marks of all later hops (16-byte granules; the
-    // first one may reach back into hop 0's own range, whose marks are never read or written)
+    // the launch of hop 0 also clears the lost marks of all later hops and the tile states of all
+    // hops, which lie behind them
     uint4* clear_begin = nullptr;
     int64_t clear_n16 = 0;
-    if (h == 0 && p.n_hops > 1) {
-      const int64_t first = hops[1].pos_base / 16 * 16;
-      const int64_t last = (p.s_max[p.n_hops] + 15) / 16 * 16;  // the array has 16 spare bytes
-      clear_begin = reinterpret_cast<uint4*>(cur.lost + first);
-      clear_n16 = last > first ? (last - first) / 16 : 0;
+    if (h == 0) {
+      const Hop& last = hops[p.n_hops - 1];
+      clear_begin = reinterpret_cast<uint4*>(cur.lost + (p.n_hops > 1 ? hops[1].pos_base : p.s_max[1] / 16 * 16));
+      const char* end = reinterpret_cast<const char*>(last.pos_state + pos_tiles_of(last.len_max));  // (two spare words follow)
+      clear_n16 = (end - reinterpret_cast<const char*>(clear_begin) + 15) / 16;
     }
     if (p.weighted) {
       const dgs_status ws = replace ? launch_fill_weighted<IdT, PtrT, TableT, true>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st)
@@ -1450,31 +1508,11 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
       DGS_LAUNCH_CHECK();
     }
 
-    const int64_t len_max = (h == 0 ? cur.s_max : 0) + cur.s_max * cur.k;
-    const int64_t pos_tiles = (len_max + kPosTile - 1) / kPosTile;
-    const int64_t row_tiles = (cur.s_max + kRowTile - 1) / kRowTile;
-    if (is_capped(pos_tiles + row_tiles))
-      hipLaunchKernelGGL((hop_flag_kernel<IdT, TableT, true>), dim3(capped_grid(pos_tiles + row_tiles)),
-                         dim3(kBlock), 0, st, cur, pos_tiles, row_tiles, table);
-    else
-      hipLaunchKernelGGL((hop_flag_kernel<IdT, TableT, false>), dim3(capped_grid(pos_tiles + row_tiles)),
-                         dim3(kBlock), 0, st, cur, pos_tiles, row_tiles, table);
-    DGS_LAUNCH_CHECK();
-    if (cur.pos_off) {
-      hipLaunchKernelGGL(pos_scan_kernel, dim3(1), dim3(1024), 0, st, cur);
-      DGS_LAUNCH_CHECK();
+    switch (pos_tile_kind(cur.len_max)) {
+      case kShortTile: launch_compact<IdT, TableT, 256, 1, 1>(cur, table, st); break;
+      case kMiddleTile: launch_compact<IdT, TableT, 256, 4, 4>(cur, table, st); break;
+      case kLongTile: launch_compact<IdT, TableT, 512, 4, 4>(cur, table, st); break;
     }
-    if (cur.tile_off) {
-      hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(1024), 0, st, cur);
-      DGS_LAUNCH_CHECK();
-    }
-    const int64_t compact_blocks = pos_tiles > 0 ? pos_tiles : 1;  // block 0 always writes the lengths
-    if (is_capped(compact_blocks))
-      hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, true>), dim3(capped_grid(compact_blocks)), dim3(kBlock),
-                         0, st, cur, compact_blocks, pos_tiles, row_tiles, table);
-    else
-      hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, false>), dim3(capped_grid(compact_blocks)), dim3(kBlock),
-                         0, st, cur, compact_blocks, pos_tiles, row_tiles, table);
     DGS_LAUNCH_CHECK();
   }
   // every length is final here: mark the point the caller may wait for
@@ -1609,6 +1647,7 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
     t.flags = sizes_dev + 2 * n_hops + 1 + h;
     t.host_sizes = sizes_host;
     t.n_hops = n_hops;
+    t.look_polls = lookback_polls();
     t.frontier = frontier;
     t.src_local = outs[h].src_local;
     t.dst_local = outs[h].dst_local;

@@ -66,13 +66,17 @@ int dgs_abi_version(void);
  *                                hash table per bucket) whatever the graph's size, 4 like 3 with
  *                                those tables cut to 256 slots (small inputs then fill them and
  *                                are gone over in parts)
+ *   DGS_DEBUG_LOOKBACK_POLLS     n > 0: a block that needs the counts of the blocks before it
+ *                                looks for them n - 1 times before it counts them itself
+ *                                (1: it never looks; the default is 256 times)
  */
 enum {
   DGS_DEBUG_FORCE_SPLIT_TABLE = 0,
   DGS_DEBUG_WEIGHTED_GROUP = 1,
   DGS_DEBUG_GATHER_LDS_BYTES = 2,
   DGS_DEBUG_SAMPLER_GRID_CAP = 3,
-  DGS_DEBUG_SAMPLER_BUCKETED = 4
+  DGS_DEBUG_SAMPLER_BUCKETED = 4,
+  DGS_DEBUG_LOOKBACK_POLLS = 5
 };
 dgs_status dgs_debug_set(int32_t option, int64_t value);
 

@@ -774,6 +774,26 @@ def test_fused_sampler_under_a_small_grid_cap(pkg, oracle, graph, cap, request, 
         assert torch.equal(x.cpu(), feats[f.cpu()])
 
 
+@pytest.mark.parametrize("n_seeds,fanouts,replace", [(1, [3], False), (900, [9, 4], False), (4000, [12, 6, 3], False),
+                                                     (6000, [30, 10], True)])
+def test_fused_sampler_whose_tiles_do_not_wait_for_each_other(pkg, oracle, graph, n_seeds, fanouts, replace, request, last_hop):
+    # a tile's block that does not find the counts of the tiles before it (here: never looks) counts
+    # them itself, with the same result; lists of one tile, of several short, middle and long tiles
+    capi = pkg.capi
+    indptr, indices = graph
+    ip_ct = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix_ct = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    seeds = np.random.default_rng(n_seeds).integers(0, 20000, size=n_seeds).astype(np.int64)
+    want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, 5, 0)
+    request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, 0))
+    for polls in (0, 1):
+        capi.check(capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, polls))
+        sampler = pkg.ChunkTensorSampler(fanouts, ip_ct, ix_ct, replace=replace, seed=5)
+        f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
+        assert np.array_equal(_np(f), want_f), polls
+        _check_blocks(blocks, want_blocks)
+
+
 def test_unique_relabel_ids_beyond_32_bits(pkg, oracle):
     # 8-byte ids are first tried in one-word table slots; an id of 2^32 - 1 or more sends the call
     # to the two-array table.  Ids that only differ above bit 31 must not be confused, present or not.

@@ -327,7 +327,7 @@ __device__ __forceinline__ void offsets_tile(const Hop& h, int64_t tile) {
 // (and loops over its virtual blocks): the length is waited for first and blocks beyond it
 // leave without having read anything.
 template <typename IdT, typename TableT, bool EARLY>
-__device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, int64_t b) {
+__device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, int64_t b, int tid) {
   const int k = h.k;
   if (k == 0) return;
   const int groups = relabel_groups(k);
@@ -345,7 +345,7 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) {
     const int chunk = group * kRelabelItems + j;
-    const int t = chunk * kBlock + threadIdx.x;  // padded pick inside the tile
+    const int t = chunk * kBlock + tid;  // padded pick inside the tile
     const int r = t / k;
     l[j] = t - r * k;
     i[j] = tile * kRowTile + r;
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
     if (vb < fill_blocks) {
       fill_rows<IdT, PtrT, TableT, G, !STRIDE>(h, vb, table, indptr, indices, replace, rng_seed);
     } else if (!STRIDE && vb < fill_blocks + relabel_count) {  // (a striding launch is given no such blocks)
-      relabel_tile<IdT, TableT, !STRIDE>(prev, table, vb - fill_blocks);
+      relabel_tile<IdT, TableT, !STRIDE>(prev, table, vb - fill_blocks, threadIdx.x);
     } else {
       const int64_t i = (vb - fill_blocks - relabel_count) * kBlock + threadIdx.x;
       if (i < clear_n16) clear_begin[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -572,32 +572,40 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
   }
 }
 
-// ---- weighted picks (race.h): one wave per seed row, a block per row for long rows ----
-
+// ---- weighted picks (race.h) ----
+//
+// Two launch shapes.  A small hop (kSharedMaxRows) is one launch of 16-wave blocks, a wave per row; rows
+// of more than kSharedRow positions are put on a list in LDS and the whole block works on them, one
+// after the other, once its waves are through with the others.  Its time is that of its longest chain:
+// what made such a hop slow was a row of 2000 positions on one wave, behind three others, and then a
+// launch of its own for the longer ones (1024 / 5.9 k rows of mean degree 50, longest 17 k, k = 5 / 10:
+// 46 and 59 us as two launches,
+// 31 and 37 as one).
+// A large hop has rows enough for every wave slot: four-wave blocks, several rows per wave, and a second
+// launch, a block per row, for the queued rows above long_row<64>() positions.
 constexpr int64_t kMaxLongGrid = 512;
+constexpr int64_t kSharedMaxRows = 16384;
+constexpr uint32_t kSharedRow = 512;  // two stretches of a wave (stretch_keys); with 256 a batch takes 2 % longer, the block's turns adding up
 
-// Lanes that one row's picks occupy when a wave writes them out: the wave races its rows one
+// Lanes that one row's picks occupy when a wave of a large hop writes them out: the wave races its rows one
 // after the other (64 lanes on a row), parks every row's picks in that row's lanes and then
 // inserts and records the picks of all its rows in one go, so that the instructions of that step
 // are not spent on a mostly idle wave.
 __host__ __device__ __forceinline__ int weighted_row_lanes(int64_t k) { return k <= 16 ? 16 : (k <= 32 ? 32 : kWave); }
 inline int64_t weighted_rows_per_block(int64_t k) { return (kBlock / kWave) * (kWave / weighted_row_lanes(k)); }
 
-// One virtual block of the weighted fill launch: four waves with 64 / weighted_row_lanes(k) seed
-// rows each.  Rows above long_row<64>() positions are queued for hop_fill_weighted_long_kernel,
-// which fills their positions; everything else about a row is what fill_rows does.
-template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
-__device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t vb, const TableT& table,
-                                                   const TierView<PtrT>& indptr, const TierView<IdT>& indices,
-                                                   const TierView<float>& probs, uint64_t rng_seed) {
+// The wave's rows [first, first + 64 / lanes) of the hop.  Rows above `long_limit` positions are only
+// announced (put_off(row of the hop, its first edge, its degree, its seed), by one lane); everything
+// else about a row is what fill_rows does.
+template <typename IdT, typename PtrT, typename TableT, bool REPLACE, typename PutOff>
+__device__ __forceinline__ void fill_wave_weighted(const Hop& h, int64_t s, int64_t first, int lanes, uint32_t long_limit,
+                                                   const TableT& table, const TierView<PtrT>& indptr,
+                                                   const TierView<IdT>& indices, const TierView<float>& probs,
+                                                   uint64_t rng_seed, PutOff put_off) {
   const Group<kWave> g;
-  const int64_t s = seeds_of(h);
   const bool look_first = look_before_insert(h, s);
-  if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   const int k = h.k;
-  const int lanes = weighted_row_lanes(k);
   const int rows = kWave / lanes;
-  const int64_t first = (vb * (kBlock / kWave) + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave)))) * rows;
   if (first >= s) return;  // whole waves leave together
   // every lane looks up the row whose picks it will write out
   const int mine = g.l / lanes;  // that row among the wave's
@@ -626,15 +634,15 @@ __device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t vb, con
     h.slot[h.pos_base + i] =
         seed_ok ? table.insert_min(seed, uint32_t(h.pos_base + i), &first_seen, &displaced) : kInvalidSlot;
   }
-  // rows that are copied need no work; long rows are queued and written by the other launch
-  const bool is_long = deg > long_row<kWave>() && (REPLACE || deg > uint32_t(k));
-  if (is_long && l == 0) h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = i;
+  // rows that are copied need no work; long rows are written by somebody else
+  const bool is_long = deg > long_limit && (REPLACE || deg > uint32_t(k));
+  if (is_long && l == 0) put_off(i, b, deg, seed);
   uint32_t pick = uint32_t(l);  // what a copied row keeps: its positions in order
   for (int r = 0; r < rows; ++r) {
     // row r of the wave, in scalar registers
     const int src = r * lanes;
     const uint32_t rdeg = lane_read(deg, src);
-    const bool rlong = rdeg > long_row<kWave>() && (REPLACE || rdeg > uint32_t(k));
+    const bool rlong = rdeg > long_limit && (REPLACE || rdeg > uint32_t(k));
     if (rdeg == 0 || rlong || (!REPLACE && rdeg <= uint32_t(k))) continue;
     const int64_t rrow = int64_t(lane_read(uint64_t(int64_t(seed)), src));
     const int64_t rb = int64_t(lane_read(uint64_t(b), src));
@@ -659,6 +667,30 @@ __device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t vb, con
                  : (REPLACE ? (deg == 0 ? 0u : uint32_t(k)) : (deg < uint32_t(k) ? deg : uint32_t(k)));
 }
 
+// The picks of one long row (a valid one: its edges are deg positions from b on), by a whole
+// kLongBlock-thread block.
+template <typename IdT, typename TableT, bool REPLACE>
+__device__ __forceinline__ void fill_long_row(const Hop& h, int64_t s, int64_t i, int64_t row, int64_t b, uint32_t deg,
+                                              LongRowScratch& lds, const TableT& table, const TierView<IdT>& indices,
+                                              const TierView<float>& probs, uint64_t rng_seed) {
+  const bool look_first = look_before_insert(h, s);
+  const bool bucketed = bucketed_now(h, s);
+  const int k = h.k;
+  const int64_t p0 = h.pos_base + seed_part(h, s) + i * k;
+  if (REPLACE) {
+    draw_long_row(lds, probs, b, int64_t(deg), int64_t(k), rng_seed, h.rng_stream, row,
+                  [&](int64_t j, int64_t pick) {
+                    if (!emit_pick<IdT>(h, table, indices, p0 + j, true, b + pick, look_first, bucketed))
+                      h.row_cnt[i] = kBadPick;
+                  });
+  } else {
+    const uint32_t pos = race_long_row(lds, probs, b, deg, k, rng_seed, h.rng_stream, row);
+    const int l = threadIdx.x;  // wave 0 holds the winners
+    if (l < k && !emit_pick<IdT>(h, table, indices, p0 + l, pos < deg, b + pos, look_first, bucketed))
+      h.row_cnt[i] = kBadPick;
+  }
+}
+
 // Same layout of virtual blocks as hop_fill_kernel (fill, previous hop's edge list, clearing).
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void hop_fill_weighted_kernel(Hop h, Hop prev, int64_t fill_blocks,
@@ -670,9 +702,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
   const int64_t total = fill_blocks + relabel_count + clear_blocks;
   for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
     if (vb < fill_blocks) {
-      fill_rows_weighted<IdT, PtrT, TableT, REPLACE>(h, vb, table, indptr, indices, probs, rng_seed);
+      const int64_t s = seeds_of(h);
+      if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
+      const int lanes = weighted_row_lanes(h.k);
+      const int64_t first = (vb * (kBlock / kWave) + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave)))) * (kWave / lanes);
+      fill_wave_weighted<IdT, PtrT, TableT, REPLACE>(
+          h, s, first, lanes, long_row<kWave>(), table, indptr, indices, probs, rng_seed, [&](int64_t i, int64_t, uint32_t, IdT) {
+            h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = i;
+          });
     } else if (vb < fill_blocks + relabel_count) {
-      relabel_tile<IdT, TableT, false>(prev, table, vb - fill_blocks);  // always a striding launch
+      relabel_tile<IdT, TableT, false>(prev, table, vb - fill_blocks, threadIdx.x);  // always a striding launch
     } else {
       const int64_t i = (vb - fill_blocks - relabel_count) * kBlock + threadIdx.x;
       if (i < clear_n16) clear_begin[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -689,27 +728,56 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_long_kernel(Hop 
   __shared__ LongRowScratch lds;
   const int64_t n_long = *h.long_count;
   const int64_t s = seeds_of(h);
-  const bool look_first = look_before_insert(h, s);
-  const bool bucketed = bucketed_now(h, s);
-  const int k = h.k;
   for (int64_t t = blockIdx.x; t < n_long; t += gridDim.x) {
     const int64_t i = h.long_rows[t];
     const int64_t row = int64_t(static_cast<const IdT*>(h.seeds)[i]);
     const int64_t b = int64_t(indptr.at(row));
     const uint32_t deg = uint32_t(int64_t(indptr.at(row + 1)) - b);  // queued rows have a valid degree
-    const int64_t p0 = h.pos_base + seed_part(h, s) + i * k;
-    if (REPLACE) {
-      draw_long_row(lds, probs, b, int64_t(deg), int64_t(k), rng_seed, h.rng_stream, row,
-                    [&](int64_t j, int64_t pick) {
-                      if (!emit_pick<IdT>(h, table, indices, p0 + j, true, b + pick, look_first, bucketed))
-                        h.row_cnt[i] = kBadPick;
-                    });
+    fill_long_row<IdT, TableT, REPLACE>(h, s, i, row, b, deg, lds, table, indices, probs, rng_seed);
+  }
+}
+
+// A small hop: blocks [0, fill_blocks) have kLongWaves seed rows each; the blocks of the previous hop's
+// edge list and of the clearing, of kBlock threads elsewhere, are taken four at a time.
+template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
+__global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Hop h, Hop prev, int64_t fill_blocks,
+                                                                              int64_t relabel_count, uint4* clear_begin,
+                                                                              int64_t clear_n16, TableT table,
+                                                                              TierView<PtrT> indptr,
+                                                                              TierView<IdT> indices,
+                                                                              TierView<float> probs, uint64_t rng_seed) {
+  if (int64_t(blockIdx.x) >= fill_blocks) {
+    const int64_t vb = (int64_t(blockIdx.x) - fill_blocks) * (kLongBlock / kBlock) + threadIdx.x / kBlock;
+    const int tid = threadIdx.x & (kBlock - 1);
+    if (vb < relabel_count) {
+      relabel_tile<IdT, TableT, false>(prev, table, vb, tid);
     } else {
-      const uint32_t pos = race_long_row(lds, probs, b, deg, k, rng_seed, h.rng_stream, row);
-      const int l = threadIdx.x;  // wave 0 holds the winners
-      if (l < k && !emit_pick<IdT>(h, table, indices, p0 + l, pos < deg, b + pos, look_first, bucketed))
-        h.row_cnt[i] = kBadPick;
+      const int64_t i = (vb - relabel_count) * kBlock + tid;
+      if (i < clear_n16) clear_begin[i] = make_uint4(0u, 0u, 0u, 0u);
     }
+    return;
+  }
+  struct Listed { int64_t row, begin; uint32_t deg; int at; };
+  __shared__ LongRowScratch lds;
+  __shared__ Listed listed[kLongWaves];
+  __shared__ int n_listed;
+  const int64_t s = seeds_of(h);
+  const int64_t first = int64_t(blockIdx.x) * kLongWaves;
+  if (h.n_seeds_out && blockIdx.x == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
+  if (first >= s) return;  // whole blocks leave together
+  if (threadIdx.x == 0) n_listed = 0;
+  __syncthreads();
+  fill_wave_weighted<IdT, PtrT, TableT, REPLACE>(
+      h, s, first + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave))), kWave, kSharedRow, table, indptr, indices, probs,
+      rng_seed, [&](int64_t i, int64_t b, uint32_t deg, IdT seed) {
+        listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(seed), b, deg, int(i - first)};  // a wave lists at most its one row
+      });
+  __syncthreads();
+  const int n = n_listed;
+  for (int t = 0; t < n; ++t) {
+    const Listed r = listed[t];
+    fill_long_row<IdT, TableT, REPLACE>(h, s, first + int64_t(wave_uniform(uint32_t(r.at))), wave_uniform(r.row),
+                                        wave_uniform(r.begin), wave_uniform(r.deg), lds, table, indices, probs, rng_seed);
   }
 }
 
@@ -1215,7 +1283,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
 
 template <typename IdT, typename TableT, bool STRIDE>
 __global__ __launch_bounds__(kBlock) void hop_relabel_kernel(Hop h, int64_t blocks, TableT table) {
-  DGS_FOR_VIRTUAL_BLOCKS(vb, blocks) relabel_tile<IdT, TableT, !STRIDE>(h, table, vb);
+  DGS_FOR_VIRTUAL_BLOCKS(vb, blocks) relabel_tile<IdT, TableT, !STRIDE>(h, table, vb, threadIdx.x);
 }
 
 __global__ void zero_sizes_kernel(int64_t* __restrict__ sizes, int n) {
@@ -1440,15 +1508,25 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
                        TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
 }
 
-// The weighted fill of one hop: the main launch (a wave per row) and the block-per-row launch for
-// the rows it queued.  Only the direct table is supported (the entry point insists on one).
+// Whether a weighted hop is one launch of kLongBlock-thread blocks (see above).
+inline bool weighted_shared(const Hop& h) { return h.s_max <= kSharedMaxRows; }
+
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
 dgs_status launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin,
                                 int64_t clear_n16, const TableT& table, const dgs_view& indptr,
                                 const dgs_view& indices, const dgs_view& probs, uint64_t rng_seed, hipStream_t st) {
+  const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
+  if (weighted_shared(cur)) {
+    const int64_t fill_blocks = (cur.s_max + kLongWaves - 1) / kLongWaves;
+    const int64_t others = (relabel_count + clear_blocks + kLongBlock / kBlock - 1) / (kLongBlock / kBlock);
+    hipLaunchKernelGGL((hop_fill_weighted_shared_kernel<IdT, PtrT, TableT, REPLACE>), dim3(uint32_t(fill_blocks + others)),
+                       dim3(kLongBlock), 0, st, cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
+                       TierView<PtrT>(indptr), TierView<IdT>(indices), TierView<float>(probs), rng_seed);
+    DGS_LAUNCH_CHECK();
+    return DGS_OK;
+  }
   const int64_t rows_per_block = weighted_rows_per_block(cur.k);
   const int64_t fill_blocks = (cur.s_max + rows_per_block - 1) / rows_per_block;
-  const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
   const int64_t total = fill_blocks + relabel_count + clear_blocks;
   hipLaunchKernelGGL((hop_fill_weighted_kernel<IdT, PtrT, TableT, REPLACE>), dim3(capped_grid(total)), dim3(kBlock),
                      0, st, cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
@@ -1467,7 +1545,7 @@ template <typename IdT, typename PtrT, typename TableT>
 dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const TableT& table, const dgs_view& indptr,
                       const dgs_view& indices, const dgs_view* probs, bool replace, uint64_t rng_seed,
                       void** sizes_ticket, hipStream_t st) {
-  if (p.weighted) {  // the long-row queues of all hops start empty (their counters are one array, hop 0's first)
+  if (p.weighted && !weighted_shared(hops[0])) {  // the long-row queues of all hops start empty (their counters are one array, hop 0's first)
     hipLaunchKernelGGL(zero_sizes_kernel, dim3(1), dim3(64), 0, st, hops[0].long_count, p.n_hops);
     DGS_LAUNCH_CHECK();
   }
@@ -1483,6 +1561,8 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
       const Hop& last = hops[p.n_hops - 1];
       clear_begin = reinterpret_cast<uint4*>(cur.lost + (p.n_hops > 1 ? hops[1].pos_base : p.s_max[1] / 16 * 16));
       const char* end = reinterpret_cast<const char*>(last.pos_state + pos_tiles_of(last.len_max));  // (two spare words follow)
+      // (where hop 0 queues no rows itself, the queues' counters as well: they come next)
+      if (p.weighted && weighted_shared(cur)) end = reinterpret_cast<const char*>(cur.long_count + DGS_MAX_HOPS);
       clear_n16 = (end - reinterpret_cast<const char*>(clear_begin) + 15) / 16;
     }
     if (p.weighted) {

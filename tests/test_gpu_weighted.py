@@ -256,6 +256,30 @@ def test_weighted_fused_long_rows_and_wide_fanout(pkg, oracle, last_hop):
             assert np.array_equal(_np(g.src_local), w[0]) and np.array_equal(_np(g.dst_local), w[1])
 
 
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n_seeds", [1, 16, 17, 16384, 16385])
+def test_weighted_fused_small_and_large_hops(pkg, oracle, last_hop, n_seeds, replace):
+    # hops of up to 16384 rows are one launch whose 16-wave blocks share the rows of more than 512
+    # positions, larger ones two launches: row lengths around both limits, several long rows a block,
+    # a small hop in front of a large one
+    rng = np.random.default_rng(n_seeds)
+    deg = np.concatenate([[256, 257, 511, 512, 513, 4096, 4097, 2047, 2048, 2049, 0, 1], rng.integers(0, 40, size=3000)])
+    n = deg.size
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int64)
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    seeds = np.concatenate([np.arange(12), rng.integers(0, n, size=n_seeds)])[:n_seeds].astype(np.int64)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    for fanouts in ([5], [4, 18]):
+        pkg.set_rng_state(77, 1)
+        sampler = pkg.ChunkTensorSampler(fanouts, cts[0], cts[1], cts[2], replace)
+        f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
+        want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, 77, 1, probs=probs)
+        assert np.array_equal(_np(f), want_f), fanouts
+        for g, w in zip(blocks, want_blocks):
+            assert np.array_equal(_np(g.src_local), w[0]) and np.array_equal(_np(g.dst_local), w[1])
+
+
 def test_weighted_rows_that_the_key_halves_leave_open(pkg, oracle, last_hop):
     # the race first compares the upper 32 bits of the keys and repeats a row on full keys when
     # those tie where it matters: infinite weights (all keys 0), fewer usable weights than picks

@@ -4,20 +4,34 @@
 // 8-byte ids that may not fit 32 bits) maps each id to the smallest position at which it occurs.
 // The atomic that inserts a position tells whether it is, so far, its id's smallest and which
 // position it displaced (marked lost): a position is a "first occurrence" when it was smallest
-// at insertion and never lost.  Flags are scanned tile by tile, first occurrences are compacted
-// in input order (which is what makes the result independent of the table layout) and the
-// table value becomes the id's rank.  Every mapping id remembers its slot, so a tensor that
-// is both mapped and relabelled (the picked neighbours of the upstream sampler
-// loop) is not probed a second time.
+// at insertion and never lost.  First occurrences are counted, ranked and compacted in input order
+// (which is what makes the result independent of the table layout) by one launch whose blocks add
+// up the tiles before theirs (lookback.h), and the first occurrence's word becomes the id's rank.
+// Every mapping id remembers its slot, so a tensor that is both mapped and relabelled (the picked
+// neighbours of the upstream sampler loop) is not probed a second time.
+//
+// Launches: clear -> insert -> rank -> lookup.  The caller waits for the count that the third one
+// leaves, so every launch in front of it is 5 us of a short call.
 #include "common.h"
+#include "lookback.h"
 #include "table.h"
 
 namespace dgs {
 namespace {
 
 constexpr int kThreads = 256;
+// Positions of a rank block: kThreads x kItems (one vector load of words and one of lost marks per
+// thread) x GROUPS.  One group up to 1024 tiles, which the look-back reads in one go (890 k ids 10.6 us,
+// 418 k 7.2 us; with four groups, a quarter of the blocks, 13.5 and 11.8); four beyond.
 constexpr int kItems = 4;
-constexpr int kTileIds = kThreads * kItems;   // ids per block in flag / compact
+constexpr int kGroupIds = kThreads * kItems;
+constexpr int kLongGroups = 4;
+constexpr int64_t kLongIds = int64_t(1024) * kGroupIds;
+inline int rank_groups(int64_t n) { return n <= kLongIds ? 1 : kLongGroups; }
+inline int64_t rank_tiles(int64_t n) {
+  const int64_t tile = int64_t(kGroupIds) * rank_groups(n);
+  return (n + tile - 1) / tile;
+}
 constexpr uint32_t kFirstBit = 0x80000000u;   // marks a first occurrence in slot[]
 constexpr int64_t kMaxMappingIds = int64_t(1) << 30;
 // slot[] word of a mapping id the table could not take (the call's results are void then: the
@@ -75,69 +89,99 @@ __global__ __launch_bounds__(kThreads) void insert_kernel(dgs_segments mapping, 
   if (displaced != kNoPosition) lost[displaced] = 1;
 }
 
-__global__ __launch_bounds__(kThreads) void flag_kernel(int64_t n, uint32_t* __restrict__ slot,
-                                                        const uint8_t* __restrict__ lost, int* __restrict__ tile_cnt) {
-  __shared__ int lds[kThreads / kWave];
-  const int64_t base = int64_t(blockIdx.x) * kTileIds + threadIdx.x * kItems;
-  int c = 0;
+// First occurrences of one tile of mapping positions: counted, added to what the tiles before hold,
+// compacted into unique_out; a first occurrence's word then holds its rank.  The block of the last tile
+// leaves counts_dev[0] = number of distinct ids, [1] = 1 if an id did not fit the table (then everything
+// else the call wrote is void), mirrored into pinned host memory when the caller gave some.
+// The arrays slot[] and lost[] reach to the end of the last tile; what lies beyond n is read and
+// written back but never counts.
+template <typename IdT, int GROUPS>
+__global__ __launch_bounds__(kThreads) void rank_kernel(dgs_segments mapping, int64_t n, uint32_t* __restrict__ slot,
+                                                        const uint8_t* __restrict__ lost, tile_state* __restrict__ state,
+                                                        int32_t max_polls, const int* __restrict__ overflow,
+                                                        IdT* __restrict__ unique_out, int64_t* __restrict__ counts_dev,
+                                                        int64_t* __restrict__ counts_host) {
+  typedef uint32_t words __attribute__((ext_vector_type(kItems)));
+  constexpr int kWaves = kThreads / kWave;
+  constexpr int64_t kTileIds = int64_t(kGroupIds) * GROUPS;
+  __shared__ LookbackLds<kThreads> look;
+  __shared__ int wave_count[GROUPS * kWaves];
+  __shared__ int lds[kWaves];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int64_t tile = blockIdx.x;
+  const int64_t base = tile * kTileIds + threadIdx.x * kItems;
+  const bool last = (tile + 1) * kTileIds >= n;
+  const int64_t bad = last ? int64_t(*overflow != 0) : 0;
+  words word[GROUPS];
+  uint32_t marks[GROUPS];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const int64_t i = base + j;
-    if (i < n) {
-      const uint32_t s = slot[i];
-      if (s & kFirstBit) {
-        if (lost[i]) slot[i] = s & ~kFirstBit; else ++c;
-      }
-    }
+  for (int g = 0; g < GROUPS; ++g) {
+    word[g] = *reinterpret_cast<const words*>(slot + base + g * kGroupIds);
+    marks[g] = *reinterpret_cast<const uint32_t*>(lost + base + g * kGroupIds);
   }
-  int total;
-  block_exclusive_scan<kThreads, int>(c, &total, lds);
-  if (threadIdx.x == 0) tile_cnt[blockIdx.x] = total;
-}
-
-// counts_dev[0] = number of distinct ids, [1] = 1 if an id did not fit the table (then everything
-// else the call wrote is void); mirrored into pinned host memory when the caller gave some.
-__global__ __launch_bounds__(1024) void unique_scan_kernel(const int* __restrict__ tile_cnt,
-                                                           int* __restrict__ tile_off, int64_t tiles,
-                                                           const int* __restrict__ overflow,
-                                                           int64_t* __restrict__ counts_dev,
-                                                           int64_t* __restrict__ counts_host) {
-  int sum;
-  single_block_scan_1024<int>(tile_cnt, tile_off, tiles, &sum);
-  if (threadIdx.x == 0) {
-    const int64_t bad = *overflow != 0;
-    counts_dev[0] = sum;
+  uint32_t first[GROUPS];   // bit j: position j of the group's is its id's first
+  int lane_before[GROUPS];  // first positions in the lanes below, then in all of the tile before
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    first[g] = 0;
+#pragma unroll
+    for (int j = 0; j < kItems; ++j)
+      if (base + g * kGroupIds + j < n && (word[g][j] & kFirstBit) != 0 && ((marks[g] >> (8 * j)) & 0xffu) == 0) first[g] |= 1u << j;
+    const int c = __builtin_popcount(first[g]);  // its bits are summed over the lanes by ballots
+    lane_before[g] = 0;
+    int sum = 0;
+#pragma unroll
+    for (int bit = 0; (1 << bit) <= kItems; ++bit) {
+      const uint64_t at = __ballot((c >> bit) & 1);
+      lane_before[g] += __builtin_popcountll(at & ((uint64_t(1) << lane) - 1)) << bit;
+      sum += __builtin_popcountll(at) << bit;
+    }
+    if (lane == 0) wave_count[g * kWaves + wave] = sum;
+  }
+  __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int q = 0; q < GROUPS * kWaves; ++q) {
+    if (q % kWaves == wave) lane_before[q / kWaves] += total;
+    total += wave_count[q];
+  }
+  const tile_state before = tile_exclusive_prefix<kThreads, false>(state, tile, tile_word(total), max_polls, look, [&](int64_t t) {
+    int c = 0;  // (a tile before this one is full; a word counts the same before and after its block has rewritten it)
+    for (int j = 0; j < GROUPS * kItems; ++j) {
+      const int64_t p = t * kTileIds + int64_t(j) * kThreads + threadIdx.x;
+      c += (slot[p] & kFirstBit) != 0 && lost[p] == 0;
+    }
+    int sum;
+    block_exclusive_scan<kThreads, int>(c, &sum, lds);
+    return tile_word(sum);
+  });
+  const int64_t rank0 = tile_sum_of(before);
+  if (last && threadIdx.x == 0) {
+    counts_dev[0] = rank0 + total;
     counts_dev[1] = bad;
     if (counts_host) {
-      mirror_to_host(counts_host, sum);
+      mirror_to_host(counts_host, rank0 + total);
       mirror_to_host(counts_host + 1, bad);
     }
   }
-}
-
-template <typename IdT, typename TableT>
-__global__ __launch_bounds__(kThreads) void compact_kernel(dgs_segments mapping, int64_t n,
-                                                           uint32_t* __restrict__ slot,
-                                                           const int* __restrict__ tile_off,
-                                                           IdT* __restrict__ unique_out) {
-  __shared__ int lds[kThreads / kWave];
-  const int64_t base = int64_t(blockIdx.x) * kTileIds + threadIdx.x * kItems;
-  uint32_t s[kItems];
-  int c = 0;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    s[j] = base + j < n ? slot[base + j] : 0u;
-    c += (s[j] & kFirstBit) != 0;
-  }
-  int total;
-  int rank = tile_off[blockIdx.x] + block_exclusive_scan<kThreads, int>(c, &total, lds);
+  for (int g = 0; g < GROUPS; ++g) {
+    const int64_t p = base + g * kGroupIds;
+    uint32_t rank = uint32_t(rank0) + uint32_t(lane_before[g]);
+    bool changed = false;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    if (s[j] & kFirstBit) {
-      unique_out[rank] = seg_load<IdT>(mapping, base + j);
-      slot[base + j] = uint32_t(rank) | kFirstBit;  // a first occurrence's word now holds its rank
-      ++rank;
+    for (int j = 0; j < kItems; ++j) {
+      if ((first[g] >> j) & 1) {
+        unique_out[rank] = seg_load<IdT>(mapping, p + j);
+        word[g][j] = rank | kFirstBit;
+        ++rank;
+        changed = true;
+      } else if (((marks[g] >> (8 * j)) & 0xffu) != 0) {
+        word[g][j] &= ~kFirstBit;
+        changed = true;
+      }
     }
+    if (changed) *reinterpret_cast<words*>(slot + p) = word[g];
   }
 }
 
@@ -327,11 +371,10 @@ __global__ __launch_bounds__(kSmallThreads) void small_relabel_kernel(dgs_segmen
 
 struct UniqueWorkspace {
   void* table;       // capacity slots of the table layout in use
-  uint8_t* lost;     // [n + 16] then the overflow word: one region to zero
+  uint8_t* lost;     // [padded to whole rank tiles], then the rank tiles' states and the overflow word: one region to zero
+  tile_state* state;
   int* overflow;
-  uint32_t* slot;    // [n]
-  int* tile_cnt;
-  int* tile_off;
+  uint32_t* slot;    // [padded to whole rank tiles]
   uint32_t capacity;
   size_t table_bytes;  // multiple of 16 (sized for the larger layout)
   size_t zero_bytes;   // multiple of 16
@@ -343,18 +386,18 @@ size_t slot_bytes(int32_t id_bytes, bool packed) { return packed ? 8 : size_t(id
 size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWorkspace* w) {
   if (n < 0) n = 0;
   if (n > kMaxMappingIds) n = kMaxMappingIds;
-  const size_t tiles = size_t((n + kTileIds - 1) / kTileIds);
+  const size_t tiles = size_t(n > 0 ? rank_tiles(n) : 1);  // (an empty list has its counts written too)
+  const size_t padded = tiles * size_t(kGroupIds) * rank_groups(n);
   Carver c(base);
   UniqueWorkspace t;
   t.capacity = table_capacity(n);
   t.table_bytes = size_t(t.capacity) * slot_bytes(id_bytes, id_bytes == 4);
   t.table = c.take<char>(t.table_bytes);
-  t.zero_bytes = (size_t(n) + 16 + sizeof(int) + 15) / 16 * 16;
+  t.zero_bytes = (padded + tiles * sizeof(tile_state) + sizeof(int) + 15) / 16 * 16;
   t.lost = c.take<uint8_t>(t.zero_bytes);
-  t.overflow = reinterpret_cast<int*>(t.lost + (size_t(n) + 16) / 16 * 16);
-  t.slot = c.take<uint32_t>(size_t(n));
-  t.tile_cnt = c.take<int>(tiles);
-  t.tile_off = c.take<int>(tiles);
+  t.state = reinterpret_cast<tile_state*>(t.lost + padded);
+  t.overflow = reinterpret_cast<int*>(t.state + tiles);
+  t.slot = c.take<uint32_t>(padded);
   if (w) *w = t;
   return c.used + 256;
 }
@@ -375,26 +418,23 @@ dgs_status run_unique_relabel(const dgs_segments& mapping, int64_t n, const dgs_
   hipLaunchKernelGGL(clear_kernel, dim3(uint32_t((table16 + zeros16 + kThreads - 1) / kThreads)), dim3(kThreads), 0,
                      st, static_cast<uint4*>(w.table), table16, reinterpret_cast<uint4*>(w.lost), zeros16);
   DGS_LAUNCH_CHECK();
-  const int64_t tiles = (n + kTileIds - 1) / kTileIds;
   if (n > 0) {
     hipLaunchKernelGGL((insert_kernel<IdT, TableT>), dim3(uint32_t((n + kThreads - 1) / kThreads)), dim3(kThreads),
                        0, st, mapping, n, table, w.slot, w.lost, w.overflow);
     DGS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(flag_kernel, dim3(uint32_t(tiles)), dim3(kThreads), 0, st, n, w.slot, w.lost, w.tile_cnt);
-    DGS_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(unique_scan_kernel, dim3(1), dim3(1024), 0, st, w.tile_cnt, w.tile_off, tiles, w.overflow,
-                     counts_dev, counts_host);
+  const dim3 tiles(uint32_t(n > 0 ? rank_tiles(n) : 1));
+  if (rank_groups(n) == 1)
+    hipLaunchKernelGGL((rank_kernel<IdT, 1>), tiles, dim3(kThreads), 0, st, mapping, n, w.slot, w.lost, w.state,
+                       lookback_polls(), w.overflow, static_cast<IdT*>(unique_out), counts_dev, counts_host);
+  else
+    hipLaunchKernelGGL((rank_kernel<IdT, kLongGroups>), tiles, dim3(kThreads), 0, st, mapping, n, w.slot, w.lost, w.state,
+                       lookback_polls(), w.overflow, static_cast<IdT*>(unique_out), counts_dev, counts_host);
   DGS_LAUNCH_CHECK();
   // the counts are final here: mark the point the caller may wait for
   if (ticket) {
     const dgs_status ts = dgs_ticket_record(st, ticket);
     if (ts != DGS_OK) return ts;
-  }
-  if (n > 0) {
-    hipLaunchKernelGGL((compact_kernel<IdT, TableT>), dim3(uint32_t(tiles)), dim3(kThreads), 0, st, mapping, n,
-                       w.slot, w.tile_off, static_cast<IdT*>(unique_out));
-    DGS_LAUNCH_CHECK();
   }
   if (m > 0) {
     SegmentAlias alias;

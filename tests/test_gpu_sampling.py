@@ -794,6 +794,28 @@ def test_fused_sampler_whose_tiles_do_not_wait_for_each_other(pkg, oracle, graph
         _check_blocks(blocks, want_blocks)
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [2049, 3072, 3073, 1 << 20, (1 << 20) + 1, (1 << 20) + 4097])
+def test_unique_relabel_at_the_edges_of_its_tiles(pkg, oracle, dtype, n, request):
+    # lists that end with a tile, one position behind it, and where the tile gets longer; every block
+    # counts the tiles before its own itself (polls 1) or learns their counts from their blocks
+    capi = pkg.capi
+    rng = np.random.default_rng(n)
+    seeds = rng.integers(0, n, size=n // 3).astype(dtype)
+    cols = rng.integers(0, n, size=n - seeds.size).astype(dtype)
+    rows = rng.choice(seeds, size=cols.size).astype(dtype)
+    want_u, want_outs = oracle.unique_relabel([seeds, cols], [rows, cols])
+    d_cols = _dev(cols)
+    request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, 0))
+    for polls in (0, 1):
+        capi.check(capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, polls))
+        for packed in (True, False):
+            u, outs = capi.unique_relabel([_dev(seeds), d_cols], [_dev(rows), d_cols], packed_table=packed)
+            assert np.array_equal(_np(u), want_u), (polls, packed)
+            for a, b in zip(outs, want_outs):
+                assert np.array_equal(_np(a), b), (polls, packed)
+
+
 def test_unique_relabel_ids_beyond_32_bits(pkg, oracle):
     # 8-byte ids are first tried in one-word table slots; an id of 2^32 - 1 or more sends the call
     # to the two-array table.  Ids that only differ above bit 31 must not be confused, present or not.

@@ -75,6 +75,7 @@ struct Table<IdT, true> {
         if (cur == kEmpty) { *first = true; return pos; }
       }
       if (uint32_t(cur >> 32) == uint32_t(key)) {
+        if (cur < packed) { *first = false; return pos; }  // (it only ever gets smaller: no atomic needed)
         const unsigned long long old = atomicMin(slots + pos, packed);
         *first = old > packed;
         if (*first) *displaced = uint32_t(old);

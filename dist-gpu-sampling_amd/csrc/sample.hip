@@ -7,8 +7,8 @@
 //   scan  : one block turns the tile totals into tile offsets and the edge count;
 //   fill  : num_picks <= 64: a group of G lanes per seed row over the whole grid (G = 8..64,
 //           the smallest power of two holding num_picks), so a wave64 serves 64/G rows;
-//           larger num_picks: one wave per row, Floyd's kept set in LDS (num_picks <= 2048) or
-//           in the row's own output slots (any num_picks).
+//           larger num_picks: one wave per row, Floyd's candidates in an LDS table (num_picks <=
+//           2048) or his kept set in the row's own output slots (any num_picks).
 // Random picks follow the "dgs-philox-1" contract: every (seed, stream, row, draw) names one
 // Philox block, so results do not depend on the launch shape.
 #include <mutex>
@@ -49,7 +49,7 @@ dgs_status static_scratch_of(void** out) {
 }
 
 constexpr int kMaxGroupPicks = 64;   // fill_group_kernel handles num_picks <= 64
-constexpr int kMaxLdsPicks = 2048;   // fill_wave_kernel keeps Floyd's set in LDS
+constexpr int kMaxLdsPicks = 2048;   // fill_wave_kernel keeps Floyd's candidates in LDS
 constexpr int kFlagDegree = 1;       // some row has degree >= 2^32, or offsets outside the edge array
 constexpr int kFlagSeed = 2;         // some seed id is not a row of the graph
 
@@ -134,61 +134,118 @@ __global__ __launch_bounds__(kTile) void fill_group_kernel(
   out_cols[o] = indices.at(row_start[i] + pos);
 }
 
-// Any num_picks: one wave per row, lanes stride over the slots; Floyd's kept set lives in LDS
-// (num_picks <= kMaxLdsPicks; the launcher sends larger requests to fill_wave_global_kernel).
+// LDS words of one wave of fill_wave_kernel for rows longer than k: the candidates of the slots, the
+// table that tells which slot drew a candidate first (less than half full), a bit per slot.
+__host__ __device__ __forceinline__ int floyd_table_slots(int k) {
+  int c = 128;
+  while (c < 2 * k) c <<= 1;
+  return c;
+}
+__host__ __device__ __forceinline__ int floyd_bit_words(int k) { return (k + 31) / 32 + 1; }
+inline size_t floyd_lds_bytes(int k) {
+  return (size_t(k) + size_t(floyd_table_slots(k)) + size_t(floyd_bit_words(k) + 1) / 2 * 2) * sizeof(uint32_t);
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// kMaxGroupPicks < num_picks <= kMaxLdsPicks: one wave per row, lanes stride over the slots.
+// Rows longer than num_picks: no walk over the slots (see pick_position, whose rule this is).  All
+// candidates go into an open-addressing table whose entries name a slot, the lowest one that drew the
+// entry's candidate; then 64 slots at a time, in order, ask the table whether a lower slot drew theirs
+// and follow the links to substitutes among the slots already settled.  Bound: LDS latency, about a
+// dozen trips per 64 slots.  Slot after slot, every candidate compared with all kept before it, it was
+// num_picks trips per row: 13.3 k rows of mean degree 50 at num_picks 100 took 32.3 us, and 9.4 now.
 template <typename IdT>
 __global__ __launch_bounds__(kTile) void fill_wave_kernel(
     const IdT* __restrict__ seeds, int64_t n_seeds, const int64_t* __restrict__ row_start,
     const uint32_t* __restrict__ row_deg, const int64_t* __restrict__ row_off,
-    const int64_t* __restrict__ tile_off, TierView<IdT> indices, int64_t k, bool replace, uint64_t rng_seed,
-    uint32_t rng_stream, IdT* __restrict__ out_rows, IdT* __restrict__ out_cols) {
-  extern __shared__ uint32_t kept_lds[];  // (kTile / kWave) * min(k, kMaxLdsPicks) entries
+    const int64_t* __restrict__ tile_off, TierView<IdT> indices, int k, bool replace, uint64_t rng_seed,
+    uint32_t rng_stream, int lds_words, IdT* __restrict__ out_rows, IdT* __restrict__ out_cols) {
+  extern __shared__ uint32_t floyd_lds[];  // lds_words for every wave of the block
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t i = int64_t(blockIdx.x) * (kTile / kWave) + wave;
+  const int64_t i = int64_t(blockIdx.x) * (blockDim.x / kWave) + wave;
   if (i >= n_seeds) return;  // whole waves leave together
-  const int64_t kk = k < kMaxLdsPicks ? k : kMaxLdsPicks;
-  uint32_t* kept = kept_lds + int64_t(wave) * kk;
   const int64_t start = row_start[i];
   const int64_t off = tile_off[i / kTile] + row_off[i];
   const int64_t row = int64_t(seeds[i]);
   const uint32_t deg = row_deg[i];
   if (replace) {
     if (deg > 0) {
-      for (int64_t s = lane; s < k; s += kWave) {
+      for (int s = lane; s < k; s += kWave) {
         const uint32_t p = philox_bounded(rng_seed, rng_stream, row, uint32_t(s), deg);
         out_rows[off + s] = IdT(row);
         out_cols[off + s] = indices.at(start + p);
       }
     }
-  } else if (int64_t(deg) <= k) {
+  } else if (deg <= uint32_t(k)) {
     for (uint32_t s = lane; s < deg; s += kWave) {
       out_rows[off + s] = IdT(row);
       out_cols[off + s] = indices.at(start + s);
     }
   } else {
-    // Floyd, 64 candidates at a time; each is checked against everything kept so far
+    constexpr uint32_t kNoSlot = 0xffffffffu;
     const uint32_t base_top = deg - uint32_t(k);
-    for (int s0 = 0; s0 < int(k); s0 += kWave) {
-      const int s = s0 + lane;
-      uint32_t cand = 0xffffffffu;
-      if (s < k) cand = philox_bounded(rng_seed, rng_stream, row, uint32_t(s), base_top + s + 1u);
-      const int batch = int(k) - s0 < kWave ? int(k) - s0 : kWave;
-      for (int b = 0; b < batch; ++b) {
-        const uint32_t c = __shfl(cand, b, kWave);
-        const int slot = s0 + b;
-        bool hit = false;
-        for (int q = lane; q < slot; q += kWave) hit |= kept[q] == c;
-        const bool any = __ballot(hit) != 0;
-        if (lane == 0) kept[slot] = any ? base_top + uint32_t(slot) : c;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int cap = floyd_table_slots(k);
+    uint32_t* taken_bits = floyd_lds + wave * lds_words;            // word pairs: 64 slots each
+    uint32_t* table = taken_bits + (floyd_bit_words(k) + 1) / 2 * 2;
+    uint32_t* drawn = table + cap;                                  // [k] candidates
+    for (int q = lane; q < cap; q += kWave) table[q] = kNoSlot;
+    for (int s = lane; s < k; s += kWave)
+      drawn[s] = philox_bounded(rng_seed, rng_stream, row, uint32_t(s), base_top + uint32_t(s) + 1u);
+    wave_lds_fence();
+    // an entry goes from empty to a slot and then only down among slots of the same candidate, so the
+    // candidate that an entry stands for never changes
+    for (int s = lane; s < k; s += kWave) {
+      const uint32_t c = drawn[s];
+      uint32_t q = (c * 0x9E3779B1u) >> 7 & uint32_t(cap - 1);
+      for (;;) {  // ends: the table has more entries than there are candidates
+        const uint32_t held = atomicCAS(&table[q], kNoSlot, uint32_t(s));
+        if (held == kNoSlot) break;
+        if (drawn[held] == c) {
+          atomicMin(&table[q], uint32_t(s));
+          break;
+        }
+        q = (q + 1) & uint32_t(cap - 1);
       }
     }
-    for (int64_t s = lane; s < k; s += kWave) {
-      out_rows[off + s] = IdT(row);
-      out_cols[off + s] = indices.at(start + kept[s]);
+    wave_lds_fence();
+    for (int s0 = 0; s0 < k; s0 += kWave) {
+      const int s = s0 + lane;
+      bool drawn_before = false, linked = false, settled = false;
+      uint32_t c = 0, link = 0;
+      if (s < k) {
+        c = drawn[s];
+        uint32_t q = (c * 0x9E3779B1u) >> 7 & uint32_t(cap - 1);
+        uint32_t held;
+        while (drawn[held = table[q]] != c) q = (q + 1) & uint32_t(cap - 1);  // every candidate is in the table
+        drawn_before = held < uint32_t(s);
+        link = c - base_top;  // the slot whose substitute this candidate is (if below s)
+        linked = link < uint32_t(s);
+        if (linked && link < uint32_t(s0)) {  // a slot settled in an earlier round
+          settled = (taken_bits[link / 32] >> (link & 31) & 1u) != 0;
+          linked = false;
+        }
+      }
+      const bool known = drawn_before || settled;
+      bool taken = known;
+      uint64_t all = __ballot(taken);
+      for (;;) {
+        taken = known || (linked && (all >> (link - uint32_t(s0) & 63u) & 1) != 0);
+        const uint64_t now = __ballot(taken);
+        if (now == all) break;  // marks are only ever added: at most 64 rounds
+        all = now;
+      }
+      if (lane < 2) taken_bits[s0 / 32 + lane] = uint32_t(all >> (32 * lane));
+      wave_lds_fence();
+      if (s < k) {
+        out_rows[off + s] = IdT(row);
+        out_cols[off + s] = indices.at(start + (taken ? base_top + uint32_t(s) : c));
+      }
     }
   }
 }
@@ -310,13 +367,13 @@ dgs_status run_fill(const void* seeds, int64_t n_seeds, const dgs_view& indices,
                        TierView<IdT>(indices), k, replace, rng_seed, rng_stream, static_cast<IdT*>(out_rows),
                        static_cast<IdT*>(out_cols));
   } else {
-    const int64_t kk = k;
-    const size_t lds = replace ? 0 : size_t(kTile / kWave) * size_t(kk) * sizeof(uint32_t);
-    const int64_t blocks = (n_seeds + kTile / kWave - 1) / (kTile / kWave);
-    hipLaunchKernelGGL((fill_wave_kernel<IdT>), dim3(uint32_t(blocks)), dim3(kTile), lds, st,
+    const size_t lds = replace ? 0 : floyd_lds_bytes(int(k));
+    const int waves = lds > 16384 ? 2 : kTile / kWave;  // a block's LDS stays within 64 KB
+    const int64_t blocks = (n_seeds + waves - 1) / waves;
+    hipLaunchKernelGGL((fill_wave_kernel<IdT>), dim3(uint32_t(blocks)), dim3(waves * kWave), lds * waves, st,
                        static_cast<const IdT*>(seeds), n_seeds, w.row_start, w.row_deg, w.row_off, w.tile_off,
-                       TierView<IdT>(indices), k, replace, rng_seed, rng_stream, static_cast<IdT*>(out_rows),
-                       static_cast<IdT*>(out_cols));
+                       TierView<IdT>(indices), int(k), replace, rng_seed, rng_stream, int(lds / sizeof(uint32_t)),
+                       static_cast<IdT*>(out_rows), static_cast<IdT*>(out_cols));
   }
   DGS_LAUNCH_CHECK();
   return DGS_OK;

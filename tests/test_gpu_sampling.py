@@ -117,6 +117,25 @@ def test_sample_any_fanout_without_replacement(pkg, oracle, id_dtype):
     assert r.numel() == sum(min(int(deg[s]), 3000) for s in seeds)
 
 
+@pytest.mark.parametrize("k", [65, 127, 128, 129, 1000, 1023, 1025, 2048])
+def test_sample_wide_fanouts_without_replacement(pkg, oracle, k):
+    # fanouts of the wave-per-row fill: a slot behind a whole stretch of 64, tables at a power of two and
+    # above, blocks of four and of two waves; rows barely longer than the fanout settle most slots by
+    # links to lower ones
+    capi = pkg.capi
+    deg = np.array([k - 1, k, k + 1, k + 2, k + 64, 2 * k, 0, 50 * k, 1], dtype=np.int64)
+    indptr = np.zeros(deg.size + 1, dtype=np.int64)
+    indptr[1:] = np.cumsum(deg)
+    indices = np.arange(int(indptr[-1]), dtype=np.int32)
+    seeds = np.tile(np.arange(deg.size, dtype=np.int32), 7)
+    ip, ix = _dev(indptr), _dev(indices)
+    for stream in range(4):
+        want_r, want_c = oracle.sample_neighbors(seeds, indptr, indices, k, False, 0x5EED, stream)
+        r, c, flags = capi.sample_neighbors(_dev(seeds), capi.tensor_view(ip), capi.tensor_view(ix), k, False, 0x5EED, stream)
+        assert flags == 0
+        assert np.array_equal(_np(r), want_r) and np.array_equal(_np(c), want_c), stream
+
+
 def test_seed_ids_outside_the_graph_are_refused(pkg, oracle, graph, last_hop):
     # a seed id is checked before it addresses indptr: its row emits nothing, the call is flagged,
     # the operators raise

@@ -46,6 +46,7 @@
 
 #include "common.h"
 #include "lookback.h"
+#include "one_block.h"
 #include "picks.h"
 #include "race.h"
 #include "table.h"
@@ -1605,10 +1606,47 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
   return DGS_OK;
 }
 
+// Whether the call is one launch of one block (one_block.h): the more launches that saves, the more
+// positions one CU may work through.  us per batch, one block against the launches: one hop, 780
+// positions 52.9 / 54.7, 2028 56.5 / 55.7; two hops, 1056 64.3 / 68.8, 2046 66.4 / 68.8, 4092 74.0 / 70.3;
+// three hops, 1536 74.2 / 84.5, 3840 82.3 / 86.1.
+inline bool one_block_fits(const Plan& p) {
+  const int64_t limit = std::min<int64_t>(kOnePositions, int64_t(1024) * p.n_hops);
+  return !p.weighted && p.kind != TableKind::kSplit && p.s_max[p.n_hops] <= limit &&
+         debug_option(DGS_DEBUG_SAMPLER_BUCKETED) == 0 && debug_option(DGS_DEBUG_SAMPLER_GRID_CAP) == 0 &&
+         debug_option(DGS_DEBUG_LOOKBACK_POLLS) == 0;  // (test hooks of the launches it replaces)
+}
+
+template <typename IdT, typename PtrT>
+dgs_status run_one_block(const Plan& p, const Hop* hops, int64_t* sizes, const dgs_view& indptr, const dgs_view& indices,
+                         bool replace, uint64_t rng_seed, void** sizes_ticket, hipStream_t st) {
+  OneBlockBatch q{};
+  q.seeds = hops[0].seeds;
+  q.n_seeds = p.s_max[0];
+  q.frontier = hops[0].frontier;
+  q.sizes = sizes;
+  q.host_sizes = hops[0].host_sizes;
+  q.id_limit = p.kind == TableKind::kDirect ? uint64_t(indptr.total - 1) : 0xffffffffull;  // what the table would hold
+  q.rng_seed = rng_seed;
+  q.first_stream = hops[0].rng_stream;
+  q.n_hops = p.n_hops;
+  q.replace = replace;
+  for (int h = 0; h < p.n_hops; ++h) {
+    q.k[h] = hops[h].k;
+    q.src_local[h] = hops[h].src_local;
+    q.dst_local[h] = hops[h].dst_local;
+  }
+  hipLaunchKernelGGL((one_block_kernel<IdT, PtrT>), dim3(1), dim3(kOneBlock), 0, st, q, TierView<PtrT>(indptr), TierView<IdT>(indices));
+  DGS_LAUNCH_CHECK();
+  return sizes_ticket ? dgs_ticket_record(st, sizes_ticket) : DGS_OK;
+}
+
 template <typename IdT, typename PtrT>
 dgs_status run_blocks_table(const Plan& p, Hop* hops, const Buckets& buckets, void* hash_table, void* node_table,
                             uint32_t epoch, const dgs_view& indptr, const dgs_view& indices, const dgs_view* probs,
                             bool replace, uint64_t rng_seed, void** sizes_ticket, hipStream_t st) {
+  if (one_block_fits(p))
+    return run_one_block<IdT, PtrT>(p, hops, hops[0].n_seeds_out, indptr, indices, replace, rng_seed, sizes_ticket, st);
   if (p.kind == TableKind::kDirect)
     return run_blocks<IdT, PtrT, DirectTable<IdT>>(p, hops, buckets, DirectTable<IdT>(node_table, epoch, uint32_t(indptr.total - 1)),
                                                    indptr, indices, probs, replace, rng_seed, sizes_ticket, st);

@@ -813,6 +813,32 @@ def test_fused_sampler_whose_tiles_do_not_wait_for_each_other(pkg, oracle, graph
         _check_blocks(blocks, want_blocks)
 
 
+@pytest.mark.parametrize("id_dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("replace", [False, True])
+def test_fused_sampler_in_one_block(pkg, oracle, id_dtype, replace, request):
+    # batches of up to 1024 positions a hop and 4096 in all are one launch, larger ones a chain of launches: the
+    # smallest, the largest that fit, the next ones, every group width, eight hops; the launches give the same (mode 1)
+    capi = pkg.capi
+    rng = np.random.default_rng(77)
+    indptr, indices = powerlaw_graph(rng, 3000, 12, 700, id_dtype=id_dtype)
+    indices[::3] = indices[::3] % 20  # ids that come up again and again
+    ip_ct = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix_ct = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_BUCKETED, 0))
+    for n, fanouts in [(1, [1]), (1, [64]), (16, [63]), (17, [63]), (8, [15, 15]), (9, [15, 15]), (3, [15, 7, 7]),
+                       (4, [15, 7, 7]), (16, [1] * 8), (17, [1] * 8), (512, [1]), (31, [32]), (60, [16]), (113, [8]),
+                       (30, [10, 5]), (5, [3, 20, 9]), (6, [4, 0, 30])]:
+        seeds = rng.integers(0, 3000, size=n).astype(id_dtype)
+        seeds[n // 2:] = seeds[:n - n // 2]  # (each twice)
+        want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, 5, 0)
+        for mode in (0, 1):
+            capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_BUCKETED, mode))
+            sampler = pkg.ChunkTensorSampler(fanouts, ip_ct, ix_ct, replace=replace, seed=5)
+            f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
+            assert np.array_equal(_np(f), want_f), (n, fanouts, mode)
+            _check_blocks(blocks, want_blocks)
+
+
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
 @pytest.mark.parametrize("n", [2049, 3072, 3073, 1 << 20, (1 << 20) + 1, (1 << 20) + 4097])
 def test_unique_relabel_at_the_edges_of_its_tiles(pkg, oracle, dtype, n, request):

@@ -83,6 +83,24 @@ torch::Tensor device_bytes(size_t n, const torch::Device& dev) {
   return torch::empty({static_cast<int64_t>(n)}, torch::TensorOptions().dtype(torch::kUInt8).device(dev));
 }
 
+// `count` elements of `type` that begin `at` bytes into the storage of `owner` (at its very beginning
+// when at = 0), as a 1-d tensor that shares it.  Made without an operator call: narrow and view cost
+// 1 us each, and a batch hands out three pieces a hop.
+torch::Tensor piece_of(const torch::Tensor& owner, int64_t at, int64_t count, c10::ScalarType type) {
+  torch::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(owner.storage()), owner.key_set(),
+                                                             c10::scalarTypeToTypeMeta(type));
+  t.unsafeGetTensorImpl()->set_storage_offset(at / static_cast<int64_t>(c10::elementSize(type)));
+  t.unsafeGetTensorImpl()->set_sizes_contiguous({count});
+  return t;
+}
+
+// A tensor that nobody else holds yet, cut to its first `count` rows in place.
+void keep_rows(const torch::Tensor& fresh, int64_t count) {
+  std::vector<int64_t> sizes = fresh.sizes().vec();
+  sizes[0] = count;
+  fresh.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+}
+
 // Blocking read of a few int64 values from the device through a pinned buffer.
 std::vector<int64_t> read_back(const torch::Tensor& dev, int64_t count) {
   thread_local torch::Tensor pinned =
@@ -440,7 +458,9 @@ std::tuple<torch::Tensor, torch::Tensor> sample_impl(const torch::Tensor& seeds_
                             rows.data_ptr(), cols.data_ptr(), ws.data_ptr(), ws_bytes, st));
   }
   check_sampling_flags(len[1], "sample_neighbors", -1);
-  return std::make_tuple(rows.narrow(0, 0, len[0]), cols.narrow(0, 0, len[0]));
+  keep_rows(rows, len[0]);
+  keep_rows(cols, len[0]);
+  return std::make_tuple(rows, cols);
 }
 
 // upstream RowWiseSamplingUniformCUDA (src/cuda/rowwise_sampling.cu:176-187)
@@ -608,7 +628,14 @@ std::tuple<torch::Tensor, std::vector<torch::Tensor>> TensorRelabel(std::vector<
     if (counts_host[1] == 0) break;
     TORCH_CHECK(packed != 0, "tensor_relabel: the table rejected an id");
   }
-  return std::make_tuple(unique.narrow(0, 0, u), relabelled.split_with_sizes(sizes, 0));
+  keep_rows(unique, u);
+  std::vector<torch::Tensor> parts;
+  int64_t at = 0;
+  for (const int64_t size : sizes) {
+    parts.push_back(piece_of(relabelled, at, size, dt));
+    at += size * w;
+  }
+  return std::make_tuple(unique, parts);
 }
 
 using BlocksResult = std::tuple<std::vector<torch::Tensor>, std::vector<torch::Tensor>, std::vector<torch::Tensor>,
@@ -641,30 +668,31 @@ class PendingBlocks : public torch::CustomClassHolder {
     const int n_sizes = 3 * hops_ + 1;
     for (int i = 0; i < n_sizes; ++i) TORCH_CHECK(sizes_host[i] >= 0, "sample_blocks: the kernels left no lengths");
     const std::vector<int64_t> sz(sizes_host, sizes_host + n_sizes);
-    std::vector<torch::Tensor> frontier(hops_);
+    std::vector<torch::Tensor> frontier(hops_), src(hops_), dst(hops_);
+    const c10::ScalarType id_type = seeds_.scalar_type();
     for (int h = 0; h < hops_; ++h) {
       check_sampling_flags(sz[2 * hops_ + 1 + h], "sample_blocks", h);
-      frontier[h] = all_.narrow(0, 0, sz[h + 1]);
-      src_[h] = src_[h].narrow(0, 0, sz[hops_ + 1 + h]);
-      dst_[h] = dst_[h].narrow(0, 0, sz[hops_ + 1 + h]);
+      frontier[h] = all_.first(sz[h + 1], id_type);
+      src[h] = src_[h].first(sz[hops_ + 1 + h], id_type);
+      dst[h] = dst_[h].first(sz[hops_ + 1 + h], id_type);
     }
     if (indptr_) indptr_->set_frontier_hint(sz[hops_]);
     if (features_) {
       const int64_t rows = sz[hops_];
       if (rows <= x_rows_) {
-        x_ = x_.narrow(0, 0, rows);
+        keep_rows(x_, rows);
       } else {
         // the frontier did not fit the capped buffer and the gather enqueued behind the last hop
         // wrote nothing: gather now into exactly `rows` rows, on the stream the batch was begun on
         // (the lengths are final, so the frontier is complete)
         const c10::StreamGuard on_begin_stream(stream_);
         x_ = torch::empty({rows, features_->elem_stride()}, x_.options());
-        check(dgs_gather_rows(features_->view(), features_->elem_stride(), all_.data_ptr(), width_, rows,
+        check(dgs_gather_rows(features_->view(), features_->elem_stride(), all_.data(), width_, rows,
                               x_.data_ptr(), DGS_TIER_ANY, features_->bad_index_word(), current_stream()));
         gathered_late_ = true;
       }
     }
-    return std::make_tuple(frontier, src_, dst_, features_ ? x_ : torch::empty({0}, seeds_.options()), seeds_);
+    return std::make_tuple(frontier, src, dst, features_ ? x_ : torch::empty({0}, seeds_.options()), seeds_);
   }
 
   static c10::intrusive_ptr<PendingBlocks> Begin(const torch::Tensor& seeds_in,
@@ -736,32 +764,30 @@ class PendingBlocks : public torch::CustomClassHolder {
     // allocator no longer matter and separate blocks are reused more freely: C4, whose worst case
     // is 511 MB of ids per batch, ran 4 % slower out of one block)
     constexpr int64_t kOneBlockBytes = int64_t(128) << 20;
-    torch::Tensor sizes_dev;
+    int64_t* sizes_dev = nullptr;
     if (carved <= kOneBlockBytes) {
-      torch::Tensor block = device_bytes(static_cast<size_t>(carved), dev);
-      const auto ids_of = [&](int64_t at, int64_t count) {
-        return block.narrow(0, at, count * w).view(p->seeds_.scalar_type());
-      };
-      p->all_ = ids_of(all_at, seeds_max[hops]);
+      const torch::Tensor block = device_bytes(static_cast<size_t>(carved), dev);
+      p->all_ = Piece{block, all_at};
       for (int h = 0; h < hops; ++h) {
-        p->src_[h] = ids_of(src_at[h], edges_max[h]);
-        p->dst_[h] = ids_of(dst_at[h], edges_max[h]);
+        p->src_[h] = Piece{block, src_at[h]};
+        p->dst_[h] = Piece{block, dst_at[h]};
       }
-      sizes_dev = block.narrow(0, sizes_at, n_sizes * 8).view(torch::kInt64);
+      sizes_dev = static_cast<int64_t*>(Piece{block, sizes_at}.data());
       p->owned_.push_back(block);
     } else {
-      p->all_ = torch::empty({seeds_max[hops]}, opt);
-      p->owned_.push_back(p->all_);
+      const auto own = [&](const torch::Tensor& t) {
+        p->owned_.push_back(t);
+        return Piece{t, 0};
+      };
+      p->all_ = own(torch::empty({seeds_max[hops]}, opt));
       for (int h = 0; h < hops; ++h) {
-        p->src_[h] = torch::empty({edges_max[h]}, opt);
-        p->dst_[h] = torch::empty({edges_max[h]}, opt);
-        p->owned_.push_back(p->src_[h]);
-        p->owned_.push_back(p->dst_[h]);
+        p->src_[h] = own(torch::empty({edges_max[h]}, opt));
+        p->dst_[h] = own(torch::empty({edges_max[h]}, opt));
       }
-      sizes_dev = torch::empty({n_sizes}, opt.dtype(torch::kInt64));
-      p->owned_.push_back(sizes_dev);  // (kept with the batch: the kernels write it after this call returns)
+      // (kept with the batch: the kernels write it after this call returns)
+      sizes_dev = static_cast<int64_t*>(own(torch::empty({n_sizes}, opt.dtype(torch::kInt64))).data());
     }
-    for (int h = 0; h < hops; ++h) outs[h] = dgs_block_out{p->src_[h].data_ptr(), p->dst_[h].data_ptr()};
+    for (int h = 0; h < hops; ++h) outs[h] = dgs_block_out{p->src_[h].data(), p->dst_[h].data()};
     const size_t ws_bytes = probs ? dgs_sample_blocks_weighted_workspace_bytes(n, fanouts.data(), hops, w)
                                   : dgs_sample_blocks_workspace_bytes(n, fanouts.data(), hops, w);
     torch::Tensor ws = device_bytes(ws_bytes, dev);  // freed on return: the allocator reuses it in stream order
@@ -774,12 +800,12 @@ class PendingBlocks : public torch::CustomClassHolder {
     if (probs)
       check(dgs_sample_blocks_weighted(p->seeds_.data_ptr(), w, n, indptr->view(), indices->view(), probs->view(),
                                        fanouts.data(), hops, replace, rng.first, rng.second, table.first,
-                                       table.second, p->all_.data_ptr(), outs.data(), sizes_dev.data_ptr<int64_t>(),
+                                       table.second, p->all_.data(), outs.data(), sizes_dev,
                                        p->pinned_.data_ptr<int64_t>(), nullptr, ws.data_ptr(), ws_bytes, st));
     else
       check(dgs_sample_blocks(p->seeds_.data_ptr(), w, n, indptr->view(), indices->view(), fanouts.data(), hops,
-                              replace, rng.first, rng.second, table.first, table.second, p->all_.data_ptr(),
-                              outs.data(), sizes_dev.data_ptr<int64_t>(), p->pinned_.data_ptr<int64_t>(),
+                              replace, rng.first, rng.second, table.first, table.second, p->all_.data(),
+                              outs.data(), sizes_dev, p->pinned_.data_ptr<int64_t>(),
                               nullptr, ws.data_ptr(), ws_bytes, st));
     if (features) {
       const auto xopt = torch::TensorOptions().dtype(features->dtype()).device(dev);
@@ -811,8 +837,8 @@ class PendingBlocks : public torch::CustomClassHolder {
         // 0.197 / 0.193 / 0.205 ms per step; the uniform sampler's kernels wait for memory, and its
         // steps are 9 % slower at 5 and 4)
         const int32_t gather_blocks_per_cu = probs ? 4 : 0;
-        p->gather_status_ = dgs_gather_rows_dyn_shared(features->view(), features->elem_stride(), p->all_.data_ptr(), w,
-                                                       buffer_rows, sizes_dev.data_ptr<int64_t>() + hops, last,
+        p->gather_status_ = dgs_gather_rows_dyn_shared(features->view(), features->elem_stride(), p->all_.data(), w,
+                                                       buffer_rows, sizes_dev + hops, last,
                                                        p->x_.data_ptr(), DGS_TIER_ANY, gather_blocks_per_cu,
                                                        features->bad_index_word(), st);
       }
@@ -849,10 +875,17 @@ class PendingBlocks : public torch::CustomClassHolder {
   TicketRef end_;               // recorded behind the last launch of Begin
   bool gathered_late_ = false;  // Finish enqueued a gather behind end_
   dgs_status gather_status_ = DGS_OK;
-  torch::Tensor pinned_, seeds_, all_, x_;
+  torch::Tensor pinned_, seeds_, x_;
+  struct Piece {  // worst-case room for ids: at a byte offset into one of owned_
+    torch::Tensor owner;
+    int64_t at = 0;
+    void* data() const { return static_cast<char*>(owner.data_ptr()) + at; }
+    torch::Tensor first(int64_t count, c10::ScalarType type) const { return piece_of(owner, at, count, type); }
+  };
   std::vector<torch::Tensor> owned_;  // the allocations behind all_, src_, dst_ and the device-side lengths
   torch::Tensor staged_seeds_;  // pinned copy of host seeds, alive until the batch is finished
-  std::vector<torch::Tensor> src_, dst_;
+  Piece all_;
+  std::vector<Piece> src_, dst_;
   // the feature gather: rows of the buffer it was enqueued into (-1: none), and what a second,
   // exact gather in Finish needs
   c10::intrusive_ptr<ChunkTensor> features_;

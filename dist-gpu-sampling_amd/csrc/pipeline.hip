@@ -257,7 +257,7 @@ __device__ __forceinline__ T block_sum(T v, T* lds /* NT/64 */) {
 // ---- packed edge list of one hop (off the critical path) -----------------------------
 
 // One block per NT * kRowItems rows: scan of the rows' pick counts.  The block of the last row publishes the
-// hop's edge count and error bits.
+// hop's edge count and error bits; in a hop without rows (every id before it was refused) tile 0 does.
 template <int NT, bool EARLY>
 __device__ __forceinline__ void offsets_tile(const Hop& h, int64_t tile) {
   constexpr int64_t kRows = NT * kRowItems;
@@ -265,12 +265,12 @@ __device__ __forceinline__ void offsets_tile(const Hop& h, int64_t tile) {
   __shared__ LookbackLds<NT> look;
   __shared__ int bad;
   const int64_t s = seeds_of(h);
-  if (!EARLY && tile * kRows >= s) return;
+  if (!EARLY && tile != 0 && tile * kRows >= s) return;
   const int64_t i = tile * kRows + threadIdx.x * kRowItems;
   uint32_t rc[kRowItems];
 #pragma unroll
   for (int j = 0; j < kRowItems; ++j) rc[j] = i + j < h.s_max ? h.row_cnt[i + j] : 0u;  // requested together with s
-  if (tile * kRows >= s) return;  // whole blocks leave together
+  if (tile != 0 && tile * kRows >= s) return;  // whole blocks leave together
   if (threadIdx.x == 0) bad = 0;
   __syncthreads();
   int c = 0;
@@ -1272,7 +1272,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
     return;
   }
   const int64_t s = seeds_of(h);
-  const int64_t rows = (s + NT * kRowItems - 1) / (NT * kRowItems);
+  const int64_t rows = s > 0 ? (s + NT * kRowItems - 1) / (NT * kRowItems) : 1;  // (tile 0 of either kind writes the lengths)
   const int64_t len = seed_part(h, s) + s * h.k;
   const int64_t total = rows + (len > 0 ? (len + kTile - 1) / kTile : 1);
   for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {

@@ -170,6 +170,38 @@ def test_seed_ids_outside_the_graph_are_refused(pkg, oracle, graph, last_hop):
     assert flags[0] == 2 and flags[1] == 0
 
 
+@pytest.mark.parametrize("cap", [0, 1])
+@pytest.mark.parametrize("fanouts", [[4, 3], [3, 5, 2], [40, 30]])
+def test_calls_whose_every_seed_is_outside_the_graph(pkg, graph, fanouts, cap, request, last_hop):
+    # the frontier stays empty: the later hops have no rows, and their edge counts and flag words are
+    # written all the same (launches that fit the grid and launches that loop, one block and many)
+    capi = pkg.capi
+    indptr, indices = graph
+    n, hops = indptr.size - 1, len(fanouts)
+    probs = (np.random.default_rng(1).random(indices.size) + 0.05).astype(np.float32)
+    ip, ix, pr = _dev(indptr), _dev(indices), _dev(probs)
+    stores = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    feats = pkg.create_chunktensor(torch.zeros((n, 4)), 1, 1 << 40)
+    node_table = torch.full((capi.lib.dgs_node_table_bytes(n) // 8,), -1, dtype=torch.int64, device="cuda")
+    capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, cap))
+    request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, 0))
+    epoch = 0
+    for n_seeds in (3, 3000):
+        seeds = _dev(np.where(np.arange(n_seeds) % 2 == 0, -1, n + 7).astype(np.int64))
+        for replace in (False, True):
+            for weights in (None, capi.tensor_view(pr)):
+                epoch += 1
+                for kw in ({}, dict(node_table=node_table, epoch=epoch)):
+                    got, _, flags = capi.sample_blocks(seeds, capi.tensor_view(ip), capi.tensor_view(ix), fanouts, replace,
+                                                       1, 0, probs_view=weights, **kw)
+                    assert list(flags) == [2] + [0] * (hops - 1), (n_seeds, replace, weights is None)
+                    assert all(t.numel() == 0 for hop in got for t in hop)
+                sampler = pkg.ChunkTensorSampler(fanouts, stores[0], stores[1], None if weights is None else stores[2], replace)
+                with pytest.raises(RuntimeError, match="seed id"):
+                    sampler.sample_blocks_and_index(None, seeds, feats)
+    torch.cuda.synchronize()
+
+
 def test_neighbour_ids_outside_the_graph_are_refused(pkg, last_hop):
     # a graph whose edge array holds an id that is no node: with the direct node table the id would
     # address the table, so it is checked first and the call raises

@@ -85,12 +85,17 @@ torch::Tensor device_bytes(size_t n, const torch::Device& dev) {
 
 // `count` elements of `type` that begin `at` bytes into the storage of `owner` (at its very beginning
 // when at = 0), as a 1-d tensor that shares it.  Made without an operator call: narrow and view cost
-// 1 us each, and a batch hands out three pieces a hop.
+// 1 us each, and a batch hands out three pieces a hop.  As a view would, it shares the owner's version
+// counter (pieces may overlap: autograd has to notice that one it saved was written through another)
+// and is an inference tensor only if the owner is one.
 torch::Tensor piece_of(const torch::Tensor& owner, int64_t at, int64_t count, c10::ScalarType type) {
+  const c10::InferenceMode as_owner(owner.is_inference());
   torch::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(owner.storage()), owner.key_set(),
                                                              c10::scalarTypeToTypeMeta(type));
-  t.unsafeGetTensorImpl()->set_storage_offset(at / static_cast<int64_t>(c10::elementSize(type)));
-  t.unsafeGetTensorImpl()->set_sizes_contiguous({count});
+  c10::TensorImpl* impl = t.unsafeGetTensorImpl();
+  if (!owner.is_inference()) impl->set_version_counter(owner.unsafeGetTensorImpl()->version_counter());
+  impl->set_storage_offset(at / static_cast<int64_t>(c10::elementSize(type)));
+  impl->set_sizes_contiguous({count});
   return t;
 }
 

@@ -634,6 +634,37 @@ def test_fused_long_tile_lists(pkg, oracle, last_hop):
     assert 60_000 * 41 > 2048 * 256 and blocks[0].num_dst > 200_000
 
 
+@pytest.mark.parametrize("n_seeds", [8, 3000])
+def test_results_that_share_memory_behave_as_views(pkg, n_seeds):
+    # the frontiers of a batch are prefixes of one array: a tensor that autograd has saved must not be
+    # written through another one unnoticed, and a batch begun outside inference mode and taken inside
+    # it consists of ordinary tensors
+    n = 20000
+    ip = pkg.create_chunktensor(torch.arange(n + 1) * 4, 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.randint(0, n, (4 * n,)), 1, 1 << 40)
+    sampler = pkg.ChunkTensorSampler([3, 3], ip, ix)
+    seeds = torch.randint(0, n, (n_seeds,)).cuda()
+    _, _, blocks = sampler.sample_blocks(None, seeds)
+    last, inner = blocks[0].src_ids, blocks[1].src_ids
+    assert last.data_ptr() == inner.data_ptr()
+    weight = torch.randn(n, 2, device="cuda", requires_grad=True)
+    rows = weight[last]
+    inner.add_(0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        rows.sum().backward()
+    weight[last].sum().backward()  # untouched since: fine
+    pending = sampler.submit(None, seeds)
+    with torch.inference_mode():
+        _, _, blocks = pending.result()
+    assert not any(t.is_inference() for b in blocks for t in (b.src_ids, b.src_local, b.dst_local))
+    with torch.inference_mode():  # all of it inside: inference tensors, as any operator's there
+        _, _, blocks = sampler.sample_blocks(None, seeds)
+    assert all(t.is_inference() for b in blocks for t in (b.src_ids, b.src_local, b.dst_local))
+    _, (a, b) = pkg.ops._CAPI_tensor_relabel([seeds], [seeds, seeds])
+    a.add_(0)
+    assert a._version == b._version == 1
+
+
 def test_host_seeds_are_accepted(pkg, oracle, graph, last_hop):
     # upstream's sampler receives host-side seed_nodes and uploads them itself
     indptr, indices = graph

@@ -264,3 +264,14 @@ def test_bench_refuses_more_than_one_gpu():
         p = subprocess.run([sys.executable, os.path.join(root, "bench.py")] + argv, capture_output=True, text=True,
                            env={**os.environ, **env}, timeout=120)
         assert p.returncode != 0 and "ONE GPU" in p.stderr and p.stdout.strip() == ""
+
+
+def test_bench_legs_have_a_batch_for_every_step():
+    # a leg may time more steps than the headline has batches: it gets further ones of the same sequence
+    import bench
+    import torch
+    cfg = {"graph_seed": 3, "nodes": 1000, "batch": 8}
+    for have, count in ((25, 45), (5, 5), (60, 45), (1, 2)):
+        got = bench.first_batches(cfg, bench.make_batches(cfg, have), count, device="cpu")
+        assert len(got) == count
+        assert all(torch.equal(a, b) for a, b in zip(got, bench.make_batches(cfg, count)))

@@ -575,18 +575,28 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
 
 // ---- weighted picks (race.h) ----
 //
-// Two launch shapes.  A small hop (kSharedMaxRows) is one launch of 16-wave blocks, a wave per row; rows
-// of more than kSharedRow positions are put on a list in LDS and the whole block works on them, one
-// after the other, once its waves are through with the others.  Its time is that of its longest chain:
-// what made such a hop slow was a row of 2000 positions on one wave, behind three others, and then a
-// launch of its own for the longer ones (1024 / 5.9 k rows of mean degree 50, longest 17 k, k = 5 / 10:
-// 46 and 59 us as two launches,
-// 31 and 37 as one).
+// Two launch shapes.  A small hop (kSharedMaxRows) is one launch of 16-wave blocks, a wave per row; long
+// rows are put on a list in LDS and the whole block works on them, one after the other, once its waves
+// are through with the others.  Its time is that of its longest chain: what made such a hop slow was a
+// row of 2000 positions on one wave, behind three others, and then a launch of its own for the longer
+// ones (1024 / 5.9 k rows of mean degree 50, longest 17 k, k = 5 / 10: 46 and 59 us as two launches, 31
+// and 37 as one).
+// A block's turns on its list add up, so a block has as few rows as still give every CU a block
+// (kSharedBlocks): with 16 rows in every block, 16 / 256 / 1024 seeds of 17 000 neighbours each took
+// 382 / 388 / 390 us (one hop of 5, the whole call) where two launches take 82 / 87 / 160; now 65 / 73 / 140.
+// A turn costs 6 us and 1 us per 1000 positions, a wave by itself 8 to 15 us per 1000: rows between
+// kSharedRow and long_row<64>() positions are listed only where the block has few of them (none but one
+// below 1024 positions, four at most), since the waves of the others run side by side.  8192 rows of 1000
+// neighbours: 127 us as two launches, 308 with all of them listed, 105 now.
 // A large hop has rows enough for every wave slot: four-wave blocks, several rows per wave, and a second
-// launch, a block per row, for the queued rows above long_row<64>() positions.
+// launch, a block per row, for the queued rows above long_row<64>() positions.  us a call of one hop,
+// one launch / two, by rows and their degree: 8192 rows of 10 / 50 / 1000 / mean 50 with hubs 59 / 71,
+// 65 / 76, 105 / 127, 88 / 118; 12 000 rows 66 / 76, 77 / 80, 135 / 141, 100 / 120; 16 384 rows 74 / 72,
+// 88 / 80, 162 / 158, 131 / 125.
 constexpr int64_t kMaxLongGrid = 512;
-constexpr int64_t kSharedMaxRows = 16384;
-constexpr uint32_t kSharedRow = 512;  // two stretches of a wave (stretch_keys); with 256 a batch takes 2 % longer, the block's turns adding up
+constexpr int64_t kSharedMaxRows = 12288;
+constexpr int64_t kSharedBlocks = 256;  // one per CU
+constexpr uint32_t kSharedRow = 512;    // two stretches of a wave (stretch_keys); with 256 a batch takes 2 % longer
 
 // Lanes that one row's picks occupy when a wave of a large hop writes them out: the wave races its rows one
 // after the other (64 lanes on a row), parks every row's picks in that row's lanes and then
@@ -595,40 +605,51 @@ constexpr uint32_t kSharedRow = 512;  // two stretches of a wave (stretch_keys);
 __host__ __device__ __forceinline__ int weighted_row_lanes(int64_t k) { return k <= 16 ? 16 : (k <= 32 ? 32 : kWave); }
 inline int64_t weighted_rows_per_block(int64_t k) { return (kBlock / kWave) * (kWave / weighted_row_lanes(k)); }
 
-// The wave's rows [first, first + 64 / lanes) of the hop.  Rows above `long_limit` positions are only
-// announced (put_off(row of the hop, its first edge, its degree, its seed), by one lane); everything
-// else about a row is what fill_rows does.
-template <typename IdT, typename PtrT, typename TableT, bool REPLACE, typename PutOff>
-__device__ __forceinline__ void fill_wave_weighted(const Hop& h, int64_t s, int64_t first, int lanes, uint32_t long_limit,
-                                                   const TableT& table, const TierView<PtrT>& indptr,
-                                                   const TierView<IdT>& indices, const TierView<float>& probs,
-                                                   uint64_t rng_seed, PutOff put_off) {
+// The row that a lane looks up: row i of the hop (no row if i >= s).
+template <typename IdT>
+struct WeightedRow {
+  int64_t i, b;   // b: its first edge
+  uint32_t deg;   // 0: nothing to pick
+  IdT seed;
+  bool seed_ok, bad;
+  __device__ __forceinline__ bool raced(int k, bool replace) const { return deg > 0 && (replace || deg > uint32_t(k)); }
+};
+template <typename IdT, typename PtrT, typename TableT>
+__device__ __forceinline__ WeightedRow<IdT> look_up_row(const Hop& h, int64_t s, int64_t i, const TableT& table,
+                                                        const TierView<PtrT>& indptr, const TierView<IdT>& indices) {
+  WeightedRow<IdT> r{i, 0, 0u, IdT(0), true, false};
+  if (i < s) {
+    r.seed = static_cast<const IdT*>(h.seeds)[i];
+    // nothing is addressed by an id or an offset before it has been checked
+    r.seed_ok = row_in_range(indptr, int64_t(r.seed)) && table.holds(r.seed);
+    int64_t deg64 = 0;
+    if (r.seed_ok) {
+      r.b = int64_t(indptr.at(int64_t(r.seed)));
+      deg64 = int64_t(indptr.at(int64_t(r.seed) + 1)) - r.b;
+    }
+    r.bad = deg64 < 0 || deg64 > 0xffffffffLL || r.b < 0 || r.b + deg64 > indices.n;
+    r.deg = r.bad ? 0u : uint32_t(deg64);
+  }
+  return r;
+}
+
+// The wave's 64 / lanes consecutive rows; every lane brings the row whose picks it will write out.  Rows
+// above `long_limit` positions are only announced (put_off(row), by one lane); everything else about a
+// row is what fill_rows does.
+template <typename IdT, typename TableT, bool REPLACE, typename PutOff>
+__device__ __forceinline__ void fill_wave_weighted(const Hop& h, int64_t s, const WeightedRow<IdT>& own, int lanes,
+                                                   uint32_t long_limit, const TableT& table, const TierView<IdT>& indices,
+                                                   const TierView<float>& probs, uint64_t rng_seed, PutOff put_off) {
   const Group<kWave> g;
   const bool look_first = look_before_insert(h, s);
   const int k = h.k;
   const int rows = kWave / lanes;
-  if (first >= s) return;  // whole waves leave together
-  // every lane looks up the row whose picks it will write out
-  const int mine = g.l / lanes;  // that row among the wave's
+  const int mine = g.l / lanes;  // the lane's row among the wave's
   const int l = g.l - mine * lanes;
-  const int64_t i = first + mine;
-  int64_t b = 0;
-  uint32_t deg = 0;
-  bool bad = false;
-  IdT seed = 0;
-  bool seed_ok = true;
-  if (i < s) {
-    seed = static_cast<const IdT*>(h.seeds)[i];
-    // nothing is addressed by an id or an offset before it has been checked
-    seed_ok = row_in_range(indptr, int64_t(seed)) && table.holds(seed);
-    int64_t deg64 = 0;
-    if (seed_ok) {
-      b = int64_t(indptr.at(int64_t(seed)));
-      deg64 = int64_t(indptr.at(int64_t(seed) + 1)) - b;
-    }
-    bad = deg64 < 0 || deg64 > 0xffffffffLL || b < 0 || b + deg64 > indices.n;
-    deg = bad ? 0u : uint32_t(deg64);
-  }
+  const int64_t i = own.i, b = own.b;
+  const uint32_t deg = own.deg;
+  const IdT seed = own.seed;
+  const bool seed_ok = own.seed_ok, bad = own.bad;
   if (i < s && l == 0 && h.index == 0) {
     bool first_seen;
     uint32_t displaced;
@@ -636,8 +657,8 @@ __device__ __forceinline__ void fill_wave_weighted(const Hop& h, int64_t s, int6
         seed_ok ? table.insert_min(seed, uint32_t(h.pos_base + i), &first_seen, &displaced) : kInvalidSlot;
   }
   // rows that are copied need no work; long rows are written by somebody else
-  const bool is_long = deg > long_limit && (REPLACE || deg > uint32_t(k));
-  if (is_long && l == 0) put_off(i, b, deg, seed);
+  const bool is_long = deg > long_limit && own.raced(k, REPLACE);
+  if (is_long && l == 0) put_off(own);
   uint32_t pick = uint32_t(l);  // what a copied row keeps: its positions in order
   for (int r = 0; r < rows; ++r) {
     // row r of the wave, in scalar registers
@@ -707,9 +728,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
       const int lanes = weighted_row_lanes(h.k);
       const int64_t first = (vb * (kBlock / kWave) + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave)))) * (kWave / lanes);
-      fill_wave_weighted<IdT, PtrT, TableT, REPLACE>(
-          h, s, first, lanes, long_row<kWave>(), table, indptr, indices, probs, rng_seed, [&](int64_t i, int64_t, uint32_t, IdT) {
-            h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = i;
+      if (first >= s) continue;  // whole waves leave together
+      const WeightedRow<IdT> own = look_up_row<IdT, PtrT>(h, s, first + (threadIdx.x & (kWave - 1)) / lanes, table, indptr, indices);
+      fill_wave_weighted<IdT, TableT, REPLACE>(
+          h, s, own, lanes, long_row<kWave>(), table, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row) {
+            h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = row.i;
           });
     } else if (vb < fill_blocks + relabel_count) {
       relabel_tile<IdT, TableT, false>(prev, table, vb - fill_blocks, threadIdx.x);  // always a striding launch
@@ -738,10 +761,11 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_long_kernel(Hop 
   }
 }
 
-// A small hop: blocks [0, fill_blocks) have kLongWaves seed rows each; the blocks of the previous hop's
-// edge list and of the clearing, of kBlock threads elsewhere, are taken four at a time.
+// A small hop: blocks [0, fill_blocks) have rows_per_block (at most kLongWaves) seed rows each; the blocks
+// of the previous hop's edge list and of the clearing, of kBlock threads elsewhere, are taken four at a time.
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
 __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Hop h, Hop prev, int64_t fill_blocks,
+                                                                              int32_t rows_per_block,
                                                                               int64_t relabel_count, uint4* clear_begin,
                                                                               int64_t clear_n16, TableT table,
                                                                               TierView<PtrT> indptr,
@@ -761,18 +785,29 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Ho
   struct Listed { int64_t row, begin; uint32_t deg; int at; };
   __shared__ LongRowScratch lds;
   __shared__ Listed listed[kLongWaves];
-  __shared__ int n_listed;
+  __shared__ int n_listed, n_between;
+  __shared__ uint32_t longest_between;
   const int64_t s = seeds_of(h);
-  const int64_t first = int64_t(blockIdx.x) * kLongWaves;
+  const int64_t first = int64_t(blockIdx.x) * rows_per_block;
   if (h.n_seeds_out && blockIdx.x == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   if (first >= s) return;  // whole blocks leave together
-  if (threadIdx.x == 0) n_listed = 0;
+  if (threadIdx.x == 0) n_listed = n_between = longest_between = 0;
   __syncthreads();
-  fill_wave_weighted<IdT, PtrT, TableT, REPLACE>(
-      h, s, first + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave))), kWave, kSharedRow, table, indptr, indices, probs,
-      rng_seed, [&](int64_t i, int64_t b, uint32_t deg, IdT seed) {
-        listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(seed), b, deg, int(i - first)};  // a wave lists at most its one row
-      });
+  const int wave = int(wave_uniform(uint32_t(threadIdx.x / kWave)));
+  const bool has_row = wave < rows_per_block && first + wave < s;
+  const WeightedRow<IdT> own = look_up_row<IdT, PtrT>(h, has_row ? s : 0, first + wave, table, indptr, indices);
+  if ((threadIdx.x & (kWave - 1)) == 0 && own.deg > kSharedRow && own.deg <= long_row<kWave>() && own.raced(h.k, REPLACE)) {
+    atomicAdd(&n_between, 1);
+    atomicMax(&longest_between, own.deg);
+  }
+  __syncthreads();
+  // (turns on all of them against the longest one's time on its wave, in about 6 us each)
+  const uint32_t limit = uint32_t(n_between) * kSharedRow <= longest_between ? kSharedRow : long_row<kWave>();
+  if (has_row)
+    fill_wave_weighted<IdT, TableT, REPLACE>(
+        h, s, own, kWave, limit, table, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row) {  // a wave lists at most its one row
+          listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(row.seed), row.b, row.deg, int(row.i - first)};
+        });
   __syncthreads();
   const int n = n_listed;
   for (int t = 0; t < n; ++t) {
@@ -1511,6 +1546,9 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
 
 // Whether a weighted hop is one launch of kLongBlock-thread blocks (see above).
 inline bool weighted_shared(const Hop& h) { return h.s_max <= kSharedMaxRows; }
+inline int64_t shared_rows_per_block(const Hop& h) {
+  return std::min<int64_t>(kLongWaves, std::max<int64_t>(1, (h.s_max + kSharedBlocks - 1) / kSharedBlocks));
+}
 
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
 dgs_status launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin,
@@ -1518,10 +1556,11 @@ dgs_status launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel
                                 const dgs_view& indices, const dgs_view& probs, uint64_t rng_seed, hipStream_t st) {
   const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
   if (weighted_shared(cur)) {
-    const int64_t fill_blocks = (cur.s_max + kLongWaves - 1) / kLongWaves;
+    const int64_t rows = shared_rows_per_block(cur);
+    const int64_t fill_blocks = (cur.s_max + rows - 1) / rows;
     const int64_t others = (relabel_count + clear_blocks + kLongBlock / kBlock - 1) / (kLongBlock / kBlock);
     hipLaunchKernelGGL((hop_fill_weighted_shared_kernel<IdT, PtrT, TableT, REPLACE>), dim3(uint32_t(fill_blocks + others)),
-                       dim3(kLongBlock), 0, st, cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
+                       dim3(kLongBlock), 0, st, cur, prev, fill_blocks, int32_t(rows), relabel_count, clear_begin, clear_n16, table,
                        TierView<PtrT>(indptr), TierView<IdT>(indices), TierView<float>(probs), rng_seed);
     DGS_LAUNCH_CHECK();
     return DGS_OK;

@@ -257,11 +257,10 @@ def test_weighted_fused_long_rows_and_wide_fanout(pkg, oracle, last_hop):
 
 
 @pytest.mark.parametrize("replace", [False, True])
-@pytest.mark.parametrize("n_seeds", [1, 16, 17, 16384, 16385])
+@pytest.mark.parametrize("n_seeds", [1, 16, 17, 12288, 12289, 16384, 16385])
 def test_weighted_fused_small_and_large_hops(pkg, oracle, last_hop, n_seeds, replace):
-    # hops of up to 16384 rows are one launch whose 16-wave blocks share the rows of more than 512
-    # positions, larger ones two launches: row lengths around both limits, several long rows a block,
-    # a small hop in front of a large one
+    # hops of up to 12288 rows are one launch whose 16-wave blocks share their long rows, larger ones two
+    # launches: row lengths around the limits, several long rows a block, a small hop in front of a large one
     rng = np.random.default_rng(n_seeds)
     deg = np.concatenate([[256, 257, 511, 512, 513, 4096, 4097, 2047, 2048, 2049, 0, 1], rng.integers(0, 40, size=3000)])
     n = deg.size
@@ -278,6 +277,54 @@ def test_weighted_fused_small_and_large_hops(pkg, oracle, last_hop, n_seeds, rep
         assert np.array_equal(_np(f), want_f), fanouts
         for g, w in zip(blocks, want_blocks):
             assert np.array_equal(_np(g.src_local), w[0]) and np.array_equal(_np(g.dst_local), w[1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n_seeds", [2, 16, 256, 257, 513, 3840, 3841, 12288, 12289])
+def test_weighted_fused_dense_rows(pkg, oracle, n_seeds, replace):
+    # how many rows a block of a small hop has goes by the hop's size (1 up to 256 rows, 16 above 3840),
+    # whether it shares its rows of 513 to 2048 positions goes by how many of them it has; hops above
+    # 12288 rows are two launches
+    rng = np.random.default_rng(n_seeds)
+    deg = np.concatenate([[513, 1023, 1024, 1025, 1536, 2048, 2049, 5000, 0, 512], rng.integers(513, 2049, size=30)])
+    n = deg.size
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int64)
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    seeds = np.concatenate([rng.integers(0, n, size=n_seeds // 2), rng.integers(8, 10, size=n_seeds - n_seeds // 2)])
+    seeds[rng.random(n_seeds) < 0.2] = 4
+    seeds = seeds.astype(np.int64)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    sampler = pkg.ChunkTensorSampler([6], cts[0], cts[1], cts[2], replace, seed=9)
+    f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
+    want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, [6], replace, 9, 0, probs=probs)
+    assert np.array_equal(_np(f), want_f)
+    assert np.array_equal(_np(blocks[0].src_local), want_blocks[0][0])
+    assert np.array_equal(_np(blocks[0].dst_local), want_blocks[0][1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
+def test_weighted_fused_small_batch_of_long_rows_uses_the_whole_gpu(pkg, replace):
+    # 16 rows of 17 000 positions are worked on side by side: not 16 times as long as one (measured:
+    # 1.01 times; one block working on all of them, 5.9 times)
+    import time
+    n, deg = 512, 17_000
+    ip = pkg.create_chunktensor(torch.arange(n + 1) * deg, 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.randint(0, n, (n * deg,)), 1, 1 << 40)
+    pr = pkg.create_chunktensor(torch.rand(n * deg) + 0.01, 1, 1 << 40)
+    sampler = pkg.ChunkTensorSampler([5], ip, ix, pr, replace)
+    best = {}
+    for n_seeds in (1, 16):
+        seeds = torch.arange(n_seeds).cuda()
+        took = []
+        for _ in range(30):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            sampler.sample_blocks(None, seeds)
+            torch.cuda.synchronize()
+            took.append(time.perf_counter() - t0)
+        best[n_seeds] = min(took)
+    assert best[16] < 3 * best[1], best
 
 
 def test_weighted_rows_that_the_key_halves_leave_open(pkg, oracle, last_hop):

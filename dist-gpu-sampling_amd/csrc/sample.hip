@@ -183,9 +183,23 @@ __global__ __launch_bounds__(kTile) void fill_wave_kernel(
       }
     }
   } else if (deg <= uint32_t(k)) {
-    for (uint32_t s = lane; s < deg; s += kWave) {
-      out_rows[off + s] = IdT(row);
-      out_cols[off + s] = indices.at(start + s);
+    // four loads in flight per lane: the LDS that the other rows need leaves a CU few waves at the widest
+    // num_picks (8192 rows of 1000 neighbours, us a call, one load / four: num_picks 1024 79 / 72, 2048 90 / 78)
+    constexpr int kAhead = 4;
+    for (uint32_t s0 = 0; s0 < deg; s0 += kAhead * kWave) {
+      IdT id[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const uint32_t s = s0 + uint32_t(u * kWave + lane);
+        id[u] = s < deg ? indices.at(start + s) : IdT(0);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const uint32_t s = s0 + uint32_t(u * kWave + lane);
+        if (s >= deg) break;
+        out_rows[off + s] = IdT(row);
+        out_cols[off + s] = id[u];
+      }
     }
   } else {
     constexpr uint32_t kNoSlot = 0xffffffffu;

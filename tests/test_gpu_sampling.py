@@ -136,6 +136,21 @@ def test_sample_wide_fanouts_without_replacement(pkg, oracle, k):
         assert np.array_equal(_np(r), want_r) and np.array_equal(_np(c), want_c), stream
 
 
+@pytest.mark.parametrize("k", [700, 2048])
+def test_sample_wide_fanouts_copy_whole_rows(pkg, oracle, k):
+    # rows no longer than the fanout, copied 256 positions at a time: lengths around the steps
+    capi = pkg.capi
+    deg = np.array([1, 0, 63, 64, 65, 191, 192, 193, 255, 256, 257, 511, 512, 513, 699, 700], dtype=np.int64)
+    indptr = np.zeros(deg.size + 1, dtype=np.int64)
+    indptr[1:] = np.cumsum(deg)
+    for id_dtype in (np.int32, np.int64):
+        indices = np.arange(int(indptr[-1])).astype(id_dtype)[::-1].copy()
+        seeds = np.tile(np.arange(deg.size), 3).astype(id_dtype)
+        want_r, want_c = oracle.sample_neighbors(seeds, indptr, indices, k, False, 5, 1)
+        r, c, flags = capi.sample_neighbors(_dev(seeds), capi.tensor_view(_dev(indptr)), capi.tensor_view(_dev(indices)), k, False, 5, 1)
+        assert flags == 0 and np.array_equal(_np(r), want_r) and np.array_equal(_np(c), want_c)
+
+
 def test_seed_ids_outside_the_graph_are_refused(pkg, oracle, graph, last_hop):
     # a seed id is checked before it addresses indptr: its row emits nothing, the call is flagged,
     # the operators raise

@@ -147,7 +147,8 @@ def test_sample_wide_fanouts_copy_whole_rows(pkg, oracle, k):
         indices = np.arange(int(indptr[-1])).astype(id_dtype)[::-1].copy()
         seeds = np.tile(np.arange(deg.size), 3).astype(id_dtype)
         want_r, want_c = oracle.sample_neighbors(seeds, indptr, indices, k, False, 5, 1)
-        r, c, flags = capi.sample_neighbors(_dev(seeds), capi.tensor_view(_dev(indptr)), capi.tensor_view(_dev(indices)), k, False, 5, 1)
+        ip, ix = _dev(indptr), _dev(indices)  # (a view does not keep its tensor alive)
+        r, c, flags = capi.sample_neighbors(_dev(seeds), capi.tensor_view(ip), capi.tensor_view(ix), k, False, 5, 1)
         assert flags == 0 and np.array_equal(_np(r), want_r) and np.array_equal(_np(c), want_c)
 
 

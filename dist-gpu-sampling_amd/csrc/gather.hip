@@ -405,9 +405,17 @@ dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index
 // Whether the launch goes to gather_ragged_kernel: rows that 16-byte chunks do not divide (or that
 // begin at odd addresses), unless they are very short (see kRaggedMinChunks); a row of
 // kRaggedMinChunks chunks has at least 16 bytes, so a 16-byte chunk meets two rows at most.
-bool is_ragged(const dgs_view& v, int64_t row_bytes, const void* out, int tier, int vec) {
+// Rows that may lie in host memory come over PCIe either way, and a wave's even chunks ask for the same
+// lines: what the odd loads add, the second one of a row's end and more requests in a row's way, is lost
+// unless the chunks are very small and the list is long.  `rows` is the caller's row count or estimate.
+// us, even chunks / 16 bytes, 40 % of the rows in HBM: 500 x 602 B 20.5 / 21.7, 30 k x 200 B 132 / 142,
+// 100 k x 300 B of float32 479 / 498, 30 k x 602 B 264 / 260, 100 k x 1002 B 1288 / 1228, 30 k x 701 B of
+// bytes 315 / 290.
+constexpr int64_t kRaggedHostRow = 600, kRaggedHostBytes = 18'000'000;
+bool is_ragged(const dgs_view& v, int64_t row_bytes, const void* out, int tier, int vec, int64_t rows) {
   if (vec == 16 || row_bytes < kRaggedMinChunks * vec || row_bytes > kRaggedMaxRow) return false;
   if (reinterpret_cast<uintptr_t>(out) & 15) return false;
+  if (tier != DGS_TIER_DEVICE && (vec > 2 || row_bytes < kRaggedHostRow || rows < kRaggedHostBytes / row_bytes)) return false;
   const int64_t thr = v.threshold * v.elem_bytes, all = v.total * v.elem_bytes / row_bytes * row_bytes;
   if (tier == DGS_TIER_DEVICE) return thr >= row_bytes;
   if (tier == DGS_TIER_HOST) return (thr + row_bytes - 1) / row_bytes * row_bytes < all;
@@ -451,7 +459,7 @@ template <int TIER>
 dgs_status dispatch_vec(int vec, const dgs_view& v, int64_t row_bytes, const void* index,
                         int32_t index_bytes, int64_t n, const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad,
                         void* out, hipStream_t st) {
-  if (is_ragged(v, row_bytes, out, TIER, vec))
+  if (is_ragged(v, row_bytes, out, TIER, vec, n_dev && n_expected > 0 ? n_expected : n))
     return index_bytes == 8 ? launch_ragged<TIER, int64_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st)
                             : launch_ragged<TIER, int32_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
   switch (vec) {

@@ -131,6 +131,45 @@ def test_gather_of_rows_that_16_byte_chunks_do_not_divide(pkg, dtype, dim):
         st.close()
 
 
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 301), (torch.uint8, 601), (torch.uint8, 703), (torch.float16, 1023)])
+def test_gather_of_odd_rows_from_host_memory(pkg, dtype, dim):
+    # rows of at least 600 bytes in 1- or 2-byte chunks, some or all of them in host memory: a list of 18 MB
+    # and more goes to the kernel of the test above (which the caller's estimate decides where the count
+    # lies on the device), a shorter one to the even chunks; both return the rows' bytes
+    capi = pkg.capi
+    rows, eb = 300, torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator().manual_seed(dim)
+    full = torch.randint(0, 256, (rows, dim * eb), generator=g, dtype=torch.uint8).view(dtype)
+    long_list = 18_000_000 // (dim * eb)
+    idx = torch.cat([torch.tensor([0, rows - 1, rows - 1, 0, 1, rows - 2]), torch.randint(0, rows, (long_list,), generator=g)])
+    bad = torch.zeros(1, dtype=torch.int64, device="cuda")
+    for cap in (0, 16, dim * eb + eb, 123 * dim * eb, 123 * dim * eb + 5 * eb, rows * dim * eb - eb):
+        st = capi.Store(rows * dim, eb, cap)
+        st.load(full)
+        ids = idx.cuda()
+        for n in (long_list - 1, long_list, long_list + 6):
+            got = capi.gather_rows(st.view, dim, ids[:n], dtype, bad_index=bad)
+            assert bad.item() == 0 and torch.equal(_bits(got.cpu()), _bits(full[idx[:n]])), (cap, n)
+        short = idx[:507].to(torch.int32).cuda()
+        wrong = short.clone()
+        wrong[3], wrong[40], wrong[-1] = -1, rows, rows + 7
+        want = full[idx[:507]].clone()
+        want[[3, 40, 506]] = 0
+        out = torch.zeros((508, dim), dtype=dtype, device="cuda")
+        for count, given, expect in ((507, short, full[idx[:507]]), (29, short, full[idx[:507]]), (0, short, full[idx[:507]]),
+                                     (508, short, full[idx[:507]]), (507, wrong, want)):
+            for expected in (1, 1 << 24):
+                out.zero_()
+                n_dev = torch.tensor([count], dtype=torch.int64, device="cuda")
+                capi.check(capi.lib.dgs_gather_rows_dyn(st.view, dim, given.data_ptr(), 4, 507, n_dev.data_ptr(), expected,
+                                                        out.data_ptr(), capi.TIER_ANY, bad.data_ptr(), capi.stream_ptr()))
+                written = count if count <= 507 else 0
+                assert torch.equal(_bits(out[:written].cpu()), _bits(expect[:written])), (cap, count, expected)
+                assert (_bits(out[written:]) == 0).all().item() and bad.item() == (given is wrong), (cap, count, expected)
+                bad.zero_()
+        st.close()
+
+
 def test_index_1d_and_empty(pkg):
     full = torch.arange(1000, dtype=torch.int32)
     ct = pkg.ChunkTensor([1000], torch.int32, 1234)

@@ -1,5 +1,6 @@
-// Exclusive prefix over the tiles of a launch inside that launch: every tile's block publishes its
-// count and adds up what the tiles before it published, so that counting, scanning and compacting a
+// Exclusive prefix over the tiles of a launch inside that launch, after Merrill and Garland's single-pass
+// scan with decoupled look-back: every tile's block publishes its count and adds up what the tiles before
+// it published, so that counting, scanning and compacting a
 // list take one launch instead of two or three (5 us of launch floor each on a short list).
 //
 // A tile's state word says how far it is: 0 nothing yet, kTileCount its own count, kTilePrefix the sum
@@ -24,10 +25,11 @@ constexpr tile_state kTilePrefix = 2ull << 62;
 constexpr int kTileFlagShift = 48;  // a word is status (2 bits), flags (8 bits, or-ed), sum (48 bits, added)
 constexpr tile_state kTileSumMask = (1ull << kTileFlagShift) - 1;
 constexpr int kLookbackPolls = 256;
-// (test hook: n > 0 makes it n - 1, so that 1 has every prefix counted afresh)
+// (test hook: n > 0 makes it n - 1, so that 1 has every prefix counted afresh; n < 0 makes it negative,
+// which withholds the prefixes, so that every block reads its way back to the first tile)
 inline int32_t lookback_polls() {
   const int64_t forced = debug_option(DGS_DEBUG_LOOKBACK_POLLS);
-  return forced > 0 ? int32_t(forced - 1) : kLookbackPolls;
+  return forced > 0 ? int32_t(forced - 1) : forced < 0 ? -kLookbackPolls : kLookbackPolls;
 }
 
 __host__ __device__ __forceinline__ tile_state tile_word(int64_t sum, uint32_t flags = 0) {
@@ -46,8 +48,8 @@ struct LookbackLds {
   tile_state one;
 };
 
-// Called by all NT threads of the block of tile `tile` with the tile's own word (no status) and the
-// number of times a word is read before it is counted instead (lookback_polls()); returns
+// Called by all NT threads of the block of tile `tile` with the tile's own word (no status) and
+// lookback_polls(), the number of times a word is read before it is counted instead; returns
 // the combined word of the tiles before it.  `recount(t)` is called by the whole block and returns
 // tile t's own word.  FLAGS: the words carry flags.
 template <int NT, bool FLAGS, typename Recount>
@@ -59,13 +61,14 @@ __device__ __forceinline__ tile_state tile_exclusive_prefix(tile_state* state, i
   const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   if (threadIdx.x == 0)
     __hip_atomic_store(state + tile, own | (tile == 0 ? kTilePrefix : kTileCount), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int32_t reads = max_polls < 0 ? -max_polls : max_polls;
   tile_state before = 0;
   for (int64_t hi = tile; hi > 0;) {
     tile_state v[kItems];
     bool missing = true;
 #pragma unroll
     for (int j = 0; j < kItems; ++j) v[j] = 0;
-    for (int polls = 0; missing && polls < max_polls; ++polls) {
+    for (int polls = 0; missing && polls < reads; ++polls) {
       missing = false;
 #pragma unroll
       for (int j = 0; j < kItems; ++j) {
@@ -119,7 +122,7 @@ __device__ __forceinline__ tile_state tile_exclusive_prefix(tile_state* state, i
     if (done) break;
     hi -= kPerWave * (NT / kWave);
   }
-  if (threadIdx.x == 0 && tile != 0)
+  if (threadIdx.x == 0 && tile != 0 && max_polls >= 0)
     __hip_atomic_store(state + tile, tile_add(before, own) | kTilePrefix, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return before;
 }

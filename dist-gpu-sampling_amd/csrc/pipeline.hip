@@ -1,5 +1,6 @@
-// Multi-hop sampling + relabel as one stream of kernels with no host round trip and no
-// synchronisation between blocks inside a kernel.
+// Multi-hop sampling + relabel as one stream of kernels with no host round trip.  Inside a kernel no
+// block depends on another one's being scheduled: the blocks of a compact launch look for the counts of
+// the tiles before theirs, and count for themselves what does not come (lookback.h).
 //
 // The per-hop operators (sample.hip, unique.hip) each read a length back to the host so
 // that they can return exactly-sized arrays.  Here every buffer has its worst-case size
@@ -33,9 +34,10 @@
 //            seed list may repeat ids, asks the table; later hops look at the lost marks),
 //            learns how many first occurrences lie in the tiles before (lookback.h), ranks its
 //            own, appends them to the frontier and records the rank at the position.
-// Off the critical path, as surplus blocks of later launches: the rows' pick counts are
-// scanned (blocks of the compact launch), and the packed edge list (src_local, dst_local) is
-// written (rank of a pick = rank recorded at its id's smallest position).
+// Off the critical path, as surplus blocks: the rows' pick counts are scanned (in the compact launch),
+// and the packed edge list (src_local, dst_local) is written (in the next hop's fill; rank of a pick =
+// rank recorded at its id's smallest position).
+// A small batch is one launch of one block instead of all this (one_block.h).
 //
 // These kernels are chains of dependent memory accesses, so what a thread will need is requested
 // as early as its address is known: a hop's length lives in device memory, but every buffer has

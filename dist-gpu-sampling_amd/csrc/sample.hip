@@ -268,7 +268,7 @@ __global__ __launch_bounds__(kTile) void fill_wave_kernel(
 // of out_cols (a position fits an id slot) and is turned into neighbour ids at the end.  Slots are
 // resolved 64 at a time: every lane first compares its candidate with all positions kept by
 // earlier batches (read 64 at a time, handed round with __shfl), then the batch settles its own
-// order lane by lane as pick_position does.
+// order slot after slot, in the words of Floyd's rule.
 template <typename IdT>
 __global__ __launch_bounds__(kTile) void fill_wave_global_kernel(
     const IdT* __restrict__ seeds, int64_t n_seeds, const int64_t* __restrict__ row_start,

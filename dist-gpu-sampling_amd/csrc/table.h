@@ -1,11 +1,10 @@
 // Device-side open-addressing tables for unique/relabel (linear probing, capacity 2^m).
 //
 // A table maps a node id to the smallest position at which it occurs in the mapping
-// list.  unique.hip later overwrites that field with the id's rank (set_value); the
-// multi-hop pipeline keeps positions and learns from insert_min() whether a position
-// is, so far, the smallest of its id and which position it displaced.
-//   packed   one 64-bit word per slot: id in the high half, position/rank in the low
-//            half (ids must be < 2^32 - 1); insertion is a single 64-bit atomic;
+// list.  insert_min() tells whether a position is, so far, the smallest of its id and
+// which position it displaced.
+//   packed   one 64-bit word per slot: id in the high half, position in the low half
+//            (ids must be < 2^32 - 1); insertion is a single 64-bit atomic;
 //   split    id array + uint32 value array (any 64-bit id >= 0).
 // Slots only ever change from empty to a key, and positions only decrease, so a plain
 // (possibly stale) load is a safe first look before the atomic.
@@ -86,9 +85,6 @@ struct Table<IdT, true> {
   }
   __device__ __forceinline__ uint32_t value(uint32_t slot) const { return uint32_t(slots[slot]); }
   __device__ __forceinline__ IdT key(uint32_t slot) const { return IdT(uint32_t(slots[slot] >> 32)); }
-  __device__ __forceinline__ void set_value(uint32_t slot, uint32_t v) const {
-    reinterpret_cast<uint32_t*>(slots)[2 * size_t(slot)] = v;  // low half (little endian)
-  }
   // slot of `key`, or mask + 1 when absent
   __device__ __forceinline__ uint32_t find(IdT key) const {
     uint32_t pos = hash_id(uint32_t(key)) & mask;
@@ -146,7 +142,6 @@ struct Table<IdT, false> {
   }
   __device__ __forceinline__ uint32_t value(uint32_t slot) const { return vals[slot]; }
   __device__ __forceinline__ IdT key(uint32_t slot) const { return keys[slot]; }
-  __device__ __forceinline__ void set_value(uint32_t slot, uint32_t v) const { vals[slot] = v; }
   __device__ __forceinline__ uint32_t find(IdT key) const {
     uint32_t pos = hash_id(uint64_t(int64_t(key))) & mask;
     for (;;) {

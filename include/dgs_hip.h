@@ -68,7 +68,9 @@ int dgs_abi_version(void);
  *                                are gone over in parts)
  *   DGS_DEBUG_LOOKBACK_POLLS     n > 0: a block that needs the counts of the blocks before it
  *                                looks for them n - 1 times before it counts them itself
- *                                (1: it never looks; the default is 256 times)
+ *                                (1: it never looks; the default is 256 times); n < 0: blocks
+ *                                leave their own counts only, no sums over the blocks before
+ *                                them, so that every block has to read all of those
  */
 enum {
   DGS_DEBUG_FORCE_SPLIT_TABLE = 0,

@@ -24,14 +24,18 @@ def np_unique_first(x):
     return u[np.argsort(first, kind="stable")]
 
 
-LAST_HOP_MODES = ["last hop by size", "last hop bucketed", "last hop bucketed by hash", "last hop bucketed by hash in parts"]
+LAST_HOP_MODES = ["last hop by size", "last hop bucketed", "last hop bucketed by hash", "last hop bucketed by hash in parts",
+                  "last hop by table"]
 
 
 def set_last_hop_mode(pkg, mode):
-    """How the fused sampler's last hop finds its first occurrences in this test: by size (small
-    test inputs then take the node table's atomics), always through the bucketed LDS pass, or
-    always through the form of that pass for graphs of any node count (buckets by a hash of the id),
-    or through that form with on-chip tables so small that buckets are gone over in parts."""
+    """How the fused sampler's last hop finds its first occurrences in this test: by size (of small test
+    inputs, the unweighted ones of up to some 1000 positions a hop are then one launch of one block, with
+    the table in LDS; larger ones and weighted ones take the node table's atomics), always through the
+    bucketed LDS pass, or always through the form of that pass for graphs of any node count (buckets by
+    a hash of the id), or through that form with on-chip tables so small that buckets are gone over in
+    parts, or always through the node table's atomics (never one block, never bucketed)."""
     capi = pkg.capi
     capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_BUCKETED, {LAST_HOP_MODES[0]: 0, LAST_HOP_MODES[1]: 2,
-                                                                    LAST_HOP_MODES[2]: 3, LAST_HOP_MODES[3]: 4}[mode]))
+                                                                    LAST_HOP_MODES[2]: 3, LAST_HOP_MODES[3]: 4,
+                                                                    LAST_HOP_MODES[4]: 1}[mode]))

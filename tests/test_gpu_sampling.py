@@ -633,7 +633,8 @@ def test_fused_sample_blocks_c_abi_and_split_table(pkg, oracle, graph, last_hop)
 
 
 def test_fused_long_tile_lists(pkg, oracle, last_hop):
-    # > 2048 position tiles and > 2048 row tiles in the last hop: the separate scan launches
+    # a worst case of 22 M positions and 2.5 M rows in the last hop, a small part of which is real: launches
+    # that loop over the tiles the hop has
     rng = np.random.default_rng(5)
     indptr, indices = powerlaw_graph(rng, 1_000_000, 6, 200, zero_frac=0.1)
     seeds = rng.permutation(1_000_000)[:60_000].astype(np.int64)
@@ -646,8 +647,27 @@ def test_fused_long_tile_lists(pkg, oracle, last_hop):
     frontier, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
     assert np.array_equal(_np(frontier), o_frontier)
     _check_blocks(blocks, o_blocks)
-    # the launch plan is sized by the worst case: 60000 * 41 rows and 9 times as many positions
-    assert 60_000 * 41 > 2048 * 256 and blocks[0].num_dst > 200_000
+    assert 60_000 * 41 > 512 * 2048 and blocks[0].num_dst > 200_000
+
+
+def test_fused_hop_of_more_tiles_than_one_look_back_reads(pkg, oracle, request):
+    # a tile's block reads the counts of the 1024 tiles before its own at a time: 2.2 M rows (2048 a tile)
+    # and 11 M positions (8192 a tile) are more.  With the sums over earlier tiles withheld, every block
+    # reads its way back over all of them.
+    capi = pkg.capi
+    rng = np.random.default_rng(12)
+    n = 300_000
+    indptr = np.arange(n + 1, dtype=np.int64) * 6
+    indices = rng.integers(0, n, size=6 * n).astype(np.int32)
+    seeds = rng.integers(0, n, size=2_200_000).astype(np.int32)
+    o_frontier, _, o_blocks = oracle.sample_blocks(seeds, indptr, indices, [4], False, 3, 0)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices)]
+    request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, 0))
+    for polls in (0, -1):
+        capi.check(capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, polls))
+        frontier, _, blocks = pkg.ChunkTensorSampler([4], *cts, seed=3).sample_blocks(None, torch.from_numpy(seeds))
+        assert np.array_equal(_np(frontier), o_frontier), polls
+        _check_blocks(blocks, o_blocks)
 
 
 @pytest.mark.parametrize("n_seeds", [8, 3000])
@@ -863,7 +883,9 @@ def test_fused_sampler_under_a_small_grid_cap(pkg, oracle, graph, cap, request, 
     seeds = rng.integers(0, 20000, size=1500).astype(np.int64)
     capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, cap))
     request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, 0))
-    for weights, fanouts, replace in ((None, [12, 6, 3], False), (None, [20, 9], True), (probs, [5, 4], False)):
+    # (weighted hops of up to 12288 rows are one launch that does not loop: the last two have hops above)
+    for weights, fanouts, replace in ((None, [12, 6, 3], False), (None, [20, 9], True), (probs, [5, 4], False),
+                                      (probs, [3, 9], False), (probs, [3, 9], True)):
         sampler = pkg.ChunkTensorSampler(fanouts, ip_ct, ix_ct, None if weights is None else pr_ct, replace=replace, seed=5)
         f, _, blocks, x = sampler.sample_blocks_and_index(None, torch.from_numpy(seeds), ft)
         want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, 5, 0, probs=weights)
@@ -938,6 +960,23 @@ def test_unique_relabel_at_the_edges_of_its_tiles(pkg, oracle, dtype, n, request
             assert np.array_equal(_np(u), want_u), (polls, packed)
             for a, b in zip(outs, want_outs):
                 assert np.array_equal(_np(a), b), (polls, packed)
+
+
+@pytest.mark.parametrize("n", [3000, (1 << 22) + 1, 4_300_001])
+def test_unique_relabel_of_more_tiles_than_one_look_back_reads(pkg, oracle, n, request):
+    # a tile's block reads the counts of the 1024 tiles of 4096 ids before its own at a time; with the sums
+    # over earlier tiles withheld, every block reads its way back over all of them
+    capi = pkg.capi
+    rng = np.random.default_rng(n)
+    for dtype, packed in ((np.int32, True), (np.int64, True), (np.int64, False)):
+        ids = rng.integers(0, n // 2, size=n).astype(dtype)
+        want_u, want_outs = oracle.unique_relabel([ids], [ids])
+        d_ids = _dev(ids)
+        request.addfinalizer(lambda: capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, 0))
+        for polls in (0, -1):
+            capi.check(capi.lib.dgs_debug_set(capi.DEBUG_LOOKBACK_POLLS, polls))
+            u, outs = capi.unique_relabel([d_ids], [d_ids], packed_table=packed)
+            assert np.array_equal(_np(u), want_u) and np.array_equal(_np(outs[0]), want_outs[0]), (polls, dtype, packed)
 
 
 def test_unique_relabel_ids_beyond_32_bits(pkg, oracle):

@@ -957,6 +957,7 @@ def main():
             el_alone, _ = timed_steps(smp, some, 1)
             ev = [[torch.cuda.Event(enable_timing=True) for _ in range(2)] for _ in range(k_other)]
             st_stats = []
+            smp.sample_blocks(None, some[0])  # (untimed: the allocator has not seen a batch without features on this stream)
             for i in range(k_other):
                 ev[i][0].record()
                 r = smp.sample_blocks(None, some[args.warmup + i])

@@ -2,8 +2,9 @@
 // in LDS.
 //
 // A batch of a few seeds is a chain of launches that each take their 5 us floor whatever they do, and a
-// host that sends them one after the other: 16 seeds over fanouts [5,10] were five sampler launches, and
-// took 68.8 us with the host's part and the features where 64.3 are needed now.
+// host that sends them one after the other: 16 seeds over fanouts [5,10] are five sampler launches, and
+// take 56.4 us with the host's part and the features where one block needs 50.1; three hops of 5 from 8
+// seeds 87.1 and 56.4.
 // Here a hop is four steps between barriers of one block: picks (G lanes per seed row) and their
 // insertion, first occurrences and ranks (a scan over positions), the rows' edge offsets (a scan over
 // rows), the edge list.  Results are those of the launches in pipeline.hip: same picks, same order of

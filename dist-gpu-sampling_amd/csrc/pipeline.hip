@@ -64,8 +64,12 @@ constexpr int kRowItems = 4;                   // rows a thread of a compact blo
 // short list can use: hop 0 reads the table at random, and two CUs alone take 6 us longer over 6 k
 // positions than twelve.  Blocks of four waves as far as it goes: beside other batches' gathers, which
 // free a CU's wave slots four at a time, blocks of eight wait (8 batches through the loader 1394 us
-// against 1433).  The longest lists need eight: with four a thread's positions spill its registers
-// (2.1 M positions 28 us, 3.6 M 32 us, against 13 and 17).
+// against 1433).  Beyond 1.3 M positions eight-wave blocks, since a launch that loops has 512 blocks
+// whatever their size.  us a call, short / middle / long tiles, by positions of its last hop: one hop
+// 100 k 50.2 / 52.1 / 59.3, 131 k 60.7 / 59.7 / 65.4, 180 k 61.5 / 57.5 / 64.0, 1.2 M 172 / 123.9 / 120.9,
+// 2.1 M 274 / 186 / 182; two hops (short, middle, and the rule's own choice, which takes shorter tiles for
+// the first one) 131 k 63.2 / 65.8 / 63.7, 180 k 69.1 / 69.3 / 64.6, 1.2 M 189 / 137.5 / 137.9, 2.1 M 277 /
+// 182 / 179.
 enum PosTile { kShortTile, kMiddleTile, kLongTile };  // NT x ITEMS x GROUPS = 256 x 1 x 1, 256 x 4 x 4, 512 x 4 x 4
 inline PosTile pos_tile_kind(int64_t len_max) { return len_max <= 131072 ? kShortTile : len_max <= 1310720 ? kMiddleTile : kLongTile; }
 inline int64_t pos_tile_size(int64_t len_max) {
@@ -1648,9 +1652,10 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
 }
 
 // Whether the call is one launch of one block (one_block.h): the more launches that saves, the more
-// positions one CU may work through.  us per batch, one block against the launches: one hop, 780
-// positions 52.9 / 54.7, 2028 56.5 / 55.7; two hops, 1056 64.3 / 68.8, 2046 66.4 / 68.8, 4092 74.0 / 70.3;
-// three hops, 1536 74.2 / 84.5, 3840 82.3 / 86.1.
+// positions one CU may work through.  us per batch with its features, one block / the launches: one hop,
+// 770 positions 44.3 / 48.8, 1023 44.9 / 49.6, 2024 49.4 / 50.2, 3960 60.1 / 50.8; two hops, 1056 50.1 / 56.4,
+// 1980 54.1 / 56.2, 2640 56.3 / 56.4, 4092 65.9 / 59.1; three hops, 1728 56.4 / 87.1, 3024 62.6 / 89.1, 3888
+// 67.3 / 89.1 (what saves them more than a launch floor is that the host sends one launch).
 inline bool one_block_fits(const Plan& p) {
   const int64_t limit = std::min<int64_t>(kOnePositions, int64_t(1024) * p.n_hops);
   return !p.weighted && p.kind != TableKind::kSplit && p.s_max[p.n_hops] <= limit &&

@@ -21,8 +21,10 @@ namespace {
 
 constexpr int kThreads = 256;
 // Positions of a rank block: kThreads x kItems (one vector load of words and one of lost marks per
-// thread) x GROUPS.  One group up to 1024 tiles, which the look-back reads in one go (890 k ids 10.6 us,
-// 418 k 7.2 us; with four groups, a quarter of the blocks, 13.5 and 11.8); four beyond.
+// thread) x GROUPS.  One group up to 1024 tiles, which the look-back reads in one go; four beyond, where the
+// line could lie higher.  us a call, one group / four: ids that are mostly new 500 k 74.3 / 76.9, 1.04 M
+// 101.4 / 103.0, 1.06 M 103.9 / 105.3, 2 M 149 / 146, 4 M 268 / 251; a tenth of them new 500 k 58.0 / 64.6,
+// 1.04 M 76.6 / 81.5, 1.06 M 78.2 / 82.2, 2 M 121 / 121, 4 M 234 / 223.
 constexpr int kItems = 4;
 constexpr int kGroupIds = kThreads * kItems;
 constexpr int kLongGroups = 4;
@@ -240,10 +242,11 @@ __global__ __launch_bounds__(kThreads) void lookup_kernel(dgs_segments requiring
 // ---- small inputs: one block, the table in LDS -----------------------------------------------
 //
 // Up to kSmallIds mapping ids are handled by a single 1024-thread block whose hash table lives in
-// LDS: one launch instead of six, LDS atomics instead of memory-side ones.  One block is one CU,
-// though: its probe chains run at one CU's pace, and beyond a few thousand ids the six launches
-// over the whole GPU are faster (measured on 8-byte ids: 1024 ids 11 us against 20 us of kernels,
-// 6144 ids 43 us against 25, 10240 ids 84 us against 35), hence the low limit.
+// LDS: one launch instead of four, LDS atomics instead of memory-side ones.  One block is one CU,
+// though: its probe chains run at one CU's pace (kernel time on 8-byte ids, 6144 ids 43 us, 10240 ids
+// 84 us).  us a call with the wait for its count, the block / the launches: 2040 ids 28.6 / 42.1 (mostly new)
+// and 27.3 / 35.4 (a tenth new); with four ids a thread in place of two, 3000 ids 32.5 / 39.0 and 29.4 / 34.9,
+// 4090 ids 36.4 / 42.2 and 30.7 / 34.9, but every shorter list takes 1.1 us more (512 ids 26.4 -> 27.5).
 // Slots are packed words (id in the high half, position / rank in the low half), so an id
 // of 2^32 - 1 or more sets the overflow word like the packed table in HBM does.
 constexpr int kSmallThreads = 1024;

@@ -598,10 +598,14 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
 // launch, a block per row, for the queued rows above long_row<64>() positions.  us a call of one hop,
 // one launch / two, by rows and their degree: 8192 rows of 10 / 50 / 1000 / mean 50 with hubs 59 / 71,
 // 65 / 76, 105 / 127, 88 / 118; 12 000 rows 66 / 76, 77 / 80, 135 / 141, 100 / 120; 16 384 rows 74 / 72,
-// 88 / 80, 162 / 158, 131 / 125.
+// 88 / 80, 162 / 158, 131 / 125.  Above 32 picks the four-wave blocks give every row a wave as well, 20 of
+// them to a CU, and the one launch is kept to what runs at once: 6000 rows, 64 picks, of 50 / 200 / 1000
+// neighbours 74 / 81, 118 / 112, 181 / 157; 4500 rows 72 / 76, 110 / 104, 166 / 147; 4000 rows (against what
+// they took as two launches of an earlier form) 67 / 77, 97 / 105, 139 / 147.
 constexpr int64_t kMaxLongGrid = 512;
 constexpr int64_t kSharedMaxRows = 12288;
-constexpr int64_t kSharedBlocks = 256;  // one per CU
+constexpr int64_t kSharedBlocks = 256;  // one per CU (and one is what fits: 90 VGPRs)
+constexpr int64_t kSharedMaxRowsWide = kSharedBlocks * kLongWaves;  // for more than 32 picks
 constexpr uint32_t kSharedRow = 512;    // two stretches of a wave (stretch_keys); with 256 a batch takes 2 % longer
 
 // Lanes that one row's picks occupy when a wave of a large hop writes them out: the wave races its rows one
@@ -1551,7 +1555,9 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
 }
 
 // Whether a weighted hop is one launch of kLongBlock-thread blocks (see above).
-inline bool weighted_shared(const Hop& h) { return h.s_max <= kSharedMaxRows; }
+inline bool weighted_shared(const Hop& h) {
+  return h.s_max <= (weighted_row_lanes(h.k) < kWave ? kSharedMaxRows : kSharedMaxRowsWide);
+}
 inline int64_t shared_rows_per_block(const Hop& h) {
   return std::min<int64_t>(kLongWaves, std::max<int64_t>(1, (h.s_max + kSharedBlocks - 1) / kSharedBlocks));
 }

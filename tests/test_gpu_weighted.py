@@ -304,6 +304,27 @@ def test_weighted_fused_dense_rows(pkg, oracle, n_seeds, replace):
 
 
 @pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("k", [32, 33, 64])
+def test_weighted_fused_wide_picks_around_the_limit_of_one_launch(pkg, oracle, k, replace):
+    # above 32 picks hops of more than 4096 rows are two launches already
+    rng = np.random.default_rng(k)
+    deg = np.concatenate([[0, 1, 32, 33, 64, 65, 513, 2048, 2049, 4097], rng.integers(20, 100, size=500)])
+    n = deg.size
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int64)
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    sampler = pkg.ChunkTensorSampler([k], cts[0], cts[1], cts[2], replace, seed=9)
+    for n_seeds in (4096, 4097):
+        seeds = np.concatenate([np.arange(10), rng.integers(0, n, size=n_seeds - 10)]).astype(np.int64)
+        f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds), batch=0)
+        want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, [k], replace, 9, 0, probs=probs)
+        assert np.array_equal(_np(f), want_f)
+        assert np.array_equal(_np(blocks[0].src_local), want_blocks[0][0])
+        assert np.array_equal(_np(blocks[0].dst_local), want_blocks[0][1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
 def test_weighted_fused_small_batch_of_long_rows_uses_the_whole_gpu(pkg, replace):
     # 16 rows of 17 000 positions are worked on side by side: not 16 times as long as one (measured:
     # 1.01 times; one block working on all of them, 5.9 times)

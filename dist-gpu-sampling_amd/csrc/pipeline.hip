@@ -46,11 +46,11 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "choose.h"
 #include "common.h"
 #include "lookback.h"
 #include "one_block.h"
 #include "picks.h"
-#include "race.h"
 #include "table.h"
 
 namespace dgs {
@@ -139,8 +139,10 @@ struct Hop {
   uint32_t* slot;           // [all positions] table slot of a position, bit 31 = first occurrence
   uint32_t* rank_at;        // [all positions] rank of the id first seen at that position
   uint8_t* lost;            // [all positions] non-zero: a smaller position of the same id exists
-  int64_t* long_rows;       // weighted only: [s_max] rows handed to the block-per-row launch
-  int64_t* long_count;      // weighted only: entries of long_rows
+  int64_t* long_rows;       // weighted only: ranks of the frontier's rows of more than kLongRow positions ...
+  int64_t* long_count;      // ... and how many there are, one array for all hops but the first
+  uint8_t* long_seeds;      // weighted only, hop 0: the long ones of every kSeedSegment seeds ...
+  int32_t* long_seed_count; // ... and how many there are
   tile_state* pos_state;    // [position tiles of this hop] first occurrences, in the course of their scan
   void* frontier;           // growing array of distinct ids
   void* src_local;          // out [nnz]
@@ -155,6 +157,8 @@ struct Hop {
   int32_t pad1_;
   int64_t bucket_pos_cap;   // ... as long as the hop's padded positions (seeds * k) are no more than this: decided on the device
   int* bucket_overflow;     // set by the pass when a bucket held more ids than its LDS table takes (the call fails)
+  dgs_view indptr;          // weighted, where a hop follows: the offsets, for finding its long rows
+  int64_t n_edges;
 };
 
 // (written without a conditional so that the read is not moved behind a test)
@@ -579,55 +583,42 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
   }
 }
 
-// ---- weighted picks (race.h) ----
+// ---- weighted picks (choose.h) ----
 //
-// Two launch shapes.  A small hop (kSharedMaxRows) is one launch of 16-wave blocks, a wave per row; long
-// rows are put on a list in LDS and the whole block works on them, one after the other, once its waves
-// are through with the others.  Its time is that of its longest chain: what made such a hop slow was a
-// row of 2000 positions on one wave, behind three others, and then a launch of its own for the longer
-// ones (1024 / 5.9 k rows of mean degree 50, longest 17 k, k = 5 / 10: 46 and 59 us as two launches, 31
-// and 37 as one).
-// A block's turns on its list add up, so a block has as few rows as still give every CU a block
-// (kSharedBlocks): with 16 rows in every block, 16 / 256 / 1024 seeds of 17 000 neighbours each took
-// 382 / 388 / 390 us (one hop of 5, the whole call) where two launches take 82 / 87 / 160; now 65 / 73 / 140.
-// A turn costs 6 us and 1 us per 1000 positions, a wave by itself 8 to 15 us per 1000: rows between
-// kSharedRow and long_row<64>() positions are listed only where the block has few of them (none but one
-// below 1024 positions, four at most), since the waves of the others run side by side.  8192 rows of 1000
-// neighbours: 127 us as two launches, 308 with all of them listed, 105 now.
-// A large hop has rows enough for every wave slot: four-wave blocks, several rows per wave, and a second
-// launch, a block per row, for the queued rows above long_row<64>() positions.  us a call of one hop,
-// one launch / two, by rows and their degree: 8192 rows of 10 / 50 / 1000 / mean 50 with hubs 59 / 71,
-// 65 / 76, 105 / 127, 88 / 118; 12 000 rows 66 / 76, 77 / 80, 135 / 141, 100 / 120; 16 384 rows 74 / 72,
-// 88 / 80, 162 / 158, 131 / 125.  Above 32 picks the four-wave blocks give every row a wave as well, 20 of
-// them to a CU, and the one launch is kept to what runs at once: 6000 rows, 64 picks, of 50 / 200 / 1000
-// neighbours 74 / 81, 118 / 112, 181 / 157; 4500 rows 72 / 76, 110 / 104, 166 / 147; 4000 rows (against what
-// they took as two launches of an earlier form) 67 / 77, 97 / 105, 139 / 147.
-constexpr int64_t kMaxLongGrid = 512;
-constexpr int64_t kSharedMaxRows = 12288;
-constexpr int64_t kSharedBlocks = 256;  // one per CU (and one is what fits: 90 VGPRs)
-constexpr int64_t kSharedMaxRowsWide = kSharedBlocks * kLongWaves;  // for more than 32 picks
-constexpr uint32_t kSharedRow = 512;    // two stretches of a wave (stretch_keys); with 256 a batch takes 2 % longer
+// A block takes up to choose_rows(k) rows: a thread looks each of them up, the block chooses their picks,
+// and then every pick is placed by a thread of its own.  Rows above kLongRow positions are raced, or drawn
+// from, by a whole block each.  They are queued before the launch, by the compact launch of the hop before
+// (announce_long_rows) or, in hop 0, by the launch that clears (announce_long_seeds), so that they are
+// worked on from its first moment, beside the others.
+// A small hop (kSharedMaxRows) is a launch of larger blocks instead, which have as few rows as still give
+// every CU a block and take their own long rows one after the other at the end; rows between kSharedRow and
+// kLongRow positions as well where the block has few of them, since its waves race the others side by side.
+// In hop 0 that reaches further (kSharedMaxSeeds): it saves the launch that queues.  us a call of one hop,
+// shared / queued: 4000 rows of 50 / 200 / 1000, 64 picks 64 / 73, 78 / 102, 89 / 120; 8192 rows of 10 / 50 /
+// 1000 57 / 59, 63 / 66, 85 / 122; 12 000 of 200 86 / 103; 65 536 of 20 180 / 93.  A second hop of up to 3072
+// rows takes 19 us shared and 23 queued, one of 6144 43 and 28.
+// kLongRow 512 / 1024 / 2048: 287 / 278 / 276 us for a batch of 1024 seeds, fanouts [5,10,15].
+constexpr uint32_t kLongRow = 2048, kSharedRow = 512;
+static_assert(kLongRow <= kDrawRow, "draw_rows takes every row that is not long");
+constexpr int64_t kLongQueueBlocks = 256;  // (512: no faster)
+constexpr int64_t kSharedMaxRows = 4096, kSharedMaxSeeds = 12288;  // of a later hop, of hop 0
+constexpr int64_t kSharedBlocks = 256;  // one per CU
+constexpr int kSharedRows = 16;
+constexpr int kSeedSegment = 256;       // seeds of one list of long rows in hop 0
 
-// Lanes that one row's picks occupy when a wave of a large hop writes them out: the wave races its rows one
-// after the other (64 lanes on a row), parks every row's picks in that row's lanes and then
-// inserts and records the picks of all its rows in one go, so that the instructions of that step
-// are not spent on a mostly idle wave.
-__host__ __device__ __forceinline__ int weighted_row_lanes(int64_t k) { return k <= 16 ? 16 : (k <= 32 ? 32 : kWave); }
-inline int64_t weighted_rows_per_block(int64_t k) { return (kBlock / kWave) * (kWave / weighted_row_lanes(k)); }
-
-// The row that a lane looks up: row i of the hop (no row if i >= s).
+// A seed row as one thread looks it up (no row if i >= s).
 template <typename IdT>
 struct WeightedRow {
-  int64_t i, b;   // b: its first edge
+  int64_t b;      // its first edge
   uint32_t deg;   // 0: nothing to pick
   IdT seed;
   bool seed_ok, bad;
-  __device__ __forceinline__ bool raced(int k, bool replace) const { return deg > 0 && (replace || deg > uint32_t(k)); }
+  __device__ __forceinline__ bool chosen(int k, bool replace) const { return deg > 0 && (replace || deg > uint32_t(k)); }
 };
 template <typename IdT, typename PtrT, typename TableT>
 __device__ __forceinline__ WeightedRow<IdT> look_up_row(const Hop& h, int64_t s, int64_t i, const TableT& table,
                                                         const TierView<PtrT>& indptr, const TierView<IdT>& indices) {
-  WeightedRow<IdT> r{i, 0, 0u, IdT(0), true, false};
+  WeightedRow<IdT> r{0, 0u, IdT(0), true, false};
   if (i < s) {
     r.seed = static_cast<const IdT*>(h.seeds)[i];
     // nothing is addressed by an id or an offset before it has been checked
@@ -643,135 +634,214 @@ __device__ __forceinline__ WeightedRow<IdT> look_up_row(const Hop& h, int64_t s,
   return r;
 }
 
-// The wave's 64 / lanes consecutive rows; every lane brings the row whose picks it will write out.  Rows
-// above `long_limit` positions are only announced (put_off(row), by one lane); everything else about a
-// row is what fill_rows does.
-template <typename IdT, typename TableT, bool REPLACE, typename PutOff>
-__device__ __forceinline__ void fill_wave_weighted(const Hop& h, int64_t s, const WeightedRow<IdT>& own, int lanes,
-                                                   uint32_t long_limit, const TableT& table, const TierView<IdT>& indices,
+template <int NT, bool REPLACE>
+struct ChooseLds {
+  std::conditional_t<REPLACE, DrawRowsLds<NT>, RaceRowsLds<NT>> rows;
+  uint32_t picks[kChooseRows];     // picks that the row has here; those of a long row come from somebody else
+  uint32_t bad_pick[kChooseRows];
+};
+constexpr uint32_t kElsewhere = 0xffffffffu;
+
+// The picks of the hop's rows [first, first + rows), by a whole block.  Long rows, and with SHARED some of
+// those above kSharedRow positions, are only announced (put_off(row, its number here), by one thread).
+template <typename IdT, typename PtrT, typename TableT, bool REPLACE, bool SHARED, int NT, typename PutOff>
+__device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t s, int64_t first, int rows,
+                                                   ChooseLds<NT, REPLACE>& lds, const TableT& table,
+                                                   const TierView<PtrT>& indptr, const TierView<IdT>& indices,
                                                    const TierView<float>& probs, uint64_t rng_seed, PutOff put_off) {
-  const Group<kWave> g;
-  const bool look_first = look_before_insert(h, s);
   const int k = h.k;
-  const int rows = kWave / lanes;
-  const int mine = g.l / lanes;  // the lane's row among the wave's
-  const int l = g.l - mine * lanes;
-  const int64_t i = own.i, b = own.b;
-  const uint32_t deg = own.deg;
-  const IdT seed = own.seed;
-  const bool seed_ok = own.seed_ok, bad = own.bad;
-  if (i < s && l == 0 && h.index == 0) {
-    bool first_seen;
-    uint32_t displaced;
-    h.slot[h.pos_base + i] =
-        seed_ok ? table.insert_min(seed, uint32_t(h.pos_base + i), &first_seen, &displaced) : kInvalidSlot;
-  }
-  // rows that are copied need no work; long rows are written by somebody else
-  const bool is_long = deg > long_limit && own.raced(k, REPLACE);
-  if (is_long && l == 0) put_off(own);
-  uint32_t pick = uint32_t(l);  // what a copied row keeps: its positions in order
-  for (int r = 0; r < rows; ++r) {
-    // row r of the wave, in scalar registers
-    const int src = r * lanes;
-    const uint32_t rdeg = lane_read(deg, src);
-    const bool rlong = rdeg > long_limit && (REPLACE || rdeg > uint32_t(k));
-    if (rdeg == 0 || rlong || (!REPLACE && rdeg <= uint32_t(k))) continue;
-    const int64_t rrow = int64_t(lane_read(uint64_t(int64_t(seed)), src));
-    const int64_t rb = int64_t(lane_read(uint64_t(b), src));
-    uint32_t won = kNoPos;  // lane j: pick j of this row
-    if (REPLACE) {  // at most 64 draws: draw j is found by lane j
-      draw_row<kWave>(g, probs, rb, int64_t(rdeg), int64_t(k), rng_seed, h.rng_stream, rrow,
-                      [&](int64_t, int64_t at) { won = uint32_t(at); });
-    } else {
-      won = race_row<kWave>(g, probs, rb, rdeg, k, rng_seed, h.rng_stream, rrow);
+  const bool look_first = look_before_insert(h, s);
+  const bool bucketed = bucketed_now(h, s);
+  if (int64_t(rows) > s - first) rows = int(s - first);
+  const int t = threadIdx.x;
+  WeightedRow<IdT> own;
+  clear_entries(lds.rows, rows, k);
+  if (t < kWave) {
+    own = look_up_row<IdT, PtrT>(h, t < rows ? s : 0, first + t, table, indptr, indices);
+    const bool chosen = k > 0 && own.chosen(k, REPLACE);
+    uint32_t long_row = kLongRow;
+    if (SHARED) {  // (the block's turns on all rows in between against the longest one's time on its wave)
+      const bool between = chosen && own.deg > kSharedRow && own.deg <= kLongRow;
+      const uint32_t n = uint32_t(__builtin_popcountll(__ballot(between)));
+      if (n * kSharedRow <= ~wave_min(between ? ~own.deg : ~0u)) long_row = kSharedRow;
     }
-    const uint32_t parked = __shfl(won, l, kWave);
-    if (mine == r) pick = parked;
+    const bool is_long = chosen && own.deg > long_row;
+    set_row(lds.rows, own.b, int64_t(own.seed), chosen && !is_long ? own.deg : 0u);
+    if (t < kChooseRows) {
+      lds.picks[t] = is_long ? kElsewhere : chosen ? uint32_t(k) : REPLACE || k == 0 ? 0u : own.deg;
+      lds.bad_pick[t] = 0;
+    }
+    if (is_long) put_off(own, t);
+    if (t < rows && h.index == 0) {  // the caller's seeds open the mapping list
+      bool first_seen;
+      uint32_t displaced;
+      h.slot[h.pos_base + first + t] =
+          own.seed_ok ? table.insert_min(own.seed, uint32_t(h.pos_base + first + t), &first_seen, &displaced) : kInvalidSlot;
+    }
   }
-  bool pick_ok = true;
-  if (i < s && l < k && !is_long)
-    pick_ok = emit_pick<IdT>(h, table, indices, h.pos_base + seed_part(h, s) + i * k + l, pick < deg, b + pick, look_first,
-                             bucketed_now(h, s));
-  const uint64_t row_mask = lanes == kWave ? ~uint64_t(0) : ((uint64_t(1) << lanes) - 1);
-  const bool picks_ok = ((__ballot(!pick_ok) >> (mine * lanes)) & row_mask) == 0;
-  if (i < s && l == 0)
-    h.row_cnt[i] = !seed_ok ? kBadSeed : bad ? kBadRow : !picks_ok ? kBadPick
-                 : (REPLACE ? (deg == 0 ? 0u : uint32_t(k)) : (deg < uint32_t(k) ? deg : uint32_t(k)));
+  __syncthreads();
+  const int64_t p0 = h.pos_base + seed_part(h, s) + first * k;
+  if (k == 0) {  // nothing to choose (a zero fanout)
+  } else if constexpr (REPLACE) {
+    draw_rows<NT>(lds.rows, rows, k, probs, rng_seed, h.rng_stream, [&](int r, int j, uint32_t pos) {
+      if (!emit_pick<IdT>(h, table, indices, p0 + int64_t(r) * k + j, true, lds.rows.begin[r] + pos, look_first, bucketed))
+        lds.bad_pick[r] = 1;
+    });
+  } else {
+    race_rows<NT>(lds.rows, rows, k, probs, rng_seed, h.rng_stream);
+  }
+  // two picks a thread at a time, so that their ids are on their way together
+  constexpr int kAhead = 2;
+  int r = k > 0 ? t / k : rows, l = k > 0 ? t % k : 0;
+  while (r < rows) {
+    int at_row[kAhead], at_slot[kAhead];
+    bool here[kAhead], have[kAhead];
+    IdT id[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      at_row[u] = r;
+      at_slot[u] = l;
+      here[u] = have[u] = false;
+      id[u] = IdT(0);
+      if (r < rows) {
+        const uint32_t n = lds.picks[r];
+        here[u] = n != kElsewhere && !(REPLACE && n != 0);
+        have[u] = here[u] && uint32_t(l) < n;
+        uint32_t pos = uint32_t(l);  // copied rows keep their positions in order
+        if constexpr (!REPLACE)
+          if (have[u] && lds.rows.deg[r] != 0) pos = lds.rows.entry_pos[r * (k + 1) + l];
+        if (have[u]) id[u] = indices.at(lds.rows.begin[r] + pos);
+      }
+      r += NT / k;
+      l += NT % k;
+      if (l >= k) {
+        l -= k;
+        ++r;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (!here[u]) continue;
+      const int64_t p = p0 + int64_t(at_row[u]) * k + at_slot[u];
+      uint32_t word = kInvalidSlot;
+      if (have[u] && !place_pick<IdT>(h, table, id[u], p, look_first, bucketed, &word)) lds.bad_pick[at_row[u]] = 1;
+      h.slot[p] = word;
+    }
+  }
+  __syncthreads();
+  if (t < rows && lds.picks[t] != kElsewhere)
+    h.row_cnt[first + t] = !own.seed_ok ? kBadSeed : own.bad ? kBadRow : lds.bad_pick[t] != 0 ? kBadPick
+                         : (REPLACE ? (own.deg == 0 ? 0u : uint32_t(k)) : (own.deg < uint32_t(k) ? own.deg : uint32_t(k)));
 }
 
-// The picks of one long row (a valid one: its edges are deg positions from b on), by a whole
-// kLongBlock-thread block.
-template <typename IdT, typename TableT, bool REPLACE>
+// The picks of one long row (a valid one: its edges are deg positions from b on), by a whole block.
+template <int NT, bool REPLACE>
+struct LongLds {
+  std::conditional_t<REPLACE, DrawLongLds<NT>, RaceLongLds<NT>> row;
+  int bad_pick;
+};
+template <typename IdT, typename TableT, bool REPLACE, int NT>
 __device__ __forceinline__ void fill_long_row(const Hop& h, int64_t s, int64_t i, int64_t row, int64_t b, uint32_t deg,
-                                              LongRowScratch& lds, const TableT& table, const TierView<IdT>& indices,
+                                              LongLds<NT, REPLACE>& lds, const TableT& table, const TierView<IdT>& indices,
                                               const TierView<float>& probs, uint64_t rng_seed) {
   const bool look_first = look_before_insert(h, s);
   const bool bucketed = bucketed_now(h, s);
   const int k = h.k;
   const int64_t p0 = h.pos_base + seed_part(h, s) + i * k;
-  if (REPLACE) {
-    draw_long_row(lds, probs, b, int64_t(deg), int64_t(k), rng_seed, h.rng_stream, row,
-                  [&](int64_t j, int64_t pick) {
-                    if (!emit_pick<IdT>(h, table, indices, p0 + j, true, b + pick, look_first, bucketed))
-                      h.row_cnt[i] = kBadPick;
-                  });
+  if (threadIdx.x == 0) lds.bad_pick = 0;
+  __syncthreads();
+  if constexpr (REPLACE) {
+    draw_long<NT>(lds.row, probs, b, deg, k, rng_seed, h.rng_stream, row, [&](int j, uint32_t pick) {
+      if (!emit_pick<IdT>(h, table, indices, p0 + j, true, b + pick, look_first, bucketed)) lds.bad_pick = 1;
+    });
   } else {
-    const uint32_t pos = race_long_row(lds, probs, b, deg, k, rng_seed, h.rng_stream, row);
+    const uint32_t pos = race_long<NT>(lds.row, probs, b, deg, k, rng_seed, h.rng_stream, row);
     const int l = threadIdx.x;  // wave 0 holds the winners
-    if (l < k && !emit_pick<IdT>(h, table, indices, p0 + l, pos < deg, b + pos, look_first, bucketed))
-      h.row_cnt[i] = kBadPick;
+    if (l < k && !emit_pick<IdT>(h, table, indices, p0 + l, pos < deg, b + pos, look_first, bucketed)) lds.bad_pick = 1;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) h.row_cnt[i] = lds.bad_pick != 0 ? kBadPick : uint32_t(k);
+  __syncthreads();
 }
 
-// Same layout of virtual blocks as hop_fill_kernel (fill, previous hop's edge list, clearing).
-template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void hop_fill_weighted_kernel(Hop h, Hop prev, int64_t fill_blocks,
-                                                                   int64_t relabel_count, uint4* clear_begin,
-                                                                   int64_t clear_n16, TableT table,
-                                                                   TierView<PtrT> indptr, TierView<IdT> indices,
-                                                                   TierView<float> probs, uint64_t rng_seed) {
-  const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
-  const int64_t total = fill_blocks + relabel_count + clear_blocks;
-  for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
-    if (vb < fill_blocks) {
-      const int64_t s = seeds_of(h);
-      if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
-      const int lanes = weighted_row_lanes(h.k);
-      const int64_t first = (vb * (kBlock / kWave) + int64_t(wave_uniform(uint32_t(threadIdx.x / kWave)))) * (kWave / lanes);
-      if (first >= s) continue;  // whole waves leave together
-      const WeightedRow<IdT> own = look_up_row<IdT, PtrT>(h, s, first + (threadIdx.x & (kWave - 1)) / lanes, table, indptr, indices);
-      fill_wave_weighted<IdT, TableT, REPLACE>(
-          h, s, own, lanes, long_row<kWave>(), table, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row) {
-            h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = row.i;
-          });
-    } else if (vb < fill_blocks + relabel_count) {
-      relabel_tile<IdT, TableT, false>(prev, table, vb - fill_blocks, threadIdx.x);  // always a striding launch
-    } else {
-      const int64_t i = (vb - fill_blocks - relabel_count) * kBlock + threadIdx.x;
-      if (i < clear_n16) clear_begin[i] = make_uint4(0u, 0u, 0u, 0u);
+// Hop 0's clearing, and the lists of its long rows: segment by segment, so that nothing has to be cleared
+// before them.
+template <typename IdT, typename PtrT>
+__global__ __launch_bounds__(kSeedSegment) void announce_long_seeds_kernel(Hop h, int64_t segments, uint4* clear_begin,
+                                                                           int64_t clear_n16, TierView<PtrT> indptr,
+                                                                           int64_t n_edges) {
+  if (int64_t(blockIdx.x) >= segments) {
+    const int64_t i = (int64_t(blockIdx.x) - segments) * kSeedSegment + threadIdx.x;
+    if (i < clear_n16) clear_begin[i] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
+  __shared__ int found;
+  if (threadIdx.x == 0) found = 0;
+  __syncthreads();
+  const int64_t i = int64_t(blockIdx.x) * kSeedSegment + threadIdx.x;
+  if (i < h.n_seeds_host) {
+    const int64_t row = int64_t(static_cast<const IdT*>(h.seeds)[i]);
+    if (row_in_range(indptr, row)) {  // (bad rows are found by the fill)
+      const int64_t b = int64_t(indptr.at(row)), deg = int64_t(indptr.at(row + 1)) - b;
+      if (deg > int64_t(kLongRow) && deg <= 0xffffffffLL && b >= 0 && b + deg <= n_edges)
+        h.long_seeds[int64_t(blockIdx.x) * kSeedSegment + atomicAdd(&found, 1)] = uint8_t(threadIdx.x);
     }
   }
+  __syncthreads();
+  if (threadIdx.x == 0) h.long_seed_count[blockIdx.x] = found;
 }
 
-// The queued long rows of a hop, a 1024-thread block per row.
+// Virtual blocks: the queued long rows, the others, the previous hop's edge list.
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
-__global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_long_kernel(Hop h, TableT table,
-                                                                            TierView<PtrT> indptr,
-                                                                            TierView<IdT> indices,
-                                                                            TierView<float> probs, uint64_t rng_seed) {
-  __shared__ LongRowScratch lds;
-  const int64_t n_long = *h.long_count;
-  const int64_t s = seeds_of(h);
-  for (int64_t t = blockIdx.x; t < n_long; t += gridDim.x) {
-    const int64_t i = h.long_rows[t];
-    const int64_t row = int64_t(static_cast<const IdT*>(h.seeds)[i]);
-    const int64_t b = int64_t(indptr.at(row));
-    const uint32_t deg = uint32_t(int64_t(indptr.at(row + 1)) - b);  // queued rows have a valid degree
-    fill_long_row<IdT, TableT, REPLACE>(h, s, i, row, b, deg, lds, table, indices, probs, rng_seed);
+__global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_kernel(Hop h, Hop prev, int64_t fill_blocks,
+                                                                   int32_t rows_per_block, int64_t relabel_count,
+                                                                   TableT table, TierView<PtrT> indptr,
+                                                                   TierView<IdT> indices, TierView<float> probs,
+                                                                   uint64_t rng_seed) {
+  __shared__ union {
+    ChooseLds<kBlock, REPLACE> choose;
+    LongLds<kBlock, REPLACE> long_row;
+  } lds;
+  const int64_t total = kLongQueueBlocks + fill_blocks + relabel_count;
+  for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
+    if (vb >= kLongQueueBlocks + fill_blocks) {
+      relabel_tile<IdT, TableT, false>(prev, table, vb - kLongQueueBlocks - fill_blocks, threadIdx.x);  // always a striding launch
+      continue;
+    }
+    const int64_t s = seeds_of(h);
+    if (vb < kLongQueueBlocks) {
+      const auto take = [&](int64_t i) {
+        const int64_t row = int64_t(static_cast<const IdT*>(h.seeds)[i]);
+        if (!table.holds(IdT(row)) || h.k == 0) return;
+        const int64_t b = int64_t(indptr.at(row));
+        const uint32_t deg = uint32_t(int64_t(indptr.at(row + 1)) - b);  // queued rows have a valid degree
+        fill_long_row<IdT, TableT, REPLACE, kBlock>(h, s, i, row, b, deg, lds.long_row, table, indices, probs, rng_seed);
+      };
+      if (h.index == 0) {  // several blocks share a segment's list where there are fewer segments than blocks
+        const int64_t segments = (s + kSeedSegment - 1) / kSeedSegment;
+        const int64_t at_once = segments < kLongQueueBlocks ? segments : kLongQueueBlocks;
+        const int64_t sharers = kLongQueueBlocks / at_once, sharer = vb / at_once;
+        if (sharer < sharers)
+          for (int64_t g = vb % at_once; g < segments; g += at_once)
+            for (int64_t j = sharer; j < h.long_seed_count[g]; j += sharers)
+              take(g * kSeedSegment + h.long_seeds[g * kSeedSegment + j]);
+      } else {
+        const int64_t n_long = *h.long_count;
+        for (int64_t t = vb; t < n_long; t += kLongQueueBlocks) take(h.long_rows[t]);
+      }
+    } else {
+      const int64_t at = vb - kLongQueueBlocks;
+      if (h.n_seeds_out && at == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
+      const int64_t first = at * rows_per_block;
+      if (first >= s) continue;  // whole blocks leave together
+      fill_rows_weighted<IdT, PtrT, TableT, REPLACE, false, kBlock>(h, s, first, rows_per_block, lds.choose, table, indptr, indices,
+                                                                    probs, rng_seed, [](const WeightedRow<IdT>&, int) {});
+    }
+    __syncthreads();  // lds is rewritten by the block's next rows
   }
 }
 
-// A small hop: blocks [0, fill_blocks) have rows_per_block (at most kLongWaves) seed rows each; the blocks
+// A small hop: blocks [0, fill_blocks) have rows_per_block (at most kSharedRows) seed rows each; the blocks
 // of the previous hop's edge list and of the clearing, of kBlock threads elsewhere, are taken four at a time.
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
 __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Hop h, Hop prev, int64_t fill_blocks,
@@ -793,37 +863,29 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Ho
     return;
   }
   struct Listed { int64_t row, begin; uint32_t deg; int at; };
-  __shared__ LongRowScratch lds;
-  __shared__ Listed listed[kLongWaves];
-  __shared__ int n_listed, n_between;
-  __shared__ uint32_t longest_between;
+  __shared__ union {
+    ChooseLds<kLongBlock, REPLACE> choose;
+    LongLds<kLongBlock, REPLACE> long_row;
+  } lds;
+  __shared__ Listed listed[kSharedRows];
+  __shared__ int n_listed;
   const int64_t s = seeds_of(h);
   const int64_t first = int64_t(blockIdx.x) * rows_per_block;
   if (h.n_seeds_out && blockIdx.x == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   if (first >= s) return;  // whole blocks leave together
-  if (threadIdx.x == 0) n_listed = n_between = longest_between = 0;
-  __syncthreads();
-  const int wave = int(wave_uniform(uint32_t(threadIdx.x / kWave)));
-  const bool has_row = wave < rows_per_block && first + wave < s;
-  const WeightedRow<IdT> own = look_up_row<IdT, PtrT>(h, has_row ? s : 0, first + wave, table, indptr, indices);
-  if ((threadIdx.x & (kWave - 1)) == 0 && own.deg > kSharedRow && own.deg <= long_row<kWave>() && own.raced(h.k, REPLACE)) {
-    atomicAdd(&n_between, 1);
-    atomicMax(&longest_between, own.deg);
-  }
-  __syncthreads();
-  // (turns on all of them against the longest one's time on its wave, in about 6 us each)
-  const uint32_t limit = uint32_t(n_between) * kSharedRow <= longest_between ? kSharedRow : long_row<kWave>();
-  if (has_row)
-    fill_wave_weighted<IdT, TableT, REPLACE>(
-        h, s, own, kWave, limit, table, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row) {  // a wave lists at most its one row
-          listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(row.seed), row.b, row.deg, int(row.i - first)};
-        });
+  if (threadIdx.x == 0) n_listed = 0;
+  wave_lds_fence();  // (the first wave lists)
+  fill_rows_weighted<IdT, PtrT, TableT, REPLACE, true, kLongBlock>(
+      h, s, first, rows_per_block, lds.choose, table, indptr, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row, int r) {
+        listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(row.seed), row.b, row.deg, r};
+      });
   __syncthreads();
   const int n = n_listed;
   for (int t = 0; t < n; ++t) {
     const Listed r = listed[t];
-    fill_long_row<IdT, TableT, REPLACE>(h, s, first + int64_t(wave_uniform(uint32_t(r.at))), wave_uniform(r.row),
-                                        wave_uniform(r.begin), wave_uniform(r.deg), lds, table, indices, probs, rng_seed);
+    fill_long_row<IdT, TableT, REPLACE, kLongBlock>(h, s, first + int64_t(wave_uniform(uint32_t(r.at))), wave_uniform(r.row),
+                                                    wave_uniform(r.begin), wave_uniform(r.deg), lds.long_row, table, indices,
+                                                    probs, rng_seed);
   }
 }
 
@@ -1201,7 +1263,8 @@ template <> struct Items<4> {
 // floor; 13 bytes per position and 12 per first occurrence otherwise (2.1 M positions, 980 k of them
 // first: 13 us).
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool EARLY>
-__device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const TableT& table) {
+__device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const TableT& table, int64_t* begin, int64_t* end) {
+  *begin = *end = 0;  // the ranks that the tile adds
   using words = typename Items<ITEMS>::words;
   constexpr int kWaves = NT / kWave;
   constexpr int kGroup = NT * ITEMS;
@@ -1272,6 +1335,8 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
     return tile_word(block_sum<NT, int>(n, wave_count));
   });
   const int64_t rank0 = first_rank(h, s) + tile_sum_of(before);
+  *begin = rank0;
+  *end = rank0 + total;
   if ((tile + 1) * kTile >= len && threadIdx.x == 0) {  // the last tile: the frontier's size is known
     *h.n_unique = rank0 + total;
     if (h.host_sizes) {
@@ -1304,16 +1369,37 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
   }
 }
 
+// The long ones among the frontier's rows of ranks [begin, end), which this block has just appended, go
+// onto the next hop's queue.
+template <typename IdT, int NT>
+__device__ __forceinline__ void announce_long_rows(const Hop& h, int64_t begin, int64_t end) {
+  const auto offset = [&](int64_t i) {
+    const int64_t at = i < h.indptr.threshold ? i : i - h.indptr.threshold;
+    const void* p = i < h.indptr.threshold ? h.indptr.dev : h.indptr.host;
+    return h.indptr.elem_bytes == 8 ? static_cast<const int64_t*>(p)[at] : int64_t(static_cast<const int32_t*>(p)[at]);
+  };
+  __syncthreads();  // the ids are there
+  for (int64_t rank = begin + threadIdx.x; rank < end; rank += NT) {
+    const int64_t row = int64_t(static_cast<const IdT*>(h.frontier)[rank]);
+    if (row < 0 || row >= h.indptr.total - 1) continue;
+    const int64_t b = offset(row), deg = offset(row + 1) - b;
+    if (deg <= int64_t(kLongRow) || deg > 0xffffffffLL || b < 0 || b + deg > h.n_edges) continue;  // (a bad row is found by the fill)
+    h.long_rows[atomicAdd(reinterpret_cast<unsigned long long*>(h.long_count), 1ull)] = rank;
+  }
+}
+
 // Virtual blocks: one per NT * kRowItems rows (scan of the rows' pick counts), then one per position tile.  A
 // launch that fits the grid cap has a block for each in the worst case; a launch that loops (STRIDE)
 // goes over the tiles the hop really has.
-template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE>
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, bool ANNOUNCE>
 __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
+  int64_t begin = 0, end = 0;
   if (!STRIDE) {
     const int64_t vb = blockIdx.x;
     if (vb < row_tiles) offsets_tile<NT, true>(h, vb);
-    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, true>(h, vb - row_tiles, table);
+    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, true>(h, vb - row_tiles, table, &begin, &end);
+    if (ANNOUNCE) announce_long_rows<IdT, NT>(h, begin, end);
     return;
   }
   const int64_t s = seeds_of(h);
@@ -1321,8 +1407,10 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
   const int64_t len = seed_part(h, s) + s * h.k;
   const int64_t total = rows + (len > 0 ? (len + kTile - 1) / kTile : 1);
   for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
+    begin = end = 0;
     if (vb < rows) offsets_tile<NT, false>(h, vb);
-    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table);
+    else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table, &begin, &end);
+    if (ANNOUNCE) announce_long_rows<IdT, NT>(h, begin, end);
     __syncthreads();  // the tiles' LDS is rewritten by the block's next one
   }
 }
@@ -1461,7 +1549,8 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     tiles += row_tiles_of(p.s_max[h], len) + pos_tiles_of(len);
   }
   tile_state* states = c.take<tile_state>(tiles + 2);
-  int64_t* long_counts = p.weighted ? c.take<int64_t>(DGS_MAX_HOPS) : nullptr;
+  int64_t* long_count = p.weighted ? c.take<int64_t>(2) : nullptr;  // (cleared with them)
+  int64_t* long_rows = p.weighted ? c.take<int64_t>(size_t(p.s_max[p.n_hops - 1])) : nullptr;
   int64_t pos_base = 0;
   for (int h = 0; h < p.n_hops; ++h) {
     const size_t s = size_t(p.s_max[h]);
@@ -1476,8 +1565,12 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     v.slot = slot;
     v.rank_at = rank_at;
     v.lost = lost;
-    v.long_rows = p.weighted ? c.take<int64_t>(s) : nullptr;
-    v.long_count = p.weighted ? long_counts + h : nullptr;
+    v.long_rows = long_rows;
+    v.long_count = long_count;
+    if (p.weighted && h == 0) {
+      v.long_seeds = c.take<uint8_t>(s + kSeedSegment);
+      v.long_seed_count = c.take<int32_t>(s / kSeedSegment + 1);
+    }
     v.s_max = p.s_max[h];
     v.pos_base = pos_base;
     v.len_max = int64_t(len);
@@ -1519,16 +1612,21 @@ void launch_relabel(const Hop& hop, const TableT& table, hipStream_t st) {
                        blocks, table);
 }
 
-template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
-void launch_compact(const Hop& hop, const TableT& table, hipStream_t st) {
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool ANNOUNCE>
+void launch_compact_as(const Hop& hop, const TableT& table, hipStream_t st) {
   const int64_t row_tiles = row_tiles_of(hop.s_max, hop.len_max);
   const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max);
   if (blocks > std::min(grid_cap(), kLookbackGrid))
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true>), dim3(uint32_t(std::min(grid_cap(), kLookbackGrid))),
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(uint32_t(std::min(grid_cap(), kLookbackGrid))),
                        dim3(NT), 0, st, hop, row_tiles, table);
   else
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false>), dim3(uint32_t(blocks)), dim3(NT), 0, st,
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(uint32_t(blocks)), dim3(NT), 0, st,
                        hop, row_tiles, table);
+}
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
+void launch_compact(const Hop& hop, bool announce, const TableT& table, hipStream_t st) {
+  if (announce) launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, true>(hop, table, st);
+  else launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, false>(hop, table, st);
 }
 
 template <typename IdT, typename PtrT, typename TableT, int G>
@@ -1554,53 +1652,40 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
                        TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
 }
 
-// Whether a weighted hop is one launch of kLongBlock-thread blocks (see above).
-inline bool weighted_shared(const Hop& h) {
-  return h.s_max <= (weighted_row_lanes(h.k) < kWave ? kSharedMaxRows : kSharedMaxRowsWide);
-}
-inline int64_t shared_rows_per_block(const Hop& h) {
-  return std::min<int64_t>(kLongWaves, std::max<int64_t>(1, (h.s_max + kSharedBlocks - 1) / kSharedBlocks));
-}
+// Whether a weighted hop is a launch of kLongBlock-thread blocks (see above).
+inline bool weighted_shared(const Hop& h) { return h.s_max <= (h.index == 0 ? kSharedMaxSeeds : kSharedMaxRows); }
 
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
-dgs_status launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin,
-                                int64_t clear_n16, const TableT& table, const dgs_view& indptr,
-                                const dgs_view& indices, const dgs_view& probs, uint64_t rng_seed, hipStream_t st) {
+void launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin, int64_t clear_n16,
+                          const TableT& table, const dgs_view& indptr, const dgs_view& indices, const dgs_view& probs,
+                          uint64_t rng_seed, hipStream_t st) {
   const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
   if (weighted_shared(cur)) {
-    const int64_t rows = shared_rows_per_block(cur);
+    const int64_t rows = std::min<int64_t>(kSharedRows, std::max<int64_t>(1, (cur.s_max + kSharedBlocks - 1) / kSharedBlocks));
     const int64_t fill_blocks = (cur.s_max + rows - 1) / rows;
     const int64_t others = (relabel_count + clear_blocks + kLongBlock / kBlock - 1) / (kLongBlock / kBlock);
     hipLaunchKernelGGL((hop_fill_weighted_shared_kernel<IdT, PtrT, TableT, REPLACE>), dim3(uint32_t(fill_blocks + others)),
                        dim3(kLongBlock), 0, st, cur, prev, fill_blocks, int32_t(rows), relabel_count, clear_begin, clear_n16, table,
                        TierView<PtrT>(indptr), TierView<IdT>(indices), TierView<float>(probs), rng_seed);
-    DGS_LAUNCH_CHECK();
-    return DGS_OK;
+    return;
   }
-  const int64_t rows_per_block = weighted_rows_per_block(cur.k);
-  const int64_t fill_blocks = (cur.s_max + rows_per_block - 1) / rows_per_block;
-  const int64_t total = fill_blocks + relabel_count + clear_blocks;
-  hipLaunchKernelGGL((hop_fill_weighted_kernel<IdT, PtrT, TableT, REPLACE>), dim3(capped_grid(total)), dim3(kBlock),
-                     0, st, cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
-                     TierView<PtrT>(indptr), TierView<IdT>(indices), TierView<float>(probs), rng_seed);
-  DGS_LAUNCH_CHECK();
-  // two 1024-thread blocks fit a CU: at most one round over the 256 CUs
-  const uint32_t long_blocks = uint32_t(cur.s_max < kMaxLongGrid ? (cur.s_max < 1 ? 1 : cur.s_max) : kMaxLongGrid);
-  hipLaunchKernelGGL((hop_fill_weighted_long_kernel<IdT, PtrT, TableT, REPLACE>), dim3(long_blocks),
-                     dim3(kLongBlock), 0, st, cur, table, TierView<PtrT>(indptr), TierView<IdT>(indices),
+  if (cur.index == 0) {
+    const int64_t segments = (cur.s_max + kSeedSegment - 1) / kSeedSegment;
+    hipLaunchKernelGGL((announce_long_seeds_kernel<IdT, PtrT>), dim3(uint32_t(segments + clear_blocks)), dim3(kSeedSegment), 0, st,
+                       cur, segments, clear_begin, clear_n16, TierView<PtrT>(indptr), indices.total);
+  }
+  const int64_t rows = choose_rows(cur.k);
+  const int64_t fill_blocks = (cur.s_max + rows - 1) / rows;
+  const int64_t total = kLongQueueBlocks + fill_blocks + relabel_count;
+  hipLaunchKernelGGL((hop_fill_weighted_kernel<IdT, PtrT, TableT, REPLACE>), dim3(capped_grid(total)), dim3(kBlock), 0, st, cur,
+                     prev, fill_blocks, int32_t(rows), relabel_count, table, TierView<PtrT>(indptr), TierView<IdT>(indices),
                      TierView<float>(probs), rng_seed);
-  DGS_LAUNCH_CHECK();
-  return DGS_OK;
 }
 
 template <typename IdT, typename PtrT, typename TableT>
 dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const TableT& table, const dgs_view& indptr,
                       const dgs_view& indices, const dgs_view* probs, bool replace, uint64_t rng_seed,
                       void** sizes_ticket, hipStream_t st) {
-  if (p.weighted && !weighted_shared(hops[0])) {  // the long-row queues of all hops start empty (their counters are one array, hop 0's first)
-    hipLaunchKernelGGL(zero_sizes_kernel, dim3(1), dim3(64), 0, st, hops[0].long_count, p.n_hops);
-    DGS_LAUNCH_CHECK();
-  }
   for (int h = 0; h < p.n_hops; ++h) {
     const Hop& cur = hops[h];
     const Hop prev = h > 0 ? hops[h - 1] : Hop{};
@@ -1613,14 +1698,12 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
       const Hop& last = hops[p.n_hops - 1];
       clear_begin = reinterpret_cast<uint4*>(cur.lost + (p.n_hops > 1 ? hops[1].pos_base : p.s_max[1] / 16 * 16));
       const char* end = reinterpret_cast<const char*>(last.pos_state + pos_tiles_of(last.len_max));  // (two spare words follow)
-      // (where hop 0 queues no rows itself, the queues' counters as well: they come next)
-      if (p.weighted && weighted_shared(cur)) end = reinterpret_cast<const char*>(cur.long_count + DGS_MAX_HOPS);
+      if (p.weighted) end = reinterpret_cast<const char*>(cur.long_count + 2);  // (which comes next)
       clear_n16 = (end - reinterpret_cast<const char*>(clear_begin) + 15) / 16;
     }
     if (p.weighted) {
-      const dgs_status ws = replace ? launch_fill_weighted<IdT, PtrT, TableT, true>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st)
-                                    : launch_fill_weighted<IdT, PtrT, TableT, false>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st);
-      if (ws != DGS_OK) return ws;
+      if (replace) launch_fill_weighted<IdT, PtrT, TableT, true>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st);
+      else launch_fill_weighted<IdT, PtrT, TableT, false>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st);
     } else if (cur.k <= 8) launch_fill<IdT, PtrT, TableT, 8>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
     else if (cur.k <= 16) launch_fill<IdT, PtrT, TableT, 16>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
     else if (cur.k <= 32) launch_fill<IdT, PtrT, TableT, 32>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
@@ -1640,10 +1723,12 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
       DGS_LAUNCH_CHECK();
     }
 
+    // (a queue holds the whole frontier: from hop 0 on, where a later hop reads it; hops only get larger)
+    const bool announce = p.weighted && h + 1 < p.n_hops && !weighted_shared(hops[p.n_hops - 1]);
     switch (pos_tile_kind(cur.len_max)) {
-      case kShortTile: launch_compact<IdT, TableT, 256, 1, 1>(cur, table, st); break;
-      case kMiddleTile: launch_compact<IdT, TableT, 256, 4, 4>(cur, table, st); break;
-      case kLongTile: launch_compact<IdT, TableT, 512, 4, 4>(cur, table, st); break;
+      case kShortTile: launch_compact<IdT, TableT, 256, 1, 1>(cur, announce, table, st); break;
+      case kMiddleTile: launch_compact<IdT, TableT, 256, 4, 4>(cur, announce, table, st); break;
+      case kLongTile: launch_compact<IdT, TableT, 512, 4, 4>(cur, announce, table, st); break;
     }
     DGS_LAUNCH_CHECK();
   }
@@ -1822,6 +1907,8 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
     t.src_local = outs[h].src_local;
     t.dst_local = outs[h].dst_local;
     t.rng_stream = first_stream + uint32_t(h);
+    t.indptr = indptr;
+    t.n_edges = indices.total;
   }
   const bool rep = replace != 0;
   if (id_bytes == 8)

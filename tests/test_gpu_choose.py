@@ -1,0 +1,87 @@
+"""GPU parity of the block-wise weighted choice (csrc/choose.h) at the edges of its row classes, against the
+CPU oracle: picks are bit-exact whatever the float32 race decides and whatever it leaves to 64-bit keys."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+# quads, the counting limit, stretches of a wave, the limits of block turns and queues, more than one go
+EDGES = [0, 1, 2, 3, 4, 5, 7, 8, 9, 31, 32, 33, 63, 64, 65, 127, 128, 129, 130, 255, 256, 257, 511, 512, 513, 1023, 1024,
+         1025, 2047, 2048, 2049, 4095, 4096, 4097, 5121, 20480, 20481]
+SEED, STREAM = 0x5eed5eed77, 3
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    return load_pkg()
+
+
+def _graph(rng, n):
+    deg = rng.integers(0, 40, size=n)
+    deg[rng.permutation(n)[:2 * len(EDGES)]] = EDGES * 2
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    return deg, indptr, rng.integers(0, n, size=int(indptr[-1])).astype(np.int32)
+
+
+def _weights(kind, rng, oracle, deg, indptr):
+    w = (rng.random(int(indptr[-1])) + 0.01).astype(np.float32)
+    if kind == "spread":   # hundreds of binades, denormal ones and huge ones among them, and no weight at all
+        w = np.exp2(rng.uniform(-148, 126, size=w.size)).astype(np.float32)
+        w[rng.random(w.size) < 0.3] = rng.choice(np.array([0, -1, np.nan], dtype=np.float32))
+    if kind == "few":      # mostly unusable: they are picked in order of their positions
+        w[rng.random(w.size) < 0.9] = 0.0
+    if kind == "infinite":
+        w[rng.random(w.size) < 0.2] = np.inf
+    if kind == "level":    # every weight is its own variate: all of a row's keys are 1 to within a float32
+        for row in range(len(deg)):
+            for p in range(min(int(deg[row]), 1100)):
+                w[indptr[row] + p] = oracle.weighted_key(SEED, STREAM, row, p, 1.0)
+    return w
+
+
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("kind", ["plain", "spread", "few", "infinite", "level"])
+def test_choice_at_the_edges_of_the_row_classes(pkg, oracle, kind, replace):
+    rng = np.random.default_rng(5)
+    n = 600
+    deg, indptr, indices = _graph(rng, n)
+    probs = _weights(kind, rng, oracle, deg, indptr)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    for n_seeds, fanouts in [(n, [7]), (n, [33]), (n, [64]), (n, [1]), (1, [5, 3]), (300, [2, 0, 4])]:
+        seeds = rng.permutation(n)[:n_seeds].astype(np.int32)
+        pkg.set_rng_state(SEED, STREAM)
+        f, _, blocks = pkg.ChunkTensorSampler(fanouts, *cts, replace=replace).sample_blocks(None, torch.from_numpy(seeds))
+        want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, SEED, STREAM, probs=probs)
+        assert np.array_equal(f.cpu().numpy(), want_f), (n_seeds, fanouts)
+        for g, w in zip(blocks, want):
+            assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n_seeds,fanouts", [(200, [6, 4, 3]),     # shared, shared, queued: long rows of every frontier
+                                             (900, [6, 4]),        # shared, then queued
+                                             (12289, [3, 2]),      # the first hop's long rows come from its segments
+                                             (70000, [2])])        # more segments than blocks
+def test_long_rows_reach_the_hop_that_has_them(pkg, oracle, n_seeds, fanouts, replace):
+    rng = np.random.default_rng(n_seeds)
+    n = 6000
+    deg = rng.integers(0, 20, size=n)
+    hubs = rng.permutation(n)[:40]
+    deg[hubs] = rng.integers(2040, 2600, size=40)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int32)
+    indices[rng.random(indices.size) < 0.02] = hubs[0]
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    seeds = rng.integers(0, n, size=n_seeds).astype(np.int32)
+    seeds[:40] = hubs
+    for _ in range(2):  # (the second call works on what the first one left in the buffers)
+        pkg.set_rng_state(SEED, STREAM)
+        f, _, blocks = pkg.ChunkTensorSampler(fanouts, *cts, replace=replace).sample_blocks(None, torch.from_numpy(seeds))
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, SEED, STREAM, probs=probs)
+    assert np.array_equal(f.cpu().numpy(), want_f)
+    for g, w in zip(blocks, want):
+        assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])

@@ -36,7 +36,8 @@
 //            own, appends them to the frontier and records the rank at the position.
 // Off the critical path, as surplus blocks: the rows' pick counts are scanned (in the compact launch),
 // and the packed edge list (src_local, dst_local) is written (in the next hop's fill; rank of a pick =
-// rank recorded at its id's smallest position).
+// rank recorded at its id's smallest position, which the pick met when it was inserted or finds by links:
+// the table is not read again).
 // A small batch is one launch of one block instead of all this (one_block.h).
 //
 // These kernels are chains of dependent memory accesses, so what a thread will need is requested
@@ -136,8 +137,8 @@ struct Hop {
   uint32_t* row_cnt;        // [s_max] picks of every row (kBadRow on error)
   uint32_t* row_off;        // [s_max] first packed edge of the row
   tile_state* row_state;    // [row tiles] the tiles' edge counts, in the course of their scan
-  uint32_t* slot;           // [all positions] table slot of a position, bit 31 = first occurrence
-  uint32_t* rank_at;        // [all positions] rank of the id first seen at that position
+  uint32_t* slot;           // [all positions] what is known of a position's id (see Slot words)
+  uint32_t* rank_at;        // [all positions] rank of the id first seen there; of a lost position: a smaller one | kLinkBit
   uint8_t* lost;            // [all positions] non-zero: a smaller position of the same id exists
   int64_t* long_rows;       // weighted only: ranks of the frontier's rows of more than kLongRow positions ...
   int64_t* long_count;      // ... and how many there are, one array for all hops but the first
@@ -244,7 +245,28 @@ __device__ __forceinline__ uint32_t bucket_of(const Buckets& b, int log_buckets,
   return (b.hashed ? hash_id(id) : id) & uint32_t((1 << log_buckets) - 1);
 }
 
-// rank of the id at position p, given p's slot word
+// ---- Slot words ----
+//
+// What the slot word of a position says when its edge is written out:
+//   kFirstBit | table slot    the first occurrence of its id: its rank is at the position itself;
+//   kRankBit | rank           the rank itself (bucketed hops);
+//   a position                of the same id and smaller, or the position's own where it has lost its bit:
+//                             the rank is there, or a link to a smaller position;
+//   table slot                in hop 0, whose first occurrences are settled by asking the table.
+// A pick that is not its id's first has met a smaller position of the id when it was inserted.  That one may
+// itself be displaced later in the same launch: whoever does so leaves a link to its own position in rank_at,
+// and positions only get smaller along the links.  Reading these words, a stream and some 4-byte reads near
+// one another, in place of the table's entry saves a random read of a table that caches do not hold: R-MAT of
+// 2^26 nodes, 3.05 M picks, two thirds of them repeats: 44 -> 25 us for the hop's edge list, 380 -> 369 for the batch.
+constexpr uint32_t kLinkBit = 0x80000000u;
+
+// rank at position `at`, or where the links from there lead
+__device__ __forceinline__ uint32_t rank_from(const Hop& h, uint32_t at) {
+  uint32_t r = h.rank_at[at];
+  while (r & kLinkBit) r = h.rank_at[r & ~kLinkBit];
+  return r;
+}
+// rank of the id at position p of hop 0, given p's slot word
 template <typename TableT>
 __device__ __forceinline__ uint32_t rank_of(const Hop& h, const TableT& table, int64_t p, uint32_t slot_word) {
   if (slot_word & kFirstBit) return h.rank_at[p];
@@ -371,9 +393,8 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
     }
   }
   if (tile * kRowTile >= s) return;  // whole blocks leave together
-  // Rank of a pick = rank recorded at the smallest position of its id: its own position when it
-  // is a first occurrence, else the position the table holds.  Two rounds of loads, each issued
-  // for all of the thread's picks before any is used.
+  // Rank of a pick = rank recorded at the smallest position of its id (see Slot words).  Rounds of
+  // loads, each issued for all of the thread's picks before any is used.
   const bool bucketed = bucketed_now(h, s);
   bool live[kRelabelItems];
   bool known[kRelabelItems];  // bucketed hop: the word of a repeat may be the rank itself
@@ -384,17 +405,20 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
     at[j] = uint32_t(p[j]);
     known[j] = false;
     if (live[j] && !(word[j] & kFirstBit)) {
-      if (bucketed) {
-        known[j] = (word[j] & kRankBit) != 0;
-        at[j] = word[j] & (kRankBit - 1);
-      } else {
+      if (h.index == 0) {
         at[j] = table.value(word[j]);
+      } else {
+        known[j] = bucketed && (word[j] & kRankBit) != 0;
+        at[j] = known[j] ? word[j] & (kRankBit - 1) : word[j];
       }
     }
   }
   uint32_t rank[kRelabelItems];
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) rank[j] = !live[j] ? 0u : known[j] ? at[j] : h.rank_at[at[j]];
+#pragma unroll
+  for (int j = 0; j < kRelabelItems; ++j)
+    if (rank[j] & kLinkBit) rank[j] = rank_from(h, rank[j] & ~kLinkBit);
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) {
     if (!live[j]) continue;
@@ -411,9 +435,10 @@ inline int64_t relabel_blocks(int64_t s_max, int k) {
 
 // ---- critical path ------------------------------------------------------------------------
 
-// Marks `displaced` (a position of this call) as no longer the smallest of its id.
-__device__ __forceinline__ void mark_lost(const Hop& h, uint32_t displaced) {
-  if (displaced != kNoPosition) h.lost[displaced] = 1;
+// Marks `displaced` (a position of this hop) as no longer the smallest of its id: p is smaller.
+__device__ __forceinline__ void mark_lost(const Hop& h, uint32_t displaced, int64_t p) {
+  h.lost[displaced] = 1;
+  h.rank_at[displaced] = uint32_t(p) | kLinkBit;
 }
 
 // The slot word of padded position p, which holds a pick of neighbour id `col`: the id goes into
@@ -430,11 +455,11 @@ __device__ __forceinline__ bool place_pick(const Hop& h, const TableT& table, Id
     return true;
   }
   bool first;
-  uint32_t displaced;
-  uint32_t w = table.insert_min(col, uint32_t(p), &first, &displaced, look_first);
+  uint32_t met;
+  uint32_t w = table.insert_min(col, uint32_t(p), &first, &met, look_first);
   if (h.index != 0) {
-    if (first) w |= kFirstBit;  // provisional: void once the position is marked lost
-    mark_lost(h, displaced);
+    if (first && met != kNoPosition) mark_lost(h, met, p);
+    w = first ? (w | kFirstBit) : met;  // (the bit is provisional: void once the position is marked lost)
   }
   *word = w;
   return true;
@@ -517,8 +542,8 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   const int64_t p = h.pos_base + seed_part(h, s) + i * k + l;
   // Draws with replacement repeat positions: on a row shorter than k most slots do.  Only the
   // lowest slot of each position reads the edge array and goes to the table; a repeat can never be
-  // its id's smallest position, so it takes its leader's id and slot word (without the first bit)
-  // and touches nothing.  Repeats are found through a small table of the wave's own in LDS: every
+  // its id's smallest position, so it takes its leader's slot word, or position where that may be the
+  // first, and touches nothing.  Repeats are found through a small table of the wave's own in LDS: every
   // slot of the row offers (position, lane) to the entry its position hashes to, the smallest
   // offer stays, and a slot that then reads its own position with a lower lane of its row has found
   // its leader.  Two positions that meet in one entry cost a missed repeat, never a wrong one.
@@ -549,7 +574,8 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
     const uint32_t leader_word = __shfl(word, leader, G);
     const int leader_ok = __shfl(int(pick_ok), leader, G);
     if (live && leader != l) {
-      word = leader_word == kInvalidSlot ? kInvalidSlot : (leader_word & ~kFirstBit);
+      word = leader_word == kInvalidSlot ? kInvalidSlot
+           : h.index != 0 && (leader_word & kFirstBit) ? uint32_t(p - l + leader) : (leader_word & ~kFirstBit);
       pick_ok = leader_ok != 0;
     }
   }
@@ -1349,7 +1375,7 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
     const int64_t p = h.pos_base + base + g * kGroup;
     uint32_t rank = uint32_t(rank0) + uint32_t(lane_before[g]);
     words ranks;
-    bool changed = false;
+    bool changed = false, any_lost = false;
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       ranks[j] = rank;
@@ -1360,11 +1386,17 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
         changed |= h.index == 0;
         if (h.index == 0) word[g][j] = bare | kFirstBit;  // the bit as relabel_tile reads it
       } else if (((lost[g] >> (8 * j)) & 0xffu) != 0) {
-        changed = true;
-        word[g][j] = bare;
+        changed = any_lost = true;
+        word[g][j] = uint32_t(p) + uint32_t(j);  // its own position, where the link to a smaller one is
       }
     }
-    *reinterpret_cast<words*>(h.rank_at + p) = ranks;  // (only the ones at first positions are ever read)
+    if (!any_lost) {
+      *reinterpret_cast<words*>(h.rank_at + p) = ranks;  // (only the ones at first positions are ever read)
+    } else {
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j)
+        if ((first[g] >> j) & 1) h.rank_at[p + j] = ranks[j];
+    }
     if (changed) *reinterpret_cast<words*>(h.slot + p) = word[g];
   }
 }

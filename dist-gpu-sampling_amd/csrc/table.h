@@ -1,8 +1,8 @@
 // Device-side open-addressing tables for unique/relabel (linear probing, capacity 2^m).
 //
 // A table maps a node id to the smallest position at which it occurs in the mapping
-// list.  insert_min() tells whether a position is, so far, the smallest of its id and
-// which position it displaced.
+// list.  insert_min() tells whether a position is, so far, the smallest of its id, and which
+// position of the id it has met: the one it displaced, or the smaller one.
 //   packed   one 64-bit word per slot: id in the high half, position in the low half
 //            (ids must be < 2^32 - 1); insertion is a single 64-bit atomic;
 //   split    id array + uint32 value array (any 64-bit id >= 0).
@@ -60,13 +60,13 @@ struct Table<IdT, true> {
       pos = (pos + 1) & mask;
     }
   }
-  // Same, reporting whether idx became the smallest position of its key (*first) and, if it
-  // replaced a larger one, which (*displaced, else kNoPosition).
-  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* displaced,
+  // Same, reporting whether idx became the smallest position of its key (*first), and the position that
+  // the key had (*met: the larger one that idx replaced, kNoPosition if there was none, or the smaller one).
+  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* met,
                                                  bool /*look_first*/ = true) const {
     const unsigned long long packed = (static_cast<unsigned long long>(uint32_t(key)) << 32) | idx;
     uint32_t pos = hash_id(uint32_t(key)) & mask;
-    *displaced = kNoPosition;
+    *met = kNoPosition;
     for (;;) {
       unsigned long long cur = slots[pos];
       if (cur == kEmpty) {
@@ -74,10 +74,10 @@ struct Table<IdT, true> {
         if (cur == kEmpty) { *first = true; return pos; }
       }
       if (uint32_t(cur >> 32) == uint32_t(key)) {
-        if (cur < packed) { *first = false; return pos; }  // (it only ever gets smaller: no atomic needed)
+        if (cur < packed) { *first = false; *met = uint32_t(cur); return pos; }  // (it only ever gets smaller: no atomic needed)
         const unsigned long long old = atomicMin(slots + pos, packed);
         *first = old > packed;
-        if (*first) *displaced = uint32_t(old);
+        *met = uint32_t(old);
         return pos;
       }
       pos = (pos + 1) & mask;
@@ -125,7 +125,7 @@ struct Table<IdT, false> {
     atomicMin(vals + pos, idx);
     return pos;
   }
-  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* displaced,
+  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* met,
                                                  bool /*look_first*/ = true) const {
     using W = typename AtomicWord<IdT>::type;
     uint32_t pos = hash_id(uint64_t(int64_t(key))) & mask;
@@ -137,7 +137,7 @@ struct Table<IdT, false> {
     }
     const uint32_t old = atomicMin(vals + pos, idx);
     *first = old > idx;
-    *displaced = (*first && old != 0xffffffffu) ? old : kNoPosition;
+    *met = old;  // (an empty value is kNoPosition)
     return pos;
   }
   __device__ __forceinline__ uint32_t value(uint32_t slot) const { return vals[slot]; }
@@ -175,15 +175,17 @@ struct DirectTable {
   // only be larger than the truth) settles the matter without an atomic, which is what keeps
   // popular ids from serialising thousands of atomics on one address; on ids that are mostly
   // new the extra read is pure cost.  The result is the same either way.
-  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* displaced,
+  __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* met,
                                                  bool look_first = true) const {
     const unsigned long long v = (static_cast<unsigned long long>(tag) << 32) | idx;
     unsigned long long* e = entries + uint32_t(key);
-    if (look_first && *e < v) { *first = false; *displaced = kNoPosition; return uint32_t(key); }
+    if (look_first) {
+      const unsigned long long seen = *e;
+      if (seen < v) { *first = false; *met = uint32_t(seen); return uint32_t(key); }
+    }
     const unsigned long long old = atomicMin(e, v);
     *first = old > v;
-    // an entry of this use that was larger: that position is no longer its id's smallest
-    *displaced = (*first && uint32_t(old >> 32) == tag) ? uint32_t(old) : kNoPosition;
+    *met = uint32_t(old >> 32) == tag ? uint32_t(old) : kNoPosition;  // (an entry of this use)
     return uint32_t(key);
   }
   __device__ __forceinline__ uint32_t value(uint32_t slot) const { return uint32_t(entries[slot]); }

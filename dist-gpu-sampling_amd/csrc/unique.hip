@@ -85,10 +85,10 @@ __global__ __launch_bounds__(kThreads) void insert_kernel(dgs_segments mapping, 
     return;
   }
   bool first;
-  uint32_t displaced;
-  const uint32_t w = table.insert_min(key, uint32_t(i), &first, &displaced);
+  uint32_t met;
+  const uint32_t w = table.insert_min(key, uint32_t(i), &first, &met);
   slot[i] = first ? (w | kFirstBit) : w;
-  if (displaced != kNoPosition) lost[displaced] = 1;
+  if (first && met != kNoPosition) lost[met] = 1;
 }
 
 // First occurrences of one tile of mapping positions: counted, added to what the tiles before hold,

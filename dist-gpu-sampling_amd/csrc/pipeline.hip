@@ -416,9 +416,11 @@ __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, 
   uint32_t rank[kRelabelItems];
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) rank[j] = !live[j] ? 0u : known[j] ? at[j] : h.rank_at[at[j]];
+  if ((rank[0] | rank[1] | rank[2] | rank[3]) & kLinkBit) {
 #pragma unroll
-  for (int j = 0; j < kRelabelItems; ++j)
-    if (rank[j] & kLinkBit) rank[j] = rank_from(h, rank[j] & ~kLinkBit);
+    for (int j = 0; j < kRelabelItems; ++j)
+      if (rank[j] & kLinkBit) rank[j] = rank_from(h, rank[j] & ~kLinkBit);
+  }
 #pragma unroll
   for (int j = 0; j < kRelabelItems; ++j) {
     if (!live[j]) continue;
@@ -1375,7 +1377,8 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
     const int64_t p = h.pos_base + base + g * kGroup;
     uint32_t rank = uint32_t(rank0) + uint32_t(lane_before[g]);
     words ranks;
-    bool changed = false, any_lost = false;
+    bool changed = false;
+    uint32_t links = 0;  // bit j: position j has lost its bit, and a link is where its rank would be
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       ranks[j] = rank;
@@ -1386,17 +1389,18 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
         changed |= h.index == 0;
         if (h.index == 0) word[g][j] = bare | kFirstBit;  // the bit as relabel_tile reads it
       } else if (((lost[g] >> (8 * j)) & 0xffu) != 0) {
-        changed = any_lost = true;
+        changed = true;
+        links |= 1u << j;
         word[g][j] = uint32_t(p) + uint32_t(j);  // its own position, where the link to a smaller one is
       }
     }
-    if (!any_lost) {
-      *reinterpret_cast<words*>(h.rank_at + p) = ranks;  // (only the ones at first positions are ever read)
-    } else {
+    if (links != 0) {
+      const words there = *reinterpret_cast<const words*>(h.rank_at + p);
 #pragma unroll
       for (int j = 0; j < ITEMS; ++j)
-        if ((first[g] >> j) & 1) h.rank_at[p + j] = ranks[j];
+        if ((links >> j) & 1) ranks[j] = there[j];
     }
+    *reinterpret_cast<words*>(h.rank_at + p) = ranks;  // (beside the links only the ones at first positions are ever read)
     if (changed) *reinterpret_cast<words*>(h.slot + p) = word[g];
   }
 }

@@ -34,6 +34,11 @@ class BlockOut(ctypes.Structure):
     _fields_ = [("src_local", c_vp), ("dst_local", c_vp)]
 
 
+class EdgeJob(ctypes.Structure):
+    """dgs_edge_job"""
+    _fields_ = [("words", c_u64 * 16)]
+
+
 class Segments(ctypes.Structure):
     """dgs_segments"""
     _fields_ = [("ptr", c_vp * MAX_SEGMENTS), ("len", c_i64 * MAX_SEGMENTS), ("count", c_i32),
@@ -84,6 +89,12 @@ SIGNATURES = {
                                          c_u64, c_u32, c_vp, c_u32, c_vp, ctypes.POINTER(BlockOut), c_vp, c_vp,
                                          ctypes.POINTER(c_vp), c_vp, c_sz, c_vp]),
     "dgs_sample_blocks_weighted_workspace_bytes": (c_sz, [c_i64, ctypes.POINTER(c_i64), c_i32, c_i32]),
+    "dgs_sample_blocks_leave_edges": (ctypes.c_int, [c_vp, c_i32, c_i64, View, View, ctypes.POINTER(View), ctypes.POINTER(c_i64),
+                                                     c_i32, c_i32, c_u64, c_u32, c_vp, c_u32, c_vp, ctypes.POINTER(BlockOut),
+                                                     c_vp, c_vp, ctypes.POINTER(EdgeJob), c_vp, c_sz, c_vp]),
+    "dgs_gather_rows_dyn_edges": (ctypes.c_int, [View, c_i64, c_vp, c_i32, c_i64, c_vp, c_i64, c_vp, c_i32, c_i32, c_vp,
+                                                 ctypes.POINTER(EdgeJob), c_vp]),
+    "dgs_write_edges": (ctypes.c_int, [ctypes.POINTER(EdgeJob), c_vp]),
     "dgs_sample_blocks_weighted": (ctypes.c_int, [c_vp, c_i32, c_i64, View, View, View, ctypes.POINTER(c_i64), c_i32,
                                                   c_i32, c_u64, c_u32, c_vp, c_u32, c_vp, ctypes.POINTER(BlockOut),
                                                   c_vp, c_vp, ctypes.POINTER(c_vp), c_vp, c_sz, c_vp]),

@@ -793,6 +793,8 @@ class PendingBlocks : public torch::CustomClassHolder {
       sizes_dev = static_cast<int64_t*>(own(torch::empty({n_sizes}, opt.dtype(torch::kInt64))).data());
     }
     for (int h = 0; h < hops; ++h) outs[h] = dgs_block_out{p->src_[h].data(), p->dst_[h].data()};
+    dgs_view probs_view{};
+    if (probs) probs_view = probs->view();
     const size_t ws_bytes = probs ? dgs_sample_blocks_weighted_workspace_bytes(n, fanouts.data(), hops, w)
                                   : dgs_sample_blocks_workspace_bytes(n, fanouts.data(), hops, w);
     torch::Tensor ws = device_bytes(ws_bytes, dev);  // freed on return: the allocator reuses it in stream order
@@ -802,16 +804,20 @@ class PendingBlocks : public torch::CustomClassHolder {
     // the caller's own (seed, first stream) when given, else the next `hops` streams of the
     // process-wide generator
     const auto rng = own_rng != nullptr ? *own_rng : next_rng(static_cast<uint32_t>(hops));
-    if (probs)
-      check(dgs_sample_blocks_weighted(p->seeds_.data_ptr(), w, n, indptr->view(), indices->view(), probs->view(),
-                                       fanouts.data(), hops, replace, rng.first, rng.second, table.first,
-                                       table.second, p->all_.data(), outs.data(), sizes_dev,
-                                       p->pinned_.data_ptr<int64_t>(), nullptr, ws.data_ptr(), ws_bytes, st));
-    else
-      check(dgs_sample_blocks(p->seeds_.data_ptr(), w, n, indptr->view(), indices->view(), fanouts.data(), hops,
-                              replace, rng.first, rng.second, table.first, table.second, p->all_.data(),
-                              outs.data(), sizes_dev, p->pinned_.data_ptr<int64_t>(),
-                              nullptr, ws.data_ptr(), ws_bytes, st));
+    // The last hop's edge list is written by the launch that gathers the feature rows, where there is one.
+    // Not where that launch waits for another batch's gather: the list would wait with it (8 batches through
+    // the loader 1351 us, and 1378 with every list in its gather).
+    dgs_edge_job edges{};
+    check(dgs_sample_blocks_leave_edges(p->seeds_.data_ptr(), w, n, indptr->view(), indices->view(),
+                                        probs ? &probs_view : nullptr, fanouts.data(), hops, replace, rng.first, rng.second,
+                                        table.first, table.second, p->all_.data(), outs.data(), sizes_dev,
+                                        p->pinned_.data_ptr<int64_t>(), &edges, ws.data_ptr(), ws_bytes, st));
+    bool edges_left = true;
+    if (features && gather_after != nullptr) {
+      check(dgs_write_edges(&edges, st));
+      edges = dgs_edge_job{};
+      edges_left = false;
+    }
     if (features) {
       const auto xopt = torch::TensorOptions().dtype(features->dtype()).device(dev);
       const int64_t row_bytes = features->elem_stride() * static_cast<int64_t>(c10::elementSize(features->dtype()));
@@ -842,12 +848,13 @@ class PendingBlocks : public torch::CustomClassHolder {
         // 0.197 / 0.193 / 0.205 ms per step; the uniform sampler's kernels wait for memory, and its
         // steps are 9 % slower at 5 and 4)
         const int32_t gather_blocks_per_cu = probs ? 4 : 0;
-        p->gather_status_ = dgs_gather_rows_dyn_shared(features->view(), features->elem_stride(), p->all_.data(), w,
-                                                       buffer_rows, sizes_dev + hops, last,
-                                                       p->x_.data_ptr(), DGS_TIER_ANY, gather_blocks_per_cu,
-                                                       features->bad_index_word(), st);
+        p->gather_status_ = dgs_gather_rows_dyn_edges(features->view(), features->elem_stride(), p->all_.data(), w,
+                                                      buffer_rows, sizes_dev + hops, last, p->x_.data_ptr(), DGS_TIER_ANY,
+                                                      gather_blocks_per_cu, features->bad_index_word(), &edges, st);
+        edges_left = edges_left && p->gather_status_ != DGS_OK;
       }
     }
+    if (edges_left) check(dgs_write_edges(&edges, st));
     // the batch's one ticket, behind its last launch: it bounds the wait for the lengths, tells the
     // next batch's gather when this one's is through, and the graph when its node table is free again
     p->end_ = record_ticket(st);

@@ -14,7 +14,10 @@
 // Index values are checked before they address anything: a row outside the rows the
 // requested tier holds is not read, its output row is filled with zero bytes and the
 // caller's flag word (if any) is set.
+#include <string.h>
+
 #include "common.h"
+#include "edges.h"
 
 namespace dgs {
 namespace {
@@ -131,30 +134,73 @@ __device__ __forceinline__ bool gather_tile(const char* __restrict__ dev, const 
   return bad;
 }
 
+// What the blocks of a launch share.
+struct FlatGather {
+  const char* dev;
+  const char* host;
+  int64_t thr_bytes, row_bytes;
+  uint32_t cpr, magic;
+  int64_t total_chunks;
+  const int64_t* n_rows_dev;
+  int64_t row_lo, row_hi;
+  int64_t* bad_index;
+  char* out;
+};
+
 // STRIDE: the grid is smaller than the tile count (a launch sized for fewer rows than the output
 // holds) and blocks stride over the tiles; otherwise a block has exactly one tile and no loop in
 // its instruction stream.  `total_chunks` is the launch's worst case: what the index array and the
 // output hold.
 template <int VEC, int TIER, typename IndexT, bool STRIDE>
-__global__ __launch_bounds__(kGatherThreads) void gather_flat_kernel(
-    const char* __restrict__ dev, const char* __restrict__ host, int64_t thr_bytes,
-    int64_t row_bytes, uint32_t cpr, uint32_t magic, const IndexT* __restrict__ index,
-    int64_t total_chunks, const int64_t* __restrict__ n_rows_dev, int64_t row_lo, int64_t row_hi,
-    int64_t* __restrict__ bad_index, char* __restrict__ out) {
-  const int64_t first = int64_t(blockIdx.x) * kChunksPerBlock;
-  if (first >= total_chunks) return;
+__device__ __forceinline__ void gather_flat(const FlatGather& a, const IndexT* __restrict__ index, int64_t block, int64_t blocks) {
+  const int64_t first = block * kChunksPerBlock;
+  if (first >= a.total_chunks) return;
   int64_t counted;
-  bool bad = gather_tile<VEC, TIER, IndexT>(dev, host, thr_bytes, row_bytes, cpr, magic, index, total_chunks,
-                                            total_chunks, n_rows_dev, row_lo, row_hi, out, first, &counted);
+  bool bad = gather_tile<VEC, TIER, IndexT>(a.dev, a.host, a.thr_bytes, a.row_bytes, a.cpr, a.magic, index, a.total_chunks,
+                                            a.total_chunks, a.n_rows_dev, a.row_lo, a.row_hi, a.out, first, &counted);
   if (STRIDE) {  // the count is known from here on
-    for (int64_t c0 = first + int64_t(gridDim.x) * kChunksPerBlock; c0 < counted;
-         c0 += int64_t(gridDim.x) * kChunksPerBlock) {
+    for (int64_t c0 = first + blocks * kChunksPerBlock; c0 < counted; c0 += blocks * kChunksPerBlock) {
       int64_t unused;
-      bad |= gather_tile<VEC, TIER, IndexT>(dev, host, thr_bytes, row_bytes, cpr, magic, index, counted, counted,
-                                            nullptr, row_lo, row_hi, out, c0, &unused);
+      bad |= gather_tile<VEC, TIER, IndexT>(a.dev, a.host, a.thr_bytes, a.row_bytes, a.cpr, a.magic, index, counted, counted,
+                                            nullptr, a.row_lo, a.row_hi, a.out, c0, &unused);
     }
   }
-  if (bad && bad_index) *bad_index = 1;
+  if (bad && a.bad_index) *a.bad_index = 1;
+}
+template <int VEC, int TIER, typename IndexT, bool STRIDE>
+__global__ __launch_bounds__(kGatherThreads) void gather_flat_kernel(FlatGather a, const IndexT* __restrict__ index) {
+  gather_flat<VEC, TIER, IndexT, STRIDE>(a, index, blockIdx.x, gridDim.x);
+}
+
+// The same behind a sampler's last hop, whose edge list the first `edge_grid` blocks write: it hangs on the
+// same launch as the gather does, and its waits for memory go under the gather's traffic.
+// 1024 seeds, fanouts [5,10,15], 400-byte rows, one batch at a time 202.9 -> 199.0 us; R-MAT of 2^26 nodes,
+// [50,50] 374 -> 366, 111 M nodes 221 -> 215.
+static_assert(kGatherThreads == kEdgeBlock, "the blocks are shared");
+constexpr int64_t kEdgeGrid = 4096;  // at most: they loop over the worst case, most of which is not there
+template <int VEC, int TIER, typename IndexT, bool STRIDE>
+__global__ __launch_bounds__(kGatherThreads) void gather_flat_edges_kernel(FlatGather a, const IndexT* __restrict__ index,
+                                                                           EdgeJob edges, int32_t edge_grid) {
+  if (int64_t(blockIdx.x) >= edge_grid) {
+    gather_flat<VEC, TIER, IndexT, STRIDE>(a, index, int64_t(blockIdx.x) - edge_grid, int64_t(gridDim.x) - edge_grid);
+    return;
+  }
+  if (edges.blocks <= edge_grid) {
+    later_edge_tile<IndexT, true>(edges, blockIdx.x, threadIdx.x);
+  } else {
+    for (int64_t b = blockIdx.x; b < edges.blocks; b += edge_grid) later_edge_tile<IndexT, false>(edges, b, threadIdx.x);
+  }
+}
+template <typename IdT>
+__global__ __launch_bounds__(kEdgeBlock) void edges_kernel(EdgeJob edges) {
+  for (int64_t b = blockIdx.x; b < edges.blocks; b += gridDim.x) later_edge_tile<IdT, false>(edges, b, threadIdx.x);
+}
+dgs_status launch_edges(const EdgeJob& e, hipStream_t st) {
+  const dim3 grid(uint32_t(e.blocks < kEdgeGrid ? e.blocks : kEdgeGrid));
+  if (e.id_bytes == 8) hipLaunchKernelGGL(edges_kernel<int64_t>, grid, dim3(kEdgeBlock), 0, st, e);
+  else hipLaunchKernelGGL(edges_kernel<int32_t>, grid, dim3(kEdgeBlock), 0, st, e);
+  DGS_LAUNCH_CHECK();
+  return DGS_OK;
 }
 
 // ---- rows that are no multiple of 16 bytes -----------------------------------------------------
@@ -363,7 +409,8 @@ inline uint32_t reserved_lds(int32_t blocks_per_cu) {
 
 template <int VEC, int TIER, typename IndexT>
 dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index, int64_t n,
-                         const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad_index, void* out, hipStream_t st) {
+                         const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad_index, void* out,
+                         const EdgeJob* edges, hipStream_t st) {
   const int64_t cpr = row_bytes / VEC;
   const int64_t thr_bytes = v.threshold * v.elem_bytes;
   // rows the tier holds whole: the device tier the rows that end at or before the boundary, the
@@ -379,17 +426,27 @@ dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index
     const int64_t blocks = gather_blocks(tiles, (n_expected * cpr + kChunksPerBlock - 1) / kChunksPerBlock, n_dev != nullptr);
     const uint32_t magic = cpr > 1 ? uint32_t((uint64_t(1) << 32) / uint64_t(cpr)) + 1u : 0u;
     const uint32_t lds = reserved_lds(blocks_per_cu);
-    if (blocks < tiles)
-      hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, true>), dim3(uint32_t(blocks)),
-                         dim3(kGatherThreads), lds, st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
-                         magic, static_cast<const IndexT*>(index), total_chunks, n_dev, row_lo, row_hi,
-                         bad_index, static_cast<char*>(out));
-    else
-      hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, false>), dim3(uint32_t(blocks)),
-                         dim3(kGatherThreads), lds, st, dev, host, thr_bytes, row_bytes, uint32_t(cpr),
-                         magic, static_cast<const IndexT*>(index), total_chunks, n_dev, row_lo, row_hi,
-                         bad_index, static_cast<char*>(out));
+    const FlatGather a{dev, host, thr_bytes, row_bytes, uint32_t(cpr), magic, total_chunks, n_dev, row_lo, row_hi, bad_index,
+                       static_cast<char*>(out)};
+    const IndexT* ids = static_cast<const IndexT*>(index);
+    const dim3 block(kGatherThreads);
+    if (edges != nullptr) {
+      const int32_t edge_grid = int32_t(edges->blocks < kEdgeGrid ? edges->blocks : kEdgeGrid);
+      const dim3 grid(uint32_t(blocks + edge_grid));
+      if (blocks < tiles)
+        hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, TIER, IndexT, true>), grid, block, lds, st, a, ids, *edges, edge_grid);
+      else
+        hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, TIER, IndexT, false>), grid, block, lds, st, a, ids, *edges, edge_grid);
+    } else if (blocks < tiles) {
+      hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, true>), dim3(uint32_t(blocks)), block, lds, st, a, ids);
+    } else {
+      hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, false>), dim3(uint32_t(blocks)), block, lds, st, a, ids);
+    }
   } else {
+    if (edges != nullptr) {
+      const dgs_status es = launch_edges(*edges, st);
+      if (es != DGS_OK) return es;
+    }
     const int64_t bpr = (cpr + kChunksPerBlock - 1) / kChunksPerBlock;
     DGS_REQUIRE(n * bpr <= 0x7fffffff, DGS_ERR_UNSUPPORTED, "gather: %lld rows of %lld B exceed one launch",
                 (long long)n, (long long)row_bytes);
@@ -450,24 +507,29 @@ dgs_status launch_ragged(const dgs_view& v, int64_t row_bytes, const void* index
 template <int VEC, int TIER>
 dgs_status dispatch_index(const dgs_view& v, int64_t row_bytes, const void* index,
                           int32_t index_bytes, int64_t n, const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad,
-                          void* out, hipStream_t st) {
-  return index_bytes == 8 ? launch_gather<VEC, TIER, int64_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st)
-                          : launch_gather<VEC, TIER, int32_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
+                          void* out, const EdgeJob* edges, hipStream_t st) {
+  return index_bytes == 8 ? launch_gather<VEC, TIER, int64_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st)
+                          : launch_gather<VEC, TIER, int32_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
 }
 
 template <int TIER>
 dgs_status dispatch_vec(int vec, const dgs_view& v, int64_t row_bytes, const void* index,
                         int32_t index_bytes, int64_t n, const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, int64_t* bad,
-                        void* out, hipStream_t st) {
-  if (is_ragged(v, row_bytes, out, TIER, vec, n_dev && n_expected > 0 ? n_expected : n))
+                        void* out, const EdgeJob* edges, hipStream_t st) {
+  if (is_ragged(v, row_bytes, out, TIER, vec, n_dev && n_expected > 0 ? n_expected : n)) {
+    if (edges != nullptr) {
+      const dgs_status es = launch_edges(*edges, st);
+      if (es != DGS_OK) return es;
+    }
     return index_bytes == 8 ? launch_ragged<TIER, int64_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st)
                             : launch_ragged<TIER, int32_t>(v, row_bytes, index, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
+  }
   switch (vec) {
-    case 16: return dispatch_index<16, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    case 8: return dispatch_index<8, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    case 4: return dispatch_index<4, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    case 2: return dispatch_index<2, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    default: return dispatch_index<1, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
+    case 16: return dispatch_index<16, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    case 8: return dispatch_index<8, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    case 4: return dispatch_index<4, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    case 2: return dispatch_index<2, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    default: return dispatch_index<1, TIER>(v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
   }
 }
 
@@ -569,7 +631,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_scatter_kernel(
 namespace {
 dgs_status gather_entry(dgs_view v, int64_t row_elems, const void* index, int32_t index_bytes, int64_t n,
                         const int64_t* n_dev, int64_t n_expected, int32_t blocks_per_cu, void* out, int32_t tier, int64_t* bad,
-                        void* stream) {
+                        const dgs::EdgeJob* edges, void* stream) {
   using namespace dgs;
   DGS_REQUIRE(width_ok(index_bytes), DGS_ERR_INVALID, "gather: index width %d is not 4 or 8", index_bytes);
   DGS_REQUIRE(n >= 0 && row_elems > 0, DGS_ERR_INVALID, "gather: n=%lld row_elems=%lld", (long long)n,
@@ -593,9 +655,9 @@ dgs_status gather_entry(dgs_view v, int64_t row_elems, const void* index, int32_
   const int vec = pick_vec(v, row_bytes, out, tier);
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (tier) {
-    case DGS_TIER_DEVICE: return dispatch_vec<DGS_TIER_DEVICE>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    case DGS_TIER_HOST: return dispatch_vec<DGS_TIER_HOST>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
-    default: return dispatch_vec<DGS_TIER_ANY>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, st);
+    case DGS_TIER_DEVICE: return dispatch_vec<DGS_TIER_DEVICE>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    case DGS_TIER_HOST: return dispatch_vec<DGS_TIER_HOST>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
+    default: return dispatch_vec<DGS_TIER_ANY>(vec, v, row_bytes, index, index_bytes, n, n_dev, n_expected, blocks_per_cu, bad, out, edges, st);
   }
 }
 }  // namespace
@@ -603,7 +665,7 @@ dgs_status gather_entry(dgs_view v, int64_t row_elems, const void* index, int32_
 DGS_API dgs_status dgs_gather_rows(dgs_view v, int64_t row_elems, const void* index,
                                    int32_t index_bytes, int64_t n, void* out, int32_t tier,
                                    int64_t* bad_index, void* stream) {
-  return gather_entry(v, row_elems, index, index_bytes, n, nullptr, 0, 0, out, tier, bad_index, stream);
+  return gather_entry(v, row_elems, index, index_bytes, n, nullptr, 0, 0, out, tier, bad_index, nullptr, stream);
 }
 
 DGS_API dgs_status dgs_gather_rows_dyn(dgs_view v, int64_t row_elems, const void* index,
@@ -611,7 +673,7 @@ DGS_API dgs_status dgs_gather_rows_dyn(dgs_view v, int64_t row_elems, const void
                                        int64_t n_expected, void* out, int32_t tier, int64_t* bad_index,
                                        void* stream) {
   DGS_REQUIRE(n_rows_dev != nullptr, DGS_ERR_INVALID, "gather_dyn: null n_rows_dev");
-  return gather_entry(v, row_elems, index, index_bytes, n_max, n_rows_dev, n_expected, 0, out, tier, bad_index, stream);
+  return gather_entry(v, row_elems, index, index_bytes, n_max, n_rows_dev, n_expected, 0, out, tier, bad_index, nullptr, stream);
 }
 
 DGS_API dgs_status dgs_gather_rows_dyn_shared(dgs_view v, int64_t row_elems, const void* index,
@@ -621,7 +683,31 @@ DGS_API dgs_status dgs_gather_rows_dyn_shared(dgs_view v, int64_t row_elems, con
   DGS_REQUIRE(n_rows_dev != nullptr, DGS_ERR_INVALID, "gather_dyn_shared: null n_rows_dev");
   DGS_REQUIRE(blocks_per_cu >= 0, DGS_ERR_INVALID, "gather_dyn_shared: blocks_per_cu %d", blocks_per_cu);
   return gather_entry(v, row_elems, index, index_bytes, n_max, n_rows_dev, n_expected, blocks_per_cu, out, tier, bad_index,
-                      stream);
+                      nullptr, stream);
+}
+
+DGS_API dgs_status dgs_gather_rows_dyn_edges(dgs_view v, int64_t row_elems, const void* index, int32_t index_bytes,
+                                             int64_t n_max, const int64_t* n_rows_dev, int64_t n_expected, void* out,
+                                             int32_t tier, int32_t blocks_per_cu, int64_t* bad_index,
+                                             const dgs_edge_job* left, void* stream) {
+  DGS_REQUIRE(n_rows_dev != nullptr && left != nullptr, DGS_ERR_INVALID, "gather_dyn_edges: null n_rows_dev or job");
+  DGS_REQUIRE(blocks_per_cu >= 0, DGS_ERR_INVALID, "gather_dyn_edges: blocks_per_cu %d", blocks_per_cu);
+  dgs::EdgeJob job;
+  memcpy(&job, left, sizeof(job));
+  if (job.blocks > 0 && (n_max == 0 || job.id_bytes != index_bytes)) {  // not in one launch
+    const dgs_status s = dgs::launch_edges(job, static_cast<hipStream_t>(stream));
+    if (s != DGS_OK) return s;
+    job.blocks = 0;
+  }
+  return gather_entry(v, row_elems, index, index_bytes, n_max, n_rows_dev, n_expected, blocks_per_cu, out, tier, bad_index,
+                      job.blocks > 0 ? &job : nullptr, stream);
+}
+
+DGS_API dgs_status dgs_write_edges(const dgs_edge_job* left, void* stream) {
+  DGS_REQUIRE(left != nullptr, DGS_ERR_INVALID, "write_edges: null job");
+  dgs::EdgeJob job;
+  memcpy(&job, left, sizeof(job));
+  return job.blocks > 0 ? dgs::launch_edges(job, static_cast<hipStream_t>(stream)) : DGS_OK;
 }
 
 DGS_API size_t dgs_split_index_workspace_bytes(int64_t n) {

@@ -44,11 +44,14 @@
 // as early as its address is known: a hop's length lives in device memory, but every buffer has
 // its worst-case size, so a thread asks for its own elements (inside the buffer whatever the
 // length turns out to be) together with the length and only then decides whether they count.
+#include <string.h>
+
 #include <algorithm>
 #include <type_traits>
 
 #include "choose.h"
 #include "common.h"
+#include "edges.h"
 #include "lookback.h"
 #include "one_block.h"
 #include "picks.h"
@@ -58,7 +61,7 @@ namespace dgs {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kRowTile = 256;                  // seed rows per relabel tile
+static_assert(kBlock == kEdgeBlock, "edge lists are written by surplus blocks of the fills");
 constexpr int kRowItems = 4;                   // rows a thread of a compact block takes
 // What a compact block's tile is, by the hop's worst case: NT threads x ITEMS consecutive positions x
 // GROUPS.  A few hundred tiles at most for the look-back (see lookback.h), but no fewer blocks than a
@@ -79,13 +82,7 @@ inline int64_t pos_tile_size(int64_t len_max) {
 }
 inline int64_t row_tile_size(int64_t len_max) { return (pos_tile_kind(len_max) == kLongTile ? 512 : 256) * kRowItems; }
 constexpr int kMaxPosTile = 8192;
-constexpr uint32_t kFirstBit = 0x80000000u;
 constexpr uint32_t kInvalidSlot = 0xffffffffu; // padded position that holds no pick
-// row_cnt markers of rows that make the call fail (bit (kBadRow - marker) of the hop's flag word)
-constexpr uint32_t kBadRow = 0xffffffffu;      // degree >= 2^32, or offsets outside the edge array
-constexpr uint32_t kBadSeed = 0xfffffffeu;     // the seed id is not a row of the graph
-constexpr uint32_t kBadPick = 0xfffffffdu;     // a picked neighbour id is outside what the table holds
-__device__ __forceinline__ bool is_bad_row(uint32_t row_cnt) { return row_cnt >= kBadPick; }
 constexpr int kErrBucketOverflow = 8;          // hop flag bit: the ids of a bucket of the hashed pass did not fit its LDS table
 constexpr int kMaxPicks = 64;
 constexpr int64_t kMaxPositions = int64_t(1) << 30;
@@ -137,7 +134,7 @@ struct Hop {
   uint32_t* row_cnt;        // [s_max] picks of every row (kBadRow on error)
   uint32_t* row_off;        // [s_max] first packed edge of the row
   tile_state* row_state;    // [row tiles] the tiles' edge counts, in the course of their scan
-  uint32_t* slot;           // [all positions] what is known of a position's id (see Slot words)
+  uint32_t* slot;           // [all positions] what is known of a position's id (see edges.h)
   uint32_t* rank_at;        // [all positions] rank of the id first seen there; of a lost position: a smaller one | kLinkBit
   uint8_t* lost;            // [all positions] non-zero: a smaller position of the same id exists
   int64_t* long_rows;       // weighted only: ranks of the frontier's rows of more than kLongRow positions ...
@@ -162,12 +159,7 @@ struct Hop {
   int64_t n_edges;
 };
 
-// (written without a conditional so that the read is not moved behind a test)
-__device__ __forceinline__ int64_t seeds_of(const Hop& h) {
-  const int64_t on_device = *h.n_seeds;
-  const int64_t use_device = h.n_seeds_host >> 63;  // all ones when the count lives on the device
-  return (on_device & use_device) | (h.n_seeds_host & ~use_device);
-}
+__device__ __forceinline__ int64_t seeds_of(const Hop& h) { return count_of(h.n_seeds, h.n_seeds_host); }
 // Whether this hop finds its first occurrences by the bucketed pass.  Its worst case may be far
 // beyond what the pass has room for (it grows with the product of the fanouts, the hop does not),
 // so the host only says whether the hop is eligible and every kernel decides from the hop's real
@@ -184,8 +176,6 @@ __device__ __forceinline__ int64_t first_rank(const Hop& h, int64_t s) { return 
 constexpr int kFoldSlotBits = 7;
 constexpr int kFoldSlots = 1 << kFoldSlotBits;
 constexpr int kFoldMaxRowPerPick = 4;
-constexpr int kRelabelItems = 4;  // padded picks per thread in relabel_tile
-__host__ __device__ __forceinline__ int relabel_groups(int k) { return (k + kRelabelItems - 1) / kRelabelItems; }
 
 // ---- a large last hop without memory-side atomics -------------------------------------------
 // The atomicMin per pick is what a large hop costs most (every device-scope atomic executes at
@@ -209,7 +199,6 @@ constexpr int kBucketRange = 8192;                   // ids per bucket at most: 
 constexpr int kMaxBucketTiles = 2048;                // tiles a bucket's block can walk (its LDS index of them)
 constexpr int64_t kBucketedMaxNodes = int64_t(kMaxBuckets) * kBucketRange;
 constexpr int64_t kBucketedMinPicks = int64_t(1) << 18;  // worst-case picks of the hop below which the table is cheaper
-constexpr uint32_t kRankBit = 0x40000000u;
 // Graphs with more nodes than kBucketedMaxNodes: buckets by a hash of the id, and a bucket's ids
 // are told apart in an open-addressing table in LDS (ids + smallest order values, 128 KB of the
 // CU's 160 KB) instead of an array indexed by the id's high bits.  A bucket may hold up to half as
@@ -245,27 +234,6 @@ __device__ __forceinline__ uint32_t bucket_of(const Buckets& b, int log_buckets,
   return (b.hashed ? hash_id(id) : id) & uint32_t((1 << log_buckets) - 1);
 }
 
-// ---- Slot words ----
-//
-// What the slot word of a position says when its edge is written out:
-//   kFirstBit | table slot    the first occurrence of its id: its rank is at the position itself;
-//   kRankBit | rank           the rank itself (bucketed hops);
-//   a position                of the same id and smaller, or the position's own where it has lost its bit:
-//                             the rank is there, or a link to a smaller position;
-//   table slot                in hop 0, whose first occurrences are settled by asking the table.
-// A pick that is not its id's first has met a smaller position of the id when it was inserted.  That one may
-// itself be displaced later in the same launch: whoever does so leaves a link to its own position in rank_at,
-// and positions only get smaller along the links.  Reading these words, a stream and some 4-byte reads near
-// one another, in place of the table's entry saves a random read of a table that caches do not hold: R-MAT of
-// 2^26 nodes, 3.05 M picks, two thirds of them repeats: 44 -> 25 us for the hop's edge list, 380 -> 369 for the batch.
-constexpr uint32_t kLinkBit = 0x80000000u;
-
-// rank at position `at`, or where the links from there lead
-__device__ __forceinline__ uint32_t rank_from(const Hop& h, uint32_t at) {
-  uint32_t r = h.rank_at[at];
-  while (r & kLinkBit) r = h.rank_at[r & ~kLinkBit];
-  return r;
-}
 // rank of the id at position p of hop 0, given p's slot word
 template <typename TableT>
 __device__ __forceinline__ uint32_t rank_of(const Hop& h, const TableT& table, int64_t p, uint32_t slot_word) {
@@ -349,90 +317,32 @@ __device__ __forceinline__ void offsets_tile(const Hop& h, int64_t tile) {
   }
 }
 
-// One block per (256-row tile, 4 x 256 padded picks): writes the rows' edges at their packed
-// offsets; a thread handles four picks, 256 apart, so that a wave has four times the loads in
-// flight and the launch a quarter of the waves.  src_local = rank of the picked id; dst_local = rank of the row's seed, which is
-// the row number itself except in hop 0, whose seeds may repeat.
-//
-// EARLY (here and in the other tile functions): the launch is about as large as the hop really
-// is, so a thread requests its own elements together with the hop's length and tests afterwards.
-// Without it the launch was sized for a worst case that may exceed the hop many times over
-// (and loops over its virtual blocks): the length is waited for first and blocks beyond it
-// leave without having read anything.
+__host__ __device__ __forceinline__ EdgeJob edge_job(const Hop& h) {
+  EdgeJob e{};
+  e.n_seeds = h.n_seeds;
+  e.n_seeds_host = h.n_seeds_host;
+  e.row_cnt = h.row_cnt;
+  e.row_off = h.row_off;
+  e.slot = h.slot;
+  e.rank_at = h.rank_at;
+  e.src_local = h.src_local;
+  e.dst_local = h.dst_local;
+  e.s_max = h.s_max;
+  e.first = h.pos_base + (h.index == 0 ? h.n_seeds_host : 0);  // (the caller's count: positions hang on no load)
+  e.bucket_pos_cap = h.bucketed != 0 ? h.bucket_pos_cap : -1;
+  e.k = h.k;
+  return e;
+}
 template <typename IdT, typename TableT, bool EARLY>
 __device__ __forceinline__ void relabel_tile(const Hop& h, const TableT& table, int64_t b, int tid) {
-  const int k = h.k;
-  if (k == 0) return;
-  const int groups = relabel_groups(k);
-  const int64_t tile = b / groups;
-  const int group = int(b - tile * groups);
-  // the hop's length and this thread's own rows and picks, requested together
-  const int64_t s = seeds_of(h);
-  if (!EARLY && tile * kRowTile >= s) return;
-  // (hop 0's seed part is the caller's count, a kernel argument: positions hang on no load)
-  const int64_t p0 = h.pos_base + (h.index == 0 ? h.n_seeds_host : 0);
-  int64_t i[kRelabelItems], p[kRelabelItems];
-  int l[kRelabelItems];
-  bool mine[kRelabelItems];
-  uint32_t rc[kRelabelItems], off[kRelabelItems], word[kRelabelItems], seed_word[kRelabelItems];
-#pragma unroll
-  for (int j = 0; j < kRelabelItems; ++j) {
-    const int chunk = group * kRelabelItems + j;
-    const int t = chunk * kBlock + tid;  // padded pick inside the tile
-    const int r = t / k;
-    l[j] = t - r * k;
-    i[j] = tile * kRowTile + r;
-    p[j] = p0 + i[j] * k + l[j];
-    mine[j] = chunk < k && i[j] < h.s_max;
-    rc[j] = off[j] = word[j] = seed_word[j] = 0;
-    if (mine[j]) {
-      rc[j] = h.row_cnt[i[j]];
-      off[j] = h.row_off[i[j]];
-      word[j] = h.slot[p[j]];
-      if (h.index == 0) seed_word[j] = h.slot[h.pos_base + i[j]];
-    }
+  const EdgeJob e = edge_job(h);
+  if (h.index != 0) {
+    later_edge_tile<IdT, EARLY>(e, b, tid);
+    return;
   }
-  if (tile * kRowTile >= s) return;  // whole blocks leave together
-  // Rank of a pick = rank recorded at the smallest position of its id (see Slot words).  Rounds of
-  // loads, each issued for all of the thread's picks before any is used.
-  const bool bucketed = bucketed_now(h, s);
-  bool live[kRelabelItems];
-  bool known[kRelabelItems];  // bucketed hop: the word of a repeat may be the rank itself
-  uint32_t at[kRelabelItems];
-#pragma unroll
-  for (int j = 0; j < kRelabelItems; ++j) {
-    live[j] = mine[j] && i[j] < s && !is_bad_row(rc[j]) && uint32_t(l[j]) < rc[j];
-    at[j] = uint32_t(p[j]);
-    known[j] = false;
-    if (live[j] && !(word[j] & kFirstBit)) {
-      if (h.index == 0) {
-        at[j] = table.value(word[j]);
-      } else {
-        known[j] = bucketed && (word[j] & kRankBit) != 0;
-        at[j] = known[j] ? word[j] & (kRankBit - 1) : word[j];
-      }
-    }
-  }
-  uint32_t rank[kRelabelItems];
-#pragma unroll
-  for (int j = 0; j < kRelabelItems; ++j) rank[j] = !live[j] ? 0u : known[j] ? at[j] : h.rank_at[at[j]];
-  if ((rank[0] | rank[1] | rank[2] | rank[3]) & kLinkBit) {
-#pragma unroll
-    for (int j = 0; j < kRelabelItems; ++j)
-      if (rank[j] & kLinkBit) rank[j] = rank_from(h, rank[j] & ~kLinkBit);
-  }
-#pragma unroll
-  for (int j = 0; j < kRelabelItems; ++j) {
-    if (!live[j]) continue;
-    const int64_t o = int64_t(off[j]) + l[j];
-    static_cast<IdT*>(h.src_local)[o] = IdT(rank[j]);
-    static_cast<IdT*>(h.dst_local)[o] =
-        h.index == 0 ? IdT(rank_of(h, table, h.pos_base + i[j], seed_word[j])) : IdT(i[j]);
-  }
-}
-
-inline int64_t relabel_blocks(int64_t s_max, int k) {
-  return ((s_max + kRowTile - 1) / kRowTile) * relabel_groups(k);
+  edge_tile<IdT, EARLY>(
+      e, b, tid, [&](int64_t, uint32_t word, bool*) { return table.value(word); },
+      [&](int64_t i) { return rank_of(h, table, h.pos_base + i, h.slot[h.pos_base + i]); });
 }
 
 // ---- critical path ------------------------------------------------------------------------
@@ -1638,7 +1548,7 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
 // The packed edge list of one hop as a launch of its own.
 template <typename IdT, typename TableT>
 void launch_relabel(const Hop& hop, const TableT& table, hipStream_t st) {
-  const int64_t blocks = relabel_blocks(hop.s_max, hop.k);
+  const int64_t blocks = edge_blocks(hop.s_max, hop.k);
   if (blocks <= 0) return;
   if (is_capped(blocks))
     hipLaunchKernelGGL((hop_relabel_kernel<IdT, TableT, true>), dim3(capped_grid(blocks)), dim3(kBlock), 0, st, hop,
@@ -1721,11 +1631,11 @@ void launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count
 template <typename IdT, typename PtrT, typename TableT>
 dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const TableT& table, const dgs_view& indptr,
                       const dgs_view& indices, const dgs_view* probs, bool replace, uint64_t rng_seed,
-                      void** sizes_ticket, hipStream_t st) {
+                      void** sizes_ticket, EdgeJob* left, hipStream_t st) {
   for (int h = 0; h < p.n_hops; ++h) {
     const Hop& cur = hops[h];
     const Hop prev = h > 0 ? hops[h - 1] : Hop{};
-    const int64_t surplus = h > 0 ? relabel_blocks(prev.s_max, prev.k) : 0;
+    const int64_t surplus = h > 0 ? edge_blocks(prev.s_max, prev.k) : 0;
     // the launch of hop 0 also clears the lost marks of all later hops and the tile states of all
     // hops, which lie behind them
     uint4* clear_begin = nullptr;
@@ -1773,7 +1683,14 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
     const dgs_status ts = dgs_ticket_record(st, sizes_ticket);
     if (ts != DGS_OK) return ts;
   }
-  launch_relabel<IdT>(hops[p.n_hops - 1], table, st);
+  const Hop& last = hops[p.n_hops - 1];
+  if (left != nullptr && p.n_hops > 1) {
+    *left = edge_job(last);
+    left->blocks = edge_blocks(last.s_max, last.k);
+    left->id_bytes = int32_t(sizeof(IdT));
+    return DGS_OK;
+  }
+  launch_relabel<IdT>(last, table, st);
   DGS_LAUNCH_CHECK();
   return DGS_OK;
 }
@@ -1817,21 +1734,21 @@ dgs_status run_one_block(const Plan& p, const Hop* hops, int64_t* sizes, const d
 template <typename IdT, typename PtrT>
 dgs_status run_blocks_table(const Plan& p, Hop* hops, const Buckets& buckets, void* hash_table, void* node_table,
                             uint32_t epoch, const dgs_view& indptr, const dgs_view& indices, const dgs_view* probs,
-                            bool replace, uint64_t rng_seed, void** sizes_ticket, hipStream_t st) {
+                            bool replace, uint64_t rng_seed, void** sizes_ticket, EdgeJob* left, hipStream_t st) {
   if (one_block_fits(p))
     return run_one_block<IdT, PtrT>(p, hops, hops[0].n_seeds_out, indptr, indices, replace, rng_seed, sizes_ticket, st);
   if (p.kind == TableKind::kDirect)
     return run_blocks<IdT, PtrT, DirectTable<IdT>>(p, hops, buckets, DirectTable<IdT>(node_table, epoch, uint32_t(indptr.total - 1)),
-                                                   indptr, indices, probs, replace, rng_seed, sizes_ticket, st);
+                                                   indptr, indices, probs, replace, rng_seed, sizes_ticket, left, st);
   const int64_t n16 = int64_t(p.table_bytes / 16);
   hipLaunchKernelGGL(clear_kernel, dim3(capped_grid((n16 + kBlock - 1) / kBlock)), dim3(kBlock), 0, st,
                      static_cast<uint4*>(hash_table), n16);
   DGS_LAUNCH_CHECK();
   if (p.kind == TableKind::kPacked)
     return run_blocks<IdT, PtrT, Table<IdT, true>>(p, hops, buckets, Table<IdT, true>(hash_table, p.capacity), indptr,
-                                                   indices, probs, replace, rng_seed, sizes_ticket, st);
+                                                   indices, probs, replace, rng_seed, sizes_ticket, left, st);
   return run_blocks<IdT, PtrT, Table<IdT, false>>(p, hops, buckets, Table<IdT, false>(hash_table, p.capacity), indptr,
-                                                  indices, probs, replace, rng_seed, sizes_ticket, st);
+                                                  indices, probs, replace, rng_seed, sizes_ticket, left, st);
 }
 
 }  // namespace
@@ -1878,8 +1795,8 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
                                dgs_view indices, const dgs_view* probs, const int64_t* fanouts, int32_t n_hops,
                                int32_t replace, uint64_t rng_seed, uint32_t first_stream, void* node_table,
                                uint32_t node_table_epoch, void* frontier, const dgs_block_out* outs,
-                               int64_t* sizes_dev, int64_t* sizes_host, void** sizes_ticket, void* workspace,
-                               size_t workspace_bytes, void* stream) {
+                               int64_t* sizes_dev, int64_t* sizes_host, void** sizes_ticket, dgs::EdgeJob* left,
+                               void* workspace, size_t workspace_bytes, void* stream) {
   using namespace dgs;
   Plan p;
   // node count = indptr entries - 1
@@ -1949,11 +1866,11 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
   const bool rep = replace != 0;
   if (id_bytes == 8)
     return indptr.elem_bytes == 8
-               ? run_blocks_table<int64_t, int64_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, st)
-               : run_blocks_table<int64_t, int32_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, st);
+               ? run_blocks_table<int64_t, int64_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, left, st)
+               : run_blocks_table<int64_t, int32_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, left, st);
   return indptr.elem_bytes == 8
-             ? run_blocks_table<int32_t, int64_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, st)
-             : run_blocks_table<int32_t, int32_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, st);
+             ? run_blocks_table<int32_t, int64_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, left, st)
+             : run_blocks_table<int32_t, int32_t>(p, hops, buckets, hash_table, node_table, node_table_epoch, indptr, indices, probs, rep, rng_seed, sizes_ticket, left, st);
 }
 }  // namespace
 
@@ -1965,7 +1882,7 @@ DGS_API dgs_status dgs_sample_blocks(const void* seeds, int32_t id_bytes, int64_
                                      void* workspace, size_t workspace_bytes, void* stream) {
   return sample_blocks_entry(seeds, id_bytes, n_seeds, indptr, indices, nullptr, fanouts, n_hops, replace, rng_seed,
                              first_stream, node_table, node_table_epoch, frontier, outs, sizes_dev, sizes_host,
-                             sizes_ticket, workspace, workspace_bytes, stream);
+                             sizes_ticket, nullptr, workspace, workspace_bytes, stream);
 }
 
 DGS_API dgs_status dgs_sample_blocks_weighted(const void* seeds, int32_t id_bytes, int64_t n_seeds, dgs_view indptr,
@@ -1977,5 +1894,22 @@ DGS_API dgs_status dgs_sample_blocks_weighted(const void* seeds, int32_t id_byte
                                               size_t workspace_bytes, void* stream) {
   return sample_blocks_entry(seeds, id_bytes, n_seeds, indptr, indices, &probs, fanouts, n_hops, replace, rng_seed,
                              first_stream, node_table, node_table_epoch, frontier, outs, sizes_dev, sizes_host,
-                             sizes_ticket, workspace, workspace_bytes, stream);
+                             sizes_ticket, nullptr, workspace, workspace_bytes, stream);
+}
+
+static_assert(sizeof(dgs::EdgeJob) <= sizeof(dgs_edge_job), "a job fits the caller's words");
+DGS_API dgs_status dgs_sample_blocks_leave_edges(const void* seeds, int32_t id_bytes, int64_t n_seeds, dgs_view indptr,
+                                                 dgs_view indices, const dgs_view* probs, const int64_t* fanouts,
+                                                 int32_t n_hops, int32_t replace, uint64_t rng_seed, uint32_t first_stream,
+                                                 void* node_table, uint32_t node_table_epoch, void* frontier,
+                                                 const dgs_block_out* outs, int64_t* sizes_dev, int64_t* sizes_host,
+                                                 dgs_edge_job* left, void* workspace, size_t workspace_bytes, void* stream) {
+  DGS_REQUIRE(left != nullptr, DGS_ERR_INVALID, "sample_blocks_leave_edges: null job");
+  dgs::EdgeJob job{};
+  const dgs_status s = sample_blocks_entry(seeds, id_bytes, n_seeds, indptr, indices, probs, fanouts, n_hops, replace, rng_seed,
+                                           first_stream, node_table, node_table_epoch, frontier, outs, sizes_dev, sizes_host,
+                                           nullptr, &job, workspace, workspace_bytes, stream);
+  *left = dgs_edge_job{};
+  memcpy(left, &job, sizeof(job));
+  return s;
 }

@@ -515,6 +515,30 @@ dgs_status dgs_sample_blocks_weighted(const void* seeds, int32_t id_bytes, int64
                                       int64_t* sizes_host, void** sizes_ticket,
                                       void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * dgs_sample_blocks (probs NULL) or dgs_sample_blocks_weighted without the launch that writes the
+ * last hop's edge list: *left says what is left to write (nothing in a call of one hop or of few
+ * seeds) and is given, once, to dgs_gather_rows_dyn_edges or dgs_write_edges on the same stream,
+ * while the workspace and the outputs are alive.  The job's words are the library's own.
+ * dgs_gather_rows_dyn_edges is dgs_gather_rows_dyn_shared with that list written by blocks of
+ * the same launch: a launch of its own is 5 to 8 us on the stream of a batch that runs alone.
+ * No counterpart in the reference.
+ */
+typedef struct dgs_edge_job { uint64_t words[16]; } dgs_edge_job;
+dgs_status dgs_sample_blocks_leave_edges(const void* seeds, int32_t id_bytes, int64_t n_seeds, dgs_view indptr,
+                                         dgs_view indices, const dgs_view* probs, const int64_t* fanouts,
+                                         int32_t n_hops, int32_t replace, uint64_t rng_seed,
+                                         uint32_t first_stream, void* node_table, uint32_t node_table_epoch,
+                                         void* frontier, const dgs_block_out* outs, int64_t* sizes_dev,
+                                         int64_t* sizes_host, dgs_edge_job* left, void* workspace,
+                                         size_t workspace_bytes, void* stream);
+dgs_status dgs_gather_rows_dyn_edges(dgs_view v, int64_t row_elems, const void* index, int32_t index_bytes,
+                                     int64_t n_max, const int64_t* n_rows_dev, int64_t n_expected, void* out,
+                                     int32_t tier, int32_t blocks_per_cu, int64_t* bad_index,
+                                     const dgs_edge_job* left, void* stream);
+dgs_status dgs_write_edges(const dgs_edge_job* left, void* stream);
+
+
 /* ------------------------------------------------------------------------ */
 /* Placement                                                                 */
 /* ------------------------------------------------------------------------ */

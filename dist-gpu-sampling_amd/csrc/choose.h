@@ -2,12 +2,16 @@
 // weights and draws instead of rows.  Half of all rows have a few dozen neighbours; a wave per row leaves
 // most of its lanes idle and pays a sort, or three passes over the weights, for each.
 //
-// Without replacement (race_rows) the race runs on 32-bit floats first.  approx_key is off by less than
+// Without replacement (race_rows) the race runs on 32-bit floats first.  An approximate key is off by less than
 // half of what surely_less asks for, so entries that it orders are ordered as the 64-bit keys are; where the
 // num_picks + 1 smallest of a row are not all surely ordered (one row in some thousands), 64-bit keys settle
 // it (race.h).  Rows of up to kShortRow positions: four positions to a lane, which is one Philox block, and
-// then every position counts the smaller ones of its row.  Longer ones: a wave per row that keeps what is
-// below a bar in an LDS list and lowers the bar when the list fills.
+// then every position counts the smaller ones of its row.  Longer ones: a wave per row, or a block, that keeps
+// what is below a bar in an LDS list and lowers the bar when the list fills.
+//
+// Any weight above 0 has a float key.  Where one weight outside 2^-120 .. 2^90 sent its row to 64-bit keys, by
+// one wave: 256 rows of 17 000 with one infinite weight each 171 us a call and now 68 (without it 67), two rows of
+// 10^6 6.7 ms and 0.8, 1024 seeds, fanouts [5,10,10], rows of 60 with a fifth of the weights infinite 288 and 130.
 //
 // Measured, before (a wave per row, sorts, three passes over the weights) and with this: the hops of a batch of
 // 1024 seeds, fanouts [5,10,15], rows of mean degree 50 up to 17 000, 28 / 36 / 84 us and 32 for the long rows'
@@ -28,6 +32,8 @@ namespace dgs {
 // positions that are ranked by counting (64: the same batch 277 us for 274; 21 k rows of 100, 64 picks 172 for 146)
 constexpr uint32_t kShortRow = 128;
 constexpr uint32_t kOutOfRace = 0xffffffffu;     // key bits of no position
+constexpr uint32_t kLeastKey = 0x01000000u;      // 2^-125; below it: positions of infinite weights, in their order
+constexpr uint32_t kLargestKey = 0x7e000000u;    // 2^125
 constexpr uint32_t kUnusableKey = 0x7e800000u;   // from here on: positions of weights that are not > 0, in their order
 constexpr float kSureRatio = 1.0f + 0x1p-19f;
 
@@ -49,17 +55,23 @@ __device__ __forceinline__ float approx_neg_log_u32(uint32_t x) {
   return x & 0x80000000u ? high : low;
 }
 
-// The race key of position p as the bits of a float (positive: they order like the values).  `odd`: the
-// weight is beyond what the float arithmetic is good for, and the row has to be raced on 64-bit keys.
-__device__ __forceinline__ uint32_t approx_key(uint32_t x, float w, uint32_t p, bool* odd) {
-  if (!(w > 0.0f)) return kUnusableKey + (p < 0xffffffu ? p : 0xffffffu);
-  *odd |= !(w >= 0x1p-120f && w <= 0x1p90f);
-  return __float_as_uint(approx_neg_log_u32(x) * __builtin_amdgcn_rcpf(w));
+// Race keys are the bits of positive floats (they order like the values).  A plain weight has its key by one
+// reciprocal.  The others have keys too: one that leaves the range from kLeastKey to kLargestKey is set to
+// the end that it left by, which surely_less orders against the keys inside as it orders the true one, and leaves
+// open against its like.
+__device__ __forceinline__ bool plain_weight(float w) { return w >= 0x1p-120f && w <= 0x1p90f; }
+__device__ __forceinline__ uint32_t uncommon_key(float e, float w, uint32_t p) {
+  const uint32_t in_order = p < 0xfffffeu ? p : 0xfffffeu;
+  if (!(w > 0.0f)) return kUnusableKey + in_order;
+  if (w > 3.4028234663852886e38f) return 1u + in_order;  // (the 64-bit keys are all 0)
+  const float scale = w < 1.0f ? 0x1p64f : 0x1p-64f;     // the reciprocal is of a number far from either end
+  const float key = e * __builtin_amdgcn_rcpf(w * scale) * scale;
+  return __float_as_uint(fminf(fmaxf(key, __uint_as_float(kLeastKey)), __uint_as_float(kLargestKey)));
 }
 
 // Whether the 64-bit key behind `a` is smaller than the one behind `b` for sure.
 __device__ __forceinline__ bool surely_less(uint32_t a, uint32_t b) {
-  return __uint_as_float(b) > __uint_as_float(a) * kSureRatio || (a >= kUnusableKey && b > a);
+  return __uint_as_float(b) > __uint_as_float(a) * kSureRatio || ((a >= kUnusableKey || a < kLeastKey) && b > a);
 }
 
 __device__ __forceinline__ void wave_lds_fence() {
@@ -80,15 +92,28 @@ __device__ __forceinline__ float4_anywhere weight_quad(const TierView<float>& pr
   return w;
 }
 
-// Approximate keys of positions [p, p + 4) (p a multiple of 4) of a row, of weights w; kOutOfRace beyond it.
+// Approximate keys of positions [p, p + 4) (p a multiple of 4) of a row, of weights w (0 beyond it); kOutOfRace
+// beyond it.
 __device__ __forceinline__ uint4 approx_key_quad(float4_anywhere w, uint32_t p, uint32_t deg, uint64_t rng_seed,
-                                                 uint32_t rng_stream, int64_t row, bool* odd) {
+                                                 uint32_t rng_stream, int64_t row) {
   const PhiloxWords x = philox4x32_10(0x80000000u | (p >> 2), rng_stream, uint32_t(uint64_t(row)),
                                       uint32_t(uint64_t(row) >> 32), uint32_t(rng_seed), uint32_t(rng_seed >> 32));
+  float e[4];  // 2^-33 to 23
   uint32_t key[4];
+  bool plain = true;
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-    key[c] = p < deg && deg - p > uint32_t(c) ? approx_key(x.w[c], w[c], p + c, odd) : kOutOfRace;
+  for (int c = 0; c < 4; ++c) {
+    e[c] = approx_neg_log_u32(x.w[c]);
+    key[c] = __float_as_uint(e[c] * __builtin_amdgcn_rcpf(w[c]));
+    plain &= plain_weight(w[c]);
+  }
+  if (!plain) {  // (one branch for all four, and for positions beyond the row: a branch for each is 5 % of a long row's time)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (!(p < deg && deg - p > uint32_t(c))) key[c] = kOutOfRace;
+      else if (!plain_weight(w[c])) key[c] = uncommon_key(e[c], w[c], p + c);
+    }
+  }
   return make_uint4(key[0], key[1], key[2], key[3]);
 }
 
@@ -109,11 +134,11 @@ struct ListRace {
   int n = 0;
   uint32_t bar = kOutOfRace;
   uint32_t dropped = kOutOfRace;
-  bool odd = false;  // this lane has met something that only 64-bit keys settle
+  bool open = false;  // only 64-bit keys of the whole row settle it
 };
 
 // Lowers the bar so that num_picks to num_picks + kListSlack entries stay.  (Equal keys may make that
-// impossible: the race is marked odd then.)
+// impossible: the race is left open then.)
 __device__ __forceinline__ void list_tighten(WaveList& list, ListRace& r, int k) {
   constexpr int kEach = kListRoom / kWave;
   const int lane = threadIdx.x & (kWave - 1);
@@ -125,7 +150,7 @@ __device__ __forceinline__ void list_tighten(WaveList& list, ListRace& r, int k)
     key[u] = e < r.n ? list.key[e] : kOutOfRace;
     pos[u] = e < r.n ? list.pos[e] : kNoPos;
   }
-  uint32_t lo = 0, hi = r.bar - 1;  // fewer than k entries are at or below lo (0 is no key unless the race is odd)
+  uint32_t lo = 0, hi = r.bar - 1;  // fewer than k entries are at or below lo (0 is no key)
   int kept = 0;
 #pragma unroll
   for (int u = 0; u < kEach; ++u) kept += __builtin_popcountll(__ballot(key[u] <= hi));
@@ -142,7 +167,7 @@ __device__ __forceinline__ void list_tighten(WaveList& list, ListRace& r, int k)
     }
   }
   const bool stuck = kept > k + kListSlack;
-  r.odd |= stuck;
+  r.open |= stuck;
   wave_lds_fence();
   int at = 0;
 #pragma unroll
@@ -232,7 +257,7 @@ __device__ __forceinline__ bool list_finish(WaveList& list, ListRace& r, int k, 
   if (lane == 0 && (r.n <= k || next < entry_key[k])) entry_key[k] = next;
   wave_lds_fence();
   const bool unsure = lane < k && !surely_less(entry_key[lane], entry_key[lane + 1]);
-  if (__ballot(r.odd) != 0) return false;
+  if (__ballot(r.open) != 0) return false;
   if (__ballot(unsure) == 0) return true;
   const uint32_t last = entry_key[k - 1];
   if (last == 0 || !surely_less(last, next)) return false;
@@ -275,7 +300,7 @@ struct RaceRowsLds {
   int64_t row[kChooseRows];
   uint32_t deg[kChooseRows];    // (0: not raced here)
   int quad0[kChooseRows + 1];   // short rows: first quad of the row's positions
-  uint32_t odd[kChooseRows];
+  uint32_t open[kChooseRows];   // the row is on the list already
   int listed[kChooseRows];      // rows that a wave takes
   int n_listed, next;
   uint32_t entry_key[kChooseEntries];  // row r's from r * (k + 1) on
@@ -317,7 +342,7 @@ __device__ __forceinline__ void set_row(RaceRowsLds<NT>& lds, int64_t begin, int
     lds.begin[lane] = begin;
     lds.row[lane] = row;
     lds.deg[lane] = deg;
-    lds.odd[lane] = 0;
+    lds.open[lane] = 0;
   }
   scan_quads(lds.quad0, deg <= kShortRow ? int(deg + 3) / 4 : 0);
   const uint64_t who = __ballot(deg > kShortRow);
@@ -342,11 +367,9 @@ __device__ __forceinline__ void race_rows(RaceRowsLds<NT>& lds, int rows, int k,
   const int quads = lds.quad0[kChooseRows];
   for (int q = threadIdx.x; q < quads; q += NT) {
     const int r = row_of_quad(lds.quad0, q);
-    bool odd = false;
     const uint32_t p = 4u * uint32_t(q - lds.quad0[r]), deg = lds.deg[r];
-    const uint4 key = approx_key_quad(weight_quad(probs, lds.begin[r], p, deg), p, deg, rng_seed, rng_stream, lds.row[r], &odd);
+    const uint4 key = approx_key_quad(weight_quad(probs, lds.begin[r], p, deg), p, deg, rng_seed, rng_stream, lds.row[r]);
     *reinterpret_cast<uint4*>(&lds.key[4 * q]) = key;
-    if (odd) lds.odd[r] = 1;
   }
   __syncthreads();
   // A position counts the smaller ones of its row; where the block has threads for all positions, each by
@@ -392,7 +415,7 @@ __device__ __forceinline__ void race_rows(RaceRowsLds<NT>& lds, int rows, int k,
     const int r = e / each;
     const uint32_t deg = lds.deg[r];
     if (deg == 0 || deg > kShortRow || e - r * each == k) continue;
-    if ((lds.odd[r] != 0 || !surely_less(lds.entry_key[e], lds.entry_key[e + 1])) && atomicExch(&lds.odd[r], 2u) != 2u)
+    if (!surely_less(lds.entry_key[e], lds.entry_key[e + 1]) && atomicExch(&lds.open[r], 1u) == 0u)
       lds.listed[atomicAdd(&lds.n_listed, 1)] = r;
   }
   __syncthreads();
@@ -418,7 +441,7 @@ __device__ __forceinline__ void race_rows(RaceRowsLds<NT>& lds, int rows, int k,
         for (int u = 0; u < kHeldQuads; ++u) {
           if (p0 + u * kStretch >= deg) break;
           const uint32_t p = p0 + u * kStretch + 4u * uint32_t(lane);
-          list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row, &race.odd), p, k);
+          list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row), p, k);
         }
       }
       settled = list_finish(list, race, k, lds.entry_key + r * each, lds.entry_pos + r * each, probs, begin, rng_seed, rng_stream, row);
@@ -437,12 +460,15 @@ __device__ __forceinline__ void race_rows(RaceRowsLds<NT>& lds, int rows, int k,
 // of them has reached holds for all, and wave 0 enters what the others kept into its list.
 template <int NT>
 struct RaceLongLds {
-  __align__(16) WaveList list[NT / kWave];
+  union __align__(16) {
+    WaveList list[NT / kWave];
+    FullRaceLds<NT> full;
+  };
   int kept[NT / kWave];
   uint32_t entry_key[kMaxWeightedPicks + 1];
   uint32_t entry_pos[kMaxWeightedPicks + 1];
   uint32_t bar, dropped;
-  int odd;
+  int open;
 };
 
 template <int NT>
@@ -454,7 +480,7 @@ __device__ __forceinline__ uint32_t race_long(RaceLongLds<NT>& lds, const TierVi
   const int lane = threadIdx.x & (kWave - 1), wave = int(wave_uniform(uint32_t(threadIdx.x / kWave)));
   if (threadIdx.x == 0) {
     lds.bar = lds.dropped = kOutOfRace;
-    lds.odd = 0;
+    lds.open = 0;
   }
   __syncthreads();
   WaveList& list = lds.list[wave];
@@ -473,7 +499,7 @@ __device__ __forceinline__ uint32_t race_long(RaceLongLds<NT>& lds, const TierVi
       const uint32_t published = wave_uniform(__atomic_load_n(&lds.bar, __ATOMIC_RELAXED));
       if (published < race.bar) race.bar = published;  // (entries at or above it do no harm)
       const uint32_t before = race.bar, p = quad_begin(u);
-      list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row, &race.odd), p, k);
+      list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row), p, k);
       if (race.bar < before && lane == 0) atomicMin(&lds.bar, race.bar);
     }
   }
@@ -486,13 +512,13 @@ __device__ __forceinline__ uint32_t race_long(RaceLongLds<NT>& lds, const TierVi
     if (wave != 0) atomicMin(&lds.dropped, least);
     lds.kept[wave] = race.n;
   }
-  if (__ballot(race.odd) != 0 && lane == 0) lds.odd = 1;
+  if (race.open && lane == 0) lds.open = 1;  // (the same in every lane)
   __syncthreads();
   uint32_t pos = kNoPos;
   if (wave == 0) {
     if (lds.dropped < race.dropped) race.dropped = lds.dropped;
     if (lds.bar < race.bar) race.bar = lds.bar;
-    race.odd |= lds.odd != 0;
+    race.open |= lds.open != 0;
     for (int w = 1; w < kWaves; ++w) {
       const int n = int(wave_uniform(uint32_t(lds.kept[w])));
       for (int e0 = 0; e0 < n; e0 += kWave) {
@@ -502,10 +528,15 @@ __device__ __forceinline__ uint32_t race_long(RaceLongLds<NT>& lds, const TierVi
     }
     if (list_finish(list, race, k, lds.entry_key, lds.entry_pos, probs, begin, rng_seed, rng_stream, row)) {
       if (lane < k) pos = lds.entry_pos[lane];
-    } else {
-      const Group<kWave> g;
-      pos = race_row<kWave>(g, probs, begin, deg, k, rng_seed, rng_stream, row);
+    } else if (lane == 0) {
+      lds.open = 1;
     }
+  }
+  __syncthreads();
+  if (lds.open != 0) {
+    Race full;
+    race_long_row_full<NT>(full, lds.full, probs, begin, deg, k, rng_seed, rng_stream, row);
+    pos = wave == 0 ? full.pos : kNoPos;
   }
   __syncthreads();  // lds is reused by the block's next row
   return pos;

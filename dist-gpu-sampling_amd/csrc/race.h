@@ -207,19 +207,21 @@ __device__ __forceinline__ void race_offer(Race& r, const Group<G>& g, uint64_t 
 // The waves of a block that share one row publish the key of their last entry once they hold
 // num_picks entries (kNoKey before); the smallest of these bounds the row's final last key from
 // above, so a candidate beyond it can be dropped unseen.  Stale reads only make the bound looser.
+template <int WAVES>
 __device__ __forceinline__ uint64_t lowest_bar(uint64_t* bars, int lane) {
-  uint64_t v = __atomic_load_n(&bars[lane & (kLongWaves - 1)], __ATOMIC_RELAXED);
+  uint64_t v = __atomic_load_n(&bars[lane & (WAVES - 1)], __ATOMIC_RELAXED);
 #pragma unroll
-  for (int stride = 1; stride < kLongWaves; stride <<= 1) {
+  for (int stride = 1; stride < WAVES; stride <<= 1) {
     const uint64_t o = lane_xor(v, stride);
     if (o < v) v = o;
   }
   return v;
 }
 
+template <int WAVES>
 __device__ __forceinline__ uint64_t lowest_bar_after_sync(uint64_t* bars, int lane) {
   __syncthreads();  // every wave of the block has published its final bar
-  return lowest_bar(bars, lane);
+  return lowest_bar<WAVES>(bars, lane);
 }
 
 // Race keys of the four G-position steps of the stretch that begins at position sb (a multiple of
@@ -253,9 +255,9 @@ __device__ __forceinline__ void stretch_keys(const Group<G>& g, const TierView<f
 }
 
 // Runs positions [begin, end) of the group's row, in steps of `stride` (begin and stride multiples
-// of 4 G), through its race.  `bars` (block-per-row kernel only) is the block's table of published
-// last keys.
-template <int G>
+// of 4 G), through its race.  `bars` (block-per-row only) is the table of the last keys that the block's
+// WAVES waves have published.
+template <int G, int WAVES = kLongWaves>
 __device__ __forceinline__ void race_scan(Race& r, const Group<G>& g, const TierView<float>& probs, int64_t start,
                                           uint64_t begin, uint64_t end, uint64_t stride, int k, uint64_t rng_seed,
                                           uint32_t rng_stream, int64_t row, uint64_t* bars = nullptr) {
@@ -264,7 +266,7 @@ __device__ __forceinline__ void race_scan(Race& r, const Group<G>& g, const Tier
   for (uint64_t sb = begin; __ballot(sb < end); sb += stride) {
     uint64_t ck[4];
     stretch_keys<G>(g, probs, start, sb, end, rng_seed, rng_stream, row, ck);
-    const uint64_t bar = bars != nullptr ? lowest_bar(bars, g.l) : kNoKey;
+    const uint64_t bar = bars != nullptr ? lowest_bar<WAVES>(bars, g.l) : kNoKey;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const uint64_t cb = sb + uint64_t(G) * c;
@@ -486,12 +488,17 @@ __device__ __forceinline__ uint64_t locate_draws(const Group<G>& g, const TierVi
   return settled;
 }
 
+// LDS of a block of NT threads that races a long row on full keys.
+template <int NT>
+struct FullRaceLds {
+  uint64_t key[NT];
+  uint32_t pos[NT];
+  uint64_t bars[NT / kWave];
+};
+
 // LDS of a block that works on long rows.
-struct LongRowScratch {
-  uint64_t key[kLongBlock];
+struct LongRowScratch : FullRaceLds<kLongBlock> {
   uint32_t half[kLongBlock];
-  uint32_t pos[kLongBlock];
-  uint64_t bars[kLongWaves];
   uint64_t sum[kLongWaves];
   float max[kLongWaves];
   uint32_t half_bars[kLongWaves];
@@ -522,22 +529,24 @@ __device__ __forceinline__ uint32_t race_row(const Group<G>& g, const TierView<f
   return pos;
 }
 
-// Without replacement, a long row raced by a whole 1024-thread block on full keys: each wave
+// Without replacement, a long row raced by a whole block of NT threads on full keys: each wave
 // races an interleaved share of the row, then the waves' winners are merged pairwise (wave w takes
 // over the entries of wave w + step: 16 lists become one in four rounds; entries beyond the lowest
 // published bar cannot be among the row's best).  On return lane l < k of wave 0 holds the l-th
 // winner in r.pos.  Every thread of the block must call it.
-__device__ __forceinline__ void race_long_row_full(Race& r, LongRowScratch& lds, const TierView<float>& probs,
+template <int NT>
+__device__ __forceinline__ void race_long_row_full(Race& r, FullRaceLds<NT>& lds, const TierView<float>& probs,
                                                    int64_t start, uint32_t deg, int k, uint64_t rng_seed,
                                                    uint32_t rng_stream, int64_t row) {
+  constexpr int kWaves = NT / kWave;
   const Group<kWave> g;
   const int wave = threadIdx.x / kWave;
-  if (threadIdx.x < kLongWaves) lds.bars[threadIdx.x] = kNoKey;
+  if (threadIdx.x < kWaves) lds.bars[threadIdx.x] = kNoKey;
   __syncthreads();
   race_reset(r);
-  race_scan<kWave>(r, g, probs, start, 256u * wave, deg, 256u * kLongWaves, k, rng_seed, rng_stream, row, lds.bars);
-  const uint64_t bar = lowest_bar_after_sync(lds.bars, g.l);
-  for (int step = 1; step < kLongWaves; step <<= 1) {
+  race_scan<kWave, kWaves>(r, g, probs, start, 256u * wave, deg, 256u * kWaves, k, rng_seed, rng_stream, row, lds.bars);
+  const uint64_t bar = lowest_bar_after_sync<kWaves>(lds.bars, g.l);
+  for (int step = 1; step < kWaves; step <<= 1) {
     lds.key[threadIdx.x] = r.key;
     lds.pos[threadIdx.x] = r.pos;
     __syncthreads();
@@ -637,7 +646,7 @@ __device__ __forceinline__ uint32_t race_long_row(LongRowScratch& lds, const Tie
   uint32_t pos = wave == 0 ? r.pos : kNoPos;
   if (again) {
     Race full;
-    race_long_row_full(full, lds, probs, start, deg, k, rng_seed, rng_stream, row);
+    race_long_row_full<kLongBlock>(full, lds, probs, start, deg, k, rng_seed, rng_stream, row);
     pos = wave == 0 ? full.pos : kNoPos;
   }
   return pos;

@@ -60,6 +60,35 @@ def test_choice_at_the_edges_of_the_row_classes(pkg, oracle, kind, replace):
             assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
 
 
+@pytest.mark.parametrize("kind", ["one", "infinite", "equal"])
+@pytest.mark.parametrize("n_seeds,fanouts", [(300, [64]), (300, [5, 3]),      # long rows by blocks of 16 waves ...
+                                             (12289, [64]), (12289, [5])])    # ... and of four, from the queue
+def test_long_rows_that_floats_alone_do_not_settle(pkg, oracle, n_seeds, fanouts, kind):
+    rng = np.random.default_rng(n_seeds)
+    n = 2000
+    deg = rng.integers(0, 20, size=n)
+    deg[:12] = [2048, 2049, 2303, 2304, 2305, 5120, 5121, 20480, 20481, 33333, 4096, 40000]
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int32)
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    if kind == "one":         # a row's first and last weight
+        probs[indptr[:-1][deg > 0]] = 1e-42
+        probs[indptr[1:][deg > 0] - 1] = np.inf
+    elif kind == "infinite":  # more of them than picks, in the order of their positions
+        probs[rng.random(probs.size) < 0.3] = np.inf
+    else:                     # keys beyond float32: 64-bit ones of whole rows
+        probs[:] = rng.choice(np.array([1e-45, 3e-45, 4e-45], dtype=np.float32), size=probs.size)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    seeds = rng.integers(0, n, size=n_seeds).astype(np.int32)
+    seeds[:24] = np.arange(24) % 12
+    pkg.set_rng_state(SEED, STREAM)
+    f, _, blocks = pkg.ChunkTensorSampler(fanouts, *cts, replace=False).sample_blocks(None, torch.from_numpy(seeds))
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, False, SEED, STREAM, probs=probs)
+    assert np.array_equal(f.cpu().numpy(), want_f)
+    for g, w in zip(blocks, want):
+        assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+
+
 @pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("n_seeds,fanouts", [(200, [6, 4, 3]),     # shared, shared, queued: long rows of every frontier
                                              (900, [6, 4]),        # shared, then queued

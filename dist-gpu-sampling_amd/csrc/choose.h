@@ -25,6 +25,8 @@
 #ifndef DGS_CSRC_CHOOSE_H_
 #define DGS_CSRC_CHOOSE_H_
 
+#include <type_traits>
+
 #include "race.h"
 
 namespace dgs {
@@ -657,7 +659,11 @@ __device__ __forceinline__ void draw_rows(DrawRowsLds<NT>& lds, int rows, int k,
 
 // A long row drawn from by a whole block of NT threads (every thread must call it): every wave owns a
 // contiguous part of it, read once as far as kHeld quads a lane go, and settles the draws that fall into
-// its own part.
+// its own part.  What is beyond is read in three passes, bound by the wait for memory: several stretches ahead
+// (16 384 rows, 8 of them of 10^6 positions, 10 draws, us a call: one stretch at a time 1593; four ahead in
+// every pass 1117, eight in the two sums and four in the search, whose registers eight would not fit, 1057; 64
+// rows of 200 000: 391, 288, 274).
+template <int N> using AheadOf = std::integral_constant<int, N>;
 template <int NT>
 struct DrawLongLds {
   float max[NT / kWave];
@@ -680,15 +686,23 @@ __device__ __forceinline__ void draw_long(DrawLongLds<NT>& lds, const TierView<f
   float4_anywhere held[kHeld];
 #pragma unroll
   for (int u = 0; u < kHeld; ++u) held[u] = quad_at(lo + u * kStretch);
-  const auto every_stretch = [&](auto each) {  // each(p0, quad) returns whether to go on
+  const auto every_stretch = [&](auto ahead, auto each) {  // each(p0, quad) returns whether to go on
+    constexpr int kAhead = decltype(ahead)::value;
     bool on = true;
 #pragma unroll
     for (int u = 0; u < kHeld; ++u)
       if (on && lo + u * kStretch < hi) on = each(lo + u * kStretch, held[u]);
-    for (uint64_t p0 = lo + kHeld * kStretch; on && p0 < hi; p0 += kStretch) on = each(p0, quad_at(p0));
+    for (uint64_t p0 = lo + kHeld * kStretch; on && p0 < hi; p0 += kAhead * kStretch) {
+      float4_anywhere next[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) next[u] = quad_at(p0 + u * kStretch);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (on && p0 + u * kStretch < hi) on = each(p0 + u * kStretch, next[u]);
+    }
   };
   float most = 0.0f;
-  every_stretch([&](uint64_t, float4_anywhere w) {
+  every_stretch(AheadOf<8>(), [&](uint64_t, float4_anywhere w) {
     const float m = quad_max(w);
     most = m > most ? m : most;
     return true;
@@ -705,7 +719,7 @@ __device__ __forceinline__ void draw_long(DrawLongLds<NT>& lds, const TierView<f
     return sum;
   };
   uint64_t mine = 0;
-  every_stretch([&](uint64_t, float4_anywhere w) {
+  every_stretch(AheadOf<8>(), [&](uint64_t, float4_anywhere w) {
     mine += share(w);
     return true;
   });
@@ -730,7 +744,7 @@ __device__ __forceinline__ void draw_long(DrawLongLds<NT>& lds, const TierView<f
     if (pending == 0) continue;
     uint32_t pick = deg - 1;
     uint64_t at = before;
-    every_stretch([&](uint64_t p0, float4_anywhere w) {
+    every_stretch(AheadOf<4>(), [&](uint64_t p0, float4_anywhere w) {
       const uint64_t sum = share(w);
       const uint64_t upto = at + group_inclusive_sum<kWave>(sum, lane);
       const uint64_t after = lane_read(upto, kWave - 1);

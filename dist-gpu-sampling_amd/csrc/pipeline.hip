@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
 // kLongRow 512 / 1024 / 2048: 287 / 278 / 276 us for a batch of 1024 seeds, fanouts [5,10,15].
 constexpr uint32_t kLongRow = 2048, kSharedRow = 512;
 static_assert(kLongRow <= kDrawRow, "draw_rows takes every row that is not long");
-constexpr int64_t kLongQueueBlocks = 256;  // (512: no faster)
+constexpr int64_t kMinQueueBlocks = 256, kMaxQueueBlocks = 512;  // (see queue_blocks)
 constexpr int64_t kSharedMaxRows = 4096, kSharedMaxSeeds = 12288;  // of a later hop, of hop 0
 constexpr int64_t kSharedBlocks = 256;  // one per CU
 constexpr int kSharedRows = 16;
@@ -731,8 +731,9 @@ __global__ __launch_bounds__(kSeedSegment) void announce_long_seeds_kernel(Hop h
 
 // Virtual blocks: the queued long rows, the others, the previous hop's edge list.
 template <typename IdT, typename PtrT, typename TableT, bool REPLACE>
-__global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_kernel(Hop h, Hop prev, int64_t fill_blocks,
-                                                                   int32_t rows_per_block, int64_t relabel_count,
+__global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_kernel(Hop h, Hop prev, int64_t queue_blocks,
+                                                                   int64_t fill_blocks, int32_t rows_per_block,
+                                                                   int64_t relabel_count,
                                                                    TableT table, TierView<PtrT> indptr,
                                                                    TierView<IdT> indices, TierView<float> probs,
                                                                    uint64_t rng_seed) {
@@ -740,14 +741,14 @@ __global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_ker
     ChooseLds<kBlock, REPLACE> choose;
     LongLds<kBlock, REPLACE> long_row;
   } lds;
-  const int64_t total = kLongQueueBlocks + fill_blocks + relabel_count;
+  const int64_t total = queue_blocks + fill_blocks + relabel_count;
   for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
-    if (vb >= kLongQueueBlocks + fill_blocks) {
-      relabel_tile<IdT, TableT, false>(prev, table, vb - kLongQueueBlocks - fill_blocks, threadIdx.x);  // always a striding launch
+    if (vb >= queue_blocks + fill_blocks) {
+      relabel_tile<IdT, TableT, false>(prev, table, vb - queue_blocks - fill_blocks, threadIdx.x);  // always a striding launch
       continue;
     }
     const int64_t s = seeds_of(h);
-    if (vb < kLongQueueBlocks) {
+    if (vb < queue_blocks) {
       const auto take = [&](int64_t i) {
         const int64_t row = int64_t(static_cast<const IdT*>(h.seeds)[i]);
         if (!table.holds(IdT(row)) || h.k == 0) return;
@@ -757,18 +758,18 @@ __global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_ker
       };
       if (h.index == 0) {  // several blocks share a segment's list where there are fewer segments than blocks
         const int64_t segments = (s + kSeedSegment - 1) / kSeedSegment;
-        const int64_t at_once = segments < kLongQueueBlocks ? segments : kLongQueueBlocks;
-        const int64_t sharers = kLongQueueBlocks / at_once, sharer = vb / at_once;
+        const int64_t at_once = segments < queue_blocks ? segments : queue_blocks;
+        const int64_t sharers = queue_blocks / at_once, sharer = vb / at_once;
         if (sharer < sharers)
           for (int64_t g = vb % at_once; g < segments; g += at_once)
             for (int64_t j = sharer; j < h.long_seed_count[g]; j += sharers)
               take(g * kSeedSegment + h.long_seeds[g * kSeedSegment + j]);
       } else {
         const int64_t n_long = *h.long_count;
-        for (int64_t t = vb; t < n_long; t += kLongQueueBlocks) take(h.long_rows[t]);
+        for (int64_t t = vb; t < n_long; t += queue_blocks) take(h.long_rows[t]);
       }
     } else {
-      const int64_t at = vb - kLongQueueBlocks;
+      const int64_t at = vb - queue_blocks;
       if (h.n_seeds_out && at == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
       const int64_t first = at * rows_per_block;
       if (first >= s) continue;  // whole blocks leave together
@@ -1598,6 +1599,19 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
                        TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
 }
 
+// Blocks of a weighted launch that take queued long rows, in front of `others`.  256 keep a block on every CU, which
+// a frontier of hubs leaves waiting for its chains: 512 where they and the others fit the GPU at once, four
+// blocks to a CU, or where there are several rounds of the others anyway.  In between the others would be dealt
+// out unevenly behind them (2048 seeds, fanouts [10,10], rows of 300: 129 us with 256, 137 with 512).
+// us a call, 256 / 512: 16 384 rows of 3000 750 / 441 (10 picks), 455 / 279 (draws); of 17 000 1572 / 926, 1360 /
+// 791; 300 of 20 000 among them 134 / 107, 129 / 104; 1024 seeds, fanouts [10,10], rows of 3000 548 / 358, 352 / 239.
+// Batches whose long rows are a few hundred: level.  1024 or 2048: 290 for the first, and 2 to 5 us more for those.
+inline int64_t queue_blocks(int64_t others) {
+  constexpr int64_t kSlots = 1024;
+  if (others >= kSlots) return kMaxQueueBlocks;
+  return std::min(kMaxQueueBlocks, std::max(kMinQueueBlocks, kSlots - others));
+}
+
 // Whether a weighted hop is a launch of kLongBlock-thread blocks (see above).
 inline bool weighted_shared(const Hop& h) { return h.s_max <= (h.index == 0 ? kSharedMaxSeeds : kSharedMaxRows); }
 
@@ -1622,9 +1636,10 @@ void launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count
   }
   const int64_t rows = choose_rows(cur.k);
   const int64_t fill_blocks = (cur.s_max + rows - 1) / rows;
-  const int64_t total = kLongQueueBlocks + fill_blocks + relabel_count;
+  const int64_t queued = queue_blocks(fill_blocks + relabel_count);
+  const int64_t total = queued + fill_blocks + relabel_count;
   hipLaunchKernelGGL((hop_fill_weighted_kernel<IdT, PtrT, TableT, REPLACE>), dim3(capped_grid(total)), dim3(kBlock), 0, st, cur,
-                     prev, fill_blocks, int32_t(rows), relabel_count, table, TierView<PtrT>(indptr), TierView<IdT>(indices),
+                     prev, queued, fill_blocks, int32_t(rows), relabel_count, table, TierView<PtrT>(indptr), TierView<IdT>(indices),
                      TierView<float>(probs), rng_seed);
 }
 

@@ -90,6 +90,28 @@ def test_long_rows_that_floats_alone_do_not_settle(pkg, oracle, n_seeds, fanouts
 
 
 @pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n_seeds,fanouts", [(14000, [5]),           # more long rows than blocks of the queue: from segments ...
+                                             (1500, [4, 12]),        # ... and from the queue, 600 blocks beside it ...
+                                             (5000, [3, 2, 9])])     # ... and more of them than the GPU holds
+def test_frontiers_of_long_rows(pkg, oracle, n_seeds, fanouts, replace):
+    rng = np.random.default_rng(n_seeds)
+    n = 1600
+    deg = rng.integers(2049, 2400, size=n)
+    deg[::97] = [3, 0, 40, 5120, 5121, 9217, 13313, 13314, 20480, 21505, 26000, 2048, 7, 5119, 8192, 17, 30000]  # (a wave's held and read-ahead stretches end between these)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int32)
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    seeds = rng.integers(0, n, size=n_seeds).astype(np.int32)
+    pkg.set_rng_state(SEED, STREAM)
+    f, _, blocks = pkg.ChunkTensorSampler(fanouts, *cts, replace=replace).sample_blocks(None, torch.from_numpy(seeds))
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, SEED, STREAM, probs=probs)
+    assert np.array_equal(f.cpu().numpy(), want_f)
+    for g, w in zip(blocks, want):
+        assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("n_seeds,fanouts", [(200, [6, 4, 3]),     # shared, shared, queued: long rows of every frontier
                                              (900, [6, 4]),        # shared, then queued
                                              (12289, [3, 2]),      # the first hop's long rows come from its segments

@@ -1,27 +1,29 @@
-// Weighted picks of many seed rows by one block: the rules of race.h, laid out so that lanes belong to
-// weights and draws instead of rows.  Half of all rows have a few dozen neighbours; a wave per row leaves
-// most of its lanes idle and pays a sort, or three passes over the weights, for each.
+// Weighted picks: the rules of race.h for the fused sampler, laid out so that lanes belong to weights and draws.
+// In a large hop many rows share a block (race_rows, draw_rows): half of all rows have a few dozen neighbours,
+// and a wave for each leaves most of its lanes idle.  In a small one, where nothing but latency counts, every
+// row has a wave that does it all without a barrier (race_by_wave, draw_by_wave).  Long rows have a block each
+// (race_long, draw_long).
 //
-// Without replacement (race_rows) the race runs on 32-bit floats first.  An approximate key is off by less than
-// half of what surely_less asks for, so entries that it orders are ordered as the 64-bit keys are; where the
-// num_picks + 1 smallest of a row are not all surely ordered (one row in some thousands), 64-bit keys settle
-// it (race.h).  Rows of up to kShortRow positions: four positions to a lane, which is one Philox block, and
-// then every position counts the smaller ones of its row.  Longer ones: a wave per row, or a block, that keeps
-// what is below a bar in an LDS list and lowers the bar when the list fills.
+// Without replacement the race runs on 32-bit floats first.  An approximate key is off by less than half of what
+// surely_less asks for, so entries that it orders are ordered as the 64-bit keys are; where the num_picks + 1
+// smallest of a row are not all surely ordered (one row in some thousands), 64-bit keys settle it (race.h).  Rows
+// of up to kShortRow positions: four positions to a lane, which is one Philox block, and then every position
+// counts the smaller ones of its row.  Longer ones: a wave, or the waves of a block, that keep what is below a
+// bar in an LDS list and lower the bar when the list fills.
+//
+// Measured, before (a wave per row, sorts, three passes over the weights) and with this: the hops of a batch of
+// 1024 seeds, fanouts [5,10,15], rows of mean degree 50 up to 17 000, 28 / 36 / 84 us and 32 for the long rows'
+// launch -> 27 / 28 / 63; 512 seeds with replacement 26 / 28 / 69 + 28 -> 18 / 19 / 31.  The whole batches
+// 328 -> 274 and 214 -> 140 us.  Bound now: without replacement the atomics of the picks (31 us of the widest
+// hop), then Philox and the counting; in a small hop the chain of waits (7 us for a wave's row) and its longest
+// row (17 000 positions by one block: 21 us).
 //
 // Any weight above 0 has a float key.  Where one weight outside 2^-120 .. 2^90 sent its row to 64-bit keys, by
 // one wave: 256 rows of 17 000 with one infinite weight each 171 us a call and now 68 (without it 67), two rows of
 // 10^6 6.7 ms and 0.8, 1024 seeds, fanouts [5,10,10], rows of 60 with a fifth of the weights infinite 288 and 130.
 //
-// Measured, before (a wave per row, sorts, three passes over the weights) and with this: the hops of a batch of
-// 1024 seeds, fanouts [5,10,15], rows of mean degree 50 up to 17 000, 28 / 36 / 84 us and 32 for the long rows'
-// launch -> 29 / 28 / 73; 512 seeds with replacement 26 / 28 / 69 + 28 -> 19 / 20 / 34.  The whole batches
-// 326 -> 274 and 220 -> 147 us.  Bound now: without replacement the atomics of the picks (31 us of the widest
-// hop), then Philox and the counting; in a small hop the chain of its phases (9 to 12 us) and its longest row
-// (20 000 positions by one block: 17 us).
-//
-// With replacement (draw_rows) the shares of many rows are summed up in one scan over LDS, and every draw
-// is a lane of its own that searches its row's part of it.
+// With replacement the shares of many rows are summed up in one scan over LDS, and every draw is a lane of its
+// own that searches its row's part of it (draw_rows; draw_by_wave: the sums of a row's quads).
 #ifndef DGS_CSRC_CHOOSE_H_
 #define DGS_CSRC_CHOOSE_H_
 
@@ -290,6 +292,80 @@ __device__ __forceinline__ bool list_finish(WaveList& list, ListRace& r, int k, 
   return true;
 }
 
+// A row of up to kShortRow positions: every position counts the smaller ones.  Returns as list_finish does.
+__device__ __forceinline__ bool race_short(uint32_t* keys, uint32_t* entry_key, uint32_t* entry_pos, int k,
+                                           const TierView<float>& probs, int64_t begin, uint32_t deg, uint64_t rng_seed,
+                                           uint32_t rng_stream, int64_t row) {
+  static_assert(kShortRow == 2 * kWave, "two positions to a lane at most");
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  if (4 * lane < deg)
+    *reinterpret_cast<uint4*>(&keys[4 * lane]) =
+        approx_key_quad(weight_quad(probs, begin, 4 * lane, deg), 4 * lane, deg, rng_seed, rng_stream, row);
+  for (int e = int(lane); e <= k; e += kWave) entry_key[e] = 0;  // stays where two keys share a rank: unsure
+  wave_lds_fence();
+  const auto enter = [&](uint32_t key, int rank, uint32_t pos) {
+    if (key == kOutOfRace || rank > k) return;
+    entry_key[rank] = key;
+    entry_pos[rank] = pos;
+  };
+  const uint32_t own = lane < deg ? keys[lane] : kOutOfRace;
+  int rank = 0;
+  if (deg <= kWave) {
+#pragma unroll 4
+    for (uint32_t j = 0; j < deg; j += 4) {
+      const uint4 o = *reinterpret_cast<const uint4*>(&keys[j]);
+      rank += int(o.x < own) + int(o.y < own) + int(o.z < own) + int(o.w < own);
+    }
+  } else {
+    const uint32_t own1 = lane + kWave < deg ? keys[lane + kWave] : kOutOfRace;
+    int rank1 = 0;
+#pragma unroll 4
+    for (uint32_t j = 0; j < deg; j += 4) {
+      const uint4 o = *reinterpret_cast<const uint4*>(&keys[j]);
+      rank += int(o.x < own) + int(o.y < own) + int(o.z < own) + int(o.w < own);
+      rank1 += int(o.x < own1) + int(o.y < own1) + int(o.z < own1) + int(o.w < own1);
+    }
+    enter(own1, rank1, lane + kWave);
+  }
+  enter(own, rank, lane);
+  wave_lds_fence();
+  return __ballot(int(lane) < k && !surely_less(entry_key[lane], entry_key[lane + 1])) == 0;
+}
+
+// A row of more than k positions by one wave: its picks in order into entry_pos[0 .. k] (the last one for
+// scratch, and entry_key[0 .. k]).  `floats`: not raced on them before.
+template <bool SHORT>
+__device__ __forceinline__ void race_by_wave(WaveList& list, uint32_t* entry_key, uint32_t* entry_pos, bool floats, int k,
+                                             const TierView<float>& probs, int64_t begin, uint32_t deg, uint64_t rng_seed,
+                                             uint32_t rng_stream, int64_t row) {
+  const int lane = threadIdx.x & (kWave - 1);
+  bool settled = false;
+  if (SHORT && deg <= kShortRow) {
+    settled = race_short(list.key, entry_key, entry_pos, k, probs, begin, deg, rng_seed, rng_stream, row);
+  } else if (floats) {
+    ListRace race;
+    constexpr uint32_t kStretch = 4 * kWave;
+    for (uint32_t p0 = 0; p0 < deg; p0 += kHeldQuads * kStretch) {
+      float4_anywhere held[kHeldQuads];
+#pragma unroll
+      for (int u = 0; u < kHeldQuads; ++u) held[u] = weight_quad(probs, begin, p0 + u * kStretch + 4u * uint32_t(lane), deg);
+#pragma unroll
+      for (int u = 0; u < kHeldQuads; ++u) {
+        if (p0 + u * kStretch >= deg) break;
+        const uint32_t p = p0 + u * kStretch + 4u * uint32_t(lane);
+        list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row), p, k);
+      }
+    }
+    settled = list_finish(list, race, k, entry_key, entry_pos, probs, begin, rng_seed, rng_stream, row);
+  }
+  if (!settled) {
+    const Group<kWave> g;
+    const uint32_t pos = race_row<kWave>(g, probs, begin, deg, k, rng_seed, rng_stream, row);
+    if (lane < k) entry_pos[lane] = pos;
+  }
+  wave_lds_fence();
+}
+
 // ---- many rows raced by one block ----
 
 constexpr int kChooseRows = 32;       // rows of a block at most ...
@@ -430,29 +506,8 @@ __device__ __forceinline__ void race_rows(RaceRowsLds<NT>& lds, int rows, int k,
     const int r = int(wave_uniform(uint32_t(lds.listed[t])));
     const int64_t begin = wave_uniform(lds.begin[r]), row = wave_uniform(lds.row[r]);
     const uint32_t deg = wave_uniform(lds.deg[r]);
-    bool settled = false;
-    if (deg > kShortRow) {
-      WaveList& list = lds.list[wave];
-      ListRace race;
-      constexpr uint32_t kStretch = 4 * kWave;
-      for (uint32_t p0 = 0; p0 < deg; p0 += kHeldQuads * kStretch) {
-        float4_anywhere held[kHeldQuads];
-#pragma unroll
-        for (int u = 0; u < kHeldQuads; ++u) held[u] = weight_quad(probs, begin, p0 + u * kStretch + 4u * uint32_t(lane), deg);
-#pragma unroll
-        for (int u = 0; u < kHeldQuads; ++u) {
-          if (p0 + u * kStretch >= deg) break;
-          const uint32_t p = p0 + u * kStretch + 4u * uint32_t(lane);
-          list_enter_quad(list, race, approx_key_quad(held[u], p, deg, rng_seed, rng_stream, row), p, k);
-        }
-      }
-      settled = list_finish(list, race, k, lds.entry_key + r * each, lds.entry_pos + r * each, probs, begin, rng_seed, rng_stream, row);
-    }
-    if (!settled) {
-      const Group<kWave> g;
-      const uint32_t pos = race_row<kWave>(g, probs, begin, deg, k, rng_seed, rng_stream, row);
-      if (lane < k) lds.entry_pos[r * each + lane] = pos;
-    }
+    race_by_wave<false>(lds.list[wave], lds.entry_key + r * each, lds.entry_pos + r * each, deg > kShortRow, k, probs, begin, deg, rng_seed,
+                 rng_stream, row);
   }
   __syncthreads();
 }
@@ -521,12 +576,26 @@ __device__ __forceinline__ uint32_t race_long(RaceLongLds<NT>& lds, const TierVi
     if (lds.dropped < race.dropped) race.dropped = lds.dropped;
     if (lds.bar < race.bar) race.bar = lds.bar;
     race.open |= lds.open != 0;
-    for (int w = 1; w < kWaves; ++w) {
-      const int n = int(wave_uniform(uint32_t(lds.kept[w])));
-      for (int e0 = 0; e0 < n; e0 += kWave) {
-        const int e = e0 + lane;
-        list_enter(list, race, e < n ? lds.list[w].key[e] : kOutOfRace, e < n ? lds.list[w].pos[e] : kNoPos, k);
+    // (a lane for every entry of the others: 64 at a time, and not one list after the other)
+    int upto = lane > 0 && lane < kWaves ? lds.kept[lane] : 0;
+#pragma unroll
+    for (int d = 1; d < kWaves; d <<= 1) {
+      const int o = __shfl_up(upto, d, kWave);
+      if (lane >= d) upto += o;
+    }
+    const int total = int(lane_read(uint32_t(upto), kWaves - 1));
+    for (int e0 = 0; e0 < total; e0 += kWave) {
+      const int e = e0 + lane;
+      int w = 1, from = 0;
+#pragma unroll
+      for (int v = 1; v < kWaves - 1; ++v) {
+        const int end = int(lane_read(uint32_t(upto), v));
+        if (e >= end) {
+          w = v + 1;
+          from = end;
+        }
       }
+      list_enter(list, race, e < total ? lds.list[w].key[e - from] : kOutOfRace, e < total ? lds.list[w].pos[e - from] : kNoPos, k);
     }
     if (list_finish(list, race, k, lds.entry_key, lds.entry_pos, probs, begin, rng_seed, rng_stream, row)) {
       if (lane < k) pos = lds.entry_pos[lane];
@@ -655,6 +724,63 @@ __device__ __forceinline__ void draw_rows(DrawRowsLds<NT>& lds, int rows, int k,
     __syncthreads();
     r0 = r1;
   }
+}
+
+// A row of up to kWaveDrawRow positions drawn from by one wave: lane j < k returns the position of draw j (k at
+// most 64).
+constexpr int kWaveDrawQuads = 8;  // quads a lane holds
+constexpr uint32_t kWaveDrawRow = 4 * kWave * kWaveDrawQuads;
+struct WaveDrawLds {
+  uint64_t upto[kWave * kWaveDrawQuads];  // shares up to and including a quad
+};
+__device__ __forceinline__ uint32_t draw_by_wave(WaveDrawLds& lds, const TierView<float>& probs, int64_t begin, uint32_t deg, int k,
+                                                 uint64_t rng_seed, uint32_t rng_stream, int64_t row) {
+  constexpr uint32_t kStretch = 4 * kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  float4_anywhere w[kWaveDrawQuads];
+  float most = 0.0f;
+#pragma unroll
+  for (int u = 0; u < kWaveDrawQuads; ++u) w[u] = weight_quad(probs, begin, u * kStretch + 4u * uint32_t(lane), deg);
+#pragma unroll
+  for (int u = 0; u < kWaveDrawQuads; ++u) {
+    if (u * kStretch >= deg) break;
+    const float m = quad_max(w[u]);
+    most = m > most ? m : most;
+  }
+  const QuantumScale scale = quantum_scale(__uint_as_float(~wave_min(~__float_as_uint(most))));
+  uint64_t total = 0;
+#pragma unroll
+  for (int u = 0; u < kWaveDrawQuads; ++u) {
+    if (u * kStretch >= deg) break;
+    uint64_t sum = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) sum += weight_quantum(w[u][c], scale);
+    const uint64_t upto = total + group_inclusive_sum<kWave>(sum, lane);
+    lds.upto[u * kWave + lane] = upto;
+    total = lane_read(upto, kWave - 1);
+  }
+  wave_lds_fence();
+  uint32_t pos = deg - 1;  // where the row has no positive share
+  if (lane < k && total > 0) {
+    const uint64_t want = philox_bounded64(rng_seed, rng_stream, row, uint32_t(lane), total);
+    uint32_t lo = 0, hi = (deg - 1) >> 2;  // the first quad whose sum is beyond it
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (lds.upto[mid] > want) hi = mid; else lo = mid + 1;
+    }
+    uint64_t s = lo > 0 ? lds.upto[lo - 1] : 0;
+    const float4_anywhere quad = weight_quad(probs, begin, 4 * lo, deg);  // (still in a cache)
+    pos = 4 * lo;
+    bool beyond = false;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      s += weight_quantum(quad[c], scale);
+      beyond |= s > want;
+      if (!beyond) ++pos;
+    }
+  }
+  wave_lds_fence();
+  return pos;
 }
 
 // A long row drawn from by a whole block of NT threads (every thread must call it): every wave owns a

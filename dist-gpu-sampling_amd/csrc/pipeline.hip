@@ -523,28 +523,32 @@ __global__ __launch_bounds__(kBlock) void hop_fill_kernel(Hop h, Hop prev, int64
 
 // ---- weighted picks (choose.h) ----
 //
-// A block takes up to choose_rows(k) rows: a thread looks each of them up, the block chooses their picks,
+// In a large hop a block takes up to choose_rows(k) rows: a thread looks each of them up, the block chooses their picks,
 // and then every pick is placed by a thread of its own.  Rows above kLongRow positions are raced, or drawn
 // from, by a whole block each.  They are queued before the launch, by the compact launch of the hop before
 // (announce_long_rows) or, in hop 0, by the launch that clears (announce_long_seeds), so that they are
 // worked on from its first moment, beside the others.
-// A small hop (kSharedMaxRows) is a launch of larger blocks instead, which have as few rows as still give
-// every CU a block and take their own long rows one after the other at the end; rows between kSharedRow and
-// kLongRow positions as well where the block has few of them, since its waves race the others side by side.
-// In hop 0 that reaches further (kSharedMaxSeeds): it saves the launch that queues.  us a call of one hop,
-// shared / queued: 4000 rows of 50 / 200 / 1000, 64 picks 64 / 73, 78 / 102, 89 / 120; 8192 rows of 10 / 50 /
-// 1000 57 / 59, 63 / 66, 85 / 122; 12 000 of 200 86 / 103; 65 536 of 20 180 / 93.  A second hop of up to 3072
-// rows takes 19 us shared and 23 queued, one of 6144 43 and 28.
+// A small hop (kSharedMaxRows) is a launch of larger blocks instead, with a wave for each row and as few rows to a
+// block as still give every CU one: nothing waits at a barrier but the long rows, which the block takes one after
+// the other at the end.  In hop 0 that reaches further (kSharedMaxSeeds): it saves the launch that queues.
+// us a call of one hop, small / queued form: 4000 rows of 50 / 200 / 1000, 64 picks 64 / 71, 75 / 99, 84 / 114;
+// 8192 rows of 10 / 50 / 1000 52 / 56, 58 / 62, 75 / 114; 12 000 of 200 77 / 99; 12 288 of 30 64 / 63 (draws 71 /
+// 62, but 8192 of 50 61 / 59 and of 1000 67 / 117); 65 536 of 20 150 / 90.  1024 seeds, fanouts [5,10]: 101 / 107.
+// The launch alone, 256 rows of 60 / 512 / 1000 / 2048 / 4000 / 17 000 positions, 5 picks: by a wave and, beyond
+// 2048, a block 6.9 / 9.6 / 12.1 / 14.8 / 18.0 / 21.2 us.  With the phases of fill_rows_weighted here too, and a
+// block's turn from 512 on, 9.3 / 13.1 / 16.8 / 18.8 / 21.3 / 25.0; with sorts of 64-bit keys (a wave up to 512)
+// 7.7 / 12.6 / 13.5 / 14.7 / 15.9 / 29.8, and with 15 picks 16.4 / 15.9 / 18.6 / 23.0 / 37.8 where it is now 10.9 /
+// 12.2 / 14.8 / 19.3 / 23.3: 1500 to 5000 positions and few picks are the one place that has lost (1 to 2 us).
 // kLongRow 512 / 1024 / 2048: 287 / 278 / 276 us for a batch of 1024 seeds, fanouts [5,10,15].
-constexpr uint32_t kLongRow = 2048, kSharedRow = 512;
-static_assert(kLongRow <= kDrawRow, "draw_rows takes every row that is not long");
+constexpr uint32_t kLongRow = 2048;
+static_assert(kLongRow <= kDrawRow && kLongRow <= kWaveDrawRow, "draw_rows and draw_by_wave take every row that is not long");
 constexpr int64_t kMinQueueBlocks = 256, kMaxQueueBlocks = 512;  // (see queue_blocks)
 constexpr int64_t kSharedMaxRows = 4096, kSharedMaxSeeds = 12288;  // of a later hop, of hop 0
 constexpr int64_t kSharedBlocks = 256;  // one per CU
-constexpr int kSharedRows = 16;
+constexpr int kSharedRows = kLongBlock / kWave;  // a wave for each
 constexpr int kSeedSegment = 256;       // seeds of one list of long rows in hop 0
 
-// A seed row as one thread looks it up (no row if i >= s).
+// A seed row as one thread looks it up.
 template <typename IdT>
 struct WeightedRow {
   int64_t b;      // its first edge
@@ -554,11 +558,11 @@ struct WeightedRow {
   __device__ __forceinline__ bool chosen(int k, bool replace) const { return deg > 0 && (replace || deg > uint32_t(k)); }
 };
 template <typename IdT, typename PtrT, typename TableT>
-__device__ __forceinline__ WeightedRow<IdT> look_up_row(const Hop& h, int64_t s, int64_t i, const TableT& table,
-                                                        const TierView<PtrT>& indptr, const TierView<IdT>& indices) {
+__device__ __forceinline__ WeightedRow<IdT> look_up_row(bool is_row, IdT seed, const TableT& table, const TierView<PtrT>& indptr,
+                                                        const TierView<IdT>& indices) {
   WeightedRow<IdT> r{0, 0u, IdT(0), true, false};
-  if (i < s) {
-    r.seed = static_cast<const IdT*>(h.seeds)[i];
+  if (is_row) {
+    r.seed = seed;
     // nothing is addressed by an id or an offset before it has been checked
     r.seed_ok = row_in_range(indptr, int64_t(r.seed)) && table.holds(r.seed);
     int64_t deg64 = 0;
@@ -580,13 +584,12 @@ struct ChooseLds {
 };
 constexpr uint32_t kElsewhere = 0xffffffffu;
 
-// The picks of the hop's rows [first, first + rows), by a whole block.  Long rows, and with SHARED some of
-// those above kSharedRow positions, are only announced (put_off(row, its number here), by one thread).
-template <typename IdT, typename PtrT, typename TableT, bool REPLACE, bool SHARED, int NT, typename PutOff>
+// The picks of the hop's rows [first, first + rows) but the long ones, by a whole block.
+template <typename IdT, typename PtrT, typename TableT, bool REPLACE, int NT>
 __device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t s, int64_t first, int rows,
                                                    ChooseLds<NT, REPLACE>& lds, const TableT& table,
                                                    const TierView<PtrT>& indptr, const TierView<IdT>& indices,
-                                                   const TierView<float>& probs, uint64_t rng_seed, PutOff put_off) {
+                                                   const TierView<float>& probs, uint64_t rng_seed) {
   const int k = h.k;
   const bool look_first = look_before_insert(h, s);
   const bool bucketed = bucketed_now(h, s);
@@ -595,21 +598,14 @@ __device__ __forceinline__ void fill_rows_weighted(const Hop& h, int64_t s, int6
   WeightedRow<IdT> own;
   clear_entries(lds.rows, rows, k);
   if (t < kWave) {
-    own = look_up_row<IdT, PtrT>(h, t < rows ? s : 0, first + t, table, indptr, indices);
+    own = look_up_row<IdT, PtrT>(t < rows, t < rows ? static_cast<const IdT*>(h.seeds)[first + t] : IdT(0), table, indptr, indices);
     const bool chosen = k > 0 && own.chosen(k, REPLACE);
-    uint32_t long_row = kLongRow;
-    if (SHARED) {  // (the block's turns on all rows in between against the longest one's time on its wave)
-      const bool between = chosen && own.deg > kSharedRow && own.deg <= kLongRow;
-      const uint32_t n = uint32_t(__builtin_popcountll(__ballot(between)));
-      if (n * kSharedRow <= ~wave_min(between ? ~own.deg : ~0u)) long_row = kSharedRow;
-    }
-    const bool is_long = chosen && own.deg > long_row;
+    const bool is_long = chosen && own.deg > kLongRow;
     set_row(lds.rows, own.b, int64_t(own.seed), chosen && !is_long ? own.deg : 0u);
     if (t < kChooseRows) {
       lds.picks[t] = is_long ? kElsewhere : chosen ? uint32_t(k) : REPLACE || k == 0 ? 0u : own.deg;
       lds.bad_pick[t] = 0;
     }
-    if (is_long) put_off(own, t);
     if (t < rows && h.index == 0) {  // the caller's seeds open the mapping list
       bool first_seen;
       uint32_t displaced;
@@ -773,11 +769,56 @@ __global__ __launch_bounds__(kBlock, REPLACE ? 3 : 4) void hop_fill_weighted_ker
       if (h.n_seeds_out && at == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
       const int64_t first = at * rows_per_block;
       if (first >= s) continue;  // whole blocks leave together
-      fill_rows_weighted<IdT, PtrT, TableT, REPLACE, false, kBlock>(h, s, first, rows_per_block, lds.choose, table, indptr, indices,
-                                                                    probs, rng_seed, [](const WeightedRow<IdT>&, int) {});
+      fill_rows_weighted<IdT, PtrT, TableT, REPLACE, kBlock>(h, s, first, rows_per_block, lds.choose, table, indptr, indices, probs,
+                                                             rng_seed);
     }
     __syncthreads();  // lds is rewritten by the block's next rows
   }
+}
+
+// The picks of one row, by one wave (all of its lanes have looked the row up): a lane has a pick, and in hop 0 the
+// lane behind them, or the first one afterwards, the seed, which opens the mapping list.
+struct WaveRaceLds {
+  __align__(16) WaveList list;
+  uint32_t entry_key[kMaxWeightedPicks + 1], entry_pos[kMaxWeightedPicks + 1];
+};
+template <bool REPLACE> using WaveLds = std::conditional_t<REPLACE, WaveDrawLds, WaveRaceLds>;
+template <typename IdT, typename TableT, bool REPLACE>
+__device__ __forceinline__ void fill_row_weighted(const Hop& h, int64_t s, int64_t i, const WeightedRow<IdT>& own, WaveLds<REPLACE>& lds,
+                                                  const TableT& table, const TierView<IdT>& indices, const TierView<float>& probs,
+                                                  uint64_t rng_seed) {
+  const bool look_first = look_before_insert(h, s);
+  const bool bucketed = bucketed_now(h, s);
+  const int k = h.k, l = threadIdx.x & (kWave - 1);
+  const bool chosen = k > 0 && own.chosen(k, REPLACE);
+  const uint32_t n = chosen ? uint32_t(k) : REPLACE || k == 0 ? 0u : own.deg;
+  const int64_t b = wave_uniform(own.b), row = wave_uniform(int64_t(own.seed));
+  const uint32_t deg = wave_uniform(own.deg);
+  uint32_t pos = uint32_t(l);  // copied rows keep their positions in order
+  if (chosen) {
+    if constexpr (REPLACE) {
+      pos = draw_by_wave(lds, probs, b, deg, k, rng_seed, h.rng_stream, row);
+    } else {
+      race_by_wave<true>(lds.list, lds.entry_key, lds.entry_pos, true, k, probs, b, deg, rng_seed, h.rng_stream, row);
+      if (l < k) pos = lds.entry_pos[l];
+    }
+  }
+  const int64_t p0 = h.pos_base + seed_part(h, s) + i * k;
+  bool ok = true;
+  const auto place = [&](bool is_seed) {
+    uint32_t word = kInvalidSlot;
+    const int64_t p = is_seed ? h.pos_base + i : p0 + l;
+    if (is_seed ? own.seed_ok : uint32_t(l) < n)
+      ok = place_pick<IdT>(h, table, is_seed ? own.seed : indices.at(b + pos), p, look_first, bucketed, &word);
+    h.slot[p] = word;
+  };
+  const bool seed_too = h.index == 0;
+  if (l < k + int(seed_too)) place(l == k);
+  if (seed_too && k == kWave && l == 0) place(true);
+  const uint64_t bad = __ballot(!ok);
+  if (l == 0)
+    h.row_cnt[i] = !own.seed_ok ? kBadSeed : own.bad ? kBadRow : bad != 0 ? kBadPick
+                 : (REPLACE ? (deg == 0 ? 0u : uint32_t(k)) : (deg < uint32_t(k) ? deg : uint32_t(k)));
 }
 
 // A small hop: blocks [0, fill_blocks) have rows_per_block (at most kSharedRows) seed rows each; the blocks
@@ -803,21 +844,35 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Ho
   }
   struct Listed { int64_t row, begin; uint32_t deg; int at; };
   __shared__ union {
-    ChooseLds<kLongBlock, REPLACE> choose;
+    WaveLds<REPLACE> wave[kSharedRows];
     LongLds<kLongBlock, REPLACE> long_row;
   } lds;
   __shared__ Listed listed[kSharedRows];
   __shared__ int n_listed;
-  const int64_t s = seeds_of(h);
   const int64_t first = int64_t(blockIdx.x) * rows_per_block;
+  const int wave = int(wave_uniform(uint32_t(threadIdx.x / kWave)));
+  const int64_t i = first + wave;
+  // (asked for together with the hop's length: the seed list has room for s_max ids)
+  const IdT seed = wave < rows_per_block && i < h.s_max ? static_cast<const IdT*>(h.seeds)[i] : IdT(0);
+  const int64_t s = seeds_of(h);
   if (h.n_seeds_out && blockIdx.x == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   if (first >= s) return;  // whole blocks leave together
   if (threadIdx.x == 0) n_listed = 0;
-  wave_lds_fence();  // (the first wave lists)
-  fill_rows_weighted<IdT, PtrT, TableT, REPLACE, true, kLongBlock>(
-      h, s, first, rows_per_block, lds.choose, table, indptr, indices, probs, rng_seed, [&](const WeightedRow<IdT>& row, int r) {
-        listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(row.seed), row.b, row.deg, r};
-      });
+  __syncthreads();
+  const bool has_row = wave < rows_per_block && i < s;
+  const WeightedRow<IdT> own = look_up_row<IdT, PtrT>(has_row, seed, table, indptr, indices);
+  if (has_row && h.k > 0 && own.deg > kLongRow) {
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+      listed[atomicAdd(&n_listed, 1)] = Listed{int64_t(own.seed), own.b, own.deg, wave};
+      if (h.index == 0) {  // (while the other waves are at their rows)
+        uint32_t word;
+        place_pick<IdT>(h, table, own.seed, h.pos_base + i, false, false, &word);
+        h.slot[h.pos_base + i] = word;
+      }
+    }
+  } else if (has_row) {
+    fill_row_weighted<IdT, TableT, REPLACE>(h, s, i, own, lds.wave[wave], table, indices, probs, rng_seed);
+  }
   __syncthreads();
   const int n = n_listed;
   for (int t = 0; t < n; ++t) {

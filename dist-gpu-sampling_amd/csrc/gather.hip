@@ -178,6 +178,7 @@ __global__ __launch_bounds__(kGatherThreads) void gather_flat_kernel(FlatGather 
 // [50,50] 374 -> 366, 111 M nodes 221 -> 215.
 static_assert(kGatherThreads == kEdgeBlock, "the blocks are shared");
 constexpr int64_t kEdgeGrid = 4096;  // at most: they loop over the worst case, most of which is not there
+constexpr int64_t kMaxEdgeGrid = 16384;  // ... and in a launch of their own
 template <int VEC, int TIER, typename IndexT, bool STRIDE>
 __global__ __launch_bounds__(kGatherThreads) void gather_flat_edges_kernel(FlatGather a, const IndexT* __restrict__ index,
                                                                            EdgeJob edges, int32_t edge_grid) {
@@ -191,14 +192,22 @@ __global__ __launch_bounds__(kGatherThreads) void gather_flat_edges_kernel(FlatG
     for (int64_t b = blockIdx.x; b < edges.blocks; b += edge_grid) later_edge_tile<IndexT, false>(edges, b, threadIdx.x);
   }
 }
-template <typename IdT>
+// The list as a launch of its own.  Where the grid takes a block for every tile of the worst case, a thread asks for
+// its elements together with the hop's length; beyond that blocks loop over what the hop really has.  The last
+// list of a batch of 1024 seeds, fanouts [5,10,15], with loops / without: 7.6 / 6.6 us; of 4096 seeds 26.1 / 25.6.
+template <typename IdT, bool STRIDE>
 __global__ __launch_bounds__(kEdgeBlock) void edges_kernel(EdgeJob edges) {
-  for (int64_t b = blockIdx.x; b < edges.blocks; b += gridDim.x) later_edge_tile<IdT, false>(edges, b, threadIdx.x);
+  if (!STRIDE) later_edge_tile<IdT, true>(edges, blockIdx.x, threadIdx.x);
+  else
+    for (int64_t b = blockIdx.x; b < edges.blocks; b += gridDim.x) later_edge_tile<IdT, false>(edges, b, threadIdx.x);
 }
 dgs_status launch_edges(const EdgeJob& e, hipStream_t st) {
-  const dim3 grid(uint32_t(e.blocks < kEdgeGrid ? e.blocks : kEdgeGrid));
-  if (e.id_bytes == 8) hipLaunchKernelGGL(edges_kernel<int64_t>, grid, dim3(kEdgeBlock), 0, st, e);
-  else hipLaunchKernelGGL(edges_kernel<int32_t>, grid, dim3(kEdgeBlock), 0, st, e);
+  const int64_t forced = debug_option(DGS_DEBUG_SAMPLER_GRID_CAP);
+  const bool loops = e.blocks > (forced > 0 ? forced : kMaxEdgeGrid);
+  const dim3 grid(uint32_t(!loops ? e.blocks : forced > 0 && forced < kEdgeGrid ? forced : kEdgeGrid));
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kEdgeBlock), 0, st, e); };
+  if (e.id_bytes == 8) loops ? go(edges_kernel<int64_t, true>) : go(edges_kernel<int64_t, false>);
+  else loops ? go(edges_kernel<int32_t, true>) : go(edges_kernel<int32_t, false>);
   DGS_LAUNCH_CHECK();
   return DGS_OK;
 }

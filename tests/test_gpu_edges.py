@@ -42,3 +42,36 @@ def test_edge_list_in_the_gathers_launch(pkg, oracle, n_seeds, fanouts, dim, dty
         for g, w in zip(blocks, want):
             assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
         assert torch.equal(rows.cpu(), x[torch.from_numpy(want_f.astype(np.int64))])
+
+
+@pytest.mark.parametrize("n_seeds,fanouts,dim,cap", [
+    (3000, [7, 4], 0, 0),        # no features: a list of its own, by a block for every tile
+    (3000, [7, 4], 0, 3),        # ... by blocks that loop
+    (3000, [7, 4], 301, 0),      # in front of a gather of odd-width rows
+    (3000, [7, 4], 301, 1),
+    (40_000, [40, 49], 0, 0),    # more tiles than a launch has blocks
+])
+def test_edge_list_in_a_launch_of_its_own(pkg, oracle, n_seeds, fanouts, dim, cap):
+    rng = np.random.default_rng(12)
+    n = 20_000
+    indptr, indices = powerlaw_graph(rng, n, 12, 300)
+    ip = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    seeds = rng.integers(0, n, size=n_seeds).astype(indices.dtype)
+    sampler = pkg.ChunkTensorSampler(fanouts, ip, ix)
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, False, 31, 4)
+    capi = pkg.capi
+    capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, cap))
+    try:
+        pkg.set_rng_state(31, 4)
+        if dim:
+            x = torch.from_numpy(rng.standard_normal((n, dim)).astype(np.float32)).to(torch.bfloat16)
+            f, _, blocks, rows = sampler.sample_blocks_and_index(None, torch.from_numpy(seeds), pkg.create_chunktensor(x, 1, 1 << 40))
+            assert torch.equal(rows.cpu(), x[torch.from_numpy(want_f.astype(np.int64))])
+        else:
+            f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds))
+        assert np.array_equal(f.cpu().numpy(), want_f)
+        for g, w in zip(blocks, want):
+            assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+    finally:
+        capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, 0))

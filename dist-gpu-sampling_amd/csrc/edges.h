@@ -28,9 +28,12 @@ __device__ __forceinline__ bool is_bad_row(uint32_t row_cnt) { return row_cnt >=
 //   table slot                in hop 0, whose first occurrences are settled by asking the table.
 // A pick that is not its id's first has met a smaller position of the id when it was inserted.  That one may
 // itself be displaced later in the same launch: whoever does so leaves a link to its own position in rank_at,
-// and positions only get smaller along the links.  Reading these words, a stream and some 4-byte reads near
+// and positions only get smaller along the links.  What makes every position met a rank or a link: one of the same
+// launch is linked when it is displaced, and one of an earlier hop is its id's smallest for good, because a hop's
+// launches end before the next hop looks (see DirectTable).  Hop 0 leaves no links: its displaced positions hold
+// numbers that mean nothing, and none of them may be met later.  Reading these words, a stream and some 4-byte reads near
 // one another, in place of the table's entry saves a random read of a table that caches do not hold: R-MAT of
-// 2^26 nodes, 3.05 M picks, two thirds of them repeats: 44 -> 25 us for the hop's edge list, 380 -> 369 for the batch.
+// 2^26 nodes, 3.05 M picks, two thirds of them repeats: 44 -> 25 us for the hop's edge list, 376 -> 365 for the batch.
 constexpr uint32_t kRankBit = 0x40000000u;
 constexpr uint32_t kLinkBit = 0x80000000u;
 
@@ -61,10 +64,15 @@ __device__ __forceinline__ int64_t count_of(const int64_t* n_dev, int64_t n_host
 __host__ __device__ __forceinline__ int edge_groups(int k) { return (k + kEdgeItems - 1) / kEdgeItems; }
 inline int64_t edge_blocks(int64_t s_max, int k) { return ((s_max + kRowTile - 1) / kRowTile) * edge_groups(k); }
 
-// rank at position `at`, or where the links from there lead
-__device__ __forceinline__ uint32_t rank_from(const uint32_t* __restrict__ rank_at, uint32_t at) {
-  uint32_t r = rank_at[at];
-  while (r & kLinkBit) r = rank_at[r & ~kLinkBit];
+// The rank that r, read at position `at`, is, or that the links from there lead to.  A link to no smaller position is
+// none that a launch has left: it is not followed (rank 0).
+__device__ __forceinline__ uint32_t rank_from(const uint32_t* __restrict__ rank_at, uint32_t at, uint32_t r) {
+  while (r & kLinkBit) {
+    const uint32_t next = r & ~kLinkBit;
+    if (next >= at) return 0;
+    at = next;
+    r = rank_at[at];
+  }
   return r;
 }
 
@@ -120,6 +128,7 @@ __device__ __forceinline__ void edge_tile(const EdgeJob& e, int64_t b, int tid, 
     at[j] = uint32_t(p[j]);
     known[j] = false;
     if (live[j] && !(word[j] & kFirstBit)) at[j] = at_of(s, word[j], &known[j]);
+    if (!known[j] && at[j] > uint32_t(p[j])) at[j] = uint32_t(p[j]);  // (words name no later position: none is read by one that does)
   }
   uint32_t rank[kEdgeItems];
 #pragma unroll
@@ -127,8 +136,7 @@ __device__ __forceinline__ void edge_tile(const EdgeJob& e, int64_t b, int tid, 
   static_assert(kEdgeItems == 4, "the ranks are looked over at once");
   if ((rank[0] | rank[1] | rank[2] | rank[3]) & kLinkBit) {
 #pragma unroll
-    for (int j = 0; j < kEdgeItems; ++j)
-      if (rank[j] & kLinkBit) rank[j] = rank_from(e.rank_at, rank[j] & ~kLinkBit);
+    for (int j = 0; j < kEdgeItems; ++j) rank[j] = rank_from(e.rank_at, at[j], rank[j]);
   }
 #pragma unroll
   for (int j = 0; j < kEdgeItems; ++j) {

@@ -174,7 +174,10 @@ struct DirectTable {
   // `look_first`: read the entry before the atomic.  A value already below v (a stale read can
   // only be larger than the truth) settles the matter without an atomic, which is what keeps
   // popular ids from serialising thousands of atomics on one address; on ids that are mostly
-  // new the extra read is pure cost.  The result is the same either way.
+  // new the extra read is pure cost.  Whether idx is first is the same either way; *met may be a
+  // position that has been displaced since, in this launch, and then holds a link to a smaller one.
+  // It must not be staler than that: every launch that inserts has to end, its entries visible,
+  // before one of a later hop looks (a position that hop 0 displaced holds no link).
   __device__ __forceinline__ uint32_t insert_min(IdT key, uint32_t idx, bool* first, uint32_t* met,
                                                  bool look_first = true) const {
     const unsigned long long v = (static_cast<unsigned long long>(tag) << 32) | idx;

@@ -259,8 +259,8 @@ def test_weighted_fused_long_rows_and_wide_fanout(pkg, oracle, last_hop):
 @pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("n_seeds", [1, 16, 17, 12288, 12289, 16384, 16385])
 def test_weighted_fused_small_and_large_hops(pkg, oracle, last_hop, n_seeds, replace):
-    # hops of up to 12288 rows are one launch whose 16-wave blocks share their long rows, larger ones two
-    # launches: row lengths around the limits, several long rows a block, a small hop in front of a large one
+    # a first hop of up to 12288 rows is one launch with a wave for each and its long rows in turn, a larger one
+    # shares blocks and has a queue: row lengths around the limits, several long rows a block, both as a later hop
     rng = np.random.default_rng(n_seeds)
     deg = np.concatenate([[256, 257, 511, 512, 513, 4096, 4097, 2047, 2048, 2049, 0, 1], rng.integers(0, 40, size=3000)])
     n = deg.size
@@ -282,9 +282,8 @@ def test_weighted_fused_small_and_large_hops(pkg, oracle, last_hop, n_seeds, rep
 @pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("n_seeds", [2, 16, 256, 257, 513, 3840, 3841, 12288, 12289])
 def test_weighted_fused_dense_rows(pkg, oracle, n_seeds, replace):
-    # how many rows a block of a small hop has goes by the hop's size (1 up to 256 rows, 16 above 3840),
-    # whether it shares its rows of 513 to 2048 positions goes by how many of them it has; hops above
-    # 12288 rows are two launches
+    # how many rows a block of a small hop has goes by the hop's size (1 up to 256 rows, 16 above 3840); rows of
+    # up to 2048 positions have a wave each, longer ones the block; a first hop above 12288 rows has a queue
     rng = np.random.default_rng(n_seeds)
     deg = np.concatenate([[513, 1023, 1024, 1025, 1536, 2048, 2049, 5000, 0, 512], rng.integers(513, 2049, size=30)])
     n = deg.size
@@ -306,7 +305,7 @@ def test_weighted_fused_dense_rows(pkg, oracle, n_seeds, replace):
 @pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("k", [32, 33, 64])
 def test_weighted_fused_wide_picks_around_the_limit_of_one_launch(pkg, oracle, k, replace):
-    # above 32 picks hops of more than 4096 rows are two launches already
+    # a wave a row up to 12288 rows of a first hop, and beyond that blocks of 32 rows up to 32 picks, of 16 above
     rng = np.random.default_rng(k)
     deg = np.concatenate([[0, 1, 32, 33, 64, 65, 513, 2048, 2049, 4097], rng.integers(20, 100, size=500)])
     n = deg.size
@@ -315,13 +314,35 @@ def test_weighted_fused_wide_picks_around_the_limit_of_one_launch(pkg, oracle, k
     probs = (rng.random(indices.size) + 0.01).astype(np.float32)
     cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
     sampler = pkg.ChunkTensorSampler([k], cts[0], cts[1], cts[2], replace, seed=9)
-    for n_seeds in (4096, 4097):
+    for n_seeds in (4096, 4097, 12288, 12289):
         seeds = np.concatenate([np.arange(10), rng.integers(0, n, size=n_seeds - 10)]).astype(np.int64)
         f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds), batch=0)
         want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, [k], replace, 9, 0, probs=probs)
         assert np.array_equal(_np(f), want_f)
         assert np.array_equal(_np(blocks[0].src_local), want_blocks[0][0])
         assert np.array_equal(_np(blocks[0].dst_local), want_blocks[0][1])
+
+
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n_seeds,k", [(256, 15), (241, 16)])  # a second hop of 4096 rows at most, and of 4097
+@pytest.mark.parametrize("k2", [7, 33, 64])
+def test_weighted_fused_later_hop_around_the_limit_of_one_launch(pkg, oracle, n_seeds, k, k2, replace):
+    rng = np.random.default_rng(n_seeds + k2)
+    deg = np.concatenate([np.full(40, 2049) + np.arange(40) * 77, rng.integers(16, 90, size=6000)])
+    n = deg.size
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    indices = rng.integers(0, n, size=int(indptr[-1])).astype(np.int64)
+    hub = rng.random(indices.size) < 0.01
+    indices[hub] = rng.integers(0, 40, size=int(hub.sum()))
+    probs = (rng.random(indices.size) + 0.01).astype(np.float32)
+    seeds = np.concatenate([np.arange(20), rng.permutation(np.arange(40, n))[:n_seeds - 20]]).astype(np.int64)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, indices, probs)]
+    sampler = pkg.ChunkTensorSampler([k2, k], cts[0], cts[1], cts[2], replace, seed=9)
+    f, _, blocks = sampler.sample_blocks(None, torch.from_numpy(seeds), batch=0)
+    want_f, _, want_blocks = oracle.sample_blocks(seeds, indptr, indices, [k2, k], replace, 9, 0, probs=probs)
+    assert np.array_equal(_np(f), want_f)
+    for g, w in zip(blocks, want_blocks):
+        assert np.array_equal(_np(g.src_local), w[0]) and np.array_equal(_np(g.dst_local), w[1])
 
 
 @pytest.mark.parametrize("replace", [False, True])

@@ -808,8 +808,8 @@ __device__ __forceinline__ void fill_row_weighted(const Hop& h, int64_t s, int64
   const auto place = [&](bool is_seed) {
     uint32_t word = kInvalidSlot;
     const int64_t p = is_seed ? h.pos_base + i : p0 + l;
-    if (is_seed ? own.seed_ok : uint32_t(l) < n)
-      ok = place_pick<IdT>(h, table, is_seed ? own.seed : indices.at(b + pos), p, look_first, bucketed, &word);
+    if (is_seed ? own.seed_ok : uint32_t(l) < n)  // (a lane may place a pick and then the seed: neither hides the other's fault)
+      ok &= place_pick<IdT>(h, table, is_seed ? own.seed : indices.at(b + pos), p, look_first, bucketed, &word);
     h.slot[p] = word;
   };
   const bool seed_too = h.index == 0;

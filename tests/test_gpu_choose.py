@@ -136,3 +136,24 @@ def test_long_rows_reach_the_hop_that_has_them(pkg, oracle, n_seeds, fanouts, re
     assert np.array_equal(f.cpu().numpy(), want_f)
     for g, w in zip(blocks, want):
         assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+
+
+@pytest.mark.parametrize("n_seeds", [40, 12289])   # a wave for each row; rows shared by a block
+@pytest.mark.parametrize("k", [1, 63, 64])         # (with 64 picks the first lane places the seed too)
+@pytest.mark.parametrize("at", [0, -1])
+def test_an_id_outside_the_graph_in_any_lane_is_refused(pkg, n_seeds, k, at):
+    n = 500
+    indptr = np.arange(n + 1, dtype=np.int64) * k
+    indices = np.random.default_rng(k).integers(0, n, size=n * k).astype(np.int64)
+    cts = [pkg.create_chunktensor(torch.from_numpy(a), 1, 1 << 40) for a in (indptr, np.ones(n * k, dtype=np.float32))]
+    seeds = torch.arange(n_seeds) % n
+    for bad_id in (None, n, -1, 2 ** 35):
+        if bad_id is not None:
+            indices[indptr[10 + 1] - 1 if at else indptr[10]] = bad_id   # of node 10, whose row is copied whole
+        ix = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+        sampler = pkg.ChunkTensorSampler([k], cts[0], ix, cts[1])
+        if bad_id is None:
+            sampler.sample_blocks(None, seeds)
+            continue
+        with pytest.raises(RuntimeError, match="neighbour id"):
+            sampler.sample_blocks(None, seeds)

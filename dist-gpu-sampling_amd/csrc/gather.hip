@@ -179,11 +179,11 @@ __global__ __launch_bounds__(kGatherThreads) void gather_flat_kernel(FlatGather 
 static_assert(kGatherThreads == kEdgeBlock, "the blocks are shared");
 constexpr int64_t kEdgeGrid = 4096;  // at most: they loop over the worst case, most of which is not there
 constexpr int64_t kMaxEdgeGrid = 16384;  // ... and in a launch of their own
-template <int VEC, typename IndexT, bool STRIDE>
+template <int VEC, int TIER, typename IndexT, bool STRIDE>
 __global__ __launch_bounds__(kGatherThreads) void gather_flat_edges_kernel(FlatGather a, const IndexT* __restrict__ index,
                                                                            EdgeJob edges, int32_t edge_grid) {
   if (int64_t(blockIdx.x) >= edge_grid) {
-    gather_flat<VEC, DGS_TIER_ANY, IndexT, STRIDE>(a, index, int64_t(blockIdx.x) - edge_grid, int64_t(gridDim.x) - edge_grid);
+    gather_flat<VEC, TIER, IndexT, STRIDE>(a, index, int64_t(blockIdx.x) - edge_grid, int64_t(gridDim.x) - edge_grid);
     return;
   }
   if (edges.blocks <= edge_grid) {
@@ -439,28 +439,25 @@ dgs_status launch_gather(const dgs_view& v, int64_t row_bytes, const void* index
                        static_cast<char*>(out)};
     const IndexT* ids = static_cast<const IndexT*>(index);
     const dim3 block(kGatherThreads);
-    bool launched = false;
-    if (edges != nullptr) {
-      // (the sampler asks for rows of either tier, and rows of 1- and 2-byte chunks are few: the list goes ahead)
-      if constexpr (VEC >= 4 && TIER == DGS_TIER_ANY) {
+    if constexpr (VEC >= 4) {
+      if (edges != nullptr) {
         const int32_t edge_grid = int32_t(edges->blocks < kEdgeGrid ? edges->blocks : kEdgeGrid);
         const dim3 grid(uint32_t(blocks + edge_grid));
         if (blocks < tiles)
-          hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, IndexT, true>), grid, block, lds, st, a, ids, *edges, edge_grid);
+          hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, TIER, IndexT, true>), grid, block, lds, st, a, ids, *edges, edge_grid);
         else
-          hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, IndexT, false>), grid, block, lds, st, a, ids, *edges, edge_grid);
-        launched = true;
-      } else {
-        const dgs_status es = launch_edges(*edges, st);
-        if (es != DGS_OK) return es;
+          hipLaunchKernelGGL((gather_flat_edges_kernel<VEC, TIER, IndexT, false>), grid, block, lds, st, a, ids, *edges, edge_grid);
+        DGS_LAUNCH_CHECK();
+        return DGS_OK;
       }
+    } else if (edges != nullptr) {  // (rows of 1- and 2-byte chunks are short or few)
+      const dgs_status es = launch_edges(*edges, st);
+      if (es != DGS_OK) return es;
     }
-    if (launched) {
-    } else if (blocks < tiles) {
+    if (blocks < tiles)
       hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, true>), dim3(uint32_t(blocks)), block, lds, st, a, ids);
-    } else {
+    else
       hipLaunchKernelGGL((gather_flat_kernel<VEC, TIER, IndexT, false>), dim3(uint32_t(blocks)), block, lds, st, a, ids);
-    }
   } else {
     if (edges != nullptr) {
       const dgs_status es = launch_edges(*edges, st);

@@ -135,8 +135,8 @@ def test_edges_left_and_written(batch, weighted):
     (4, None, 4, 20, 0),   # ... which leaves wave slots to others
     (8, None, 0, 20, 0),   # indices of another width than the ids
     (4, 0, 0, 20, 0),      # no rows to gather
-    (4, None, 0, 20, 1),   # rows of one tier, chunks of 1 or 2 bytes: lists of their own
-    (4, None, 0, 1, 0)])
+    (4, None, 0, 20, 1),   # one tier
+    (4, None, 0, 1, 0)])   # chunks of 1 or 2 bytes: a list of its own
 def test_edges_left_to_a_gather(batch, weighted, index_bytes, n_max, blocks_per_cu, elems, tier):
     capi, x, leave, check = batch
     b = leave(weighted)

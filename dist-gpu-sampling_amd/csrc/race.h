@@ -1,5 +1,7 @@
-// The two weighted pick rules as device procedures over one seed row, shared by the per-hop
-// weighted operator (weighted.hip) and the fused multi-hop sampler (pipeline.hip).
+// The two weighted pick rules as device procedures over one seed row.  The per-hop weighted operator
+// (weighted.hip) runs them as they are; the fused sampler lays the same rules out over many rows and over 32-bit keys
+// first (choose.h) and comes here for the rows that these leave open (race_row, race_long_row_full) and for the
+// sums and shares.
 //   without replacement: every position races with the key E / w (E a unit exponential variate
 //     from the row's Philox stream); a group of G lanes keeps the num_picks smallest
 //     (key, position) pairs in order, lane l holding the l-th;
@@ -10,7 +12,7 @@
 // oracle's bit for bit whatever the launch shape.  Loops that contain cross-lane operations run a
 // wave-uniform number of times: a group that has run out of work keeps executing with empty
 // candidates.  Rows above long_row<G>() positions are meant for the *_long_row procedures, which
-// spread a row over the 16 waves of a 1024-thread block.
+// spread a row over the waves of a block.
 #ifndef DGS_CSRC_RACE_H_
 #define DGS_CSRC_RACE_H_
 

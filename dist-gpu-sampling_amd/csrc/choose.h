@@ -788,7 +788,8 @@ __device__ __forceinline__ uint32_t draw_by_wave(WaveDrawLds& lds, const TierVie
 // its own part.  What is beyond is read in three passes, bound by the wait for memory: several stretches ahead
 // (16 384 rows, 8 of them of 10^6 positions, 10 draws, us a call: one stretch at a time 1593; four ahead in
 // every pass 1117, eight in the two sums and four in the search, whose registers eight would not fit, 1057; 64
-// rows of 200 000: 391, 288, 274).
+// rows of 200 000: 391, 288, 274).  Rows that end soon after the held part gain nothing: 4000 seeds, fanouts [5,10], rows of
+// 6000, one stretch at a time 449; eight asked for whether or not they are there 521, those that are there 470.
 template <int N> using AheadOf = std::integral_constant<int, N>;
 template <int NT>
 struct DrawLongLds {
@@ -802,6 +803,8 @@ __device__ __forceinline__ void draw_long(DrawLongLds<NT>& lds, const TierView<f
   constexpr int kHeld = 5;
   constexpr uint64_t kStretch = 4 * kWave;
   const int lane = threadIdx.x & (kWave - 1), wave = int(wave_uniform(uint32_t(threadIdx.x / kWave)));
+  begin = wave_uniform(begin);
+  deg = wave_uniform(deg);
   const uint64_t part = ((deg + uint64_t(kWaves) - 1) / kWaves + kStretch - 1) / kStretch * kStretch;
   const uint64_t lo = part * uint32_t(wave) < deg ? part * uint32_t(wave) : deg;
   const uint64_t hi = lo + part < deg ? lo + part : deg;
@@ -821,7 +824,8 @@ __device__ __forceinline__ void draw_long(DrawLongLds<NT>& lds, const TierView<f
     for (uint64_t p0 = lo + kHeld * kStretch; on && p0 < hi; p0 += kAhead * kStretch) {
       float4_anywhere next[kAhead];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) next[u] = quad_at(p0 + u * kStretch);
+      for (int u = 0; u < kAhead; ++u)  // (the last stretches are few: none is asked for beyond them)
+        next[u] = p0 + u * kStretch < hi ? quad_at(p0 + u * kStretch) : float4_anywhere(0.0f);
 #pragma unroll
       for (int u = 0; u < kAhead; ++u)
         if (on && p0 + u * kStretch < hi) on = each(p0 + u * kStretch, next[u]);

@@ -1656,15 +1656,16 @@ void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* 
 
 // Blocks of a weighted launch that take queued long rows, in front of `others`.  256 keep a block on every CU, which
 // a frontier of hubs leaves waiting for its chains: 512 where they and the others fit the GPU at once, four
-// blocks to a CU, or where there are several rounds of the others anyway.  In between the others would be dealt
+// blocks to a CU (three where the picks are drawn), or where there are several rounds of the others anyway.  In between the others would be dealt
 // out unevenly behind them (2048 seeds, fanouts [10,10], rows of 300: 129 us with 256, 137 with 512).
 // us a call, 256 / 512: 16 384 rows of 3000 750 / 441 (10 picks), 455 / 279 (draws); of 17 000 1572 / 926, 1360 /
 // 791; 300 of 20 000 among them 134 / 107, 129 / 104; 1024 seeds, fanouts [10,10], rows of 3000 548 / 358, 352 / 239.
+// Draws by 12 289 seeds of 1000 positions, no long row among them: 133 with 256 or 383, 141 with 512.
 // Batches whose long rows are a few hundred: level.  1024 or 2048: 290 for the first, and 2 to 5 us more for those.
-inline int64_t queue_blocks(int64_t others) {
-  constexpr int64_t kSlots = 1024;
-  if (others >= kSlots) return kMaxQueueBlocks;
-  return std::min(kMaxQueueBlocks, std::max(kMinQueueBlocks, kSlots - others));
+inline int64_t queue_blocks(int64_t others, bool replace) {
+  if (others >= 1024) return kMaxQueueBlocks;
+  const int64_t slots = replace ? 768 : 1024;
+  return std::min(kMaxQueueBlocks, std::max(kMinQueueBlocks, slots - others));
 }
 
 // Whether a weighted hop is a launch of kLongBlock-thread blocks (see above).
@@ -1691,7 +1692,7 @@ void launch_fill_weighted(const Hop& cur, const Hop& prev, int64_t relabel_count
   }
   const int64_t rows = choose_rows(cur.k);
   const int64_t fill_blocks = (cur.s_max + rows - 1) / rows;
-  const int64_t queued = queue_blocks(fill_blocks + relabel_count);
+  const int64_t queued = queue_blocks(fill_blocks + relabel_count, REPLACE);
   const int64_t total = queued + fill_blocks + relabel_count;
   hipLaunchKernelGGL((hop_fill_weighted_kernel<IdT, PtrT, TableT, REPLACE>), dim3(capped_grid(total)), dim3(kBlock), 0, st, cur,
                      prev, queued, fill_blocks, int32_t(rows), relabel_count, table, TierView<PtrT>(indptr), TierView<IdT>(indices),

@@ -21,7 +21,7 @@ TORCH_LIB = os.path.join(HERE, "libdgs.so")
 OBJ_DIR = os.path.join(HERE, "build")  # objects of the HIP sources (not tracked)
 
 HIP_SOURCES = ["store.hip", "gather.hip", "sample.hip", "weighted.hip", "placement.hip", "unique.hip", "pipeline.hip"]
-HIP_HEADERS = ["common.h", "table.h", "picks.h", "weights.h", "race.h", "choose.h", "edges.h", "sample_workspace.h", "lookback.h", "one_block.h"]
+HIP_HEADERS = ["common.h", "table.h", "picks.h", "weights.h", "race.h", "buckets.h", "choose.h", "edges.h", "sample_workspace.h", "lookback.h", "one_block.h"]
 ARCH = "gfx950"
 
 

@@ -23,9 +23,9 @@
 //     device-scope atomic being executed at the memory side), and a hop costs two of them
 //     per pick: the indices read and the table atomic.
 //
-// A large last hop of uniform picks does without the table altogether (see Buckets below): its
-// fill records the picked ids, two launches group them by id and take the smallest position of
-// every id in LDS, and compact / relabel read the same slot words as on the table path.
+// A large last hop of uniform picks does without the table altogether (buckets.h): its fill records the
+// picked ids, two launches group them by id and find the first position of every id in LDS, and a
+// compact launch of its own leaves the slot words that relabel reads on the table path.
 //
 // Critical path per hop (2 launches): fill -> compact.
 //   fill     G lanes per seed row (G = 8..64): indptr pair, picks by the dgs-philox-1
@@ -49,6 +49,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "buckets.h"
 #include "choose.h"
 #include "common.h"
 #include "edges.h"
@@ -151,10 +152,10 @@ struct Hop {
   int32_t k;
   int32_t index;            // hop number
   uint32_t rng_stream;
-  int32_t bucketed;         // non-zero: first occurrences come from the bucketed pass (see Buckets) ...
+  int32_t bucketed;         // non-zero: first occurrences come from the bucketed pass (see below) ...
   int32_t pad1_;
   int64_t bucket_pos_cap;   // ... as long as the hop's padded positions (seeds * k) are no more than this: decided on the device
-  int* bucket_overflow;     // set by the pass when a bucket held more ids than its LDS table takes (the call fails)
+  const int* bucket_overflow;  // set by the pass when a bucket held more ids than its LDS table takes (the call fails)
   dgs_view indptr;          // weighted, where a hop follows: the offsets, for finding its long rows
   int64_t n_edges;
 };
@@ -181,58 +182,25 @@ constexpr int kFoldMaxRowPerPick = 4;
 // The atomicMin per pick is what a large hop costs most (every device-scope atomic executes at
 // the memory side: 26.7 G/s, 31 us for the 832 k picks of a 1024 x [5,10,15] batch, and as much
 // again while other batches share the GPU).  The last hop needs no table entry afterwards, so its
-// first occurrences can be found without the table.  The hop's units -- the ids the frontier
-// already holds (order value = rank) and the padded positions (order value = position, above
-// every rank) -- are cut into tiles of 4096; a block puts its tile's units in bucket order
-// (bucket = low bits of the id) and notes where every bucket's piece begins; then one block per
-// bucket walks that bucket's pieces in all tiles and takes the smallest order value of every id in
-// an LDS array indexed by the id's high bits.  A pick's slot word then says everything the later
-// stages need: first occurrence (id | kFirstBit, as the fill left it), a repeat of an id the
-// frontier held before this hop (its rank | kRankBit: final, no further lookup), or a repeat of
-// a pick of this hop (that pick's position, whose rank the compaction records).  Same result as
-// the table gives.
-constexpr int kBucketTile = 4096;                    // units per tile
-constexpr int kBucketTileItems = kBucketTile / kBlock;
-constexpr int kMinBuckets = 512;
-constexpr int kMaxBuckets = 2048;
-constexpr int kBucketRange = 8192;                   // ids per bucket at most: 32 KB of LDS
-constexpr int kMaxBucketTiles = 2048;                // tiles a bucket's block can walk (its LDS index of them)
-constexpr int64_t kBucketedMaxNodes = int64_t(kMaxBuckets) * kBucketRange;
-constexpr int64_t kBucketedMinPicks = int64_t(1) << 18;  // worst-case picks of the hop below which the table is cheaper
-// Graphs with more nodes than kBucketedMaxNodes: buckets by a hash of the id, and a bucket's ids
-// are told apart in an open-addressing table in LDS (ids + smallest order values, 128 KB of the
-// CU's 160 KB) instead of an array indexed by the id's high bits.  A bucket may hold up to half as
-// many units as the table has slots on average, which bounds the hop the pass accepts.
-constexpr int kHashBlock = 1024;
-constexpr int kHashSlots = 16384;
-constexpr uint32_t kHashEmpty = 0xffffffffu;         // no id: ids are below 2^31
-
-struct Buckets {
-  uint2* items;      // [tiles_max][kBucketTile] (id, order value), every tile's units in bucket order
-  uint16_t* piece;   // [tiles_max][buckets + 1] where every bucket's piece begins inside its tile; [buckets] = the tile's units
-  int32_t tiles_max; // tiles of units: front_tiles over the frontier array, the rest over the hop's padded positions
-  int32_t front_tiles;
-  int32_t log_buckets;
-  uint32_t n_nodes;
-  int32_t hashed;    // buckets by a hash of the id, ids told apart in an LDS hash table (any node count)
-  int32_t hash_slots;  // slots of that table the kernels use: kHashSlots (a test hook makes it small, so that small inputs fill it)
-};
-// Buckets of the hop.  The direct form's count follows from the node count (host); the hashed
-// form's follows from the hop's real size, on the device: as few buckets as keep a bucket's units
-// within its table's slots on average (a bucket that is fuller than that goes over its units in
-// parts), because every bucket costs its block a fixed chain of waits: a hop that fits 256 buckets
-// is one block per CU, all at once.
-constexpr int kMinHashLogBuckets = 8;
-__device__ __forceinline__ int log_buckets_of(const Buckets& b, const Hop& h, int64_t s) {
-  if (!b.hashed) return b.log_buckets;
-  const int64_t units = s + s * h.k;  // at most: short rows leave padded positions empty, ids repeat
-  int lb = kMinHashLogBuckets;
-  while (lb < b.log_buckets && (int64_t(b.hash_slots) << lb) < units) ++lb;
-  return lb;
-}
-__device__ __forceinline__ uint32_t bucket_of(const Buckets& b, int log_buckets, uint32_t id) {
-  return (b.hashed ? hash_id(id) : id) & uint32_t((1 << log_buckets) - 1);
-}
+// first occurrences can be found without the table (buckets.h).  The hop's units are the ids the frontier
+// already holds, their number rounded up to a multiple of 16, then the padded positions.  The fill leaves
+// the picked ids in the slot words; the compact launch has every pick's smallest unit from the pass: its own
+// (a first occurrence), that of an id the frontier held before this hop (its rank | kRankBit: final, no further
+// lookup), or that of an earlier pick of this hop (whose position becomes the slot word, and whose rank
+// the compaction records there).  Same result as the table gives.
+//
+// It takes two launches more than the table does, and pays where the hop is large (by its worst case: that is what the
+// host knows) and the table beyond the caches.  us a batch with rows of 64 bytes, table / pass: 2.4 M nodes, fanouts
+// [5,10,15], 640 seeds (0.63 M picks at most) 83 / 87, 768 85 / 88, 896 (0.89 M) 89 / 89; 4 M nodes, [5,10] from 16 384
+// seeds (0.98 M) 100 / 90, [5,10,15] from 2048 (2.0 M) 127 / 112, from 4096 228 / 193; 16 M nodes 103 / 94, 135 / 120,
+// 259 / 226.  Small graphs repeat their ids, and the table sits in the caches: 2048 and 4096 seeds, 100 k nodes 97 /
+// 100 and 112 / 122, 250 k 106 / 103 and 133 / 135, 500 k 115 / 103 and 157 / 140.  8 batches through the loader,
+// 400-byte rows, 2.4 M nodes: 512 seeds 737 / 772, 768 823 / 842, 1024 995 / 971, 2048 1679 / 1570; 20 M nodes,
+// 64-byte rows, 1024 seeds 675 / 690.
+constexpr int64_t kBucketedMinNodes = 262144, kBucketedMaxNodes = 16777216;
+constexpr int64_t kBucketedMinPicks = 917504;
+static_assert(kBucketedMaxNodes <= kDirectMaxIds, "the direct form takes them");
+__host__ __device__ __forceinline__ int64_t front_units(int64_t s) { return (s + 15) / 16 * 16; }
 
 // rank of the id at position p of hop 0, given p's slot word
 template <typename TableT>
@@ -883,351 +851,62 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Ho
   }
 }
 
-// ---- the bucketed pass (see Buckets) --------------------------------------------------------
+// ---- the bucketed pass (buckets.h) ----------------------------------------------------------
 
-// Tiles are laid out so that no address depends on the hop's length: front_tiles tiles over the
-// frontier array as large as it can get, then the tiles of the padded positions.  A block can
-// therefore ask for its units at once and decide afterwards which of them count.
-struct TileOfUnits {
-  bool front;      // a tile of frontier ids
-  int64_t first;   // its first rank, or its first position relative to the hop's pos_base
-};
-__device__ __forceinline__ TileOfUnits bucket_tile(const Buckets& b, int64_t tile) {
-  TileOfUnits t;
-  t.front = tile < b.front_tiles;
-  t.first = (t.front ? tile : tile - b.front_tiles) * kBucketTile;
-  return t;
-}
-// whether the tile holds anything at the hop's real length
-__device__ __forceinline__ bool bucket_tile_live(const Hop& h, const TileOfUnits& t, int64_t s) {
-  return t.first < (t.front ? s : s * h.k);
-}
-// A thread's units of a tile, requested without knowing the hop's length (every address lies inside
-// its array whatever the length turns out to be); `valid` then says which of them count.
-template <typename IdT>
-struct UnitsOfThread {
-  uint32_t id[kBucketTileItems];
-  uint32_t order[kBucketTileItems];
-  bool inside[kBucketTileItems];  // the address was inside the array, so id[] was loaded
-  __device__ __forceinline__ void load(const Hop& h, const TileOfUnits& t) {
+template <typename IdT, bool HASHED>
+__global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Buckets b) {
+  __shared__ SortLds<HASHED> lds;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *b.overflow = 0;  // (the per-bucket launch comes behind this one)
+  const int64_t s = wave_uniform(seeds_of(h));
+  if (!bucketed_now(h, s)) return;  // the hop outgrew the pass: it runs on the table
+  const uint32_t front = uint32_t(front_units(s)), units = front + uint32_t(s * h.k);
+  const int log_buckets = log_buckets_of(b, units);
+  const uint32_t* slot = h.slot + h.pos_base;
+  for (uint32_t tile = blockIdx.x; tile * kBucketTile < units; tile += gridDim.x) {
+    uint32_t id[kBucketItems];
 #pragma unroll
-    for (int j = 0; j < kBucketTileItems; ++j) {
-      const int64_t at = t.first + j * kBlock + threadIdx.x;
-      if (t.front) {
-        inside[j] = at < h.s_max;
-        id[j] = inside[j] ? uint32_t(static_cast<const IdT*>(h.frontier)[at]) : 0u;
-        order[j] = uint32_t(at);
-      } else {
-        inside[j] = at < h.len_max;
-        const uint32_t word = inside[j] ? h.slot[h.pos_base + at] : kInvalidSlot;  // id | kFirstBit as the fill left it
-        inside[j] = inside[j] && word != kInvalidSlot;
-        id[j] = word & ~kFirstBit;
-        order[j] = uint32_t(h.pos_base + at);
+    for (int j = 0; j < kBucketItems; ++j) {
+      const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x;
+      id[j] = u >= front && u < units ? nth(slot, u - front) : kNoId;  // (id | kFirstBit, or kInvalidSlot)
+    }
+    if (tile * kBucketTile < front) {
+#pragma unroll
+      for (int j = 0; j < kBucketItems; ++j) {
+        const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x;
+        if (u < uint32_t(s)) id[j] = uint32_t(nth(static_cast<const IdT*>(h.frontier), u));
       }
     }
-  }
-  __device__ __forceinline__ bool valid(const Hop& h, const TileOfUnits& t, int64_t s, int j) const {
-    const int64_t at = t.first + j * kBlock + threadIdx.x;
-    return inside[j] && at < (t.front ? s : s * h.k);
-  }
-};
-
-// One block per tile: the tile's units in bucket order (counted, placed and staged in LDS, then
-// written as one contiguous run), and where every bucket's piece begins.
-template <typename IdT>
-__global__ __launch_bounds__(kBlock) void bucket_sort_kernel(Hop h, Buckets b) {
-  __shared__ int cnt[kMaxBuckets];     // units per bucket, then the next free place of every bucket in the stage
-  __shared__ uint2 stage[kBucketTile];
-  __shared__ int lds[kBlock / kWave];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *h.bucket_overflow = 0;  // (the per-bucket launch comes behind this one)
-  for (int64_t tile = blockIdx.x; tile < b.tiles_max; tile += gridDim.x) {
-    const TileOfUnits t = bucket_tile(b, tile);
-    UnitsOfThread<IdT> units;
-    units.load(h, t);
-    const int64_t s = seeds_of(h);
-    if (!bucketed_now(h, s)) return;           // the hop outgrew the pass: it runs on the table
-    if (!bucket_tile_live(h, t, s)) continue;  // whole blocks skip a tile together
-    const int log_buckets = log_buckets_of(b, h, s);
-    const int buckets = 1 << log_buckets;
-    const int mine = buckets / kBlock;  // 1..8 consecutive buckets per thread
-    for (int j = threadIdx.x; j < buckets; j += kBlock) cnt[j] = 0;
-    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kBucketTileItems; ++j)
-      if (units.valid(h, t, s, j)) atomicAdd(&cnt[bucket_of(b, log_buckets, units.id[j])], 1);
-    __syncthreads();
-    int own[kMaxBuckets / kBlock];
-    int sum = 0;
-#pragma unroll
-    for (int j = 0; j < kMaxBuckets / kBlock; ++j) {
-      own[j] = j < mine ? cnt[threadIdx.x * mine + j] : 0;
-      sum += own[j];
-    }
-    int all;
-    int at = block_exclusive_scan<kBlock, int>(sum, &all, lds);
-    uint16_t* piece = b.piece + tile * (buckets + 1);
-#pragma unroll
-    for (int j = 0; j < kMaxBuckets / kBlock; ++j) {
-      if (j < mine) {
-        cnt[threadIdx.x * mine + j] = at;  // (the scan's barriers lie between the reads above and this)
-        piece[threadIdx.x * mine + j] = uint16_t(at);
-        at += own[j];
-      }
-    }
-    if (threadIdx.x == 0) piece[buckets] = uint16_t(all);  // <= 4096
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kBucketTileItems; ++j) {
-      if (units.valid(h, t, s, j)) {
-        const int to = atomicAdd(&cnt[bucket_of(b, log_buckets, units.id[j])], 1);
-        if (to >= 0 && to < kBucketTile) stage[to] = make_uint2(units.id[j], units.order[j]);
-      }
-    }
-    __syncthreads();
-    const int staged = all < kBucketTile ? all : kBucketTile;
-    for (int e = threadIdx.x; e < staged; e += kBlock) b.items[tile * kBucketTile + e] = stage[e];
-    __syncthreads();
+    for (int j = 0; j < kBucketItems; ++j)
+      if (id[j] != kNoId) id[j] &= ~kFirstBit;
+    sort_tile<HASHED>(b, log_buckets, tile, id, lds);
+    __syncthreads();  // lds is rewritten by the block's next tile
   }
 }
+static_assert(kInvalidSlot == kNoId, "a position without a pick is an entry without an id");
 
-// One block per bucket.  It lists the bucket's pieces in the live tiles (LDS: where each begins in
-// items[] and how many units came before it), so that its threads can share the bucket's units
-// evenly whatever their spread over the tiles; then the smallest order value of every id (LDS,
-// indexed by id / buckets), then the slot word of every pick that is not its id's first occurrence.
-__global__ __launch_bounds__(kBlock) void bucket_first_kernel(Hop h, Buckets b) {
-  __shared__ uint32_t best[kBucketRange];
-  __shared__ int piece_at[kMaxBucketTiles];      // first unit of the tile's piece, as an index into items[]
-  __shared__ int piece_before[kMaxBucketTiles];  // units of the bucket in the tiles before
-  __shared__ int lds[kBlock / kWave];
-  const int buckets = 1 << b.log_buckets;
-  const uint32_t range = (b.n_nodes + uint32_t(buckets) - 1) >> b.log_buckets;  // <= kBucketRange by the plan
-  const uint32_t pos_begin = uint32_t(h.pos_base), pos_end = uint32_t(h.pos_base + h.len_max);
-  const int64_t s = seeds_of(h);
+__global__ __launch_bounds__(kBucketBlock, 8) void bucket_first_kernel(Hop h, Buckets b) {
+  __shared__ __align__(16) uint32_t best[kBucketRange];
+  __shared__ uint32_t counts[kMaxBucketTiles];
+  const int64_t s = wave_uniform(seeds_of(h));
   if (!bucketed_now(h, s)) return;
-  const int tiles = b.tiles_max < kMaxBucketTiles ? b.tiles_max : kMaxBucketTiles;
-  const int64_t item_count = int64_t(b.tiles_max) * kBucketTile;
-  for (int bucket = blockIdx.x; bucket < buckets; bucket += gridDim.x) {
-    for (uint32_t j = threadIdx.x; j < range && j < uint32_t(kBucketRange); j += kBlock) best[j] = 0xffffffffu;
-    // the bucket's pieces: every thread asks for those of its tiles (tile = round * kBlock + thread)
-    // at once, then the rounds are scanned one after the other, a running total carried along
-    constexpr int kRounds = kMaxBucketTiles / kBlock;
-    int from[kRounds], upto[kRounds];
-#pragma unroll
-    for (int q = 0; q < kRounds; ++q) {
-      const int tile = q * kBlock + threadIdx.x;
-      from[q] = upto[q] = 0;
-      if (tile < tiles && bucket_tile_live(h, bucket_tile(b, tile), s)) {
-        const uint16_t* piece = b.piece + int64_t(tile) * (buckets + 1);
-        from[q] = piece[bucket];
-        upto[q] = piece[bucket + 1];
-      }
-    }
-    int total = 0;
-#pragma unroll
-    for (int q = 0; q < kRounds; ++q) {
-      if (q * kBlock >= tiles) break;  // the same for every thread
-      const int tile = q * kBlock + threadIdx.x;
-      const int count = from[q] <= upto[q] && upto[q] <= kBucketTile ? upto[q] - from[q] : 0;
-      int sum;
-      const int before = block_exclusive_scan<kBlock, int>(count, &sum, lds);
-      if (tile < tiles) {
-        piece_at[tile] = tile * kBucketTile + from[q];
-        piece_before[tile] = total + before;
-      }
-      total += sum;
-    }
-    __syncthreads();
-    // unit j of the bucket lives in the last tile whose piece_before is <= j
-    const auto unit = [&](int j) {
-      int lo = 0, hi = tiles - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (piece_before[mid] <= j) lo = mid; else hi = mid - 1;
-      }
-      const int64_t at = int64_t(piece_at[lo]) + (j - piece_before[lo]);
-      return at >= 0 && at < item_count ? b.items[at] : make_uint2(0u, 0u);
-    };
-    // a thread's first kKept units stay in registers for the second pass
-    constexpr int kKept = 8;
-    uint2 kept[kKept];
-#pragma unroll
-    for (int r = 0; r < kKept; ++r) {
-      const int j = threadIdx.x + r * kBlock;
-      kept[r] = j < total ? unit(j) : make_uint2(0u, 0u);
-    }
-    for (int j = threadIdx.x, r = 0; j < total; j += kBlock, ++r) {
-      uint2 it = make_uint2(0u, 0u);
-      if (r < kKept) {
-#pragma unroll
-        for (int q = 0; q < kKept; ++q) if (q == r) it = kept[q];
-      } else {
-        it = unit(j);
-      }
-      const uint32_t at = it.x >> b.log_buckets;
-      if (at < range && at < uint32_t(kBucketRange)) atomicMin(&best[at], it.y);
-    }
-    __syncthreads();
-    for (int j = threadIdx.x, r = 0; j < total; j += kBlock, ++r) {
-      uint2 it = make_uint2(0u, 0u);
-      if (r < kKept) {
-#pragma unroll
-        for (int q = 0; q < kKept; ++q) if (q == r) it = kept[q];
-      } else {
-        it = unit(j);
-      }
-      const uint32_t at = it.x >> b.log_buckets;
-      if (it.y < pos_begin || it.y >= pos_end || at >= range || at >= uint32_t(kBucketRange)) continue;  // a frontier id
-      const uint32_t least = best[at];  // first occurrences keep the word the fill gave them
-      if (least != it.y) h.slot[it.y] = least < pos_begin ? (least | kRankBit) : least;
-    }
-    __syncthreads();
-  }
+  const uint32_t front = uint32_t(front_units(s)), tiles = (front + uint32_t(s * h.k) + kBucketTile - 1) / kBucketTile;
+  clear_counts(counts, tiles);
+  for (int i = blockIdx.x; i < 1 << b.log_buckets; i += gridDim.x)
+    first_of_bucket_direct(b, bucket_in_turn(i, b.log_buckets), tiles, front, best, counts);
+  add_counts(b, counts, tiles);
 }
 
-// The per-bucket kernel for graphs of any node count: as bucket_first_kernel, but a bucket's ids
-// are told apart in an open-addressing table in LDS (the id claims a slot with a compare-and-swap,
-// the slot's second word takes the smallest order value), since an array indexed by the id itself
-// would not fit.  Buckets are chosen by low bits of a hash of the id, slots by the next bits.
-// A bucket with more units than three quarters of the table's slots (its ids might not fit) is
-// gone over in parts, by yet other bits of the hash, one table's worth at a time.  Ids that crowd
-// one part all the same (more than kHashSlots distinct ones: not by chance) set the hop's overflow
-// word, which fails the call.
-__global__ __launch_bounds__(kHashBlock) void bucket_first_hashed_kernel(Hop h, Buckets b) {
-  __shared__ uint32_t owner[kHashSlots];
-  __shared__ uint32_t best[kHashSlots];
-  __shared__ int piece_at[kMaxBucketTiles];      // first unit of the tile's piece, as an index into items[]
-  __shared__ int piece_before[kMaxBucketTiles];  // units of the bucket in the tiles before
-  __shared__ int lds[kHashBlock / kWave];
-  __shared__ int overflow;
-  const uint32_t pos_begin = uint32_t(h.pos_base), pos_end = uint32_t(h.pos_base + h.len_max);
-  const int64_t s = seeds_of(h);
+__global__ __launch_bounds__(kBucketBlock) void bucket_first_hashed_kernel(Hop h, Buckets b) {
+  __shared__ HashedLds lds;
+  const int64_t s = wave_uniform(seeds_of(h));
   if (!bucketed_now(h, s)) return;
-  const int log_buckets = log_buckets_of(b, h, s);
-  const int buckets = 1 << log_buckets;
-  const int tiles = b.tiles_max < kMaxBucketTiles ? b.tiles_max : kMaxBucketTiles;
-  const int64_t item_count = int64_t(b.tiles_max) * kBucketTile;
-  for (int bucket = blockIdx.x; bucket < buckets; bucket += gridDim.x) {
-    if (threadIdx.x == 0) overflow = 0;
-    constexpr int kRounds = kMaxBucketTiles / kHashBlock;
-    int from[kRounds], upto[kRounds];
-#pragma unroll
-    for (int q = 0; q < kRounds; ++q) {
-      const int tile = q * kHashBlock + threadIdx.x;
-      from[q] = upto[q] = 0;
-      if (tile < tiles && bucket_tile_live(h, bucket_tile(b, tile), s)) {
-        const uint16_t* piece = b.piece + int64_t(tile) * (buckets + 1);
-        from[q] = piece[bucket];
-        upto[q] = piece[bucket + 1];
-      }
-    }
-    int total = 0;
-#pragma unroll
-    for (int q = 0; q < kRounds; ++q) {
-      if (q * kHashBlock >= tiles) break;  // the same for every thread
-      const int tile = q * kHashBlock + threadIdx.x;
-      const int count = from[q] <= upto[q] && upto[q] <= kBucketTile ? upto[q] - from[q] : 0;
-      int sum;
-      const int before = block_exclusive_scan<kHashBlock, int>(count, &sum, lds);
-      if (tile < tiles) {
-        piece_at[tile] = tile * kBucketTile + from[q];
-        piece_before[tile] = total + before;
-      }
-      total += sum;
-    }
-    // The table is as large as the bucket needs: at least twice its units (all of them may be
-    // distinct ids), all of the array when that is not enough; beyond three quarters of the array
-    // the bucket is split into parts.
-    const int capacity = b.hash_slots;
-    const int parts = total <= capacity * 3 / 4 ? 1 : (total + capacity / 2 - 1) / (capacity / 2);
-    int slots = capacity < 1024 ? capacity : 1024;
-    while (slots < 2 * (total / parts + 1) && slots < capacity) slots <<= 1;
-    const uint32_t slot_mask = uint32_t(slots - 1);
-    __syncthreads();  // piece_at / piece_before are complete
-    const auto unit = [&](int j) {
-      int lo = 0, hi = tiles - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (piece_before[mid] <= j) lo = mid; else hi = mid - 1;
-      }
-      const int64_t at = int64_t(piece_at[lo]) + (j - piece_before[lo]);
-      return at >= 0 && at < item_count ? b.items[at] : make_uint2(kHashEmpty, 0u);
-    };
-    // where an id's slot search starts, and which part it belongs to: bits of its hash that the
-    // choice of the bucket did not use
-    const auto home = [&](uint32_t hash) { return (hash >> log_buckets) & slot_mask; };
-    const auto part_of = [&](uint32_t hash) { return int((hash >> 23) % uint32_t(parts)); };
-    constexpr int kKept = 8;  // a thread's first units stay in registers across the passes
-    uint2 kept[kKept];
-#pragma unroll
-    for (int r = 0; r < kKept; ++r) {
-      const int j = threadIdx.x + r * kHashBlock;
-      kept[r] = j < total ? unit(j) : make_uint2(kHashEmpty, 0u);
-    }
-    for (int part = 0; part < parts; ++part) {
-      for (int j = threadIdx.x; j < slots; j += kHashBlock) {
-        owner[j] = kHashEmpty;
-        best[j] = 0xffffffffu;
-      }
-      __syncthreads();
-      // every unit of the part claims its id's slot (or finds it claimed by the same id) and offers its order value
-      uint32_t kept_slot[kKept];
-#pragma unroll
-      for (int r = 0; r < kKept; ++r) kept_slot[r] = kHashEmpty;
-      for (int j = threadIdx.x, r = 0; j < total; j += kHashBlock, ++r) {
-        uint2 it = make_uint2(kHashEmpty, 0u);
-        if (r < kKept) {
-#pragma unroll
-          for (int q = 0; q < kKept; ++q) if (q == r) it = kept[q];
-        } else {
-          it = unit(j);
-        }
-        if (it.x == kHashEmpty) continue;
-        const uint32_t hash = hash_id(it.x);
-        if (parts > 1 && part_of(hash) != part) continue;
-        uint32_t slot = home(hash);
-        bool placed = false;
-        for (int probes = 0; probes < slots; ++probes) {
-          uint32_t seen = owner[slot];
-          if (seen == kHashEmpty) seen = atomicCAS(&owner[slot], kHashEmpty, it.x);
-          if (seen == kHashEmpty || seen == it.x) {
-            placed = true;
-            break;
-          }
-          slot = (slot + 1) & slot_mask;
-        }
-        if (placed) atomicMin(&best[slot], it.y); else overflow = 1;
-        if (r < kKept) {
-#pragma unroll
-          for (int q = 0; q < kKept; ++q) if (q == r) kept_slot[q] = placed ? slot : kHashEmpty;
-        }
-      }
-      __syncthreads();
-      if (overflow == 0) {  // (an overflowing part's answers are void: the call fails, nothing is rewritten)
-        for (int j = threadIdx.x, r = 0; j < total; j += kHashBlock, ++r) {
-          uint2 it = make_uint2(kHashEmpty, 0u);
-          uint32_t slot = kHashEmpty;
-          if (r < kKept) {
-#pragma unroll
-            for (int q = 0; q < kKept; ++q) if (q == r) { it = kept[q]; slot = kept_slot[q]; }
-          } else {
-            it = unit(j);
-          }
-          if (it.x == kHashEmpty || it.y < pos_begin || it.y >= pos_end) continue;  // not a pick of this hop
-          const uint32_t hash = hash_id(it.x);
-          if (parts > 1 && part_of(hash) != part) continue;
-          if (slot == kHashEmpty) {  // beyond what the registers kept: find the id's slot again
-            slot = home(hash);
-            for (int probes = 0; probes < slots && owner[slot] != it.x; ++probes) slot = (slot + 1) & slot_mask;
-          }
-          const uint32_t least = best[slot];  // first occurrences keep the word the fill gave them
-          if (least != it.y) h.slot[it.y] = least < pos_begin ? (least | kRankBit) : least;
-        }
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0 && overflow != 0) *h.bucket_overflow = 1;
-    __syncthreads();
-  }
+  const uint32_t front = uint32_t(front_units(s)), units = front + uint32_t(s * h.k), tiles = (units + kBucketTile - 1) / kBucketTile;
+  const int log_buckets = log_buckets_of(b, units);
+  clear_counts(lds.counts, tiles);
+  for (int i = blockIdx.x; i < 1 << log_buckets; i += gridDim.x)
+    first_of_bucket_hashed(b, log_buckets, bucket_in_turn(i, log_buckets), tiles, front, lds);
+  add_counts(b, lds.counts, tiles);
 }
 
 // Whether the position `rel` of the hop, of slot word `word`, is the first one of its id (`rel` is below
@@ -1371,6 +1050,100 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
   }
 }
 
+// The same for a tile of the bucketed pass: what a position's id is in the order of its first occurrences is known,
+// in the order of the buckets.
+template <typename IdT, bool HASHED>
+__device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets& b, int64_t s, uint32_t tile) {
+  constexpr int ITEMS = 4, GROUPS = kBucketItems / ITEMS, kWaves = kBucketBlock / kWave;
+  constexpr uint32_t kGroup = kBucketBlock * ITEMS;
+  using words = typename Items<ITEMS>::words;
+  __shared__ __align__(16) uint32_t least_of[kBucketTile];
+  __shared__ uint32_t wave_before[kWaves];  // first occurrences in tiles before this one
+  __shared__ int wave_count[GROUPS * kWaves];
+  const uint32_t front = uint32_t(front_units(s)), units = front + uint32_t(s * h.k);
+  const int log_buckets = log_buckets_of(b, units);
+  const uint32_t at = threadIdx.x * ITEMS, first_unit = tile * kBucketTile;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  uint32_t* slot = h.slot + h.pos_base;
+  words word[GROUPS];  // (positions and units are multiples of 4 together)
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const uint32_t u = first_unit + g * kGroup + at;
+    word[g] = words(kInvalidSlot);
+    if (u >= front && u < units) word[g] = nth(reinterpret_cast<const words*>(slot), (u - front) / ITEMS);
+  }
+  uint32_t before = firsts_before(b, tile);
+  unsort_tile<HASHED>(b, log_buckets, tile, least_of);
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d, kWave);
+  if (lane == 0) wave_before[wave] = before;
+  __syncthreads();
+  uint32_t first[GROUPS];
+  int lane_before[GROUPS];
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    first[g] = 0;
+    const uint32_t u = first_unit + g * kGroup + at;
+    const words least = *reinterpret_cast<const words*>(least_of + g * kGroup + at);
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (u + j >= units) word[g][j] = kInvalidSlot;
+      if (word[g][j] != kInvalidSlot && least[j] == u + j) first[g] |= 1u << j;
+    }
+    const int c = __builtin_popcount(first[g]);  // its bits are summed over the lanes by ballots
+    lane_before[g] = 0;
+    int sum = 0;
+#pragma unroll
+    for (int bit = 0; (1 << bit) <= ITEMS; ++bit) {
+      const uint64_t mask = __ballot((c >> bit) & 1);
+      lane_before[g] += __builtin_popcountll(mask & ((uint64_t(1) << lane) - 1)) << bit;
+      sum += __builtin_popcountll(mask) << bit;
+    }
+    if (lane == 0) wave_count[g * kWaves + wave] = sum;
+  }
+  __syncthreads();
+  // the groups' and waves' counts, in the order of the positions: one a lane, summed over the lanes
+  static_assert(GROUPS * kWaves <= kWave, "a count per lane");
+  const int own = lane < GROUPS * kWaves ? wave_count[lane] : 0;
+  int upto = own;
+#pragma unroll
+  for (int d = 1; d < GROUPS * kWaves; d <<= 1) {
+    const int lower = __shfl_up(upto, d, kWave);
+    if (lane >= d) upto += lower;
+  }
+  uint32_t rank0 = wave_before[lane & (kWaves - 1)];
+#pragma unroll
+  for (int d = kWaves / 2; d > 0; d >>= 1) rank0 += __shfl_xor(rank0, d, kWave);
+  rank0 += uint32_t(first_rank(h, s));
+  if (first_unit + kBucketTile >= units && threadIdx.x == GROUPS * kWaves - 1) {  // the last tile: the frontier's size is known
+    *h.n_unique = int64_t(rank0) + upto;
+    if (h.host_sizes) mirror_to_host(h.host_sizes + h.index + 1, int64_t(rank0) + upto);
+  }
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const uint32_t u = first_unit + g * kGroup + at;
+    uint32_t rank = rank0 + uint32_t(lane_before[g] + __shfl(upto - own, g * kWaves + wave, kWave));
+    if (u < front || u >= units) continue;
+    const words least = *reinterpret_cast<const words*>(least_of + g * kGroup + at);
+    words ranks;
+    bool changed = false;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      ranks[j] = rank;
+      if ((first[g] >> j) & 1) {
+        nth(static_cast<IdT*>(h.frontier), rank) = IdT(word[g][j] & ~kFirstBit);
+        ++rank;
+      } else if (word[g][j] != kInvalidSlot) {
+        changed = true;
+        const uint32_t met = least[j] < u + j ? least[j] : u + j;  // (one that is not before its own is none that the pass left)
+        word[g][j] = met < front ? met | kRankBit : uint32_t(h.pos_base) + (met - front);
+      }
+    }
+    nth(reinterpret_cast<words*>(h.rank_at + h.pos_base), (u - front) / ITEMS) = ranks;  // (only the ones at first positions are ever read)
+    if (changed) nth(reinterpret_cast<words*>(slot), (u - front) / ITEMS) = word[g];
+  }
+}
+
 // The long ones among the frontier's rows of ranks [begin, end), which this block has just appended, go
 // onto the next hop's queue.
 template <typename IdT, int NT>
@@ -1397,6 +1170,7 @@ template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STR
 __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
   int64_t begin = 0, end = 0;
+  if (h.bucketed != 0 && bucketed_now(h, seeds_of(h))) return;
   if (!STRIDE) {
     const int64_t vb = blockIdx.x;
     if (vb < row_tiles) offsets_tile<NT, true>(h, vb);
@@ -1413,6 +1187,23 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
     if (vb < rows) offsets_tile<NT, false>(h, vb);
     else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table, &begin, &end);
     if (ANNOUNCE) announce_long_rows<IdT, NT>(h, begin, end);
+    __syncthreads();  // the tiles' LDS is rewritten by the block's next one
+  }
+}
+
+// The same of a bucketed hop (nothing, where the hop has outgrown the pass): virtual blocks of kBucketBlock threads.
+template <typename IdT, bool HASHED, bool STRIDE>
+__global__ __launch_bounds__(kBucketBlock) void hop_compact_sorted_kernel(Hop h, Buckets b) {
+  constexpr int64_t kRows = kBucketBlock * kRowItems;
+  const int64_t s = wave_uniform(seeds_of(h));
+  if (!bucketed_now(h, s)) return;
+  const uint32_t rows = uint32_t(s > 0 ? (s + kRows - 1) / kRows : 1);  // (tile 0 of either kind writes the lengths)
+  const uint32_t units = uint32_t(front_units(s) + s * h.k);
+  const uint32_t total = rows + (units > 0 ? (units + kBucketTile - 1) / kBucketTile : 1);
+  for (uint32_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
+    if (vb < rows) offsets_tile<kBucketBlock, false>(h, vb);
+    else compact_sorted_tile<IdT, HASHED>(h, b, s, vb - rows);
+    if (!STRIDE) return;
     __syncthreads();  // the tiles' LDS is rewritten by the block's next one
   }
 }
@@ -1444,24 +1235,22 @@ struct Plan {
   size_t table_bytes = 0;    // 0 for the direct table
   bool weighted = false;     // picks by edge weight: per-hop queues for long rows
   bool bucketed = false;     // the last hop may find its first occurrences by the bucketed pass (if it turns out to fit)
-  bool bucket_hashed = false; // ... with ids told apart by an LDS hash table (graphs beyond kBucketedMaxNodes)
+  bool bucket_hashed = false; // ... with ids told apart by an LDS hash table (on request)
   bool bucket_space = false; // the workspace has room for that pass
-  int32_t bucket_front_tiles = 0;  // tiles over the frontier array as large as it can be before the last hop
-  int32_t bucket_pos_tiles = 0;    // tiles over the last hop's padded positions: all of them, or as many as there is room for
+  int64_t bucket_tiles = 0;   // its tiles: all of the hop's units in the worst case, or as many as there is room for
+  int64_t bucket_pos_cap = 0; // padded positions of the hop that these hold
   int32_t log_buckets = 0;
   int32_t hash_slots = kHashSlots;
   uint32_t n_nodes = 0;
 };
 
 // Tiles of the bucketed pass: the frontier before the last hop at its worst case, and as many of the
-// hop's padded positions as the per-bucket kernels can index (a hop beyond that runs on the table).
+// hop's padded positions as there is room for (a hop beyond that runs on the table).
 inline void plan_bucket_tiles(Plan* p) {
-  const int64_t front = (p->s_max[p->n_hops - 1] + kBucketTile - 1) / kBucketTile;
-  const int64_t pos = (p->nnz_max[p->n_hops - 1] + kBucketTile - 1) / kBucketTile;
-  const int64_t room = int64_t(kMaxBucketTiles) - 2 - front;
-  p->bucket_space = p->n_hops >= 2 && room >= 1;
-  p->bucket_front_tiles = int32_t(front);
-  p->bucket_pos_tiles = int32_t(pos < room ? pos : (room > 0 ? room : 0));
+  const int64_t front = front_units(p->s_max[p->n_hops - 1]), pos = p->nnz_max[p->n_hops - 1], tile = kBucketTile;
+  p->bucket_tiles = std::min<int64_t>(kMaxBucketTiles, (front + pos + tile - 1) / tile);
+  p->bucket_pos_cap = p->bucket_tiles * tile - front;
+  p->bucket_space = p->n_hops >= 2 && p->bucket_pos_cap > 0;
 }
 
 dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, int32_t id_bytes,
@@ -1487,32 +1276,23 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
     DGS_REQUIRE(n_nodes >= 0 && n_nodes < 0x7fffffffLL, DGS_ERR_UNSUPPORTED,
                 "sample_blocks: a node table needs fewer than 2^31 nodes (have %lld)", (long long)n_nodes);
     p->kind = TableKind::kDirect;
-    // the bucketed pass: slot words are ids (the direct table's), and the hop is large enough for
-    // its two extra launches to cost less than the atomics they replace.  Ids that fit the LDS
-    // array of a bucket (kBucketRange ids in each of at most kMaxBuckets buckets) index it directly;
-    // larger graphs take the hashed form.
-    // (test hook: 1 never, 2 whatever the size, 3 whatever the size and hashed whatever the graph,
-    // 4 like 3 with on-chip tables of 256 slots, so that small inputs fill them and go over their
-    // buckets in parts)
+    // The bucketed pass: slot words are ids (the direct table's).  By size only the direct form runs.  The hashed form
+    // gives the same results on any graph and takes the atomics out of the hop just the same, but does not pay: 111 M nodes,
+    // 944 k picks of mostly new ids: fill 57 -> 30 us, against 12 + 27 us for its two launches; R-MAT with two thirds
+    // repeats 149 -> 75 against 15 + 50.  It runs when the test hook asks for it (1 never, 2 whatever the size,
+    // 3 whatever the size and hashed whatever the graph, 4 like 3 with on-chip tables of 256 slots, so that small
+    // inputs fill them and go over their buckets in parts).
     const int64_t mode = debug_option(DGS_DEBUG_SAMPLER_BUCKETED);
-    const bool large = p->nnz_max[n_hops - 1] >= kBucketedMinPicks;
+    const bool large = p->nnz_max[n_hops - 1] >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
     p->bucket_hashed = n_nodes > kBucketedMaxNodes || mode == 3 || mode == 4;
-    // By size only the direct form runs.  The hashed form gives the same results on any graph and
-    // takes the atomics out of the hop just the same, but it does not pay: 111 M nodes, 944 k picks
-    // of mostly new ids: fill 64 -> 35 us and relabel 14 -> 12, against 19 + 22 us for its two
-    // launches (0.187-0.200 ms per step in flight against 0.191); R-MAT with two thirds repeats: every
-    // repeat costs a scattered 4-byte store where the table's look before the atomic gets cheaper
-    // (0.382 against 0.373 ms).  It runs when the test hook asks for it.
     p->bucketed = p->bucket_space && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
                   (p->bucket_hashed ? mode >= 2 : (large || mode >= 2));
     p->hash_slots = mode == 4 ? 256 : kHashSlots;
-    int log_b = 0;
-    if (p->bucket_hashed) {
-      // a bucket's LDS table takes kHashSlots ids: at most half as many units per bucket on average
-      const int64_t units = int64_t(p->bucket_front_tiles + p->bucket_pos_tiles) * kBucketTile;
-      while ((1 << log_b) < kMinBuckets || ((int64_t(kHashSlots) << log_b) < units && (1 << log_b) < kMaxBuckets)) ++log_b;
+    int log_b = kMinLogBuckets;
+    if (p->bucket_hashed) {  // (as many as its units may need: log_buckets_of)
+      while (log_b < kMaxLogBuckets && (int64_t(kHashSlots / 2) << log_b) < p->bucket_tiles * kBucketTile) ++log_b;
     } else {
-      while ((1 << log_b) < kMinBuckets || (int64_t(kBucketRange) << log_b) < n_nodes) ++log_b;
+      while ((int64_t(kBucketRange) << log_b) < n_nodes) ++log_b;
     }
     p->log_buckets = log_b;
     p->n_nodes = uint32_t(n_nodes);
@@ -1560,6 +1340,7 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     Hop v{};
     v.row_cnt = c.take<uint32_t>(s);
     v.row_off = c.take<uint32_t>(s);
+    v.bucketed = p.bucketed && h == p.n_hops - 1;
     v.row_state = states;
     states += row_tiles_of(int64_t(s), int64_t(len));
     v.pos_state = states;
@@ -1578,25 +1359,25 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     v.len_max = int64_t(len);
     v.k = int32_t(fanouts[h]);
     v.index = h;
-    v.bucketed = p.bucketed && h == p.n_hops - 1;
-    v.bucket_pos_cap = int64_t(p.bucket_pos_tiles) * kBucketTile;
+    v.bucket_pos_cap = p.bucket_pos_cap;
     if (hops) hops[h] = v;
     pos_base += (int64_t(len) + 15) / 16 * 16;
   }
   if (p.bucket_space) {
     Buckets b{};
-    b.front_tiles = p.bucket_front_tiles;
-    b.tiles_max = p.bucket_front_tiles + p.bucket_pos_tiles;
-    b.items = c.take<uint2>(size_t(b.tiles_max) * kBucketTile);
+    b.tiles_max = int32_t(p.bucket_tiles);
+    b.items = c.take<uint2>(size_t(b.tiles_max) * kBucketTile);  // (the larger form's)
+    b.least = c.take<uint32_t>(size_t(b.tiles_max) * kBucketTile);
     b.piece = c.take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
-    int* overflow = c.take<int>(4);
+    b.firsts = c.take<uint32_t>(kCounters * kMaxBucketTiles);
+    b.overflow = c.take<int>(4);
     b.log_buckets = p.log_buckets;
-    b.n_nodes = p.n_nodes;
+    b.n_ids = p.n_nodes;
     b.hashed = p.bucket_hashed ? 1 : 0;
     b.hash_slots = p.hash_slots;
     if (buckets) *buckets = b;
     if (hops)
-      for (int h = 0; h < p.n_hops; ++h) hops[h].bucket_overflow = overflow;
+      for (int h = 0; h < p.n_hops; ++h) hops[h].bucket_overflow = b.overflow;
   }
   return c.used + 256;
 }
@@ -1629,6 +1410,21 @@ template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
 void launch_compact(const Hop& hop, bool announce, const TableT& table, hipStream_t st) {
   if (announce) launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, true>(hop, table, st);
   else launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, false>(hop, table, st);
+}
+
+// The bucketed pass and the compact launch behind it.
+template <typename IdT, bool HASHED>
+void launch_bucketed(const Hop& hop, const Buckets& b, hipStream_t st) {
+  const uint32_t at_most = uint32_t(std::min(grid_cap(), kLookbackGrid));
+  hipLaunchKernelGGL((bucket_sort_kernel<IdT, HASHED>), dim3(std::min(at_most, uint32_t(b.tiles_max))), dim3(kBucketBlock), 0, st, hop, b);
+  const uint32_t buckets = std::min(at_most, 1u << b.log_buckets);
+  if constexpr (HASHED) hipLaunchKernelGGL(bucket_first_hashed_kernel, dim3(buckets), dim3(kBucketBlock), 0, st, hop, b);
+  else hipLaunchKernelGGL(bucket_first_kernel, dim3(buckets), dim3(kBucketBlock), 0, st, hop, b);
+  const int64_t blocks = (hop.s_max + kBucketBlock * kRowItems - 1) / (kBucketBlock * kRowItems) + b.tiles_max;
+  if (is_capped(blocks))
+    hipLaunchKernelGGL((hop_compact_sorted_kernel<IdT, HASHED, true>), dim3(capped_grid(blocks)), dim3(kBucketBlock), 0, st, hop, b);
+  else
+    hipLaunchKernelGGL((hop_compact_sorted_kernel<IdT, HASHED, false>), dim3(uint32_t(blocks)), dim3(kBucketBlock), 0, st, hop, b);
 }
 
 template <typename IdT, typename PtrT, typename TableT, int G>
@@ -1727,19 +1523,14 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
     else launch_fill<IdT, PtrT, TableT, 64>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
     DGS_LAUNCH_CHECK();
 
-    if (cur.bucketed) {  // the picks' slot words hold ids so far: group them and find the first occurrences
-      const int n_buckets = 1 << buckets.log_buckets;
-      hipLaunchKernelGGL(bucket_sort_kernel<IdT>, dim3(capped_grid(buckets.tiles_max)), dim3(kBlock), 0, st, cur,
-                         buckets);
-      DGS_LAUNCH_CHECK();
-      if (buckets.hashed)
-        hipLaunchKernelGGL(bucket_first_hashed_kernel, dim3(capped_grid(n_buckets)), dim3(kHashBlock), 0, st, cur,
-                           buckets);
-      else
-        hipLaunchKernelGGL(bucket_first_kernel, dim3(capped_grid(n_buckets)), dim3(kBlock), 0, st, cur, buckets);
-      DGS_LAUNCH_CHECK();
+    if constexpr (std::is_same_v<TableT, DirectTable<IdT>>) {
+      if (cur.bucketed) {  // (the last hop)
+        if (buckets.hashed) launch_bucketed<IdT, true>(cur, buckets, st);
+        else launch_bucketed<IdT, false>(cur, buckets, st);
+        DGS_LAUNCH_CHECK();
+        if (cur.len_max <= cur.bucket_pos_cap) break;  // (it cannot outgrow the pass)
+      }
     }
-
     // (a queue holds the whole frontier: from hop 0 on, where a later hop reads it; hops only get larger)
     const bool announce = p.weighted && h + 1 < p.n_hops && !weighted_shared(hops[p.n_hops - 1]);
     switch (pos_tile_kind(cur.len_max)) {

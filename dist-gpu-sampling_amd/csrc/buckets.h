@@ -22,9 +22,9 @@
 // Two forms.  Direct: bucket = low bits of the id, and the high bits index an array of kBucketRange entries;
 // items are one word (the high bits and the unit's place in its tile).  Hashed, for any number of ids:
 // bucket = low bits of a hash that takes no two ids to one value, hashes are told apart in an open-addressing table of
-// packed words (hash, unit), items are the hash and the unit.  A bucket whose units might not fit that table is gone over in parts, by other bits
-// of the hash, one table's worth at a time; ids that crowd one part all the same (not by chance) are
-// reported.
+// packed words (hash, unit), items are the hash and the unit.  A bucket whose ids do not fit that table is gone over
+// again in parts, by other bits of the hash, one table's worth at a time; ids that crowd one part all the same (not by
+// chance) are reported.
 #ifndef DGS_CSRC_BUCKETS_H_
 #define DGS_CSRC_BUCKETS_H_
 
@@ -45,6 +45,7 @@ constexpr int kMinLogBuckets = 8, kMaxLogBuckets = 11;
 constexpr int kMaxBuckets = 1 << kMaxLogBuckets;
 constexpr int kBucketRange = 16384;                  // direct: ids per bucket at most, 64 KB of LDS
 constexpr int64_t kDirectMaxIds = int64_t(kMaxBuckets) * kBucketRange;
+constexpr int kFewProbes = 64;                       // ... of which an id sees this many at first
 constexpr int kHashSlots = 16384;                    // hashed: entries of a bucket's table, 128 KB of LDS
 
 // A tile's first occurrences are counted by the blocks of all buckets, each of which adds its counts of all tiles with a
@@ -78,7 +79,7 @@ __device__ __forceinline__ T& nth(T* base, uint32_t i) {
 __device__ __forceinline__ int log_buckets_of(const Buckets& b, uint32_t units) {
   if (!b.hashed) return b.log_buckets;
   int lb = kMinLogBuckets;
-  while (lb < b.log_buckets && (uint32_t(b.hash_slots / 2) << lb) < units) ++lb;
+  while (lb < b.log_buckets && (uint32_t(b.hash_slots) << lb) < units) ++lb;
   return lb;
 }
 // Bucket number i of a launch.  Blocks go to the 8 XCDs in turn: buckets whose pieces lie side by side go to one of
@@ -162,12 +163,13 @@ __device__ __forceinline__ void sort_tile(const Buckets& b, int log_buckets, uin
 // A bucket's units, as the threads of its block come by them: 16 lanes have a piece, four pieces at a time, of
 // each of which the first 48 units are read at once.
 constexpr int kPieceLanes = 16, kPieceGroups = kBucketBlock / kPieceLanes;
-constexpr int kPieces = 4, kPieceChunks = 3;
-constexpr uint32_t kRoundTiles = kPieceGroups * kPieces;
+constexpr int kPieceChunks = 3;
 
 template <bool HASHED>
 struct PieceRound {
   using Item = BucketItem<HASHED>;
+  static constexpr int kPieces = HASHED ? 6 : 4;
+  static constexpr uint32_t kTiles = kPieceGroups * kPieces;  // of a round
   uint32_t at[kPieces];   // the lane's first item
   uint32_t end[kPieces];  // the piece's end
   typename Item::type item[kPieces][kPieceChunks];
@@ -223,7 +225,16 @@ struct PieceRound {
 #pragma unroll
       for (int c = 0; c < kPieceChunks; ++c)
         if (at[q] + c * kPieceLanes < end[q]) one(at[q] + c * kPieceLanes, item[q][c]);
-      for (uint32_t e = at[q] + kPieceChunks * kPieceLanes; e < end[q]; e += kPieceLanes) one(e, nth(items(b), e));
+      // (longer pieces: of ids that come up again and again, four more at a time)
+      for (uint32_t e = at[q] + kPieceChunks * kPieceLanes; e < end[q]; e += 4 * kPieceLanes) {
+        typename Item::type more[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (e + c * kPieceLanes < end[q]) more[c] = nth(items(b), e + c * kPieceLanes);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (e + c * kPieceLanes < end[q]) one(e + c * kPieceLanes, more[c]);
+      }
       if (n > 0 && (threadIdx.x & (kPieceLanes - 1)) == 0) count(tile, uint32_t(n));
     }
   }
@@ -252,7 +263,7 @@ __device__ __forceinline__ void first_of_bucket_direct(const Buckets& b, int buc
   for (uint32_t j = threadIdx.x * 4; j < range && j < uint32_t(kBucketRange); j += kBucketBlock * 4)
     *reinterpret_cast<uint4*>(best + j) = make_uint4(~0u, ~0u, ~0u, ~0u);
   __syncthreads();
-  for (uint32_t t0 = 0; t0 < tiles; t0 += kRoundTiles) {
+  for (uint32_t t0 = 0; t0 < tiles; t0 += PieceRound<false>::kTiles) {
     if (t0 > 0) round.load(b, b.log_buckets, bucket, t0, tiles);
     round.each(b, [&](uint32_t, uint32_t item, uint32_t unit) {
       const uint32_t at = item >> kLocalBits;
@@ -260,8 +271,8 @@ __device__ __forceinline__ void first_of_bucket_direct(const Buckets& b, int buc
     });
   }
   __syncthreads();
-  for (uint32_t t0 = 0; t0 < tiles; t0 += kRoundTiles) {
-    if (tiles > kRoundTiles) round.load(b, b.log_buckets, bucket, t0, tiles);  // (a single round is in registers still)
+  for (uint32_t t0 = 0; t0 < tiles; t0 += PieceRound<false>::kTiles) {
+    if (tiles > PieceRound<false>::kTiles) round.load(b, b.log_buckets, bucket, t0, tiles);  // (a single round is in registers still)
     round.each(b, [&](uint32_t e, uint32_t item, uint32_t unit) {
       const uint32_t at = item >> kLocalBits;
       if (unit < first_unit || at >= uint32_t(kBucketRange)) return false;
@@ -279,67 +290,77 @@ struct HashedLds {
   int units;
   int overflow;
 };
-__device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles,
-                                                       uint32_t first_unit, HashedLds& lds) {
+// All units of the bucket whose ids belong to part `part` of `parts`; returns whether the table took them (the same in
+// all threads), within max_probes probes each.
+__device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles, uint32_t first_unit,
+                                                     int part, int parts, int max_probes, HashedLds& lds) {
   using ItemT = BucketItem<true>::type;
   const int slots = b.hash_slots;
   const uint32_t mask = uint32_t(slots - 1);
+  // where a search starts, and which part an id belongs to: bits of its hash that did not choose the bucket
+  const auto elsewhere = [&](uint32_t hash) { return parts > 1 && int((hash >> 23) % uint32_t(parts)) != part; };
   PieceRound<true> round;
-  if (threadIdx.x == 0) lds.units = lds.overflow = 0;
+  round.load(b, log_buckets, bucket, 0, tiles);
+  for (int j = threadIdx.x; j < slots / 2; j += kBucketBlock) reinterpret_cast<uint4*>(lds.table)[j] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (threadIdx.x == 0) lds.overflow = 0;
+  __syncthreads();
+  for (uint32_t t0 = 0; t0 < tiles; t0 += PieceRound<true>::kTiles) {
+    if (t0 > 0) round.load(b, log_buckets, bucket, t0, tiles);
+    round.each(b, [&](uint32_t, ItemT item, uint32_t unit) {
+      if (elsewhere(item.x)) return;
+      const unsigned long long packed = (static_cast<unsigned long long>(item.x) << 32) | unit;
+      uint32_t slot = (item.x >> log_buckets) & mask;
+      bool placed = false;
+      for (int probes = 0; probes < max_probes && !placed; ++probes) {
+        unsigned long long cur = lds.table[slot];
+        if (cur == ~0ull) cur = atomicCAS(&lds.table[slot], ~0ull, packed);
+        placed = cur == ~0ull || uint32_t(cur >> 32) == item.x;
+        if (placed && cur > packed && cur != ~0ull) atomicMin(&lds.table[slot], packed);
+        slot = (slot + 1) & mask;
+      }
+      if (!placed) lds.overflow = 1;
+    });
+  }
+  __syncthreads();
+  const bool took = lds.overflow == 0;
+  if (took) {
+    for (uint32_t t0 = 0; t0 < tiles; t0 += PieceRound<true>::kTiles) {
+      if (tiles > PieceRound<true>::kTiles) round.load(b, log_buckets, bucket, t0, tiles);  // (a single round is in registers still)
+      round.each(b, [&](uint32_t e, ItemT item, uint32_t unit) {
+        if (unit < first_unit) return false;
+        if (elsewhere(item.x)) return false;
+        uint32_t slot = (item.x >> log_buckets) & mask;
+        unsigned long long held = lds.table[slot];
+        for (int probes = 0; probes < slots && uint32_t(held >> 32) != item.x; ++probes) {
+          slot = (slot + 1) & mask;
+          held = lds.table[slot];
+        }
+        nth(b.least, e) = uint32_t(held);
+        return uint32_t(held) == unit;
+      }, [&](uint32_t tile, uint32_t n) { lds.counts[tile] += n; });  // (nobody else has the tile's piece of this bucket)
+    }
+  }
+  __syncthreads();  // the table is rewritten
+  return took;
+}
+// A bucket of many units may be one of few ids: it is gone over in parts only where the table has not taken them all.
+__device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles,
+                                                       uint32_t first_unit, HashedLds& lds) {
+  if (first_of_part_hashed(b, log_buckets, bucket, tiles, first_unit, 0, 1, kFewProbes < b.hash_slots ? kFewProbes : b.hash_slots, lds)) return;
+  if (threadIdx.x == 0) lds.units = 0;
   __syncthreads();
   int n = 0;
-  for (uint32_t t0 = 0; t0 < tiles; t0 += kRoundTiles) {
+  for (uint32_t t0 = 0; t0 < tiles; t0 += PieceRound<true>::kTiles) {
+    PieceRound<true> round;
     round.load(b, log_buckets, bucket, t0, tiles);
     n += round.units();
   }
   if (n > 0) atomicAdd(&lds.units, n);
   __syncthreads();
-  const int total = lds.units;
-  const int parts = total <= slots * 3 / 4 ? 1 : (total + slots / 2 - 1) / (slots / 2);
-  for (int part = 0; part < parts; ++part) {
-    // where a search starts, and which part an id belongs to: bits of its hash that did not choose the bucket
-    const auto elsewhere = [&](uint32_t hash) { return parts > 1 && int((hash >> 23) % uint32_t(parts)) != part; };
-    for (int j = threadIdx.x; j < slots / 2; j += kBucketBlock) reinterpret_cast<uint4*>(lds.table)[j] = make_uint4(~0u, ~0u, ~0u, ~0u);
-    __syncthreads();
-    for (uint32_t t0 = 0; t0 < tiles; t0 += kRoundTiles) {
-      if (tiles > kRoundTiles) round.load(b, log_buckets, bucket, t0, tiles);  // (a single round is in registers still)
-      round.each(b, [&](uint32_t, ItemT item, uint32_t unit) {
-        if (elsewhere(item.x)) return;
-        const unsigned long long packed = (static_cast<unsigned long long>(item.x) << 32) | unit;
-        uint32_t slot = (item.x >> log_buckets) & mask;
-        bool placed = false;
-        for (int probes = 0; probes < slots && !placed; ++probes) {
-          unsigned long long cur = lds.table[slot];
-          if (cur == ~0ull) cur = atomicCAS(&lds.table[slot], ~0ull, packed);
-          placed = cur == ~0ull || uint32_t(cur >> 32) == item.x;
-          if (placed && cur > packed && cur != ~0ull) atomicMin(&lds.table[slot], packed);
-          slot = (slot + 1) & mask;
-        }
-        if (!placed) lds.overflow = 1;
-      });
-    }
-    __syncthreads();
-    if (lds.overflow == 0) {  // (an overflowing part's answers are void: the call fails)
-      for (uint32_t t0 = 0; t0 < tiles; t0 += kRoundTiles) {
-        if (tiles > kRoundTiles) round.load(b, log_buckets, bucket, t0, tiles);
-        round.each(b, [&](uint32_t e, ItemT item, uint32_t unit) {
-          if (unit < first_unit) return false;
-          if (elsewhere(item.x)) return false;
-          uint32_t slot = (item.x >> log_buckets) & mask;
-          unsigned long long held = lds.table[slot];
-          for (int probes = 0; probes < slots && uint32_t(held >> 32) != item.x; ++probes) {
-            slot = (slot + 1) & mask;
-            held = lds.table[slot];
-          }
-          nth(b.least, e) = uint32_t(held);
-          return uint32_t(held) == unit;
-        }, [&](uint32_t tile, uint32_t m) { lds.counts[tile] += m; });  // (nobody else has the tile's piece of this bucket)
-      }
-    }
-    __syncthreads();  // the table is rewritten
-  }
-  if (threadIdx.x == 0 && lds.overflow != 0) *b.overflow = 1;
-  __syncthreads();
+  const int parts = (lds.units + b.hash_slots / 2 - 1) / (b.hash_slots / 2);  // that fill half of the table, were all units' ids different
+  bool took = true;
+  for (int part = 0; part < parts; ++part) took &= first_of_part_hashed(b, log_buckets, bucket, tiles, first_unit, part, parts, b.hash_slots, lds);
+  if (threadIdx.x == 0 && !took) *b.overflow = 1;
 }
 
 // into[place of a unit in the tile] = its id's smallest unit, for all of the tile's units.

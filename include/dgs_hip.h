@@ -386,13 +386,15 @@ typedef struct dgs_segments {
  * out[t][i] = position of requiring[t][i] in unique, or -1 when absent.
  * Replaces TensorRelabelCUDA / Unique / Relabel / RelabelHashmap
  * (src/cuda/tensor_reindex.cu:11-205).
- *   packed_table   : 8-byte ids only.  Non-zero: the table keeps id and position in one 64-bit
- *                    slot (one atomic per id instead of two), which holds ids below 2^32 - 1; an
- *                    id beyond that sets counts_dev[1] and voids the call's results (call again
- *                    with 0).  Zero: id array + value array, any id >= 0.
+ *   packed_table   : Non-zero: an attempt for ids below 2^32 - 1.  8-byte ids: the table keeps id and
+ *                    position in one 64-bit slot (one atomic per id instead of two); an id beyond
+ *                    sets counts_dev[1] and voids the call's results (call again with 0).  Long lists
+ *                    of either width are gone over in buckets instead of on a table; more distinct ids in
+ *                    one part of the library's hash than an on-chip table holds (not by chance)
+ *                    void the attempt as well.  Zero: id array + value array, any id >= 0.
  *   unique_out     : device, capacity sum(mapping.len) ids
- *   counts_dev     : device int64[2]: [0] number of distinct ids, [1] non-zero if an id did not
- *                    fit the packed table
+ *   counts_dev     : device int64[2]: [0] number of distinct ids, [1] non-zero if the attempt that
+ *                    packed_table asks for is void
  *   counts_host / counts_ticket : optional (a ticket only with counts_host; counts_host alone
  *                    is for callers that poll it, dgs_stream_wait_words).  counts_host is pinned host memory
  *                    that the device can write; the kernels mirror counts_dev into it, and

@@ -45,3 +45,78 @@ def test_bucketed_pass_at_its_edges(pkg, oracle, mode, id_dtype, nodes, seeds, k
             assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
     finally:
         set_last_hop_mode(pkg, LAST_HOP_MODES[0])
+
+
+def _dev(x):
+    return torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+def _relabel_both_ways(pkg, oracle, mapping, requiring):
+    want_u, want = oracle.unique_relabel(mapping, requiring)
+    held = {}  # (a tensor that is given twice is one tensor)
+    dev = [[held.setdefault(id(x), _dev(x)) for x in part] for part in (mapping, requiring)]
+    for u, outs in (pkg.ops._CAPI_tensor_relabel(*dev), pkg.capi.unique_relabel(*dev)):
+        assert np.array_equal(u.cpu().numpy(), want_u)
+        for a, b in zip(outs, want):
+            assert np.array_equal(a.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [131_071, 131_072, 131_073, 139_263, 1_200_000])  # where buckets begin, 16 and 17 tiles, 147 tiles
+@pytest.mark.parametrize("distinct", [1, 3000, 1 << 30])
+def test_relabel_of_long_lists(pkg, oracle, dtype, n, distinct):
+    rng = np.random.default_rng(n)
+    seeds = rng.integers(0, distinct, size=n // 16).astype(dtype)
+    cols = rng.integers(0, distinct, size=n - seeds.size).astype(dtype)
+    rows = np.repeat(seeds, 16)[:cols.size]  # runs that begin and end anywhere in a tile
+    _relabel_both_ways(pkg, oracle, [seeds, cols], [rows, cols])
+    # ids in no order, ids that are not there, no mapped ones, all mapped ones
+    others = np.concatenate([rng.permutation(cols)[:20_000], rng.integers(0, 1 << 31, size=9000).astype(dtype), cols[:1]])
+    _relabel_both_ways(pkg, oracle, [seeds, cols], [others])
+    _relabel_both_ways(pkg, oracle, [cols, seeds], [cols, seeds])
+
+
+def test_relabel_of_long_lists_in_many_segments(pkg, oracle):
+    rng = np.random.default_rng(5)
+    sizes = [70_000, 1, 0, 8191, 8192, 8193, 60_000]
+    parts = [rng.integers(0, 200_000, size=s).astype(np.int64) for s in sizes]
+    _relabel_both_ways(pkg, oracle, parts, [parts[3], parts[0][:9000].copy(), parts[2], parts[6], parts[4][::-1].copy(), parts[1]])
+    # more ids to look up than are mapped: the table serves them
+    _relabel_both_ways(pkg, oracle, parts, [np.tile(parts[0], 3)])
+    # a segment that lies where the one before it would go on, were it not for the one in between
+    whole, between = _dev(parts[0]), _dev(parts[3])
+    mapping = [whole[:20_000], between, whole[20_000 + between.numel():], _dev(parts[6]), _dev(parts[4])]
+    host = [m.cpu().numpy() for m in mapping]
+    want_u, want = oracle.unique_relabel(host, host)
+    u, outs = pkg.ops._CAPI_tensor_relabel(mapping, mapping)
+    assert np.array_equal(u.cpu().numpy(), want_u) and all(np.array_equal(a.cpu().numpy(), b) for a, b in zip(outs, want))
+
+
+def test_relabel_of_long_lists_with_ids_beyond_32_bits(pkg, oracle):
+    rng = np.random.default_rng(6)
+    cols = rng.integers(0, 500_000, size=150_000).astype(np.int64)
+    odd = cols[:30_000].copy()
+    odd[::7] += 1 << 32   # not there, though their low halves are
+    odd[1::7] = -1
+    odd[5000:5100] = (1 << 32) - 1  # a run of them
+    _relabel_both_ways(pkg, oracle, [cols], [odd, cols])
+    cols[77_777] += 1 << 33  # among the mapped ones: the attempt is void
+    _relabel_both_ways(pkg, oracle, [cols], [odd, cols])
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_relabel_of_ids_that_crowd_a_bucket(pkg, oracle, dtype):
+    # 40 000 ids of one bucket (of 256, by the library's hash, restated here) go over its table of 16 384 in 5 parts; if they
+    # are of one part as well, the attempt is void and the table answers
+    ids = np.arange(60_000_000, dtype=np.uint32)
+    h = ids.copy()
+    h ^= h >> np.uint32(16); h *= np.uint32(0x85EBCA6B)
+    h ^= h >> np.uint32(13); h *= np.uint32(0xC2B2AE35)
+    h ^= h >> np.uint32(16)
+    bucket = ids[(h & 255) == 0]
+    part = ids[((h & 255) == 0) & ((h >> 23) % 5 == 0)]
+    others = ids[(h & 255) == 1][:100_000]
+    for crowd in (bucket[:40_000], part[:40_000]):
+        assert crowd.size == 40_000
+        mapping = [np.concatenate([crowd, others]).astype(dtype)]
+        _relabel_both_ways(pkg, oracle, mapping, [mapping[0], crowd[::-1].astype(dtype)])

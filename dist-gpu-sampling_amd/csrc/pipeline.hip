@@ -187,7 +187,8 @@ constexpr int kFoldMaxRowPerPick = 4;
 // the picked ids in the slot words; the compact launch has every pick's smallest unit from the pass: its own
 // (a first occurrence), that of an id the frontier held before this hop (its rank | kRankBit: final, no further
 // lookup), or that of an earlier pick of this hop (whose position becomes the slot word, and whose rank
-// the compaction records there).  Same result as the table gives.
+// the compaction records there).  A draw that repeats another one of its row is no unit: its slot word is that
+// draw's position from the fill on, where it finds a rank, or the link to one.  Same result as the table gives.
 //
 // It takes two launches more than the table does, and pays where the hop is large (by its worst case: that is what the
 // host knows) and the table beyond the caches.  us a batch with rows of 64 bytes, table / pass: 2.4 M nodes, fanouts
@@ -200,6 +201,14 @@ constexpr int kFoldMaxRowPerPick = 4;
 constexpr int64_t kBucketedMinNodes = 262144, kBucketedMaxNodes = 16777216;
 constexpr int64_t kBucketedMinPicks = 917504;
 static_assert(kBucketedMaxNodes <= kDirectMaxIds, "the direct form takes them");
+// Larger graphs take the hashed form, which pays for draws with replacement of a very large hop: without it many of the
+// positions are empty, which the pass goes over all the same (111 M nodes, 0.94 M picks in 2.8 M positions: 215 us a batch
+// on the table, 216 by the pass).  us a batch of draws, 64-byte rows, table / pass: 20 M nodes, fanouts [10,20] from
+// 4096 seeds (0.9 M picks at most) 78 / 88, [10,40] (1.8 M) 82 / 94, [5,10,15] (4.1 M) 180 / 172, [10,25] from 16 384 (4.5 M)
+// 193 / 188; 60 M nodes 77 / 88, 84 / 94, 189 / 173, 200 / 193; 8 batches of [5,10,15] through the loader 1295 / 1188;
+// R-MAT of 2^26 nodes, [50,50] from 16 384 (41.8 M, 3.05 M in fact, two thirds of them repeats) 372 / 354: fill 149 -> 76,
+// sort 14.4, first 35.
+constexpr int64_t kHashedMinPicks = int64_t(3) << 20;
 __host__ __device__ __forceinline__ int64_t front_units(int64_t s) { return (s + 15) / 16 * 16; }
 
 // rank of the id at position p of hop 0, given p's slot word
@@ -393,7 +402,7 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   const int64_t s = seeds_of(h);
   const bool look_first = look_before_insert(h, s);
   const bool bucketed = bucketed_now(h, s);
-  const bool fold = replace && !bucketed;
+  const bool fold = replace;
   if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   if (i >= s) return;  // whole groups leave together
   const int group_lane0 = (threadIdx.x & (kWave - 1)) - l;
@@ -877,8 +886,9 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Bucket
       }
     }
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j)
-      if (id[j] != kNoId) id[j] &= ~kFirstBit;
+    for (int j = 0; j < kBucketItems; ++j)  // (a position's word: a draw that repeats one of its own row's, no unit)
+      if (id[j] != kNoId) id[j] = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x < front ? id[j]
+                                : (id[j] & kFirstBit) != 0 ? id[j] & ~kFirstBit : kNoId;
     sort_tile<HASHED>(b, log_buckets, tile, id, lds);
     __syncthreads();  // lds is rewritten by the block's next tile
   }
@@ -1088,7 +1098,7 @@ __device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets&
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       if (u + j >= units) word[g][j] = kInvalidSlot;
-      if (word[g][j] != kInvalidSlot && least[j] == u + j) first[g] |= 1u << j;
+      if (word[g][j] != kInvalidSlot && (word[g][j] & kFirstBit) != 0 && least[j] == u + j) first[g] |= 1u << j;
     }
     const int c = __builtin_popcount(first[g]);  // its bits are summed over the lanes by ballots
     lane_before[g] = 0;
@@ -1133,13 +1143,15 @@ __device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets&
       if ((first[g] >> j) & 1) {
         nth(static_cast<IdT*>(h.frontier), rank) = IdT(word[g][j] & ~kFirstBit);
         ++rank;
-      } else if (word[g][j] != kInvalidSlot) {
+      } else if (word[g][j] != kInvalidSlot && (word[g][j] & kFirstBit) != 0) {
         changed = true;
         const uint32_t met = least[j] < u + j ? least[j] : u + j;  // (one that is not before its own is none that the pass left)
-        word[g][j] = met < front ? met | kRankBit : uint32_t(h.pos_base) + (met - front);
+        const uint32_t p = uint32_t(h.pos_base) + (met - front);
+        word[g][j] = met < front ? met | kRankBit : p;
+        ranks[j] = met < front ? met : p | kLinkBit;  // for the draws of the row that repeat this one
       }
     }
-    nth(reinterpret_cast<words*>(h.rank_at + h.pos_base), (u - front) / ITEMS) = ranks;  // (only the ones at first positions are ever read)
+    nth(reinterpret_cast<words*>(h.rank_at + h.pos_base), (u - front) / ITEMS) = ranks;
     if (changed) nth(reinterpret_cast<words*>(slot), (u - front) / ITEMS) = word[g];
   }
 }
@@ -1235,7 +1247,7 @@ struct Plan {
   size_t table_bytes = 0;    // 0 for the direct table
   bool weighted = false;     // picks by edge weight: per-hop queues for long rows
   bool bucketed = false;     // the last hop may find its first occurrences by the bucketed pass (if it turns out to fit)
-  bool bucket_hashed = false; // ... with ids told apart by an LDS hash table (on request)
+  bool bucket_hashed = false; // ... with ids told apart by an LDS hash table (graphs beyond kBucketedMaxNodes)
   bool bucket_space = false; // the workspace has room for that pass
   int64_t bucket_tiles = 0;   // its tiles: all of the hop's units in the worst case, or as many as there is room for
   int64_t bucket_pos_cap = 0; // padded positions of the hop that these hold
@@ -1254,7 +1266,7 @@ inline void plan_bucket_tiles(Plan* p) {
 }
 
 dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, int32_t id_bytes,
-                     int64_t n_nodes, bool have_node_table, Plan* p) {
+                     int64_t n_nodes, bool have_node_table, bool replace, Plan* p) {
   DGS_REQUIRE(n_hops >= 1 && n_hops <= DGS_MAX_HOPS, DGS_ERR_INVALID, "sample_blocks: %d hops (1..%d)", n_hops,
               DGS_MAX_HOPS);
   DGS_REQUIRE(fanouts != nullptr && n_seeds >= 0, DGS_ERR_INVALID, "sample_blocks: bad argument");
@@ -1276,17 +1288,15 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
     DGS_REQUIRE(n_nodes >= 0 && n_nodes < 0x7fffffffLL, DGS_ERR_UNSUPPORTED,
                 "sample_blocks: a node table needs fewer than 2^31 nodes (have %lld)", (long long)n_nodes);
     p->kind = TableKind::kDirect;
-    // The bucketed pass: slot words are ids (the direct table's).  By size only the direct form runs.  The hashed form
-    // gives the same results on any graph and takes the atomics out of the hop just the same, but does not pay: 111 M nodes,
-    // 944 k picks of mostly new ids: fill 57 -> 30 us, against 12 + 27 us for its two launches; R-MAT with two thirds
-    // repeats 149 -> 75 against 15 + 50.  It runs when the test hook asks for it (1 never, 2 whatever the size,
-    // 3 whatever the size and hashed whatever the graph, 4 like 3 with on-chip tables of 256 slots, so that small
-    // inputs fill them and go over their buckets in parts).
+    // The bucketed pass: slot words are ids (the direct table's).  (Test hook: 1 never, 2 whatever the size, 3 whatever the
+    // size and hashed whatever the graph, 4 like 3 with on-chip tables of 256 slots, so that small inputs fill them
+    // and go over their buckets in parts.)
     const int64_t mode = debug_option(DGS_DEBUG_SAMPLER_BUCKETED);
-    const bool large = p->nnz_max[n_hops - 1] >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
+    const int64_t picks = p->nnz_max[n_hops - 1];
     p->bucket_hashed = n_nodes > kBucketedMaxNodes || mode == 3 || mode == 4;
+    const bool large = p->bucket_hashed ? replace && picks >= kHashedMinPicks : picks >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
     p->bucketed = p->bucket_space && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
-                  (p->bucket_hashed ? mode >= 2 : (large || mode >= 2));
+                  (large || mode >= 2);
     p->hash_slots = mode == 4 ? 256 : kHashSlots;
     int log_b = kMinLogBuckets;
     if (p->bucket_hashed) {  // (as many as its units may need: log_buckets_of)
@@ -1619,7 +1629,7 @@ dgs_status run_blocks_table(const Plan& p, Hop* hops, const Buckets& buckets, vo
 DGS_API dgs_status dgs_sample_blocks_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops,
                                           int64_t* seeds_max, int64_t* edges_max) {
   dgs::Plan p;
-  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, false, &p);
+  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, false, false, &p);
   if (s != DGS_OK) return s;
   DGS_REQUIRE(seeds_max && edges_max, DGS_ERR_INVALID, "sample_blocks_plan: null output");
   for (int h = 0; h <= n_hops; ++h) seeds_max[h] = p.s_max[h];
@@ -1631,7 +1641,7 @@ DGS_API size_t dgs_sample_blocks_workspace_bytes(int64_t n_seeds, const int64_t*
                                                  int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   return dgs::layout(p, fanouts, nullptr, nullptr, nullptr);
@@ -1645,7 +1655,7 @@ DGS_API size_t dgs_sample_blocks_weighted_workspace_bytes(int64_t n_seeds, const
                                                           int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts (used when there is no node table)
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   p.weighted = true;
@@ -1662,7 +1672,7 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
   using namespace dgs;
   Plan p;
   // node count = indptr entries - 1
-  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, node_table != nullptr, &p);
+  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, node_table != nullptr, replace != 0, &p);
   if (s != DGS_OK) return s;
   if (probs != nullptr) {
     DGS_REQUIRE(probs->elem_bytes == 4 && probs->total == indices.total, DGS_ERR_INVALID,

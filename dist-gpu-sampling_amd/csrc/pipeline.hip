@@ -1178,10 +1178,25 @@ __device__ __forceinline__ void announce_long_rows(const Hop& h, int64_t begin, 
 // Virtual blocks: one per NT * kRowItems rows (scan of the rows' pick counts), then one per position tile.  A
 // launch that fits the grid cap has a block for each in the worst case; a launch that loops (STRIDE)
 // goes over the tiles the hop really has.
+//
+// Blocks from compact_blocks on, behind all that others wait for, write the previous hop's edge list where the fill had to
+// leave it (launch_fill): a launch of its own is 5 us at the floor, and this one, of two blocks a CU that wait for one another, has
+// the room.  111 M nodes, 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us.
+constexpr bool takes_edges(int items, bool announce) { return items > 1 && !announce; }  // (fills that leave the list are not in front of the others)
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, bool ANNOUNCE>
-__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table) {
+__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, Hop prev, int64_t row_tiles, uint32_t compact_blocks,
+                                                            int64_t relabel_count, TableT table) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
   int64_t begin = 0, end = 0;
+  if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
+    if (blockIdx.x >= compact_blocks) {
+      constexpr int kPer = NT / kEdgeBlock;
+      for (int64_t vb = int64_t(blockIdx.x - compact_blocks) * kPer + threadIdx.x / kEdgeBlock; vb < relabel_count;
+           vb += int64_t(gridDim.x - compact_blocks) * kPer)
+        relabel_tile<IdT, TableT, false>(prev, table, vb, int(threadIdx.x % kEdgeBlock));
+      return;
+    }
+  }
   if (h.bucketed != 0 && bucketed_now(h, seeds_of(h))) return;
   if (!STRIDE) {
     const int64_t vb = blockIdx.x;
@@ -1194,7 +1209,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
   const int64_t rows = s > 0 ? (s + NT * kRowItems - 1) / (NT * kRowItems) : 1;  // (tile 0 of either kind writes the lengths)
   const int64_t len = seed_part(h, s) + s * h.k;
   const int64_t total = rows + (len > 0 ? (len + kTile - 1) / kTile : 1);
-  for (int64_t vb = blockIdx.x; vb < total; vb += gridDim.x) {
+  for (int64_t vb = blockIdx.x; vb < total; vb += compact_blocks) {
     begin = end = 0;
     if (vb < rows) offsets_tile<NT, false>(h, vb);
     else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table, &begin, &end);
@@ -1405,21 +1420,25 @@ void launch_relabel(const Hop& hop, const TableT& table, hipStream_t st) {
                        blocks, table);
 }
 
+// `left`: blocks of the previous hop's edge list that are to be written too; set to 0 where the launch takes them.
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool ANNOUNCE>
-void launch_compact_as(const Hop& hop, const TableT& table, hipStream_t st) {
+void launch_compact_as(const Hop& hop, const Hop& prev, int64_t* left, const TableT& table, hipStream_t st) {
   const int64_t row_tiles = row_tiles_of(hop.s_max, hop.len_max);
-  const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max);
-  if (blocks > std::min(grid_cap(), kLookbackGrid))
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(uint32_t(std::min(grid_cap(), kLookbackGrid))),
-                       dim3(NT), 0, st, hop, row_tiles, table);
+  const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max), at_once = std::min(grid_cap(), kLookbackGrid);
+  int64_t relabel_count = 0;
+  if (takes_edges(ITEMS, ANNOUNCE)) std::swap(relabel_count, *left);
+  const uint32_t more = uint32_t(std::min((relabel_count + NT / kEdgeBlock - 1) / (NT / kEdgeBlock), kLoopGrid));
+  if (blocks > at_once)
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(uint32_t(at_once) + more),
+                       dim3(NT), 0, st, hop, prev, row_tiles, uint32_t(at_once), relabel_count, table);
   else
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(uint32_t(blocks)), dim3(NT), 0, st,
-                       hop, row_tiles, table);
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(uint32_t(blocks) + more), dim3(NT), 0, st,
+                       hop, prev, row_tiles, uint32_t(blocks), relabel_count, table);
 }
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
-void launch_compact(const Hop& hop, bool announce, const TableT& table, hipStream_t st) {
-  if (announce) launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, true>(hop, table, st);
-  else launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, false>(hop, table, st);
+void launch_compact(const Hop& hop, const Hop& prev, int64_t* left, bool announce, const TableT& table, hipStream_t st) {
+  if (announce) launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, true>(hop, prev, left, table, st);
+  else launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, false>(hop, prev, left, table, st);
 }
 
 // The bucketed pass and the compact launch behind it.
@@ -1437,27 +1456,28 @@ void launch_bucketed(const Hop& hop, const Buckets& b, hipStream_t st) {
     hipLaunchKernelGGL((hop_compact_sorted_kernel<IdT, HASHED, false>), dim3(uint32_t(blocks)), dim3(kBucketBlock), 0, st, hop, b);
 }
 
+// Returns the blocks of the previous hop's edge list that are left to be written behind this launch.
 template <typename IdT, typename PtrT, typename TableT, int G>
-void launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin, int64_t clear_n16,
-                 const TableT& table, const dgs_view& indptr, const dgs_view& indices, bool replace,
-                 uint64_t rng_seed, hipStream_t st) {
+int64_t launch_fill(const Hop& cur, const Hop& prev, int64_t relabel_count, uint4* clear_begin, int64_t clear_n16,
+                    const TableT& table, const dgs_view& indptr, const dgs_view& indices, bool replace,
+                    uint64_t rng_seed, hipStream_t st) {
   const int64_t fill_blocks = (cur.s_max * G + kBlock - 1) / kBlock;
   const int64_t clear_blocks = (clear_n16 + kBlock - 1) / kBlock;
-  int64_t total = fill_blocks + relabel_count + clear_blocks;
+  const int64_t total = fill_blocks + relabel_count + clear_blocks;
   if (is_capped(total)) {
     // A launch that loops over its virtual blocks keeps the previous hop's edge list out of the
     // loop: with it the kernel needs 85-90 vector registers and five waves fit a SIMD instead of
-    // seven (measured on a 136 k-row hop: 46 us against 39).  That list becomes a launch of its own,
+    // seven (measured on a 136 k-row hop: 46 us against 39).  That list goes with the compact launch or is one of its own,
     // behind this one (the previous hop's table entries do not change any more: positions only grow).
-    total -= relabel_count;
-    hipLaunchKernelGGL((hop_fill_kernel<IdT, PtrT, TableT, G, true>), dim3(capped_grid(total)), dim3(kBlock), 0, st,
+    hipLaunchKernelGGL((hop_fill_kernel<IdT, PtrT, TableT, G, true>), dim3(capped_grid(total - relabel_count)), dim3(kBlock), 0, st,
                        cur, prev, fill_blocks, int64_t(0), clear_begin, clear_n16, table,
                        TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
-    if (relabel_count > 0) launch_relabel<IdT>(prev, table, st);
-  } else
-    hipLaunchKernelGGL((hop_fill_kernel<IdT, PtrT, TableT, G, false>), dim3(capped_grid(total)), dim3(kBlock), 0, st,
-                       cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
-                       TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
+    return relabel_count;
+  }
+  hipLaunchKernelGGL((hop_fill_kernel<IdT, PtrT, TableT, G, false>), dim3(capped_grid(total)), dim3(kBlock), 0, st,
+                     cur, prev, fill_blocks, relabel_count, clear_begin, clear_n16, table,
+                     TierView<PtrT>(indptr), TierView<IdT>(indices), replace, rng_seed);
+  return 0;
 }
 
 // Blocks of a weighted launch that take queued long rows, in front of `others`.  256 keep a block on every CU, which
@@ -1524,13 +1544,14 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
       if (p.weighted) end = reinterpret_cast<const char*>(cur.long_count + 2);  // (which comes next)
       clear_n16 = (end - reinterpret_cast<const char*>(clear_begin) + 15) / 16;
     }
+    int64_t left_over = 0;
     if (p.weighted) {
       if (replace) launch_fill_weighted<IdT, PtrT, TableT, true>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st);
       else launch_fill_weighted<IdT, PtrT, TableT, false>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, *probs, rng_seed, st);
-    } else if (cur.k <= 8) launch_fill<IdT, PtrT, TableT, 8>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
-    else if (cur.k <= 16) launch_fill<IdT, PtrT, TableT, 16>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
-    else if (cur.k <= 32) launch_fill<IdT, PtrT, TableT, 32>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
-    else launch_fill<IdT, PtrT, TableT, 64>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
+    } else if (cur.k <= 8) left_over = launch_fill<IdT, PtrT, TableT, 8>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
+    else if (cur.k <= 16) left_over = launch_fill<IdT, PtrT, TableT, 16>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
+    else if (cur.k <= 32) left_over = launch_fill<IdT, PtrT, TableT, 32>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
+    else left_over = launch_fill<IdT, PtrT, TableT, 64>(cur, prev, surplus, clear_begin, clear_n16, table, indptr, indices, replace, rng_seed, st);
     DGS_LAUNCH_CHECK();
 
     if constexpr (std::is_same_v<TableT, DirectTable<IdT>>) {
@@ -1538,16 +1559,21 @@ dgs_status run_blocks(const Plan& p, Hop* hops, const Buckets& buckets, const Ta
         if (buckets.hashed) launch_bucketed<IdT, true>(cur, buckets, st);
         else launch_bucketed<IdT, false>(cur, buckets, st);
         DGS_LAUNCH_CHECK();
-        if (cur.len_max <= cur.bucket_pos_cap) break;  // (it cannot outgrow the pass)
+        if (cur.len_max <= cur.bucket_pos_cap) {  // (it cannot outgrow the pass)
+          if (left_over > 0) launch_relabel<IdT>(prev, table, st);
+          DGS_LAUNCH_CHECK();
+          break;
+        }
       }
     }
     // (a queue holds the whole frontier: from hop 0 on, where a later hop reads it; hops only get larger)
     const bool announce = p.weighted && h + 1 < p.n_hops && !weighted_shared(hops[p.n_hops - 1]);
     switch (pos_tile_kind(cur.len_max)) {
-      case kShortTile: launch_compact<IdT, TableT, 256, 1, 1>(cur, announce, table, st); break;
-      case kMiddleTile: launch_compact<IdT, TableT, 256, 4, 4>(cur, announce, table, st); break;
-      case kLongTile: launch_compact<IdT, TableT, 512, 4, 4>(cur, announce, table, st); break;
+      case kShortTile: launch_compact<IdT, TableT, 256, 1, 1>(cur, prev, &left_over, announce, table, st); break;
+      case kMiddleTile: launch_compact<IdT, TableT, 256, 4, 4>(cur, prev, &left_over, announce, table, st); break;
+      case kLongTile: launch_compact<IdT, TableT, 512, 4, 4>(cur, prev, &left_over, announce, table, st); break;
     }
+    if (left_over > 0) launch_relabel<IdT>(prev, table, st);
     DGS_LAUNCH_CHECK();
   }
   // every length is final here: mark the point the caller may wait for

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import load_pkg, powerlaw_graph
+from helpers import LAST_HOP_MODES, load_pkg, powerlaw_graph, set_last_hop_mode
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +77,34 @@ def test_edge_list_in_a_launch_of_its_own(pkg, oracle, n_seeds, fanouts, dim, ca
             assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
     finally:
         capi.check(capi.lib.dgs_debug_set(capi.DEBUG_SAMPLER_GRID_CAP, 0))
+
+
+@pytest.mark.parametrize("last_hop", [LAST_HOP_MODES[0], LAST_HOP_MODES[1], LAST_HOP_MODES[4]])
+@pytest.mark.parametrize("n_seeds,fanouts,replace", [
+    (33_000, [33, 1], False),    # a fill that loops, a compact launch that does not (hop 0's list, through the table)
+    (33_000, [33, 1], True),
+    (4096, [15, 10, 5], False),  # both loop (a later hop's list)
+    (9000, [64, 3, 4], True),    # ... and the hop may outgrow the bucketed pass
+    (300_000, [4, 1], True),     # ... with tiles of 4096 positions
+])
+def test_edge_list_in_the_compact_launch(pkg, oracle, last_hop, n_seeds, fanouts, replace):
+    rng = np.random.default_rng(n_seeds)
+    n = 300_000
+    indptr, indices = powerlaw_graph(rng, n, 12, 300, id_dtype=np.int32)
+    ip = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    seeds = rng.integers(0, n, size=n_seeds).astype(indices.dtype)
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, indices, fanouts, replace, 8, 1)
+    try:
+        set_last_hop_mode(pkg, last_hop)
+        for _ in range(2):  # (the second one finds the node table used)
+            pkg.set_rng_state(8, 1)
+            f, _, blocks = pkg.ChunkTensorSampler(fanouts, ip, ix, replace=replace).sample_blocks(None, torch.from_numpy(seeds))
+            assert np.array_equal(f.cpu().numpy(), want_f)
+            for g, w in zip(blocks, want):
+                assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+    finally:
+        set_last_hop_mode(pkg, LAST_HOP_MODES[0])
 
 
 @pytest.fixture(scope="module")

@@ -1181,11 +1181,12 @@ __device__ __forceinline__ void announce_long_rows(const Hop& h, int64_t begin, 
 //
 // Blocks from compact_blocks on, behind all that others wait for, write the previous hop's edge list where the fill had to
 // leave it (launch_fill): a launch of its own is 5 us at the floor, and this one, of two blocks a CU that wait for one another, has
-// the room.  111 M nodes, 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us.
+// the room.  111 M nodes, 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us, on another card 221.5 ->
+// 217.3.  (Their arguments come last: a launch without them reads none of those, 0.25 us.)
 constexpr bool takes_edges(int items, bool announce) { return items > 1 && !announce; }  // (fills that leave the list are not in front of the others)
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, bool ANNOUNCE>
-__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, Hop prev, int64_t row_tiles, uint32_t compact_blocks,
-                                                            int64_t relabel_count, TableT table) {
+__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table, Hop prev,
+                                                            uint32_t compact_blocks, int64_t relabel_count) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
   int64_t begin = 0, end = 0;
   if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
@@ -1430,10 +1431,10 @@ void launch_compact_as(const Hop& hop, const Hop& prev, int64_t* left, const Tab
   const uint32_t more = uint32_t(std::min((relabel_count + NT / kEdgeBlock - 1) / (NT / kEdgeBlock), kLoopGrid));
   if (blocks > at_once)
     hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(uint32_t(at_once) + more),
-                       dim3(NT), 0, st, hop, prev, row_tiles, uint32_t(at_once), relabel_count, table);
+                       dim3(NT), 0, st, hop, row_tiles, table, prev, uint32_t(at_once), relabel_count);
   else
     hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(uint32_t(blocks) + more), dim3(NT), 0, st,
-                       hop, prev, row_tiles, uint32_t(blocks), relabel_count, table);
+                       hop, row_tiles, table, prev, uint32_t(blocks), relabel_count);
 }
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
 void launch_compact(const Hop& hop, const Hop& prev, int64_t* left, bool announce, const TableT& table, hipStream_t st) {

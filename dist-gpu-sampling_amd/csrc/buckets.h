@@ -23,8 +23,8 @@
 // items are one word (the high bits and the unit's place in its tile).  Hashed, for any number of ids:
 // bucket = low bits of a hash that takes no two ids to one value, hashes are told apart in an open-addressing table of
 // packed words (hash, unit), items are the hash and the unit.  A bucket whose ids do not fit that table is gone over
-// again in parts, by other bits of the hash, one table's worth at a time; ids that crowd one part all the same (not by
-// chance) are reported.
+// again in parts, by other bits of the hash, one table's worth at a time; a part whose ids crowd it all the same (not by
+// chance) in as many ranges of hashes as there are tables' worths of them, each of which a table takes whatever the ids.
 #ifndef DGS_CSRC_BUCKETS_H_
 #define DGS_CSRC_BUCKETS_H_
 
@@ -58,7 +58,7 @@ struct Buckets {
   uint32_t* least;     // [tiles_max][kBucketTile] smallest unit of the item's id
   uint16_t* piece;     // [tiles_max][buckets + 1]; the last one: units of the tile
   uint32_t* firsts;    // [kCounters][kMaxBucketTiles] units that are their ids' smallest (of those that count, see below)
-  int* overflow;       // set when the ids of a part did not fit its table
+  int* overflow;       // set when the ids of a part did not fit its table (only one that a test hook makes small)
   int32_t tiles_max;
   int32_t log_buckets; // hashed: at most
   uint32_t n_ids;      // direct: ids are below it
@@ -290,15 +290,23 @@ struct HashedLds {
   int units;
   int overflow;
 };
-// All units of the bucket whose ids belong to part `part` of `parts`; returns whether the table took them (the same in
-// all threads), within max_probes probes each.
+// Part `part` of `parts` of a bucket, by bits of the hash that did not choose the bucket, and of it the hashes whose other
+// bits are `span` numbers from `lo` on.
+struct HashPart {
+  int part, parts;
+  uint32_t lo, span;
+};
+// All units of the bucket, or (PARTS) of a part of it; returns whether the table took them (the same in all threads),
+// within max_probes probes each.
+template <bool PARTS>
 __device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles, uint32_t first_unit,
-                                                     int part, int parts, int max_probes, HashedLds& lds) {
+                                                     HashPart part, int max_probes, HashedLds& lds) {
   using ItemT = BucketItem<true>::type;
   const int slots = b.hash_slots;
   const uint32_t mask = uint32_t(slots - 1);
-  // where a search starts, and which part an id belongs to: bits of its hash that did not choose the bucket
-  const auto elsewhere = [&](uint32_t hash) { return parts > 1 && int((hash >> 23) % uint32_t(parts)) != part; };
+  const auto elsewhere = [&](uint32_t hash) {
+    return PARTS && (int((hash >> 23) % uint32_t(part.parts)) != part.part || (hash >> log_buckets) - part.lo >= part.span);
+  };
   PieceRound<true> round;
   round.load(b, log_buckets, bucket, 0, tiles);
   for (int j = threadIdx.x; j < slots / 2; j += kBucketBlock) reinterpret_cast<uint4*>(lds.table)[j] = make_uint4(~0u, ~0u, ~0u, ~0u);
@@ -346,7 +354,8 @@ __device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_b
 // A bucket of many units may be one of few ids: it is gone over in parts only where the table has not taken them all.
 __device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles,
                                                        uint32_t first_unit, HashedLds& lds) {
-  if (first_of_part_hashed(b, log_buckets, bucket, tiles, first_unit, 0, 1, kFewProbes < b.hash_slots ? kFewProbes : b.hash_slots, lds)) return;
+  const int few = kFewProbes < b.hash_slots ? kFewProbes : b.hash_slots;
+  if (first_of_part_hashed<false>(b, log_buckets, bucket, tiles, first_unit, HashPart{0, 1, 0u, ~0u}, few, lds)) return;
   if (threadIdx.x == 0) lds.units = 0;
   __syncthreads();
   int n = 0;
@@ -359,7 +368,15 @@ __device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log
   __syncthreads();
   const int parts = (lds.units + b.hash_slots / 2 - 1) / (b.hash_slots / 2);  // that fill half of the table, were all units' ids different
   bool took = true;
-  for (int part = 0; part < parts; ++part) took &= first_of_part_hashed(b, log_buckets, bucket, tiles, first_unit, part, parts, b.hash_slots, lds);
+  for (int part = 0; part < parts; ++part) {
+    bool fits = first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, HashPart{part, parts, 0u, ~0u}, b.hash_slots, lds);
+    if (!fits && b.hash_slots == kHashSlots) {
+      fits = true;
+      for (uint32_t lo = 0; lo < 1u << (32 - log_buckets); lo += kHashSlots)  // (no two ids have one hash)
+        fits &= first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, HashPart{part, parts, lo, uint32_t(kHashSlots)}, kHashSlots, lds);
+    }
+    took &= fits;
+  }
   if (threadIdx.x == 0 && !took) *b.overflow = 1;
 }
 

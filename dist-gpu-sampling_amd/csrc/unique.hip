@@ -874,7 +874,7 @@ DGS_API dgs_status dgs_unique_relabel(dgs_segments mapping, dgs_segments requiri
     DGS_LAUNCH_CHECK();
     return counts_ticket ? dgs_ticket_record(st, counts_ticket) : DGS_OK;
   }
-  // (an attempt that packed_table asks for: ids that do not fit a word, or crowd a bucket, void it)
+  // (an attempt that packed_table asks for: ids that do not fit a word void it)
   if (packed_table != 0 && may_be_bucketed(n) && lookback_polls() == kLookbackPolls) {  // (test hook of the launches that it replaces)
     const SplitRequiring r = split_requiring(mapping, requiring, out, w.slot);
     if (bucket_tiles(seg_total(r.queries)) <= bucket_tiles(n))

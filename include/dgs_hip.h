@@ -389,9 +389,8 @@ typedef struct dgs_segments {
  *   packed_table   : Non-zero: an attempt for ids below 2^32 - 1.  8-byte ids: the table keeps id and
  *                    position in one 64-bit slot (one atomic per id instead of two); an id beyond
  *                    sets counts_dev[1] and voids the call's results (call again with 0).  Long lists
- *                    of either width are gone over in buckets instead of on a table; more distinct ids in
- *                    one part of the library's hash than an on-chip table holds (not by chance)
- *                    void the attempt as well.  Zero: id array + value array, any id >= 0.
+ *                    of either width are gone over in buckets instead of on a table.  Zero: id array +
+ *                    value array, any id >= 0.
  *   unique_out     : device, capacity sum(mapping.len) ids
  *   counts_dev     : device int64[2]: [0] number of distinct ids, [1] non-zero if the attempt that
  *                    packed_table asks for is void
@@ -453,8 +452,8 @@ typedef struct dgs_block_out {
  *                                                          bucketed pass met a bucket with more distinct ids
  *                                                          than its on-chip table holds (the hop's results are
  *                                                          void; ids that crowd one bucket of the library's
- *                                                          hash: run the call again with
- *                                                          DGS_DEBUG_SAMPLER_BUCKETED = 1)
+ *                                                          hash, and only with the tables that
+ *                                                          DGS_DEBUG_SAMPLER_BUCKETED = 4 cuts)
  *   sizes_host / ticket    : optional (a ticket only with sizes_host).  sizes_host is pinned host
  *                            memory that the device can write (hipHostMalloc); the kernels mirror
  *                            sizes_dev into it, and *sizes_ticket marks the point on `stream`

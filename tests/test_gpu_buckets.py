@@ -107,7 +107,7 @@ def test_relabel_of_long_lists_with_ids_beyond_32_bits(pkg, oracle):
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
 def test_relabel_of_ids_that_crowd_a_bucket(pkg, oracle, dtype):
     # 40 000 ids of one bucket (of 256, by the library's hash, restated here) go over its table of 16 384 in 5 parts; if they
-    # are of one part as well, the attempt is void and the table answers
+    # are of one part as well, that part goes over it range by range
     ids = np.arange(60_000_000, dtype=np.uint32)
     h = ids.copy()
     h ^= h >> np.uint32(16); h *= np.uint32(0x85EBCA6B)
@@ -120,3 +120,27 @@ def test_relabel_of_ids_that_crowd_a_bucket(pkg, oracle, dtype):
         assert crowd.size == 40_000
         mapping = [np.concatenate([crowd, others]).astype(dtype)]
         _relabel_both_ways(pkg, oracle, mapping, [mapping[0], crowd[::-1].astype(dtype)])
+
+
+def test_draws_that_crowd_a_bucket(pkg, oracle):
+    # 20 000 ids of one bucket (of 256) and of one of the 3 parts that its 22 000 units make: more than a table's 16 384 slots
+    n = 1 << 24
+    h = np.arange(n, dtype=np.uint32)
+    h ^= h >> np.uint32(16); h *= np.uint32(0x85EBCA6B)
+    h ^= h >> np.uint32(13); h *= np.uint32(0xC2B2AE35)
+    h ^= h >> np.uint32(16)
+    crowd = np.flatnonzero(((h & 255) == 0) & ((h >> 23) % 3 == 0))[:20_000].astype(np.int32)
+    assert crowd.size == 20_000
+    seeds = np.arange(2000, dtype=np.int32)
+    indptr = np.minimum(np.arange(n + 1, dtype=np.int64), 2000) * 10
+    ip = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.from_numpy(crowd), 1, 1 << 40)
+    want_f, _, want = oracle.sample_blocks(seeds, indptr, crowd, [10, 0], False, 2, 0)
+    try:
+        set_last_hop_mode(pkg, LAST_HOP_MODES[2])
+        pkg.set_rng_state(2, 0)
+        f, _, blocks = pkg.ChunkTensorSampler([10, 0], ip, ix).sample_blocks(None, torch.from_numpy(seeds))
+        assert np.array_equal(f.cpu().numpy(), want_f)
+        assert np.array_equal(blocks[0].src_local.cpu().numpy(), want[0][0])
+    finally:
+        set_last_hop_mode(pkg, LAST_HOP_MODES[0])

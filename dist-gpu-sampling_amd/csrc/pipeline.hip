@@ -1179,22 +1179,30 @@ __device__ __forceinline__ void announce_long_rows(const Hop& h, int64_t begin, 
 // launch that fits the grid cap has a block for each in the worst case; a launch that loops (STRIDE)
 // goes over the tiles the hop really has.
 //
-// Blocks from compact_blocks on, behind all that others wait for, write the previous hop's edge list where the fill had to
+// Blocks from LeftEdges::compact_blocks on, behind all that others wait for, write the previous hop's edge list where the fill had to
 // leave it (launch_fill): a launch of its own is 5 us at the floor, and this one, of two blocks a CU that wait for one another, has
 // the room.  111 M nodes, 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us, on another card 221.5 ->
-// 217.3.  (Their arguments come last: a launch without them reads none of those, 0.25 us.)
+// 217.3.  Launches that never have them are not given their arguments.
 constexpr bool takes_edges(int items, bool announce) { return items > 1 && !announce; }  // (fills that leave the list are not in front of the others)
+struct LeftEdges {
+  Hop prev;
+  int64_t relabel_count;    // virtual blocks of its list
+  uint32_t compact_blocks;
+};
+struct NoEdges {};
+template <int ITEMS, bool ANNOUNCE> using EdgesToo = std::conditional_t<takes_edges(ITEMS, ANNOUNCE), LeftEdges, NoEdges>;
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, bool ANNOUNCE>
-__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table, Hop prev,
-                                                            uint32_t compact_blocks, int64_t relabel_count) {
+__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table, EdgesToo<ITEMS, ANNOUNCE> also) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
   int64_t begin = 0, end = 0;
+  uint32_t blocks = gridDim.x;
   if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
-    if (blockIdx.x >= compact_blocks) {
+    blocks = also.compact_blocks;
+    if (blockIdx.x >= blocks) {
       constexpr int kPer = NT / kEdgeBlock;
-      for (int64_t vb = int64_t(blockIdx.x - compact_blocks) * kPer + threadIdx.x / kEdgeBlock; vb < relabel_count;
-           vb += int64_t(gridDim.x - compact_blocks) * kPer)
-        relabel_tile<IdT, TableT, false>(prev, table, vb, int(threadIdx.x % kEdgeBlock));
+      for (int64_t vb = int64_t(blockIdx.x - blocks) * kPer + threadIdx.x / kEdgeBlock; vb < also.relabel_count;
+           vb += int64_t(gridDim.x - blocks) * kPer)
+        relabel_tile<IdT, TableT, false>(also.prev, table, vb, int(threadIdx.x % kEdgeBlock));
       return;
     }
   }
@@ -1210,7 +1218,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
   const int64_t rows = s > 0 ? (s + NT * kRowItems - 1) / (NT * kRowItems) : 1;  // (tile 0 of either kind writes the lengths)
   const int64_t len = seed_part(h, s) + s * h.k;
   const int64_t total = rows + (len > 0 ? (len + kTile - 1) / kTile : 1);
-  for (int64_t vb = blockIdx.x; vb < total; vb += compact_blocks) {
+  for (int64_t vb = blockIdx.x; vb < total; vb += blocks) {
     begin = end = 0;
     if (vb < rows) offsets_tile<NT, false>(h, vb);
     else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table, &begin, &end);
@@ -1426,15 +1434,20 @@ template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool ANN
 void launch_compact_as(const Hop& hop, const Hop& prev, int64_t* left, const TableT& table, hipStream_t st) {
   const int64_t row_tiles = row_tiles_of(hop.s_max, hop.len_max);
   const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max), at_once = std::min(grid_cap(), kLookbackGrid);
-  int64_t relabel_count = 0;
-  if (takes_edges(ITEMS, ANNOUNCE)) std::swap(relabel_count, *left);
-  const uint32_t more = uint32_t(std::min((relabel_count + NT / kEdgeBlock - 1) / (NT / kEdgeBlock), kLoopGrid));
+  const uint32_t grid = uint32_t(std::min(blocks, at_once));
+  uint32_t more = 0;
+  EdgesToo<ITEMS, ANNOUNCE> also{};
+  if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
+    also = LeftEdges{prev, *left, grid};
+    more = uint32_t(std::min((*left + NT / kEdgeBlock - 1) / (NT / kEdgeBlock), kLoopGrid));
+    *left = 0;
+  }
   if (blocks > at_once)
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(uint32_t(at_once) + more),
-                       dim3(NT), 0, st, hop, row_tiles, table, prev, uint32_t(at_once), relabel_count);
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(grid + more), dim3(NT), 0, st, hop,
+                       row_tiles, table, also);
   else
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(uint32_t(blocks) + more), dim3(NT), 0, st,
-                       hop, row_tiles, table, prev, uint32_t(blocks), relabel_count);
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(grid + more), dim3(NT), 0, st, hop,
+                       row_tiles, table, also);
 }
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
 void launch_compact(const Hop& hop, const Hop& prev, int64_t* left, bool announce, const TableT& table, hipStream_t st) {

@@ -24,7 +24,7 @@
 // bucket = low bits of a hash that takes no two ids to one value, hashes are told apart in an open-addressing table of
 // packed words (hash, unit), items are the hash and the unit.  A bucket whose ids do not fit that table is gone over
 // again in parts, by other bits of the hash, one table's worth at a time; a part whose ids crowd it all the same (not by
-// chance) in as many ranges of hashes as there are tables' worths of them, each of which a table takes whatever the ids.
+// chance) in ranges of its hashes, each of which a table takes whatever the ids (in_parts).
 #ifndef DGS_CSRC_BUCKETS_H_
 #define DGS_CSRC_BUCKETS_H_
 
@@ -296,6 +296,28 @@ struct HashPart {
   int part, parts;
   uint32_t lo, span;
 };
+constexpr int kPartBit = 23, kPartValues = 1 << (32 - kPartBit);  // what the choice of a part looks at
+// Goes over a bucket of so many units in parts that fill half a table, were all units' ids different; a part that
+// `attempt` says its table has not taken, value by value of the bits that chose the part, in ranges of as many hashes as
+// a table has slots: no two ids have one hash, so each is taken whatever the ids are.  A sweep reads the
+// whole bucket, and there are no more than kPartValues for the parts and as many (256 buckets: twice as many) for the ranges.
+// 2 M ids that were made for one of 256 buckets: 244 + 226 sweeps.
+template <typename Attempt>
+__device__ __forceinline__ bool in_parts(int units, int slots, int log_buckets, Attempt attempt) {
+  const int half_tables = (units + slots / 2 - 1) / (slots / 2), parts = half_tables < kPartValues ? half_tables : kPartValues;
+  const uint32_t hashes = 1u << (kPartBit - log_buckets), span = hashes < uint32_t(kHashSlots) ? hashes : uint32_t(kHashSlots);  // of a value; of a range
+  bool took = true;
+  for (int part = 0; part < parts; ++part) {
+    bool fits = attempt(HashPart{part, parts, 0u, ~0u});
+    if (!fits && slots == kHashSlots) {
+      fits = true;
+      for (uint32_t value = part; value < uint32_t(kPartValues); value += parts)
+        for (uint32_t lo = value * hashes; lo < (value + 1) * hashes; lo += span) fits &= attempt(HashPart{part, parts, lo, span});
+    }
+    took &= fits;
+  }
+  return took;
+}
 // All units of the bucket, or (PARTS) of a part of it; returns whether the table took them (the same in all threads),
 // within max_probes probes each.
 template <bool PARTS>
@@ -305,7 +327,7 @@ __device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_b
   const int slots = b.hash_slots;
   const uint32_t mask = uint32_t(slots - 1);
   const auto elsewhere = [&](uint32_t hash) {
-    return PARTS && (int((hash >> 23) % uint32_t(part.parts)) != part.part || (hash >> log_buckets) - part.lo >= part.span);
+    return PARTS && (int((hash >> kPartBit) % uint32_t(part.parts)) != part.part || (hash >> log_buckets) - part.lo >= part.span);
   };
   PieceRound<true> round;
   round.load(b, log_buckets, bucket, 0, tiles);
@@ -366,17 +388,9 @@ __device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log
   }
   if (n > 0) atomicAdd(&lds.units, n);
   __syncthreads();
-  const int parts = (lds.units + b.hash_slots / 2 - 1) / (b.hash_slots / 2);  // that fill half of the table, were all units' ids different
-  bool took = true;
-  for (int part = 0; part < parts; ++part) {
-    bool fits = first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, HashPart{part, parts, 0u, ~0u}, b.hash_slots, lds);
-    if (!fits && b.hash_slots == kHashSlots) {
-      fits = true;
-      for (uint32_t lo = 0; lo < 1u << (32 - log_buckets); lo += kHashSlots)  // (no two ids have one hash)
-        fits &= first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, HashPart{part, parts, lo, uint32_t(kHashSlots)}, kHashSlots, lds);
-    }
-    took &= fits;
-  }
+  const bool took = in_parts(lds.units, b.hash_slots, log_buckets, [&](HashPart part) {
+    return first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, part, b.hash_slots, lds);
+  });
   if (threadIdx.x == 0 && !took) *b.overflow = 1;
 }
 

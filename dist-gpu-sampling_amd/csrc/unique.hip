@@ -665,18 +665,37 @@ struct UniqueWorkspace {
 // 1466 / 1171, but 4 M of them 353 / 625 and 1575 / 4650.
 constexpr int64_t kBucketedMinIds = int64_t(1) << 17;
 inline int64_t bucket_tiles(int64_t n) { return (n + kBucketTile - 1) / kBucketTile; }
-inline bool may_be_bucketed(int64_t n) { return n >= kBucketedMinIds && 2 * bucket_tiles(n) <= kMaxBucketTiles; }
+constexpr int64_t kBucketedMaxTiles = kMaxBucketTiles / 2;  // of mapping ids (as many of queries)
+inline bool may_be_bucketed(int64_t n) { return n >= kBucketedMinIds && bucket_tiles(n) <= kBucketedMaxTiles; }
 
 // packed 64-bit slots, or id array + value array (the larger: what the workspace is sized for)
 size_t slot_bytes(int32_t id_bytes, bool packed) { return packed ? 8 : size_t(id_bytes) + 4; }
 
+void take_buckets(Carver* c, int64_t map_tiles, UniqueWorkspace* t) {
+  Buckets& b = t->buckets;
+  b.hashed = 1;
+  b.hash_slots = kHashSlots;
+  b.tiles_max = int32_t(2 * map_tiles);
+  b.items = c->take<uint2>(size_t(b.tiles_max) * kBucketTile);
+  b.least = c->take<uint32_t>(size_t(b.tiles_max) * kBucketTile);
+  b.piece = c->take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
+  b.firsts = c->take<uint32_t>(kCounters * kMaxBucketTiles);
+  b.overflow = c->take<int>(4);
+  t->bad = c->take<uint32_t>(size_t(b.tiles_max));
+}
+
+// The slot words, then either the table with its marks or the buckets: an attempt uses one of them, and the one that follows a
+// void attempt comes behind it on the stream.  The size never falls as lists grow (a caller sizes one workspace for its longest
+// list): lists beyond those that go by buckets have the room of the longest one that does.
 size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWorkspace* w) {
   if (n < 0) n = 0;
   if (n > kMaxMappingIds) n = kMaxMappingIds;
   const size_t tiles = size_t(n > 0 ? rank_tiles(n) : 1);  // (an empty list has its counts written too)
   const size_t padded = tiles * size_t(kGroupIds) * rank_groups(n);
+  UniqueWorkspace t{};
   Carver c(base);
-  UniqueWorkspace t;
+  t.slot = c.take<uint32_t>(std::max(padded, may_be_bucketed(n) ? size_t(bucket_tiles(n)) * kBucketTile : 0));
+  Carver d = c;
   t.capacity = table_capacity(n);
   t.table_bytes = size_t(t.capacity) * slot_bytes(id_bytes, id_bytes == 4);
   t.table = c.take<char>(t.table_bytes);
@@ -684,25 +703,9 @@ size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWo
   t.lost = c.take<uint8_t>(t.zero_bytes);
   t.state = reinterpret_cast<tile_state*>(t.lost + padded);
   t.overflow = reinterpret_cast<int*>(t.state + tiles);
-  const size_t map_tiles = size_t(bucket_tiles(n));
-  const bool bucketed = may_be_bucketed(n);
-  t.slot = c.take<uint32_t>(std::max(padded, bucketed ? map_tiles * kBucketTile : 0));
-  t.buckets = Buckets{};
-  t.bad = nullptr;
-  if (bucketed) {
-    Buckets& b = t.buckets;
-    b.hashed = 1;
-    b.hash_slots = kHashSlots;
-    b.tiles_max = int32_t(2 * map_tiles);
-    b.items = c.take<uint2>(size_t(b.tiles_max) * kBucketTile);
-    b.least = c.take<uint32_t>(size_t(b.tiles_max) * kBucketTile);
-    b.piece = c.take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
-    b.firsts = c.take<uint32_t>(kCounters * kMaxBucketTiles);
-    b.overflow = c.take<int>(4);
-    t.bad = c.take<uint32_t>(size_t(b.tiles_max));
-  }
+  if (n >= kBucketedMinIds) take_buckets(&d, std::min(bucket_tiles(n), kBucketedMaxTiles), &t);
   if (w) *w = t;
-  return c.used + 256;
+  return std::max(c.used, d.used) + 256;
 }
 
 int64_t seg_total(const dgs_segments& s) {

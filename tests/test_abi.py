@@ -66,6 +66,19 @@ def test_workspace_queries_are_monotone():
     assert lib.dgs_split_index_workspace_bytes(0) > 0
 
 
+@pytest.mark.parametrize("id_bytes", [4, 8])
+def test_relabel_workspace_never_falls(id_bytes):
+    # one workspace sized for the longest list serves every shorter one; and lists that go by buckets take little more than
+    # the table and its marks do (1.4 to 2.8 slots of 8 or 12 bytes, 5 bytes), since an attempt uses one of them
+    lib = load_pkg().capi.lib
+    marks = {1024, 2048, 131_072, 139_264, 1 << 20, 1 << 22, (1 << 22) + 8192, 5_991_862, 1 << 23, 1 << 24}
+    marks |= {n for e in range(11, 25) for n in (int((1 << e) / 1.4),)} | set(range(0, 1 << 23, 65_521))
+    sizes = [(n, lib.dgs_unique_relabel_workspace_bytes(n, id_bytes)) for n in sorted({m + d for m in marks for d in (-1, 0, 1) if m + d >= 0})]
+    for (n, size), (more, larger) in zip(sizes, sizes[1:]):
+        assert size <= larger, (n, more)
+    assert all(size <= max(30 * n, 6 * n + 2.9 * n * (8 if id_bytes == 4 else 12)) + 200_000 for n, size in sizes)
+
+
 def test_operator_surface_is_registered():
     import torch
     load_pkg()

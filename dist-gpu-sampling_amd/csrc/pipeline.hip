@@ -201,14 +201,11 @@ constexpr int kFoldMaxRowPerPick = 4;
 constexpr int64_t kBucketedMinNodes = 262144, kBucketedMaxNodes = 16777216;
 constexpr int64_t kBucketedMinPicks = 917504;
 static_assert(kBucketedMaxNodes <= kDirectMaxIds, "the direct form takes them");
-// Larger graphs take the hashed form, which pays for draws with replacement of a very large hop: without it many of the
-// positions are empty, which the pass goes over all the same (111 M nodes, 0.94 M picks in 2.8 M positions: 215 us a batch
-// on the table, 216 by the pass).  us a batch of draws, 64-byte rows, table / pass: 20 M nodes, fanouts [10,20] from
-// 4096 seeds (0.9 M picks at most) 78 / 88, [10,40] (1.8 M) 82 / 94, [5,10,15] (4.1 M) 180 / 172, [10,25] from 16 384 (4.5 M)
-// 193 / 188; 60 M nodes 77 / 88, 84 / 94, 189 / 173, 200 / 193; 8 batches of [5,10,15] through the loader 1295 / 1188;
-// R-MAT of 2^26 nodes, [50,50] from 16 384 (41.8 M, 3.05 M in fact, two thirds of them repeats) 372 / 354: fill 149 -> 76,
-// sort 14.4, first 35.
-constexpr int64_t kHashedMinPicks = int64_t(3) << 20;
+// Larger graphs stay on the table: the hashed form (test hook) goes over every position, with a pick or without, and a
+// hub's draws are one block's work.  us a batch of draws, 64-byte rows, table / hashed pass: 20 M nodes of 15 neighbours,
+// fanouts [5,10,15] from 4096 seeds 225 / 212, with a node that 5 % of the edges lead to 306 / 371, 50 % 205 / 480; 60 M
+// nodes, [50,50] from 8192 316 / 383; R-MAT of 2^26 nodes, [50,50] from 16 384 368 / 356.  Nothing that the host knows tells
+// the last one from the others.  Without replacement, 111 M nodes, 0.94 M picks in 2.8 M positions: 215 / 216.
 __host__ __device__ __forceinline__ int64_t front_units(int64_t s) { return (s + 15) / 16 * 16; }
 
 // rank of the id at position p of hop 0, given p's slot word
@@ -1290,7 +1287,7 @@ inline void plan_bucket_tiles(Plan* p) {
 }
 
 dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, int32_t id_bytes,
-                     int64_t n_nodes, bool have_node_table, bool replace, Plan* p) {
+                     int64_t n_nodes, bool have_node_table, Plan* p) {
   DGS_REQUIRE(n_hops >= 1 && n_hops <= DGS_MAX_HOPS, DGS_ERR_INVALID, "sample_blocks: %d hops (1..%d)", n_hops,
               DGS_MAX_HOPS);
   DGS_REQUIRE(fanouts != nullptr && n_seeds >= 0, DGS_ERR_INVALID, "sample_blocks: bad argument");
@@ -1318,7 +1315,7 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
     const int64_t mode = debug_option(DGS_DEBUG_SAMPLER_BUCKETED);
     const int64_t picks = p->nnz_max[n_hops - 1];
     p->bucket_hashed = n_nodes > kBucketedMaxNodes || mode == 3 || mode == 4;
-    const bool large = p->bucket_hashed ? replace && picks >= kHashedMinPicks : picks >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
+    const bool large = !p->bucket_hashed && picks >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
     p->bucketed = p->bucket_space && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
                   (large || mode >= 2);
     p->hash_slots = mode == 4 ? 256 : kHashSlots;
@@ -1669,7 +1666,7 @@ dgs_status run_blocks_table(const Plan& p, Hop* hops, const Buckets& buckets, vo
 DGS_API dgs_status dgs_sample_blocks_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops,
                                           int64_t* seeds_max, int64_t* edges_max) {
   dgs::Plan p;
-  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, false, false, &p);
+  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, false, &p);
   if (s != DGS_OK) return s;
   DGS_REQUIRE(seeds_max && edges_max, DGS_ERR_INVALID, "sample_blocks_plan: null output");
   for (int h = 0; h <= n_hops; ++h) seeds_max[h] = p.s_max[h];
@@ -1681,7 +1678,7 @@ DGS_API size_t dgs_sample_blocks_workspace_bytes(int64_t n_seeds, const int64_t*
                                                  int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   return dgs::layout(p, fanouts, nullptr, nullptr, nullptr);
@@ -1695,7 +1692,7 @@ DGS_API size_t dgs_sample_blocks_weighted_workspace_bytes(int64_t n_seeds, const
                                                           int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts (used when there is no node table)
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   p.weighted = true;
@@ -1712,7 +1709,7 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
   using namespace dgs;
   Plan p;
   // node count = indptr entries - 1
-  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, node_table != nullptr, replace != 0, &p);
+  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, node_table != nullptr, &p);
   if (s != DGS_OK) return s;
   if (probs != nullptr) {
     DGS_REQUIRE(probs->elem_bytes == 4 && probs->total == indices.total, DGS_ERR_INVALID,

@@ -1176,24 +1176,26 @@ __device__ __forceinline__ void announce_long_rows(const Hop& h, int64_t begin, 
 // launch that fits the grid cap has a block for each in the worst case; a launch that loops (STRIDE)
 // goes over the tiles the hop really has.
 //
-// Blocks from LeftEdges::compact_blocks on, behind all that others wait for, write the previous hop's edge list where the fill had to
-// leave it (launch_fill): a launch of its own is 5 us at the floor, and this one, of two blocks a CU that wait for one another, has
-// the room.  111 M nodes, 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us, on another card 221.5 ->
-// 217.3.  Launches that never have them are not given their arguments.
-constexpr bool takes_edges(int items, bool announce) { return items > 1 && !announce; }  // (fills that leave the list are not in front of the others)
+// What else the launch may do (ALSO): queue the long rows among those it appends; or write the previous hop's edge list, in blocks
+// from LeftEdges::compact_blocks on, behind all that others wait for, where the fill had to leave it (launch_fill): a launch of
+// its own is 5 us at the floor, and this one, of two blocks a CU that wait for one another, has the room.  111 M nodes,
+// 4096 seeds, fanouts [5,10,15], a batch with its features: 217.5 -> 210.4 us, on two other cards 221.5 -> 217.3, 219.8 -> 218.1.
+// Launches that do neither are kernels of their own, of 4 registers less: a weighted batch of 1024 seeds, [5,10,15], with its features
+// 265.3 -> 262.7 us.
+enum CompactAlso { kNothing, kLongRows, kEdgeList };
 struct LeftEdges {
   Hop prev;
   int64_t relabel_count;    // virtual blocks of its list
   uint32_t compact_blocks;
 };
 struct NoEdges {};
-template <int ITEMS, bool ANNOUNCE> using EdgesToo = std::conditional_t<takes_edges(ITEMS, ANNOUNCE), LeftEdges, NoEdges>;
-template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, bool ANNOUNCE>
-__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table, EdgesToo<ITEMS, ANNOUNCE> also) {
+template <CompactAlso ALSO> using EdgesToo = std::conditional_t<ALSO == kEdgeList, LeftEdges, NoEdges>;
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool STRIDE, CompactAlso ALSO>
+__global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_tiles, TableT table, EdgesToo<ALSO> also) {
   constexpr int64_t kTile = int64_t(NT) * ITEMS * GROUPS;
   int64_t begin = 0, end = 0;
   uint32_t blocks = gridDim.x;
-  if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
+  if constexpr (ALSO == kEdgeList) {
     blocks = also.compact_blocks;
     if (blockIdx.x >= blocks) {
       constexpr int kPer = NT / kEdgeBlock;
@@ -1208,7 +1210,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
     const int64_t vb = blockIdx.x;
     if (vb < row_tiles) offsets_tile<NT, true>(h, vb);
     else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, true>(h, vb - row_tiles, table, &begin, &end);
-    if (ANNOUNCE) announce_long_rows<IdT, NT>(h, begin, end);
+    if (ALSO == kLongRows) announce_long_rows<IdT, NT>(h, begin, end);
     return;
   }
   const int64_t s = seeds_of(h);
@@ -1219,7 +1221,7 @@ __global__ __launch_bounds__(NT, 4) void hop_compact_kernel(Hop h, int64_t row_t
     begin = end = 0;
     if (vb < rows) offsets_tile<NT, false>(h, vb);
     else compact_tile<IdT, TableT, NT, ITEMS, GROUPS, false>(h, vb - rows, table, &begin, &end);
-    if (ANNOUNCE) announce_long_rows<IdT, NT>(h, begin, end);
+    if (ALSO == kLongRows) announce_long_rows<IdT, NT>(h, begin, end);
     __syncthreads();  // the tiles' LDS is rewritten by the block's next one
   }
 }
@@ -1427,29 +1429,32 @@ void launch_relabel(const Hop& hop, const TableT& table, hipStream_t st) {
 }
 
 // `left`: blocks of the previous hop's edge list that are to be written too; set to 0 where the launch takes them.
-template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, bool ANNOUNCE>
+template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS, CompactAlso ALSO>
 void launch_compact_as(const Hop& hop, const Hop& prev, int64_t* left, const TableT& table, hipStream_t st) {
   const int64_t row_tiles = row_tiles_of(hop.s_max, hop.len_max);
   const int64_t blocks = row_tiles + pos_tiles_of(hop.len_max), at_once = std::min(grid_cap(), kLookbackGrid);
   const uint32_t grid = uint32_t(std::min(blocks, at_once));
   uint32_t more = 0;
-  EdgesToo<ITEMS, ANNOUNCE> also{};
-  if constexpr (takes_edges(ITEMS, ANNOUNCE)) {
+  EdgesToo<ALSO> also{};
+  if constexpr (ALSO == kEdgeList) {
     also = LeftEdges{prev, *left, grid};
     more = uint32_t(std::min((*left + NT / kEdgeBlock - 1) / (NT / kEdgeBlock), kLoopGrid));
     *left = 0;
   }
   if (blocks > at_once)
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ANNOUNCE>), dim3(grid + more), dim3(NT), 0, st, hop,
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, true, ALSO>), dim3(grid + more), dim3(NT), 0, st, hop,
                        row_tiles, table, also);
   else
-    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ANNOUNCE>), dim3(grid + more), dim3(NT), 0, st, hop,
+    hipLaunchKernelGGL((hop_compact_kernel<IdT, TableT, NT, ITEMS, GROUPS, false, ALSO>), dim3(grid + more), dim3(NT), 0, st, hop,
                        row_tiles, table, also);
 }
 template <typename IdT, typename TableT, int NT, int ITEMS, int GROUPS>
 void launch_compact(const Hop& hop, const Hop& prev, int64_t* left, bool announce, const TableT& table, hipStream_t st) {
-  if (announce) launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, true>(hop, prev, left, table, st);
-  else launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, false>(hop, prev, left, table, st);
+  if (announce) return launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, kLongRows>(hop, prev, left, table, st);
+  if constexpr (ITEMS > 1) {  // (fills that leave the list are not in front of the others)
+    if (*left > 0) return launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, kEdgeList>(hop, prev, left, table, st);
+  }
+  launch_compact_as<IdT, TableT, NT, ITEMS, GROUPS, kNothing>(hop, prev, left, table, st);
 }
 
 // The bucketed pass and the compact launch behind it.

@@ -198,8 +198,15 @@ constexpr int kFoldMaxRowPerPick = 4;
 // 100 and 112 / 122, 250 k 106 / 103 and 133 / 135, 500 k 115 / 103 and 157 / 140.  8 batches through the loader,
 // 400-byte rows, 2.4 M nodes: 512 seeds 737 / 772, 768 823 / 842, 1024 995 / 971, 2048 1679 / 1570; 20 M nodes,
 // 64-byte rows, 1024 seeds 675 / 690.
+// That is for graphs whose rows leave many of the positions empty, which the pass goes over all the same.  Where the mean degree is
+// twice the fanout it pays earlier, the more so the wider the rows that are gathered behind it or beside it.  The same, table / the
+// pass before it had tiles of 8192 units / pass: 2.4 M nodes of 50 neighbours, 400-byte rows, a batch of 640 seeds
+// 136 / 140 / 133, 704 (0.7 M) 145 / 147 / 139, 896 181 / 180 / 168, 8 through the loader 1033 / 1024 / 1010, 1065 / 1066 /
+// 1065, 1262 / 1233 / 1221; 512-byte rows, 704 seeds 156 / 157 / 146 and 1169 / 1098 / 1107; 64-byte rows 101 / 107 / 101;
+// 8 M nodes of 50 neighbours, 256-byte rows, 704 122 / 127 / 117; 35 neighbours, 400-byte rows, 704 128 / 134 / 127; 25 108 / 117 / 111,
+// 896 123 / 131 / 125; 16 M nodes of 19, 64-byte rows, 704 91 / 109 / 104; draws, 50 neighbours, 704 115 / 123 / 114.
 constexpr int64_t kBucketedMinNodes = 262144, kBucketedMaxNodes = 16777216;
-constexpr int64_t kBucketedMinPicks = 917504;
+constexpr int64_t kBucketedMinPicks = 917504, kBucketedMinPicksFull = 655360;
 static_assert(kBucketedMaxNodes <= kDirectMaxIds, "the direct form takes them");
 // Larger graphs stay on the table: the hashed form (test hook) goes over every position, with a pick or without, and a
 // hub's draws are one block's work.  us a batch of draws, 64-byte rows, table / hashed pass: 20 M nodes of 15 neighbours,
@@ -1289,7 +1296,7 @@ inline void plan_bucket_tiles(Plan* p) {
 }
 
 dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, int32_t id_bytes,
-                     int64_t n_nodes, bool have_node_table, Plan* p) {
+                     int64_t n_nodes, int64_t n_edges, bool have_node_table, Plan* p) {
   DGS_REQUIRE(n_hops >= 1 && n_hops <= DGS_MAX_HOPS, DGS_ERR_INVALID, "sample_blocks: %d hops (1..%d)", n_hops,
               DGS_MAX_HOPS);
   DGS_REQUIRE(fanouts != nullptr && n_seeds >= 0, DGS_ERR_INVALID, "sample_blocks: bad argument");
@@ -1317,7 +1324,8 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
     const int64_t mode = debug_option(DGS_DEBUG_SAMPLER_BUCKETED);
     const int64_t picks = p->nnz_max[n_hops - 1];
     p->bucket_hashed = n_nodes > kBucketedMaxNodes || mode == 3 || mode == 4;
-    const bool large = !p->bucket_hashed && picks >= kBucketedMinPicks && n_nodes >= kBucketedMinNodes;
+    const bool full = n_edges / 2 >= n_nodes * fanouts[n_hops - 1];  // (the rows' positions, as a rule)
+    const bool large = !p->bucket_hashed && picks >= (full ? kBucketedMinPicksFull : kBucketedMinPicks) && n_nodes >= kBucketedMinNodes;
     p->bucketed = p->bucket_space && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
                   (large || mode >= 2);
     p->hash_slots = mode == 4 ? 256 : kHashSlots;
@@ -1671,7 +1679,7 @@ dgs_status run_blocks_table(const Plan& p, Hop* hops, const Buckets& buckets, vo
 DGS_API dgs_status dgs_sample_blocks_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops,
                                           int64_t* seeds_max, int64_t* edges_max) {
   dgs::Plan p;
-  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, false, &p);
+  dgs_status s = dgs::make_plan(n_seeds, fanouts, n_hops, 8, -1, -1, false, &p);
   if (s != DGS_OK) return s;
   DGS_REQUIRE(seeds_max && edges_max, DGS_ERR_INVALID, "sample_blocks_plan: null output");
   for (int h = 0; h <= n_hops; ++h) seeds_max[h] = p.s_max[h];
@@ -1683,7 +1691,7 @@ DGS_API size_t dgs_sample_blocks_workspace_bytes(int64_t n_seeds, const int64_t*
                                                  int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, -1, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   return dgs::layout(p, fanouts, nullptr, nullptr, nullptr);
@@ -1697,7 +1705,7 @@ DGS_API size_t dgs_sample_blocks_weighted_workspace_bytes(int64_t n_seeds, const
                                                           int32_t id_bytes) {
   dgs::Plan p;
   // sized for the split hash table, the largest of the layouts (used when there is no node table)
-  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, false, &p) != DGS_OK) return 0;
+  if (dgs::make_plan(n_seeds, fanouts, n_hops, id_bytes, -1, -1, false, &p) != DGS_OK) return 0;
   p.kind = dgs::TableKind::kSplit;
   p.table_bytes = size_t(p.capacity) * (size_t(id_bytes) + 4);
   p.weighted = true;
@@ -1714,7 +1722,7 @@ dgs_status sample_blocks_entry(const void* seeds, int32_t id_bytes, int64_t n_se
   using namespace dgs;
   Plan p;
   // node count = indptr entries - 1
-  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, node_table != nullptr, &p);
+  dgs_status s = make_plan(n_seeds, fanouts, n_hops, id_bytes, indptr.total - 1, indices.total, node_table != nullptr, &p);
   if (s != DGS_OK) return s;
   if (probs != nullptr) {
     DGS_REQUIRE(probs->elem_bytes == 4 && probs->total == indices.total, DGS_ERR_INVALID,

@@ -47,6 +47,27 @@ def test_bucketed_pass_at_its_edges(pkg, oracle, mode, id_dtype, nodes, seeds, k
         set_last_hop_mode(pkg, LAST_HOP_MODES[0])
 
 
+@pytest.mark.parametrize("nodes,degree,seeds", [
+    (262_144, 30, 700),  # 0.69 M picks at most, and rows that fill their positions: the pass
+    (262_144, 29, 700),  # the table
+    (262_143, 30, 700),  # the table
+    (262_144, 12, 930),  # 0.92 M picks at most: the pass
+])
+def test_last_hop_by_size(pkg, oracle, nodes, degree, seeds):
+    rng = np.random.default_rng(nodes + degree)
+    indptr = np.arange(nodes + 1, dtype=np.int64) * degree
+    indices = rng.integers(0, nodes, size=nodes * degree).astype(np.int32)
+    start = rng.permutation(nodes)[:seeds].astype(np.int32)
+    ip = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    want_f, _, want = oracle.sample_blocks(start, indptr, indices, [15, 10, 5], False, 4, 0)
+    pkg.set_rng_state(4, 0)
+    f, _, blocks = pkg.ChunkTensorSampler([15, 10, 5], ip, ix).sample_blocks(None, torch.from_numpy(start))
+    assert np.array_equal(f.cpu().numpy(), want_f)
+    for g, w in zip(blocks, want):
+        assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+
+
 def _dev(x):
     return torch.from_numpy(np.ascontiguousarray(x)).cuda()
 

@@ -41,12 +41,13 @@ constexpr int kBucketTile = kBucketBlock * kBucketItems;
 constexpr int kLocalBits = 13;
 static_assert(1 << kLocalBits == kBucketTile, "a unit's place in its tile");
 constexpr int kMaxBucketTiles = 8388608 / kBucketTile;  // 8.4 M units
-constexpr int kMinLogBuckets = 8, kMaxLogBuckets = 11;
+constexpr int kMinLogBuckets = 8, kMaxLogBuckets = 10;
 constexpr int kMaxBuckets = 1 << kMaxLogBuckets;
 constexpr int kBucketRange = 16384;                  // direct: ids per bucket at most, 64 KB of LDS
 constexpr int64_t kDirectMaxIds = int64_t(kMaxBuckets) * kBucketRange;
-constexpr int kFewProbes = 64;                       // ... of which an id sees this many at first
 constexpr int kHashSlots = 16384;                    // hashed: entries of a bucket's table, 128 KB of LDS
+constexpr int kFewProbes = 64;                       // ... of which an id sees this many at first
+static_assert(int64_t(kHashSlots / 2) * kMaxBuckets >= int64_t(kMaxBucketTiles) * kBucketTile, "half full, were all units' ids different");
 
 // A tile's first occurrences are counted by the blocks of all buckets, each of which adds its counts of all tiles with a
 // few atomics of whole lines (one for every piece took 44 us); several counters, so that few blocks meet at one.  The

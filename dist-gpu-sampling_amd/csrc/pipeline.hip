@@ -188,7 +188,8 @@ constexpr int kFoldMaxRowPerPick = 4;
 // (a first occurrence), that of an id the frontier held before this hop (its rank | kRankBit: final, no further
 // lookup), or that of an earlier pick of this hop (whose position becomes the slot word, and whose rank
 // the compaction records there).  A draw that repeats another one of its row is no unit: its slot word is that
-// draw's position from the fill on, where it finds a rank, or the link to one.  Same result as the table gives.
+// draw's position from the fill on, where it finds a rank, or the link to one; nor is a pick of an id that its tile holds again and
+// again (sort_tile), whose slot word becomes the first one's position or rank.  Same result as the table gives.
 //
 // It takes two launches more than the table does, and pays where the hop is large (by its worst case: that is what the
 // host knows) and the table beyond the caches.  us a batch with rows of 64 bytes, table / pass: 2.4 M nodes, fanouts
@@ -874,7 +875,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Bucket
   if (!bucketed_now(h, s)) return;  // the hop outgrew the pass: it runs on the table
   const uint32_t front = uint32_t(front_units(s)), units = front + uint32_t(s * h.k);
   const int log_buckets = log_buckets_of(b, units);
-  const uint32_t* slot = h.slot + h.pos_base;
+  uint32_t* slot = h.slot + h.pos_base;
   for (uint32_t tile = blockIdx.x; tile * kBucketTile < units; tile += gridDim.x) {
     uint32_t id[kBucketItems];
 #pragma unroll
@@ -893,7 +894,10 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Bucket
     for (int j = 0; j < kBucketItems; ++j)  // (a position's word: a draw that repeats one of its own row's, no unit)
       if (id[j] != kNoId) id[j] = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x < front ? id[j]
                                 : (id[j] & kFirstBit) != 0 ? id[j] & ~kFirstBit : kNoId;
-    sort_tile<HASHED>(b, log_buckets, tile, id, lds);
+    sort_tile<HASHED>(b, log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // (a pick: frontier ids are different ones)
+      const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x, met = tile * kBucketTile + before;
+      if (u >= front) nth(slot, u - front) = met < front ? met | kRankBit : uint32_t(h.pos_base) + (met - front);
+    });
     __syncthreads();  // lds is rewritten by the block's next tile
   }
 }
@@ -1153,6 +1157,8 @@ __device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets&
         const uint32_t p = uint32_t(h.pos_base) + (met - front);
         word[g][j] = met < front ? met | kRankBit : p;
         ranks[j] = met < front ? met : p | kLinkBit;  // for the draws of the row that repeat this one
+      } else if (word[g][j] != kInvalidSlot) {  // no unit: the same, where the sort has folded it
+        ranks[j] = (word[g][j] & kRankBit) != 0 ? word[g][j] & (kRankBit - 1) : word[g][j] | kLinkBit;
       }
     }
     nth(reinterpret_cast<words*>(h.rank_at + h.pos_base), (u - front) / ITEMS) = ranks;

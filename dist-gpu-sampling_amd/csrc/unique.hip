@@ -289,15 +289,29 @@ struct TileSpan {
   __device__ __forceinline__ T& at(const dgs_segments& s, uint32_t e) const { return whole ? nth(begin, e) : *seg_at<T>(s, first + e); }
 };
 
-// The mapping ids that the table would hold as well; a tile that has met another one says so in bad[].
+// Units that sort_tile has folded: (place of the one before it that it is equal to, its own place) each, from the end of the tile's
+// items downwards, which that many units less leave free.
+using Item = BucketItem<true>::type;
+__device__ __forceinline__ Item* folded_items(const Buckets& b, uint32_t tile) {
+  return static_cast<Item*>(b.items) + (size_t(tile) + 1) * kBucketTile - 1;
+}
+__device__ __forceinline__ void unfold_tile(const Buckets& b, uint32_t tile, uint32_t folds, uint32_t* into /* [kBucketTile] in LDS */) {
+  for (uint32_t e = threadIdx.x; e < folds && e < uint32_t(kBucketTile); e += kBucketBlock) {
+    const Item it = folded_items(b, tile)[-int64_t(e)];
+    into[it.y & (kBucketTile - 1)] = into[it.x & (kBucketTile - 1)];
+  }
+  __syncthreads();
+}
+
+// The mapping ids that the table would hold as well.  notes[]: 1 if the tile has met another one, and twice its folded units.
 template <typename IdT>
 __global__ __launch_bounds__(kBucketBlock) void bucketed_sort_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, dgs_segments queries,
-                                                                     int64_t m, Buckets b, uint32_t* __restrict__ bad) {
+                                                                     int64_t m, Buckets b, uint32_t* __restrict__ notes) {
   __shared__ SortLds<true> lds;
-  __shared__ uint32_t any_bad;
+  __shared__ uint32_t any_bad, folds;
   const uint32_t tile = blockIdx.x;
   if (tile == 0 && threadIdx.x == 0) *b.overflow = 0;  // (the per-bucket launch comes behind this one)
-  if (threadIdx.x == 0) any_bad = 0;
+  if (threadIdx.x == 0) any_bad = folds = 0;
   __syncthreads();
   const bool query = tile >= map_tiles;
   IdT key[kBucketItems], front[kBucketItems];  // (front: of a wave's first lane, the query in front of its own)
@@ -329,8 +343,15 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_sort_kernel(dgs_segment
     id[j] = e < count && held && !again ? uint32_t(key[j]) : kNoId;
   }
   if (refused) any_bad = 1;
-  sort_tile<true>(b, b.log_buckets, tile, id, lds);
-  if (threadIdx.x == 0) bad[tile] = any_bad;  // (sort_tile has barriers)
+  sort_tile<true>(b, b.log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // noted from the end of the tile's items on
+    const uint64_t here = __ballot(1);
+    const int lower = __builtin_popcountll(here & ((uint64_t(1) << (threadIdx.x & (kWave - 1))) - 1));
+    uint32_t at = 0;
+    if (lower == 0) at = atomicAdd(&folds, uint32_t(__builtin_popcountll(here)));
+    at = __builtin_amdgcn_readfirstlane(at) + uint32_t(lower);
+    folded_items(b, tile)[-int64_t(at)] = Item{before, uint32_t(j * kBucketBlock) + threadIdx.x};
+  });
+  if (threadIdx.x == 0) notes[tile] = any_bad | folds << 1;  // (sort_tile has barriers)
 }
 
 __global__ __launch_bounds__(kBucketBlock) void bucketed_first_kernel(Buckets b, uint32_t tiles) {
@@ -343,7 +364,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_first_kernel(Buckets b,
 // rank_kernel's work on one tile of the mapping list.
 template <typename IdT>
 __global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, Buckets b,
-                                                                     const uint32_t* __restrict__ bad, uint32_t* __restrict__ slot,
+                                                                     const uint32_t* __restrict__ notes, uint32_t* __restrict__ slot,
                                                                      IdT* __restrict__ unique_out, int64_t* __restrict__ counts_dev,
                                                                      int64_t* __restrict__ counts_host) {
   typedef uint32_t words __attribute__((ext_vector_type(kItems)));
@@ -359,7 +380,8 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segment
   const TileSpan<const IdT> span(mapping, tile, n);
   uint32_t before = firsts_before(b, tile);
   uint32_t refused = last && threadIdx.x == 0 ? uint32_t(*b.overflow) : 0u;
-  for (uint32_t t = threadIdx.x; last && t < map_tiles; t += kBucketBlock) refused |= bad[t];
+  for (uint32_t t = threadIdx.x; last && t < map_tiles; t += kBucketBlock) refused |= notes[t] & 1;
+  const uint32_t folds = notes[tile] >> 1;
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) *reinterpret_cast<words*>(least_of + g * kGroup + at) = words(kAbsent);  // (ids that are no units)
   if (threadIdx.x == 0) any_bad = 0;
@@ -370,6 +392,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segment
   for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d, kWave);
   if (lane == 0) wave_before[wave] = before;
   __syncthreads();
+  if (folds != 0) unfold_tile(b, tile, folds, least_of);
   words word[kGroups];
   uint32_t first[kGroups];  // bit j: position j of the group's is its id's first
   int lane_before[kGroups];
@@ -435,7 +458,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segment
 // then blocks of kBucketTile requiring ids that are mapping ids, given by their words.
 template <typename IdT>
 __global__ __launch_bounds__(kBucketBlock) void bucketed_lookup_kernel(dgs_segments queries, int64_t m, uint32_t map_tiles, uint32_t query_tiles,
-                                                                       Buckets b, const uint32_t* __restrict__ bad,
+                                                                       Buckets b, const uint32_t* __restrict__ notes,
                                                                        const uint32_t* __restrict__ slot, int64_t n, dgs_segments query_out,
                                                                        dgs_segments words, int64_t n_words, dgs_segments words_out) {
   __shared__ uint32_t least_of[kBucketTile];
@@ -463,11 +486,13 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_lookup_kernel(dgs_segme
   const uint32_t tile = map_tiles + blockIdx.x;
   const TileSpan<IdT> to(query_out, blockIdx.x, m);
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const bool odd_ones = bad[tile] != 0;
+  const bool odd_ones = (notes[tile] & 1) != 0;
+  const uint32_t folds = notes[tile] >> 1;
   for (int e = threadIdx.x; e < kBucketTile; e += kBucketBlock) least_of[e] = kAbsent;
   __syncthreads();
   unsort_tile<true>(b, b.log_buckets, tile, least_of);
   __syncthreads();
+  if (folds != 0) unfold_tile(b, tile, folds, least_of);
   // a thread has eight ids in a row: where the last run begins that does so before or at each
   int own[kBucketItems], latest = -1;
 #pragma unroll
@@ -651,7 +676,7 @@ struct UniqueWorkspace {
   int* overflow;
   uint32_t* slot;    // [padded to whole rank tiles, and bucket tiles]
   Buckets buckets;   // of lists that may be bucketed: room for the mapping ids and as many queries
-  uint32_t* bad;     // [bucket tiles]
+  uint32_t* notes;   // [bucket tiles]
   uint32_t capacity;
   size_t table_bytes;  // multiple of 16 (sized for the larger layout)
   size_t zero_bytes;   // multiple of 16
@@ -681,7 +706,7 @@ void take_buckets(Carver* c, int64_t map_tiles, UniqueWorkspace* t) {
   b.piece = c->take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
   b.firsts = c->take<uint32_t>(kCounters * kMaxBucketTiles);
   b.overflow = c->take<int>(4);
-  t->bad = c->take<uint32_t>(size_t(b.tiles_max));
+  t->notes = c->take<uint32_t>(size_t(b.tiles_max));
 }
 
 // The slot words, then either the table with its marks or the buckets: an attempt uses one of them, and the one that follows a
@@ -789,11 +814,11 @@ dgs_status run_bucketed_relabel(const dgs_segments& mapping, int64_t n, const Sp
   Buckets b = w.buckets;
   b.log_buckets = kMinLogBuckets;
   while (b.log_buckets < kMaxLogBuckets && (int64_t(kHashSlots / 2) << b.log_buckets) < n + m) ++b.log_buckets;
-  hipLaunchKernelGGL(bucketed_sort_kernel<IdT>, dim3(tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, r.queries, m, b, w.bad);
+  hipLaunchKernelGGL(bucketed_sort_kernel<IdT>, dim3(tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, r.queries, m, b, w.notes);
   DGS_LAUNCH_CHECK();
   hipLaunchKernelGGL(bucketed_first_kernel, dim3(1u << b.log_buckets), dim3(kBucketBlock), 0, st, b, tiles);
   DGS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bucketed_rank_kernel<IdT>, dim3(map_tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, b, w.bad, w.slot,
+  hipLaunchKernelGGL(bucketed_rank_kernel<IdT>, dim3(map_tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, b, w.notes, w.slot,
                      static_cast<IdT*>(unique_out), counts_dev, counts_host);
   DGS_LAUNCH_CHECK();
   // the counts are final here: mark the point the caller may wait for
@@ -804,7 +829,7 @@ dgs_status run_bucketed_relabel(const dgs_segments& mapping, int64_t n, const Sp
   const uint32_t blocks = query_tiles + uint32_t(bucket_tiles(n_words));
   if (blocks > 0)
     hipLaunchKernelGGL(bucketed_lookup_kernel<IdT>, dim3(blocks), dim3(kBucketBlock), 0, st, r.queries, m, map_tiles, query_tiles, b,
-                       w.bad, w.slot, n, r.query_out, r.words, n_words, r.words_out);
+                       w.notes, w.slot, n, r.query_out, r.words, n_words, r.words_out);
   DGS_LAUNCH_CHECK();
   return DGS_OK;
 }

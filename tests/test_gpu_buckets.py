@@ -47,6 +47,36 @@ def test_bucketed_pass_at_its_edges(pkg, oracle, mode, id_dtype, nodes, seeds, k
         set_last_hop_mode(pkg, LAST_HOP_MODES[0])
 
 
+@pytest.mark.parametrize("mode", LAST_HOP_MODES[1:4])
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("hubs,share", [(1, 0.03), (1, 0.5), (12, 0.7), (1, 1.0)])
+def test_bucketed_pass_with_hubs(pkg, oracle, mode, replace, hubs, share):
+    # ids that come up again and again in a tile, in rows of their own and of others, among the seeds (the even ones of them)
+    # and not: the sort hands on the first of each
+    rng = np.random.default_rng(hubs * 100 + int(share * 10))
+    n = 50_000
+    indptr, indices = powerlaw_graph(rng, n, 25, 400, id_dtype=np.int32)
+    hub = rng.permutation(n)[:hubs].astype(np.int32)
+    at = rng.random(indices.size) < share
+    indices[at] = rng.choice(hub, size=int(at.sum()))
+    start = rng.permutation(np.setdiff1d(np.arange(n, dtype=np.int32), hub[1::2]))[:4000].astype(np.int32)
+    start[-len(hub[::2]):] = hub[::2]
+    start = start[np.sort(np.unique(start, return_index=True)[1])]
+    ip = pkg.create_chunktensor(torch.from_numpy(indptr), 1, 1 << 40)
+    ix = pkg.create_chunktensor(torch.from_numpy(indices), 1, 1 << 40)
+    for fanouts in ([15, 0], [12, 4]):
+        want_f, _, want = oracle.sample_blocks(start, indptr, indices, fanouts, replace, 3, 0)
+        try:
+            set_last_hop_mode(pkg, mode)
+            pkg.set_rng_state(3, 0)
+            f, _, blocks = pkg.ChunkTensorSampler(fanouts, ip, ix, replace=replace).sample_blocks(None, torch.from_numpy(start))
+            assert np.array_equal(f.cpu().numpy(), want_f)
+            for g, w in zip(blocks, want):
+                assert np.array_equal(g.src_local.cpu().numpy(), w[0]) and np.array_equal(g.dst_local.cpu().numpy(), w[1])
+        finally:
+            set_last_hop_mode(pkg, LAST_HOP_MODES[0])
+
+
 @pytest.mark.parametrize("nodes,degree,seeds", [
     (262_144, 30, 700),  # 0.69 M picks at most, and rows that fill their positions: the pass
     (262_144, 29, 700),  # the table
@@ -95,6 +125,40 @@ def test_relabel_of_long_lists(pkg, oracle, dtype, n, distinct):
     others = np.concatenate([rng.permutation(cols)[:20_000], rng.integers(0, 1 << 31, size=9000).astype(dtype), cols[:1]])
     _relabel_both_ways(pkg, oracle, [seeds, cols], [others])
     _relabel_both_ways(pkg, oracle, [cols, seeds], [cols, seeds])
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [140_000, 600_000])
+@pytest.mark.parametrize("hubs,share", [(1, 0.02), (1, 0.2), (7, 0.5), (40, 0.9)])
+def test_relabel_of_lists_with_hubs(pkg, oracle, dtype, n, hubs, share):
+    # ids that come up again and again, mapped and looked up, in no runs; the last hub is looked up alone, so that it is not there
+    rng = np.random.default_rng(n + hubs)
+    hub = rng.integers(0, 1 << 30, size=hubs + 1).astype(dtype)
+    ids = rng.integers(0, 1 << 30, size=n).astype(dtype)
+    at = rng.random(n) < share
+    ids[at] = rng.choice(hub[:-1], size=int(at.sum()))
+    look = rng.permutation(ids)
+    at = rng.random(n) < share
+    look[at] = rng.choice(hub, size=int(at.sum()))
+    look[n // 2 - 3000:n // 2] = hub[-1]
+    _relabel_both_ways(pkg, oracle, [ids], [look, ids])
+
+
+def test_relabel_of_hubs_that_meet_in_the_filter(pkg, oracle):
+    # ids of one bucket (of 256) and of one entry of the filter (the hash's top 13 bits, by the library's hash, restated here):
+    # the smallest of them that a tile holds has the entry, the others go on as they are
+    ids = np.arange(1 << 25, dtype=np.uint32)
+    h = ids.copy()
+    h ^= h >> np.uint32(16); h *= np.uint32(0x85EBCA6B)
+    h ^= h >> np.uint32(13); h *= np.uint32(0xC2B2AE35)
+    h ^= h >> np.uint32(16)
+    meet = ids[((h & 255) == 9) & ((h >> 19) == 77)]
+    assert meet.size >= 4
+    rng = np.random.default_rng(1)
+    for n in (200_000, 700_000):
+        mapping = rng.choice(meet, size=n)
+        mapping[::5] = rng.integers(0, 1 << 30, size=mapping[::5].size)
+        _relabel_both_ways(pkg, oracle, [mapping.astype(np.int64)], [rng.permutation(mapping).astype(np.int64)])
 
 
 def test_relabel_of_long_lists_in_many_segments(pkg, oracle):

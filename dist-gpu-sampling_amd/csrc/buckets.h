@@ -35,9 +35,12 @@
 
 namespace dgs {
 
-constexpr int kBucketBlock = 1024;
-constexpr int kBucketItems = 8;                      // units a thread takes of a tile
-constexpr int kBucketTile = kBucketBlock * kBucketItems;
+constexpr int kBucketBlock = 1024;                   // threads of the launch that finds the first ones
+template <int THREADS, int ITEMS> struct TileShape {  // of the launches that go over tiles: a block's threads, units a thread takes
+  static constexpr int kThreads = THREADS, kItems = ITEMS, kTile = THREADS * ITEMS;
+};
+using BucketShape = TileShape<1024, 8>;
+constexpr int kBucketTile = BucketShape::kTile;      // units of a tile, at most
 constexpr int kLocalBits = 13;
 static_assert(1 << kLocalBits == kBucketTile, "a unit's place in its tile");
 constexpr int kMaxBucketTiles = 8388608 / kBucketTile;  // 8.4 M units
@@ -62,6 +65,7 @@ struct Buckets {
   int* overflow;       // set when the ids of a part did not fit its table (only one that a test hook makes small)
   int32_t tiles_max;
   int32_t log_buckets; // hashed: at most
+  int32_t log_tile;    // units of a tile
   uint32_t n_ids;      // direct: ids are below it
   int32_t hashed;
   int32_t hash_slots;  // kHashSlots (a test hook makes it small, so that small inputs fill it)
@@ -102,36 +106,37 @@ template <> struct BucketItem<true> {
   static __device__ __forceinline__ uint32_t local(type item) { return item.y; }
 };
 
-template <bool HASHED>
+template <bool HASHED, typename Shape>
 struct SortLds {
   int count[kMaxBuckets];  // units of every bucket, then where its piece begins
-  __align__(8) typename BucketItem<HASHED>::type stage[kBucketTile];
-  int scan[kBucketBlock / kWave];
+  __align__(8) typename BucketItem<HASHED>::type stage[Shape::kTile];
+  int scan[Shape::kThreads / kWave];
   int hot;
 };
 // A piece of that many units (four times the average, or more) is one id's or a few ids', as a rule.
-constexpr int kHotPiece = kBucketTile / 64;
+template <typename Shape> constexpr int kHotPiece = Shape::kTile / 64;
 
 // The units in hot buckets whose id has one before them in the tile are none: folded(j, place of that one in the tile).  An entry of
 // the filter goes to the smallest of the ids that meet there, and to its smallest unit; the others stay as they are.
-template <bool HASHED, typename Folded>
-__device__ __forceinline__ void fold_tile(int log_buckets, uint32_t (&id)[kBucketItems], SortLds<HASHED>& lds, Folded folded) {
+template <bool HASHED, typename Shape, typename Folded>
+__device__ __forceinline__ void fold_tile(int log_buckets, uint32_t (&id)[Shape::kItems], SortLds<HASHED, Shape>& lds, Folded folded) {
   using Item = BucketItem<HASHED>;
+  constexpr int NT = Shape::kThreads, ITEMS = Shape::kItems;
   constexpr int kEntries = sizeof(lds.stage) / sizeof(unsigned long long), kLogEntries = __builtin_ctz(kEntries);
   unsigned long long* filter = reinterpret_cast<unsigned long long*>(lds.stage);
-  for (int j = threadIdx.x; j < kEntries; j += kBucketBlock) filter[j] = ~0ull;
+  for (int j = threadIdx.x; j < kEntries; j += NT) filter[j] = ~0ull;
   __syncthreads();
-  const auto packed = [&](int j) { return (static_cast<unsigned long long>(id[j]) << 32) | (uint32_t(j * kBucketBlock) + threadIdx.x); };
-  const auto hot = [&](int j) { return id[j] != kNoId && lds.count[Item::bucket(id[j], log_buckets)] > kHotPiece; };
+  const auto packed = [&](int j) { return (static_cast<unsigned long long>(id[j]) << 32) | (uint32_t(j * NT) + threadIdx.x); };
+  const auto hot = [&](int j) { return id[j] != kNoId && lds.count[Item::bucket(id[j], log_buckets)] > kHotPiece<Shape>; };
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     if (!hot(j)) continue;
     unsigned long long* entry = filter + (hash_id(id[j]) >> (32 - kLogEntries));
     if (*entry > packed(j)) atomicMin(entry, packed(j));
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     if (!hot(j)) continue;
     const unsigned long long held = filter[hash_id(id[j]) >> (32 - kLogEntries)];
     if (uint32_t(held >> 32) != id[j] || held == packed(j)) continue;
@@ -141,42 +146,43 @@ __device__ __forceinline__ void fold_tile(int log_buckets, uint32_t (&id)[kBucke
   __syncthreads();
 }
 
-// The tile's units in bucket order.  id[j] is that of unit tile * kBucketTile + j * kBucketBlock + thread, or kNoId.  A bucket's units
+// The tile's units in bucket order.  id[j] is that of unit tile * kTile + j * kThreads + thread, or kNoId.  A bucket's units
 // are one block's work in the launch behind this one, and meet at one word of LDS if they are one id's: a tile that an id comes up
 // in again and again hands on the first one alone (fold_tile).  us a relabel call, without / with it: 4 M ids, one different
 // 4630 / 175, ten 625 / 178, a fifth of them one id 1133 / 246; 890 k 1150 / 50, 157 / 49, 221 / 58; without any such id 211 / 213
 // and 49.8 / 49.6.  A batch of 4096 seeds, [5,10,15], 2.4 M nodes of 50 neighbours, one node on 5 / 20 / 50 % of the edges: 576
 // / 845 / 1035 -> 389 / 253 / 234, none 255 / 254.
-template <bool HASHED, typename Folded>
-__device__ __forceinline__ void sort_tile(const Buckets& b, int log_buckets, uint32_t tile, uint32_t (&id)[kBucketItems],
-                                         SortLds<HASHED>& lds, Folded folded) {
+template <bool HASHED, typename Shape, typename Folded>
+__device__ __forceinline__ void sort_tile(const Buckets& b, int log_buckets, uint32_t tile, uint32_t (&id)[Shape::kItems],
+                                         SortLds<HASHED, Shape>& lds, Folded folded) {
   using Item = BucketItem<HASHED>;
+  constexpr int NT = Shape::kThreads, ITEMS = Shape::kItems;
   const int buckets = 1 << log_buckets;
-  constexpr int kMine = (kMaxBuckets + kBucketBlock - 1) / kBucketBlock;  // consecutive buckets of a thread, at most
-  const int mine = buckets > kBucketBlock ? buckets / kBucketBlock : 1, b0 = int(threadIdx.x) * mine;
-  int before[kBucketItems];      // units of its bucket that were counted before it
+  constexpr int kMine = (kMaxBuckets + NT - 1) / NT;  // consecutive buckets of a thread, at most
+  const int mine = buckets > NT ? buckets / NT : 1, b0 = int(threadIdx.x) * mine;
+  int before[ITEMS];      // units of its bucket that were counted before it
   const auto count = [&] {
-    for (int j = threadIdx.x; j < buckets; j += kBucketBlock) lds.count[j] = 0;
+    for (int j = threadIdx.x; j < buckets; j += NT) lds.count[j] = 0;
     if (threadIdx.x == 0) lds.hot = 0;
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
       before[j] = 0;
       if (id[j] != kNoId) before[j] = atomicAdd(&lds.count[Item::bucket(id[j], log_buckets)], 1);
     }
     int most = 0;
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) most = before[j] > most ? before[j] : most;
-    if (most >= kHotPiece) lds.hot = 1;
+    for (int j = 0; j < ITEMS; ++j) most = before[j] > most ? before[j] : most;
+    if (most >= kHotPiece<Shape>) lds.hot = 1;
     __syncthreads();
   };
   count();
   if (lds.hot != 0) {
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) asm volatile("" : "+v"(id[j]));  // (what hangs on them is worked out anew, not kept: 47 registers, 85)
-    fold_tile<HASHED>(log_buckets, id, lds, folded);
+    for (int j = 0; j < ITEMS; ++j) asm volatile("" : "+v"(id[j]));  // (what hangs on them is worked out anew, not kept: 47 registers, 85)
+    fold_tile<HASHED, Shape>(log_buckets, id, lds, folded);
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) asm volatile("" : "+v"(id[j]));
+    for (int j = 0; j < ITEMS; ++j) asm volatile("" : "+v"(id[j]));
     count();
   }
   int own[kMine], sum = 0;
@@ -186,7 +192,7 @@ __device__ __forceinline__ void sort_tile(const Buckets& b, int log_buckets, uin
     sum += own[j];
   }
   int all;
-  int at = block_exclusive_scan<kBucketBlock, int>(sum, &all, lds.scan);  // (has barriers)
+  int at = block_exclusive_scan<NT, int>(sum, &all, lds.scan);  // (has barriers)
   uint16_t* piece = b.piece + size_t(tile) * (buckets + 1);
 #pragma unroll
   for (int j = 0; j < kMine; ++j) {
@@ -200,15 +206,15 @@ __device__ __forceinline__ void sort_tile(const Buckets& b, int log_buckets, uin
   if (threadIdx.x < kCounters) b.firsts[threadIdx.x * kMaxBucketTiles + tile] = 0;  // (for the launch behind this one)
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j)
+  for (int j = 0; j < ITEMS; ++j)
     if (id[j] != kNoId)
       lds.stage[lds.count[Item::bucket(id[j], log_buckets)] + before[j]] =
-          Item::make(id[j], log_buckets, uint32_t(j * kBucketBlock) + threadIdx.x);
+          Item::make(id[j], log_buckets, uint32_t(j * NT) + threadIdx.x);
   __syncthreads();
-  typename Item::type* items = static_cast<typename Item::type*>(b.items) + size_t(tile) * kBucketTile;
+  typename Item::type* items = static_cast<typename Item::type*>(b.items) + size_t(tile) * Shape::kTile;
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
-    const int e = j * kBucketBlock + int(threadIdx.x);
+  for (int j = 0; j < ITEMS; ++j) {
+    const int e = j * NT + int(threadIdx.x);
     if (e < all) nth(items, uint32_t(e)) = lds.stage[e];
   }
 }
@@ -243,9 +249,9 @@ struct PieceRound {
 #pragma unroll
     for (int q = 0; q < kPieces; ++q) {
       const uint32_t tile = first_tile + uint32_t(q * kPieceGroups) + threadIdx.x / kPieceLanes;
-      if (upto[q] > uint32_t(kBucketTile)) upto[q] = kBucketTile;  // (sizes that no tile has are not followed)
-      at[q] = tile * kBucketTile + from[q] + (threadIdx.x & (kPieceLanes - 1));
-      end[q] = tile * kBucketTile + upto[q];
+      if (upto[q] > 1u << b.log_tile) upto[q] = 1u << b.log_tile;  // (sizes that no tile has are not followed)
+      at[q] = (tile << b.log_tile) + from[q] + (threadIdx.x & (kPieceLanes - 1));
+      end[q] = (tile << b.log_tile) + upto[q];
     }
 #pragma unroll
     for (int q = 0; q < kPieces; ++q)
@@ -268,10 +274,10 @@ struct PieceRound {
     const int group = int(threadIdx.x & (kWave - 1)) / kPieceLanes * kPieceLanes;
 #pragma unroll
     for (int q = 0; q < kPieces; ++q) {
-      const uint32_t tile = at[q] / kBucketTile;  // (an item's place is in its tile)
+      const uint32_t tile = at[q] >> b.log_tile;  // (an item's place is in its tile)
       int n = 0;
       const auto one = [&](uint32_t e, typename Item::type it) {
-        const bool yes = see(e, it, tile * kBucketTile + Item::local(it));
+        const bool yes = see(e, it, (tile << b.log_tile) + Item::local(it));
         // (the group's first lane is there as long as any of its lanes is)
         n += __builtin_popcountll((__ballot(yes) >> group) & ((1u << kPieceLanes) - 1));
       };
@@ -448,28 +454,30 @@ __device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log
 }
 
 // into[place of a unit in the tile] = its id's smallest unit, for all of the tile's units.
-template <bool HASHED>
-__device__ __forceinline__ void unsort_tile(const Buckets& b, int log_buckets, uint32_t tile, uint32_t* into /* [kBucketTile] in LDS */) {
+template <bool HASHED, typename Shape>
+__device__ __forceinline__ void unsort_tile(const Buckets& b, int log_buckets, uint32_t tile, uint32_t* into /* [kTile] in LDS */) {
   using Item = BucketItem<HASHED>;
-  const auto* items = static_cast<const typename Item::type*>(b.items) + size_t(tile) * kBucketTile;
-  const uint32_t* least = b.least + size_t(tile) * kBucketTile;
+  constexpr int NT = Shape::kThreads, ITEMS = Shape::kItems;
+  const auto* items = static_cast<const typename Item::type*>(b.items) + size_t(tile) * Shape::kTile;
+  const uint32_t* least = b.least + size_t(tile) * Shape::kTile;
   const int count = b.piece[size_t(tile) * ((1 << log_buckets) + 1) + (1 << log_buckets)];
-  typename Item::type item[kBucketItems];
-  uint32_t value[kBucketItems];
+  typename Item::type item[ITEMS];
+  uint32_t value[ITEMS];
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {  // (the arrays hold whole tiles)
-    item[j] = nth(items, uint32_t(j * kBucketBlock) + threadIdx.x);
-    value[j] = nth(least, uint32_t(j * kBucketBlock) + threadIdx.x);
+  for (int j = 0; j < ITEMS; ++j) {  // (the arrays hold whole tiles)
+    item[j] = nth(items, uint32_t(j * NT) + threadIdx.x);
+    value[j] = nth(least, uint32_t(j * NT) + threadIdx.x);
   }
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j)
-    if (j * kBucketBlock + int(threadIdx.x) < count) into[Item::local(item[j]) & (kBucketTile - 1)] = value[j];
+  for (int j = 0; j < ITEMS; ++j)
+    if (j * NT + int(threadIdx.x) < count) into[Item::local(item[j]) & (Shape::kTile - 1)] = value[j];
 }
 
 // First occurrences in the tiles before `tile`: the sum over the block's threads of what each is returned.
+template <int NT>
 __device__ __forceinline__ uint32_t firsts_before(const Buckets& b, uint32_t tile) {
   uint32_t n = 0;
-  for (uint32_t t = threadIdx.x; t < tile; t += kBucketBlock) {
+  for (uint32_t t = threadIdx.x; t < tile; t += NT) {
 #pragma unroll
     for (int c = 0; c < kCounters; ++c) n += b.firsts[c * kMaxBucketTiles + t];
   }

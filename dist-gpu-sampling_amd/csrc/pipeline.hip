@@ -869,7 +869,7 @@ __global__ __launch_bounds__(kLongBlock) void hop_fill_weighted_shared_kernel(Ho
 
 template <typename IdT, bool HASHED>
 __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Buckets b) {
-  __shared__ SortLds<HASHED> lds;
+  __shared__ SortLds<HASHED, BucketShape> lds;
   if (blockIdx.x == 0 && threadIdx.x == 0) *b.overflow = 0;  // (the per-bucket launch comes behind this one)
   const int64_t s = wave_uniform(seeds_of(h));
   if (!bucketed_now(h, s)) return;  // the hop outgrew the pass: it runs on the table
@@ -877,24 +877,24 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(Hop h, Bucket
   const int log_buckets = log_buckets_of(b, units);
   uint32_t* slot = h.slot + h.pos_base;
   for (uint32_t tile = blockIdx.x; tile * kBucketTile < units; tile += gridDim.x) {
-    uint32_t id[kBucketItems];
+    uint32_t id[BucketShape::kItems];
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
+    for (int j = 0; j < BucketShape::kItems; ++j) {
       const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x;
       id[j] = u >= front && u < units ? nth(slot, u - front) : kNoId;  // (id | kFirstBit, or kInvalidSlot)
     }
     if (tile * kBucketTile < front) {
 #pragma unroll
-      for (int j = 0; j < kBucketItems; ++j) {
+      for (int j = 0; j < BucketShape::kItems; ++j) {
         const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x;
         if (u < uint32_t(s)) id[j] = uint32_t(nth(static_cast<const IdT*>(h.frontier), u));
       }
     }
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j)  // (a position's word: a draw that repeats one of its own row's, no unit)
+    for (int j = 0; j < BucketShape::kItems; ++j)  // (a position's word: a draw that repeats one of its own row's, no unit)
       if (id[j] != kNoId) id[j] = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x < front ? id[j]
                                 : (id[j] & kFirstBit) != 0 ? id[j] & ~kFirstBit : kNoId;
-    sort_tile<HASHED>(b, log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // (a pick: frontier ids are different ones)
+    sort_tile<HASHED, BucketShape>(b, log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // (a pick: frontier ids are different ones)
       const uint32_t u = tile * kBucketTile + uint32_t(j * kBucketBlock) + threadIdx.x, met = tile * kBucketTile + before;
       if (u >= front) nth(slot, u - front) = met < front ? met | kRankBit : uint32_t(h.pos_base) + (met - front);
     });
@@ -1072,7 +1072,7 @@ __device__ __forceinline__ void compact_tile(const Hop& h, int64_t tile, const T
 // in the order of the buckets.
 template <typename IdT, bool HASHED>
 __device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets& b, int64_t s, uint32_t tile) {
-  constexpr int ITEMS = 4, GROUPS = kBucketItems / ITEMS, kWaves = kBucketBlock / kWave;
+  constexpr int ITEMS = 4, GROUPS = BucketShape::kItems / ITEMS, kWaves = kBucketBlock / kWave;
   constexpr uint32_t kGroup = kBucketBlock * ITEMS;
   using words = typename Items<ITEMS>::words;
   __shared__ __align__(16) uint32_t least_of[kBucketTile];
@@ -1090,8 +1090,8 @@ __device__ __forceinline__ void compact_sorted_tile(const Hop& h, const Buckets&
     word[g] = words(kInvalidSlot);
     if (u >= front && u < units) word[g] = nth(reinterpret_cast<const words*>(slot), (u - front) / ITEMS);
   }
-  uint32_t before = firsts_before(b, tile);
-  unsort_tile<HASHED>(b, log_buckets, tile, least_of);
+  uint32_t before = firsts_before<kBucketBlock>(b, tile);
+  unsort_tile<HASHED, BucketShape>(b, log_buckets, tile, least_of);
 #pragma unroll
   for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d, kWave);
   if (lane == 0) wave_before[wave] = before;
@@ -1422,6 +1422,7 @@ size_t layout(const Plan& p, const int64_t* fanouts, void* base, Hop* hops, void
     b.n_ids = p.n_nodes;
     b.hashed = p.bucket_hashed ? 1 : 0;
     b.hash_slots = p.hash_slots;
+    b.log_tile = kLocalBits;
     if (buckets) *buckets = b;
     if (hops)
       for (int h = 0; h < p.n_hops; ++h) hops[h].bucket_overflow = b.overflow;

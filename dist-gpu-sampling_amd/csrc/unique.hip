@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kThreads) void lookup_kernel(dgs_segments requiring
 // and lookup 13.2.
 constexpr uint32_t kAbsent = kNoId;
 
-// Where a tile of kBucketTile entries of a segment list lies: one after the other in one segment, as a rule.  (No segment is
+// Where a tile of entries of a segment list lies: one after the other in one segment, as a rule.  (No segment is
 // named by a number that is not a constant: the list would be copied to memory for it.)
 template <typename T>
 __device__ __forceinline__ T* seg_at(const dgs_segments& s, int64_t i, int* seg = nullptr) {
@@ -272,15 +272,15 @@ __device__ __forceinline__ T* seg_at(const dgs_segments& s, int64_t i, int* seg 
   }
   return p;
 }
-template <typename T>
+template <typename T, int TILE>
 struct TileSpan {
   int64_t first;  // the tile's first entry
   uint32_t count; // its entries
   T* begin;       // where the first one lies
   bool whole;     // and all others behind it
   __device__ __forceinline__ TileSpan(const dgs_segments& s, uint32_t tile, int64_t total) {
-    first = int64_t(tile) * kBucketTile;
-    count = uint32_t(total - first < kBucketTile ? total - first : kBucketTile);
+    first = int64_t(tile) * TILE;
+    count = uint32_t(total - first < TILE ? total - first : TILE);
     int from, upto;
     begin = seg_at<T>(s, first, &from);
     seg_at<T>(s, first + count - 1, &upto);
@@ -292,47 +292,49 @@ struct TileSpan {
 // Units that sort_tile has folded: (place of the one before it that it is equal to, its own place) each, from the end of the tile's
 // items downwards, which that many units less leave free.
 using Item = BucketItem<true>::type;
+template <typename Shape>
 __device__ __forceinline__ Item* folded_items(const Buckets& b, uint32_t tile) {
-  return static_cast<Item*>(b.items) + (size_t(tile) + 1) * kBucketTile - 1;
+  return static_cast<Item*>(b.items) + (size_t(tile) + 1) * Shape::kTile - 1;
 }
-__device__ __forceinline__ void unfold_tile(const Buckets& b, uint32_t tile, uint32_t folds, uint32_t* into /* [kBucketTile] in LDS */) {
-  for (uint32_t e = threadIdx.x; e < folds && e < uint32_t(kBucketTile); e += kBucketBlock) {
-    const Item it = folded_items(b, tile)[-int64_t(e)];
-    into[it.y & (kBucketTile - 1)] = into[it.x & (kBucketTile - 1)];
+template <typename Shape>
+__device__ __forceinline__ void unfold_tile(const Buckets& b, uint32_t tile, uint32_t folds, uint32_t* into /* [kTile] in LDS */) {
+  for (uint32_t e = threadIdx.x; e < folds && e < uint32_t(Shape::kTile); e += Shape::kThreads) {
+    const Item it = folded_items<Shape>(b, tile)[-int64_t(e)];
+    into[it.y & (Shape::kTile - 1)] = into[it.x & (Shape::kTile - 1)];
   }
   __syncthreads();
 }
 
 // The mapping ids that the table would hold as well.  notes[]: 1 if the tile has met another one, and twice its folded units.
-template <typename IdT>
-__global__ __launch_bounds__(kBucketBlock) void bucketed_sort_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, dgs_segments queries,
+template <typename IdT, typename Shape>
+__global__ __launch_bounds__(Shape::kThreads) void bucketed_sort_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, dgs_segments queries,
                                                                      int64_t m, Buckets b, uint32_t* __restrict__ notes) {
-  __shared__ SortLds<true> lds;
+  __shared__ SortLds<true, Shape> lds;
   __shared__ uint32_t any_bad, folds;
   const uint32_t tile = blockIdx.x;
   if (tile == 0 && threadIdx.x == 0) *b.overflow = 0;  // (the per-bucket launch comes behind this one)
   if (threadIdx.x == 0) any_bad = folds = 0;
   __syncthreads();
   const bool query = tile >= map_tiles;
-  IdT key[kBucketItems], front[kBucketItems];  // (front: of a wave's first lane, the query in front of its own)
+  IdT key[Shape::kItems], front[Shape::kItems];  // (front: of a wave's first lane, the query in front of its own)
   uint32_t count;
   const auto load = [&](const dgs_segments& list, uint32_t list_tile, int64_t total, bool fronts) {
-    const TileSpan<const IdT> span(list, list_tile, total);
+    const TileSpan<const IdT, Shape::kTile> span(list, list_tile, total);
     count = span.count;
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
-      const uint32_t e = uint32_t(j * kBucketBlock) + threadIdx.x;
+    for (int j = 0; j < Shape::kItems; ++j) {
+      const uint32_t e = uint32_t(j * Shape::kThreads) + threadIdx.x;
       key[j] = e < count ? span.at(list, e) : IdT(-1);
       front[j] = fronts && (threadIdx.x & (kWave - 1)) == 0 && e > 0 && e < count ? span.at(list, e - 1) : IdT(-1);
     }
   };
   if (query) load(queries, tile - map_tiles, m, true);
   else load(mapping, tile, n, false);
-  uint32_t id[kBucketItems];
+  uint32_t id[Shape::kItems];
   bool refused = false;
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
-    const uint32_t e = uint32_t(j * kBucketBlock) + threadIdx.x;
+  for (int j = 0; j < Shape::kItems; ++j) {
+    const uint32_t e = uint32_t(j * Shape::kThreads) + threadIdx.x;
     const bool held = uint64_t(int64_t(key[j])) < 0xffffffffull;
     bool again = false;  // a query equal to the one in front of it
     if (query) {
@@ -343,13 +345,13 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_sort_kernel(dgs_segment
     id[j] = e < count && held && !again ? uint32_t(key[j]) : kNoId;
   }
   if (refused) any_bad = 1;
-  sort_tile<true>(b, b.log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // noted from the end of the tile's items on
+  sort_tile<true, Shape>(b, b.log_buckets, tile, id, lds, [&](int j, uint32_t before) {  // noted from the end of the tile's items on
     const uint64_t here = __ballot(1);
     const int lower = __builtin_popcountll(here & ((uint64_t(1) << (threadIdx.x & (kWave - 1))) - 1));
     uint32_t at = 0;
     if (lower == 0) at = atomicAdd(&folds, uint32_t(__builtin_popcountll(here)));
     at = __builtin_amdgcn_readfirstlane(at) + uint32_t(lower);
-    folded_items(b, tile)[-int64_t(at)] = Item{before, uint32_t(j * kBucketBlock) + threadIdx.x};
+    folded_items<Shape>(b, tile)[-int64_t(at)] = Item{before, uint32_t(j * Shape::kThreads) + threadIdx.x};
   });
   if (threadIdx.x == 0) notes[tile] = any_bad | folds << 1;  // (sort_tile has barriers)
 }
@@ -362,37 +364,37 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_first_kernel(Buckets b,
 }
 
 // rank_kernel's work on one tile of the mapping list.
-template <typename IdT>
-__global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, Buckets b,
+template <typename IdT, typename Shape>
+__global__ __launch_bounds__(Shape::kThreads) void bucketed_rank_kernel(dgs_segments mapping, int64_t n, uint32_t map_tiles, Buckets b,
                                                                      const uint32_t* __restrict__ notes, uint32_t* __restrict__ slot,
                                                                      IdT* __restrict__ unique_out, int64_t* __restrict__ counts_dev,
                                                                      int64_t* __restrict__ counts_host) {
   typedef uint32_t words __attribute__((ext_vector_type(kItems)));
-  constexpr int kGroups = kBucketItems / kItems, kWaves = kBucketBlock / kWave;
-  constexpr uint32_t kGroup = kBucketBlock * kItems;
-  __shared__ __align__(16) uint32_t least_of[kBucketTile];
+  constexpr int kGroups = Shape::kItems / kItems, kWaves = Shape::kThreads / kWave;
+  constexpr uint32_t kGroup = Shape::kThreads * kItems;
+  __shared__ __align__(16) uint32_t least_of[Shape::kTile];
   __shared__ uint32_t wave_before[kWaves];
   __shared__ int wave_count[kGroups * kWaves];
   __shared__ int any_bad;
-  const uint32_t tile = blockIdx.x, first_unit = tile * kBucketTile, at = threadIdx.x * kItems;
+  const uint32_t tile = blockIdx.x, first_unit = tile * Shape::kTile, at = threadIdx.x * kItems;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const bool last = tile + 1 == map_tiles;
-  const TileSpan<const IdT> span(mapping, tile, n);
-  uint32_t before = firsts_before(b, tile);
+  const TileSpan<const IdT, Shape::kTile> span(mapping, tile, n);
+  uint32_t before = firsts_before<Shape::kThreads>(b, tile);
   uint32_t refused = last && threadIdx.x == 0 ? uint32_t(*b.overflow) : 0u;
-  for (uint32_t t = threadIdx.x; last && t < map_tiles; t += kBucketBlock) refused |= notes[t] & 1;
+  for (uint32_t t = threadIdx.x; last && t < map_tiles; t += Shape::kThreads) refused |= notes[t] & 1;
   const uint32_t folds = notes[tile] >> 1;
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) *reinterpret_cast<words*>(least_of + g * kGroup + at) = words(kAbsent);  // (ids that are no units)
   if (threadIdx.x == 0) any_bad = 0;
   __syncthreads();
-  unsort_tile<true>(b, b.log_buckets, tile, least_of);
+  unsort_tile<true, Shape>(b, b.log_buckets, tile, least_of);
   if (refused != 0) any_bad = 1;
 #pragma unroll
   for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d, kWave);
   if (lane == 0) wave_before[wave] = before;
   __syncthreads();
-  if (folds != 0) unfold_tile(b, tile, folds, least_of);
+  if (folds != 0) unfold_tile<Shape>(b, tile, folds, least_of);
   words word[kGroups];
   uint32_t first[kGroups];  // bit j: position j of the group's is its id's first
   int lane_before[kGroups];
@@ -455,49 +457,49 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_rank_kernel(dgs_segment
 }
 
 // Blocks [0, query_tiles): a tile of the queries each, whose ids have their smallest units at the first of every run;
-// then blocks of kBucketTile requiring ids that are mapping ids, given by their words.
-template <typename IdT>
-__global__ __launch_bounds__(kBucketBlock) void bucketed_lookup_kernel(dgs_segments queries, int64_t m, uint32_t map_tiles, uint32_t query_tiles,
+// then blocks of Shape::kTile requiring ids that are mapping ids, given by their words.
+template <typename IdT, typename Shape>
+__global__ __launch_bounds__(Shape::kThreads) void bucketed_lookup_kernel(dgs_segments queries, int64_t m, uint32_t map_tiles, uint32_t query_tiles,
                                                                        Buckets b, const uint32_t* __restrict__ notes,
                                                                        const uint32_t* __restrict__ slot, int64_t n, dgs_segments query_out,
                                                                        dgs_segments words, int64_t n_words, dgs_segments words_out) {
-  __shared__ uint32_t least_of[kBucketTile];
-  __shared__ uint16_t head[kBucketTile];  // where the run begins that an id belongs to
-  __shared__ int wave_head[kBucketBlock / kWave];
+  __shared__ uint32_t least_of[Shape::kTile];
+  __shared__ uint16_t head[Shape::kTile];  // where the run begins that an id belongs to
+  __shared__ int wave_head[Shape::kThreads / kWave];
   if (blockIdx.x >= query_tiles) {
-    const TileSpan<const uint32_t> in(words, blockIdx.x - query_tiles, n_words);
-    const TileSpan<IdT> to(words_out, blockIdx.x - query_tiles, n_words);
-    uint32_t word[kBucketItems];
+    const TileSpan<const uint32_t, Shape::kTile> in(words, blockIdx.x - query_tiles, n_words);
+    const TileSpan<IdT, Shape::kTile> to(words_out, blockIdx.x - query_tiles, n_words);
+    uint32_t word[Shape::kItems];
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
-      const uint32_t e = uint32_t(j * kBucketBlock) + threadIdx.x;
+    for (int j = 0; j < Shape::kItems; ++j) {
+      const uint32_t e = uint32_t(j * Shape::kThreads) + threadIdx.x;
       word[j] = e < in.count ? in.at(words, e) : kNoSlot;
     }
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j)
+    for (int j = 0; j < Shape::kItems; ++j)
       if ((word[j] & kFirstBit) == 0) word[j] = int64_t(word[j]) < n ? slot[word[j]] : kNoSlot;
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
-      const uint32_t e = uint32_t(j * kBucketBlock) + threadIdx.x;
+    for (int j = 0; j < Shape::kItems; ++j) {
+      const uint32_t e = uint32_t(j * Shape::kThreads) + threadIdx.x;
       if (e < in.count) to.at(words_out, e) = (word[j] & kFirstBit) != 0 ? IdT(word[j] & ~kFirstBit) : IdT(-1);
     }
     return;
   }
   const uint32_t tile = map_tiles + blockIdx.x;
-  const TileSpan<IdT> to(query_out, blockIdx.x, m);
+  const TileSpan<IdT, Shape::kTile> to(query_out, blockIdx.x, m);
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const bool odd_ones = (notes[tile] & 1) != 0;
   const uint32_t folds = notes[tile] >> 1;
-  for (int e = threadIdx.x; e < kBucketTile; e += kBucketBlock) least_of[e] = kAbsent;
+  for (int e = threadIdx.x; e < Shape::kTile; e += Shape::kThreads) least_of[e] = kAbsent;
   __syncthreads();
-  unsort_tile<true>(b, b.log_buckets, tile, least_of);
+  unsort_tile<true, Shape>(b, b.log_buckets, tile, least_of);
   __syncthreads();
-  if (folds != 0) unfold_tile(b, tile, folds, least_of);
+  if (folds != 0) unfold_tile<Shape>(b, tile, folds, least_of);
   // a thread has eight ids in a row: where the last run begins that does so before or at each
-  int own[kBucketItems], latest = -1;
+  int own[Shape::kItems], latest = -1;
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
-    const int e = int(threadIdx.x) * kBucketItems + j;
+  for (int j = 0; j < Shape::kItems; ++j) {
+    const int e = int(threadIdx.x) * Shape::kItems + j;
     if (least_of[e] != kAbsent) latest = e;
     own[j] = latest;
   }
@@ -512,23 +514,23 @@ __global__ __launch_bounds__(kBucketBlock) void bucketed_lookup_kernel(dgs_segme
   if (lane == 0) prior = -1;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kBucketBlock / kWave; ++w)
+  for (int w = 0; w < Shape::kThreads / kWave; ++w)
     if (w < wave && wave_head[w] > prior) prior = wave_head[w];
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
+  for (int j = 0; j < Shape::kItems; ++j) {
     const int h = own[j] >= 0 ? own[j] : prior;
-    head[int(threadIdx.x) * kBucketItems + j] = uint16_t(h >= 0 ? h : 0);  // (the first id of a tile is a head, or no id)
+    head[int(threadIdx.x) * Shape::kItems + j] = uint16_t(h >= 0 ? h : 0);  // (the first id of a tile is a head, or no id)
   }
   __syncthreads();
-  uint32_t word[kBucketItems];
+  uint32_t word[Shape::kItems];
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
-    const uint32_t least = least_of[head[j * kBucketBlock + threadIdx.x]];
+  for (int j = 0; j < Shape::kItems; ++j) {
+    const uint32_t least = least_of[head[j * Shape::kThreads + threadIdx.x]];
     word[j] = int64_t(least) < n ? slot[least] : kNoSlot;  // (one of the queries: the id is not in the mapping list)
   }
 #pragma unroll
-  for (int j = 0; j < kBucketItems; ++j) {
-    const uint32_t e = uint32_t(j * kBucketBlock) + threadIdx.x;
+  for (int j = 0; j < Shape::kItems; ++j) {
+    const uint32_t e = uint32_t(j * Shape::kThreads) + threadIdx.x;
     if (e >= to.count) continue;
     IdT rank = (word[j] & kFirstBit) != 0 ? IdT(word[j] & ~kFirstBit) : IdT(-1);
     if (odd_ones && uint64_t(int64_t(*seg_at<const IdT>(queries, to.first + e))) >= 0xffffffffull) rank = IdT(-1);  // (in no run)
@@ -683,26 +685,34 @@ struct UniqueWorkspace {
 };
 
 // Lists that may go by buckets: long enough for the table's atomics to cost more than the chains of waits, and short enough
-// for the tiles that a block has room to count.  us a call with the wait for its count, table / buckets, of ids mostly new,
-// of as many different ones as there are ids, of a tenth new: 101 k 37 / 36, 36 / 37, 32 / 38; 131 k 42 / 36, 37 / 37, 33 / 38;
-// 180 k 66 / 36, 44 / 38, 34 / 39; 400 k 55 / 39, 52 / 41, 45 / 41; 890 k 82 / 48, 79 / 48, 65 / 47; 4 M 262 / 203, 258 /
-// 207, 235 / 195.  A bucket's units are one block's work however few ids they are: 890 k of ten ids 355 / 152, of one
-// 1466 / 1171, but 4 M of them 353 / 625 and 1575 / 4650.
-constexpr int64_t kBucketedMinIds = int64_t(1) << 17;
-inline int64_t bucket_tiles(int64_t n) { return (n + kBucketTile - 1) / kBucketTile; }
+// for the tiles that a block has room to count.  us a call with the wait for its count, table / buckets, of ids mostly new and of
+// a tenth new: 131 k 44 / 33, 35 / 33; 180 k 67 / 34, 37 / 35; 250 k of a tenth new 39 / 35; 400 k 56 / 38, 46 / 38; 890 k 83 / 50,
+// 65 / 47; 4 M 262 / 213, 239 / 199.
+// Short lists have smaller tiles, which are more blocks and less of a chain each.  Tiles of 8192 / 2048 units: 131 k 38 / 33, 41 / 33;
+// 180 k 39 / 34, 42 / 35; 400 k 42 / 38, 45 / 38, 890 k 50 / 60 (of 4096, by 512 or 1024 threads, 34 / 35, 36 / 36, 38 / 39, 53; of
+// 2048 by 256 threads 35, 36, 40, 60; of 1024 35, 37, 47).
+using LongLists = BucketShape;
+using ShortLists = TileShape<512, 4>;
+constexpr int64_t kBucketedMinIds = int64_t(1) << 17, kShortListIds = int64_t(1) << 19;
+inline int64_t bucket_tile(int64_t n) { return n <= kShortListIds ? ShortLists::kTile : LongLists::kTile; }
+inline int64_t bucket_tiles(int64_t ids, int64_t tile) { return (ids + tile - 1) / tile; }
 constexpr int64_t kBucketedMaxTiles = kMaxBucketTiles / 2;  // of mapping ids (as many of queries)
-inline bool may_be_bucketed(int64_t n) { return n >= kBucketedMinIds && bucket_tiles(n) <= kBucketedMaxTiles; }
+constexpr int64_t kBucketedMaxIds = kBucketedMaxTiles * LongLists::kTile;
+static_assert(kShortListIds / ShortLists::kTile <= kBucketedMaxTiles, "room to count them");
+inline bool may_be_bucketed(int64_t n) { return n >= kBucketedMinIds && n <= kBucketedMaxIds; }
 
 // packed 64-bit slots, or id array + value array (the larger: what the workspace is sized for)
 size_t slot_bytes(int32_t id_bytes, bool packed) { return packed ? 8 : size_t(id_bytes) + 4; }
 
-void take_buckets(Carver* c, int64_t map_tiles, UniqueWorkspace* t) {
+void take_buckets(Carver* c, int64_t n, UniqueWorkspace* t) {
+  const int64_t tile = bucket_tile(n);
   Buckets& b = t->buckets;
   b.hashed = 1;
   b.hash_slots = kHashSlots;
-  b.tiles_max = int32_t(2 * map_tiles);
-  b.items = c->take<uint2>(size_t(b.tiles_max) * kBucketTile);
-  b.least = c->take<uint32_t>(size_t(b.tiles_max) * kBucketTile);
+  b.log_tile = __builtin_ctzll(uint64_t(tile));
+  b.tiles_max = int32_t(2 * bucket_tiles(n, tile));
+  b.items = c->take<uint2>(size_t(b.tiles_max) * size_t(tile));
+  b.least = c->take<uint32_t>(size_t(b.tiles_max) * size_t(tile));
   b.piece = c->take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
   b.firsts = c->take<uint32_t>(kCounters * kMaxBucketTiles);
   b.overflow = c->take<int>(4);
@@ -711,7 +721,8 @@ void take_buckets(Carver* c, int64_t map_tiles, UniqueWorkspace* t) {
 
 // The slot words, then either the table with its marks or the buckets: an attempt uses one of them, and the one that follows a
 // void attempt comes behind it on the stream.  The size never falls as lists grow (a caller sizes one workspace for its longest
-// list): lists beyond those that go by buckets have the room of the longest one that does.
+// list): lists beyond those that go by buckets have the room of the longest one that does, and those of large tiles that of the
+// longest one of small tiles.
 size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWorkspace* w) {
   if (n < 0) n = 0;
   if (n > kMaxMappingIds) n = kMaxMappingIds;
@@ -719,8 +730,8 @@ size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWo
   const size_t padded = tiles * size_t(kGroupIds) * rank_groups(n);
   UniqueWorkspace t{};
   Carver c(base);
-  t.slot = c.take<uint32_t>(std::max(padded, may_be_bucketed(n) ? size_t(bucket_tiles(n)) * kBucketTile : 0));
-  Carver d = c;
+  t.slot = c.take<uint32_t>(std::max(padded, may_be_bucketed(n) ? size_t(bucket_tiles(n, bucket_tile(n)) * bucket_tile(n)) : 0));
+  Carver buckets = c;
   t.capacity = table_capacity(n);
   t.table_bytes = size_t(t.capacity) * slot_bytes(id_bytes, id_bytes == 4);
   t.table = c.take<char>(t.table_bytes);
@@ -728,9 +739,16 @@ size_t unique_workspace_layout(int64_t n, int32_t id_bytes, void* base, UniqueWo
   t.lost = c.take<uint8_t>(t.zero_bytes);
   t.state = reinterpret_cast<tile_state*>(t.lost + padded);
   t.overflow = reinterpret_cast<int*>(t.state + tiles);
-  if (n >= kBucketedMinIds) take_buckets(&d, std::min(bucket_tiles(n), kBucketedMaxTiles), &t);
+  size_t used = c.used;
+  if (n >= kBucketedMinIds) {
+    for (const int64_t ids : {std::min(n, kShortListIds), std::min(n, kBucketedMaxIds)}) {
+      c = buckets;
+      take_buckets(&c, ids, &t);
+      used = std::max(used, c.used);
+    }
+  }
   if (w) *w = t;
-  return std::max(c.used, d.used) + 256;
+  return used + 256;
 }
 
 int64_t seg_total(const dgs_segments& s) {
@@ -806,19 +824,19 @@ SplitRequiring split_requiring(const dgs_segments& mapping, const dgs_segments& 
   }
   return r;
 }
-template <typename IdT>
+template <typename IdT, typename Shape>
 dgs_status run_bucketed_relabel(const dgs_segments& mapping, int64_t n, const SplitRequiring& r, void* unique_out,
                                 int64_t* counts_dev, int64_t* counts_host, void** ticket, const UniqueWorkspace& w, hipStream_t st) {
   const int64_t m = seg_total(r.queries), n_words = seg_total(r.words);
-  const uint32_t map_tiles = uint32_t(bucket_tiles(n)), query_tiles = uint32_t(bucket_tiles(m)), tiles = map_tiles + query_tiles;
+  const uint32_t map_tiles = uint32_t(bucket_tiles(n, Shape::kTile)), query_tiles = uint32_t(bucket_tiles(m, Shape::kTile)), tiles = map_tiles + query_tiles;
   Buckets b = w.buckets;
   b.log_buckets = kMinLogBuckets;
   while (b.log_buckets < kMaxLogBuckets && (int64_t(kHashSlots / 2) << b.log_buckets) < n + m) ++b.log_buckets;
-  hipLaunchKernelGGL(bucketed_sort_kernel<IdT>, dim3(tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, r.queries, m, b, w.notes);
+  hipLaunchKernelGGL((bucketed_sort_kernel<IdT, Shape>), dim3(tiles), dim3(Shape::kThreads), 0, st, mapping, n, map_tiles, r.queries, m, b, w.notes);
   DGS_LAUNCH_CHECK();
   hipLaunchKernelGGL(bucketed_first_kernel, dim3(1u << b.log_buckets), dim3(kBucketBlock), 0, st, b, tiles);
   DGS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bucketed_rank_kernel<IdT>, dim3(map_tiles), dim3(kBucketBlock), 0, st, mapping, n, map_tiles, b, w.notes, w.slot,
+  hipLaunchKernelGGL((bucketed_rank_kernel<IdT, Shape>), dim3(map_tiles), dim3(Shape::kThreads), 0, st, mapping, n, map_tiles, b, w.notes, w.slot,
                      static_cast<IdT*>(unique_out), counts_dev, counts_host);
   DGS_LAUNCH_CHECK();
   // the counts are final here: mark the point the caller may wait for
@@ -826,9 +844,9 @@ dgs_status run_bucketed_relabel(const dgs_segments& mapping, int64_t n, const Sp
     const dgs_status ts = dgs_ticket_record(st, ticket);
     if (ts != DGS_OK) return ts;
   }
-  const uint32_t blocks = query_tiles + uint32_t(bucket_tiles(n_words));
+  const uint32_t blocks = query_tiles + uint32_t(bucket_tiles(n_words, Shape::kTile));
   if (blocks > 0)
-    hipLaunchKernelGGL(bucketed_lookup_kernel<IdT>, dim3(blocks), dim3(kBucketBlock), 0, st, r.queries, m, map_tiles, query_tiles, b,
+    hipLaunchKernelGGL((bucketed_lookup_kernel<IdT, Shape>), dim3(blocks), dim3(Shape::kThreads), 0, st, r.queries, m, map_tiles, query_tiles, b,
                        w.notes, w.slot, n, r.query_out, r.words, n_words, r.words_out);
   DGS_LAUNCH_CHECK();
   return DGS_OK;
@@ -905,9 +923,14 @@ DGS_API dgs_status dgs_unique_relabel(dgs_segments mapping, dgs_segments requiri
   // (an attempt that packed_table asks for: ids that do not fit a word void it)
   if (packed_table != 0 && may_be_bucketed(n) && lookback_polls() == kLookbackPolls) {  // (test hook of the launches that it replaces)
     const SplitRequiring r = split_requiring(mapping, requiring, out, w.slot);
-    if (bucket_tiles(seg_total(r.queries)) <= bucket_tiles(n))
-      return id_bytes == 4 ? run_bucketed_relabel<int32_t>(mapping, n, r, unique_out, counts_dev, counts_host, counts_ticket, w, st)
-                           : run_bucketed_relabel<int64_t>(mapping, n, r, unique_out, counts_dev, counts_host, counts_ticket, w, st);
+    const int64_t tile = bucket_tile(n);
+    if (bucket_tiles(seg_total(r.queries), tile) <= bucket_tiles(n, tile)) {
+      const auto run = [&](auto id, auto shape) {
+        return run_bucketed_relabel<decltype(id), decltype(shape)>(mapping, n, r, unique_out, counts_dev, counts_host, counts_ticket, w, st);
+      };
+      if (tile == ShortLists::kTile) return id_bytes == 4 ? run(int32_t(0), ShortLists{}) : run(int64_t(0), ShortLists{});
+      return id_bytes == 4 ? run(int32_t(0), LongLists{}) : run(int64_t(0), LongLists{});
+    }
   }
   if (id_bytes == 4)
     return run_unique_relabel<int32_t, Table<int32_t, true>>(mapping, n, requiring, m, unique_out, counts_dev,

@@ -113,7 +113,7 @@ def _relabel_both_ways(pkg, oracle, mapping, requiring):
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
-@pytest.mark.parametrize("n", [131_071, 131_072, 131_073, 139_263, 1_200_000])  # where buckets begin, 16 and 17 tiles, 147 tiles
+@pytest.mark.parametrize("n", [131_071, 131_072, 131_073, 139_263, 524_288, 524_289, 1_200_000])  # where buckets, a tile of 2048, tiles of 8192 begin
 @pytest.mark.parametrize("distinct", [1, 3000, 1 << 30])
 def test_relabel_of_long_lists(pkg, oracle, dtype, n, distinct):
     rng = np.random.default_rng(n)
@@ -128,7 +128,7 @@ def test_relabel_of_long_lists(pkg, oracle, dtype, n, distinct):
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
-@pytest.mark.parametrize("n", [140_000, 600_000])
+@pytest.mark.parametrize("n", [140_000, 600_000])  # of small tiles and of large ones
 @pytest.mark.parametrize("hubs,share", [(1, 0.02), (1, 0.2), (7, 0.5), (40, 0.9)])
 def test_relabel_of_lists_with_hubs(pkg, oracle, dtype, n, hubs, share):
     # ids that come up again and again, mapped and looked up, in no runs; the last hub is looked up alone, so that it is not there

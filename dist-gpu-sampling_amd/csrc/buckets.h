@@ -62,7 +62,7 @@ struct Buckets {
   uint32_t* least;     // [tiles_max][kBucketTile] smallest unit of the item's id
   uint16_t* piece;     // [tiles_max][buckets + 1]; the last one: units of the tile
   uint32_t* firsts;    // [kCounters][kMaxBucketTiles] units that are their ids' smallest (of those that count, see below)
-  int* overflow;       // set when the ids of a part did not fit its table (only one that a test hook makes small)
+  int* overflow;       // the sampler's: a bucket was not answered
   int32_t tiles_max;
   int32_t log_buckets; // hashed: at most
   int32_t log_tile;    // units of a tile
@@ -432,11 +432,12 @@ __device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_b
   __syncthreads();  // the table is rewritten
   return took;
 }
-// A bucket of many units may be one of few ids: it is gone over in parts only where the table has not taken them all.
-__device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles,
+// A bucket of many units may be one of few ids: it is gone over in parts only where the table has not taken them all.  Returns
+// whether it was answered: it is, but for one that crowds a part of it where a test hook has made the tables small.
+__device__ __forceinline__ bool first_of_bucket_hashed(const Buckets& b, int log_buckets, int bucket, uint32_t tiles,
                                                        uint32_t first_unit, HashedLds& lds) {
   const int few = kFewProbes < b.hash_slots ? kFewProbes : b.hash_slots;
-  if (first_of_part_hashed<false>(b, log_buckets, bucket, tiles, first_unit, HashPart{0, 1, 0u, ~0u}, few, lds)) return;
+  if (first_of_part_hashed<false>(b, log_buckets, bucket, tiles, first_unit, HashPart{0, 1, 0u, ~0u}, few, lds)) return true;
   if (threadIdx.x == 0) lds.units = 0;
   __syncthreads();
   int n = 0;
@@ -447,10 +448,9 @@ __device__ __forceinline__ void first_of_bucket_hashed(const Buckets& b, int log
   }
   if (n > 0) atomicAdd(&lds.units, n);
   __syncthreads();
-  const bool took = in_parts(lds.units, b.hash_slots, log_buckets, [&](HashPart part) {
+  return in_parts(lds.units, b.hash_slots, log_buckets, [&](HashPart part) {
     return first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, part, b.hash_slots, lds);
   });
-  if (threadIdx.x == 0 && !took) *b.overflow = 1;
 }
 
 // into[place of a unit in the tile] = its id's smallest unit, for all of the tile's units.

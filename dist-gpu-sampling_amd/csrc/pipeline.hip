@@ -407,7 +407,6 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   const int64_t s = seeds_of(h);
   const bool look_first = look_before_insert(h, s);
   const bool bucketed = bucketed_now(h, s);
-  const bool fold = replace;
   if (h.n_seeds_out && vb == 0 && threadIdx.x == 0) *h.n_seeds_out = s;
   if (i >= s) return;  // whole groups leave together
   const int group_lane0 = (threadIdx.x & (kWave - 1)) - l;
@@ -443,7 +442,7 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   // its leader.  Two positions that meet in one entry cost a missed repeat, never a wrong one.
   // Long rows (whose draws rarely repeat) skip the search.
   int leader = l;
-  if (fold) {
+  if (replace) {
     unsigned long long* offers = fold_lds[threadIdx.x / kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const bool search = live && deg <= uint32_t(kFoldMaxRowPerPick * k);
@@ -464,7 +463,7 @@ __device__ __forceinline__ void fill_rows(const Hop& h, int64_t vb, const TableT
   uint32_t word = kInvalidSlot;
   bool pick_ok = true;
   if (live && leader == l) pick_ok = place_pick<IdT>(h, table, indices.at(b + pos), p, look_first, bucketed, &word);
-  if (fold) {
+  if (replace) {
     const uint32_t leader_word = __shfl(word, leader, G);
     const int leader_ok = __shfl(int(pick_ok), leader, G);
     if (live && leader != l) {
@@ -923,7 +922,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_first_hashed_kernel(Hop h
   const int log_buckets = log_buckets_of(b, units);
   clear_counts(lds.counts, tiles);
   for (int i = blockIdx.x; i < 1 << log_buckets; i += gridDim.x)
-    first_of_bucket_hashed(b, log_buckets, bucket_in_turn(i, log_buckets), tiles, front, lds);
+    if (!first_of_bucket_hashed(b, log_buckets, bucket_in_turn(i, log_buckets), tiles, front, lds) && threadIdx.x == 0) *b.overflow = 1;
   add_counts(b, lds.counts, tiles);
 }
 

@@ -312,7 +312,6 @@ __global__ __launch_bounds__(Shape::kThreads) void bucketed_sort_kernel(dgs_segm
   __shared__ SortLds<true, Shape> lds;
   __shared__ uint32_t any_bad, folds;
   const uint32_t tile = blockIdx.x;
-  if (tile == 0 && threadIdx.x == 0) *b.overflow = 0;  // (the per-bucket launch comes behind this one)
   if (threadIdx.x == 0) any_bad = folds = 0;
   __syncthreads();
   const bool query = tile >= map_tiles;
@@ -381,7 +380,7 @@ __global__ __launch_bounds__(Shape::kThreads) void bucketed_rank_kernel(dgs_segm
   const bool last = tile + 1 == map_tiles;
   const TileSpan<const IdT, Shape::kTile> span(mapping, tile, n);
   uint32_t before = firsts_before<Shape::kThreads>(b, tile);
-  uint32_t refused = last && threadIdx.x == 0 ? uint32_t(*b.overflow) : 0u;
+  uint32_t refused = 0;
   for (uint32_t t = threadIdx.x; last && t < map_tiles; t += Shape::kThreads) refused |= notes[t] & 1;
   const uint32_t folds = notes[tile] >> 1;
 #pragma unroll
@@ -715,7 +714,6 @@ void take_buckets(Carver* c, int64_t n, UniqueWorkspace* t) {
   b.least = c->take<uint32_t>(size_t(b.tiles_max) * size_t(tile));
   b.piece = c->take<uint16_t>(size_t(b.tiles_max) * (kMaxBuckets + 1));
   b.firsts = c->take<uint32_t>(kCounters * kMaxBucketTiles);
-  b.overflow = c->take<int>(4);
   t->notes = c->take<uint32_t>(size_t(b.tiles_max));
 }
 

@@ -1297,7 +1297,7 @@ inline void plan_bucket_tiles(Plan* p) {
   const int64_t front = front_units(p->s_max[p->n_hops - 1]), pos = p->nnz_max[p->n_hops - 1], tile = kBucketTile;
   p->bucket_tiles = std::min<int64_t>(kMaxBucketTiles, (front + pos + tile - 1) / tile);
   p->bucket_pos_cap = p->bucket_tiles * tile - front;
-  p->bucket_space = p->n_hops >= 2 && p->bucket_pos_cap > 0;
+  p->bucket_space = p->n_hops >= 2;  // (also where the frontier leaves the positions none: a call's workspace never gets smaller as it grows)
 }
 
 dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, int32_t id_bytes,
@@ -1331,7 +1331,7 @@ dgs_status make_plan(int64_t n_seeds, const int64_t* fanouts, int32_t n_hops, in
     p->bucket_hashed = n_nodes > kBucketedMaxNodes || mode == 3 || mode == 4;
     const bool full = n_edges / 2 >= n_nodes * fanouts[n_hops - 1];  // (the rows' positions, as a rule)
     const bool large = !p->bucket_hashed && picks >= (full ? kBucketedMinPicksFull : kBucketedMinPicks) && n_nodes >= kBucketedMinNodes;
-    p->bucketed = p->bucket_space && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
+    p->bucketed = p->bucket_space && p->bucket_pos_cap > 0 && n_nodes >= 1 && fanouts[n_hops - 1] >= 1 && mode != 1 &&
                   (large || mode >= 2);
     p->hash_slots = mode == 4 ? 256 : kHashSlots;
     int log_b = kMinLogBuckets;

@@ -79,6 +79,25 @@ def test_relabel_workspace_never_falls(id_bytes):
     assert all(size <= max(30 * n, 6 * n + 2.9 * n * (8 if id_bytes == 4 else 12)) + 200_000 for n, size in sizes)
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("fanouts", [[5], [5, 10], [5, 10, 15], [50, 50], [3, 3, 3, 3]])
+def test_sampler_workspace_never_falls(weighted, fanouts):
+    # a frontier beyond what the bucketed pass has room for (8.4 M ids) keeps that room
+    lib = load_pkg().capi.lib
+    query = lib.dgs_sample_blocks_weighted_workspace_bytes if weighted else lib.dgs_sample_blocks_workspace_bytes
+    hops = (ctypes.c_int64 * len(fanouts))(*fanouts)
+    front = 1
+    for k in fanouts[:-1]:
+        front *= k + 1
+    last, n = 0, 1
+    for n in sorted({int(1.03 ** e) for e in range(2, 600)} | {-(-8388608 // front) + d for d in (-2, -1, 0, 1)}):
+        size = query(n, hops, len(fanouts), 8)
+        if size == 0:  # beyond what a call takes
+            break
+        assert size >= last, n
+        last = size
+
+
 def test_operator_surface_is_registered():
     import torch
     load_pkg()

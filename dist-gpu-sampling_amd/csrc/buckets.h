@@ -17,7 +17,9 @@
 // launch behind them 10.4; before (256 threads with 16 units and items of two words; a block of 256 threads that
 // searched the pieces for its units; repeats' slot words stored at random) 11.5, 16.2 and 9.9, and 204 -> 191 for the
 // batch with its features.  The three together with 512 threads and 8 / 16 units, 256 and 16: 25.7, 28.2,
-// 35.2 (25.9 with 1024; 512 buckets).
+// 35.2 (25.9 with 1024; 512 buckets).  8 batches through the loader, of 1024 / 2048 seeds: 1354 / 2195, with 512 threads and 8 units
+// 1356 / 2214, 16 1366 / 2200, 256 and 8 1370 / 2232, 16 1358 / 2197, the pass before 1355 / 2290; sort and compact held to 64
+// registers, which spills, 1387.
 //
 // Two forms.  Direct: bucket = low bits of the id, and the high bits index an array of kBucketRange entries;
 // items are one word (the high bits and the unit's place in its tile).  Hashed, for any number of ids:
@@ -360,7 +362,8 @@ constexpr int kPartBit = 23, kPartValues = 1 << (32 - kPartBit);  // what the ch
 // `attempt` says its table has not taken, value by value of the bits that chose the part, in ranges of as many hashes as
 // a table has slots: no two ids have one hash, so each is taken whatever the ids are.  A sweep reads the
 // whole bucket, and there are no more than kPartValues for the parts and as many (256 buckets: twice as many) for the ranges.
-// 2 M ids that were made for one of 256 buckets: 244 + 226 sweeps.
+// 2 M ids that were made for one of 256 buckets: 244 + 226 sweeps.  A relabel call of such ids, by far the longest that there is:
+// 131 k 17 ms, 262 k 31, 1 M 240, 2 M 613 (on the table, where they meet too, 0.7 to 1.3).
 template <typename Attempt>
 __device__ __forceinline__ bool in_parts(int units, int slots, int log_buckets, Attempt attempt) {
   const int half_tables = (units + slots / 2 - 1) / (slots / 2), parts = half_tables < kPartValues ? half_tables : kPartValues;
@@ -397,6 +400,7 @@ __device__ __forceinline__ bool first_of_part_hashed(const Buckets& b, int log_b
     if (t0 > 0) round.load(b, log_buckets, bucket, t0, tiles);
     round.each(b, [&](uint32_t, ItemT item, uint32_t unit) {
       if (elsewhere(item.x)) return;
+      if (PARTS && *const_cast<volatile int*>(&lds.overflow) != 0) return;  // (a full table is searched to its end by whoever comes too late)
       const unsigned long long packed = (static_cast<unsigned long long>(item.x) << 32) | unit;
       uint32_t slot = (item.x >> log_buckets) & mask;
       bool placed = false;
@@ -449,7 +453,9 @@ __device__ __forceinline__ bool first_of_bucket_hashed(const Buckets& b, int log
   if (n > 0) atomicAdd(&lds.units, n);
   __syncthreads();
   return in_parts(lds.units, b.hash_slots, log_buckets, [&](HashPart part) {
-    return first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, part, b.hash_slots, lds);
+    // (a part that would take longer searches is gone over in ranges, whose hashes all begin at slots of their own)
+    const int probes = part.span == ~0u && b.hash_slots == kHashSlots ? kFewProbes : b.hash_slots;
+    return first_of_part_hashed<true>(b, log_buckets, bucket, tiles, first_unit, part, probes, lds);
   });
 }
 

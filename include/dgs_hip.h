@@ -389,8 +389,8 @@ typedef struct dgs_segments {
  *   packed_table   : Non-zero: an attempt for ids below 2^32 - 1.  8-byte ids: the table keeps id and
  *                    position in one 64-bit slot (one atomic per id instead of two); an id beyond
  *                    sets counts_dev[1] and voids the call's results (call again with 0).  Long lists
- *                    of either width are gone over in buckets instead of on a table.  Zero: id array +
- *                    value array, any id >= 0.
+ *                    of either width are gone over in buckets instead of on a table.  Zero: a table that
+ *                    takes any id >= 0 (8-byte ids: id array + value array; 4-byte ids: the one of 64-bit slots).
  *   unique_out     : device, capacity sum(mapping.len) ids
  *   counts_dev     : device int64[2]: [0] number of distinct ids, [1] non-zero if the attempt that
  *                    packed_table asks for is void

@@ -24,7 +24,8 @@ def pkg():
     (20_000, 16, 64, True),        # a small hop of the widest fanout
     (90, 90, 40, True),            # 90 ids, so that a bucket's piece is far beyond 32 units
     (512 * 7, 3000, 20, False),    # ids up to a multiple of the buckets
-    (400_000, 140_000, 15, False), # 274 tiles: a second round of them
+    (400_000, 140_000, 15, False), # 274 tiles: a second round of them in the direct form, which reads 256 at once
+    (600_000, 215_000, 15, False), # 420 tiles: in the hashed one as well, which reads 384
 ])
 def test_bucketed_pass_at_its_edges(pkg, oracle, mode, id_dtype, nodes, seeds, k, replace):
     rng = np.random.default_rng(seeds + k)
@@ -128,6 +129,13 @@ def test_relabel_of_long_lists(pkg, oracle, dtype, n, distinct):
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n,m", [(193 * 8192, 192 * 8192), (1 << 22, 1 << 22)])  # 385 tiles, one more than a round; all that there may be
+def test_relabel_of_the_longest_lists(pkg, oracle, dtype, n, m):
+    rng = np.random.default_rng(n)
+    _relabel_both_ways(pkg, oracle, [rng.integers(0, n, size=n).astype(dtype)], [rng.integers(0, 2 * n, size=m).astype(dtype)])
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
 @pytest.mark.parametrize("n", [140_000, 600_000])  # of small tiles and of large ones
 @pytest.mark.parametrize("hubs,share", [(1, 0.02), (1, 0.2), (7, 0.5), (40, 0.9)])
 def test_relabel_of_lists_with_hubs(pkg, oracle, dtype, n, hubs, share):
@@ -191,8 +199,8 @@ def test_relabel_of_long_lists_with_ids_beyond_32_bits(pkg, oracle):
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
 def test_relabel_of_ids_that_crowd_a_bucket(pkg, oracle, dtype):
-    # 40 000 ids of one bucket (of 256, by the library's hash, restated here) go over its table of 16 384 in 5 parts; if they
-    # are of one part as well, that part goes over it range by range
+    # 40 000 ids of one bucket (of 256, by the library's hash, restated here), twice, are its table of 16 384 in 10 parts; if they
+    # are of two of these as well, those go range by range
     ids = np.arange(60_000_000, dtype=np.uint32)
     h = ids.copy()
     h ^= h >> np.uint32(16); h *= np.uint32(0x85EBCA6B)

@@ -1161,9 +1161,9 @@ def test_batch_pipeline_with_a_sampler_that_has_its_own_generator(pkg, oracle, g
 
 @pytest.mark.parametrize("n_nodes", [1 << 24, (1 << 24) + 1])
 def test_bucketed_last_hop_at_its_largest_graph(pkg, oracle, n_nodes):
-    # 2^24 nodes is the most the bucketed pass takes (2048 buckets x 8192 ids in LDS); one node
-    # more and the hop stays on the table.  Ids from the very top of the range are picked and
-    # seeded, so the last LDS entries of the last buckets are in use.
+    # 2^24 nodes is the most that the direct form of the bucketed pass takes (1024 buckets x 16 384 ids in LDS);
+    # one node more and the pass, asked for here, is the hashed form.  Ids from the very top of the range are
+    # picked and seeded, so the last LDS entries of the last buckets are in use.
     rng = np.random.default_rng(n_nodes & 0xff)
     deg = np.zeros(n_nodes, dtype=np.int64)
     busy = np.concatenate([rng.integers(0, n_nodes, size=40000), np.arange(n_nodes - 3000, n_nodes)])
@@ -1193,8 +1193,8 @@ def test_bucketed_last_hop_at_its_largest_graph(pkg, oracle, n_nodes):
 
 def test_bucketed_last_hop_near_its_largest_worst_case(pkg, oracle, graph):
     # 1024 seeds x [7, 30, 31] (hop order): the last hop's worst case is 8.1 M units, just inside what
-    # the bucketed pass has room for (1985 of its 2048 tiles; most of them stay empty on this graph,
-    # whose 20,000 nodes the frontier soon exhausts), and the pass is chosen by size
+    # the bucketed pass has room for (992 of its 1024 tiles; most of them stay empty on this graph,
+    # whose 20,000 nodes the frontier soon exhausts); by size a graph this small stays on the table
     indptr, indices = graph
     rng = np.random.default_rng(17)
     seeds = rng.permutation(20000)[:1024].astype(np.int64)
